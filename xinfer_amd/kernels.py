@@ -945,10 +945,17 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return out
 
 
+def gemm_f32_form(M: int, N: int) -> int:
+    """The form in which `gemm_tn` makes a float32 product of M rows and N features: 0, 1 the kernel for few rows with 16 or
+    32 features a workgroup; 2, 3, 4 tiles of 32 x 64, 64 x 64 and 128 x 128 (rows x features).  All give the same bits."""
+    return int(lib().xi_gemm_f32_form(int(M), int(N)))
+
+
 def gemm_tn(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
-            out: Optional[torch.Tensor] = None, accumulate: bool = False) -> torch.Tensor:
-    """y = x @ w.T with x [M, K], w [N, K]; float32 accumulation in ascending k.
-    `accumulate` adds the product to `out` instead of overwriting it."""
+            out: Optional[torch.Tensor] = None, accumulate: bool = False, form: int = -1) -> torch.Tensor:
+    """y = x @ w.T with x [M, K], w [N, K]; float32 accumulation in an order that depends on K alone.
+    `accumulate` adds the product to `out` instead of overwriting it.  `form` of a float32 product: see `gemm_f32_form`
+    (-1: chosen from the sizes; 0 and 1 take up to 64 rows)."""
     _dev(x, w, out)
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         raise KernelError(f"gemm: x {tuple(x.shape)} and w {tuple(w.shape)} do not match")
@@ -963,7 +970,7 @@ def gemm_tn(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     elif out.shape != (M, N) or (out_dtype is not None and out.dtype != out_dtype):
         raise KernelError("gemm: out has the wrong shape or dtype")
     _ok(lib().xi_gemm_tn(_p(x), _p(w), _p(out), M, N, K, _code(x, "gemm"), _code(out, "gemm"),
-                         int(bool(accumulate)), _stream()))
+                         int(bool(accumulate)), int(form), _stream()))
     return out
 
 
