@@ -44,3 +44,80 @@ def test_product_form_refused():
         kernels.gemm_tn(x, w, form=0)
     with pytest.raises(kernels.KernelError):
         kernels.gemm_tn(x, w, form=5)
+
+
+def _plain_attention(q, k, v, scale, window, chunk, cap, slopes, sinks):
+    """q [T, H, d] at the last T of the positions of k [L, G, d], v [L, G, dv]; float64."""
+    T, H, L = q.shape[0], q.shape[1], k.shape[0]
+    i, j = torch.arange(L - T, L)[:, None], torch.arange(L)[None]
+    seen = j <= i
+    if window:
+        seen = seen & (i - j < window)
+    if chunk:
+        seen = seen & (i // chunk == j // chunk)
+    out = []
+    for h in range(H):
+        g = h // (H // k.shape[1])
+        s = (q[:, h] @ k[:, g].T) * scale
+        s = cap * torch.tanh(s / cap) if cap else s
+        if slopes is not None:
+            s = s - slopes[h] * (i - j)
+        s = s.masked_fill(~seen, float("-inf"))
+        z = sinks[h].reshape(1, 1).expand(T, 1) if sinks is not None else torch.full((T, 1), float("-inf"), dtype=s.dtype)
+        w = torch.softmax(torch.cat([s, z], dim=1), dim=1)[:, :L]
+        out.append(torch.where(seen, w, 0.0) @ v[:, g].nan_to_num(0.0, 0.0, 0.0) if window else w @ v[:, g])
+    return torch.stack(out, dim=1)
+
+
+@pytest.mark.parametrize("nq,nkv,d,dv,page,window,chunk,cap,slopes,sinks,latent", [
+    (4, 2, 16, 16, 8, 0, 0, 0.0, False, False, False), (6, 2, 48, 80, 16, 0, 0, 0.0, False, False, False),
+    (8, 2, 128, 128, 64, 33, 0, 0.0, False, True, False), (17, 1, 64, 112, 16, 0, 40, 5.0, False, True, False),
+    (4, 4, 96, 32, 12, 0, 0, 3.0, True, False, False), (40, 1, 256, 192, 64, 0, 0, 0.0, False, True, True),
+    (2, 1, 208, 256, 32, 100, 64, 0.0, False, False, False)])
+def test_attention(nq, nkv, d, dv, page, window, chunk, cap, slopes, sinks, latent):
+    """Portions and single tokens of two requests against float64, every token's bits alone and in the step, and beside the kernel
+    for every size; outside the window the first request's keys and values are undefined and must stay unread."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d + dv)
+    lens, news = [300, 41], [37, 41]
+    pages = [-(-n // page) for n in lens]
+    perm = torch.randperm(sum(pages) + 2, generator=g).tolist()
+    bt = torch.zeros(2, max(pages) + 1, dtype=torch.int32)
+    kc = torch.full((len(perm), nkv, page, d), float("nan"))
+    vc = kc if latent else torch.full((len(perm), nkv, page, dv), float("nan"))
+    scale, qs, want = d ** -0.5, [], []
+    sl = torch.rand(nq, generator=g) * 0.1 if slopes else None
+    sk = torch.randn(nq, generator=g) if sinks else None
+    dbl = lambda t: None if t is None else t.double()
+    for b, (n, new) in enumerate(zip(lens, news)):
+        k = torch.randn(n, nkv, d, generator=g)
+        v = k[..., :dv] if latent else torch.randn(n, nkv, dv, generator=g)
+        qb = torch.randn(new, nq, d, generator=g) * 2
+        qs.append(qb)
+        want.append(_plain_attention(qb.double(), k.double(), v.double(), scale, window, chunk, cap, dbl(sl), dbl(sk)))
+        first = n - new + 1 - window if window and b == 0 else 0       # what no query of this step sees
+        for i in range(n):
+            p = perm[sum(pages[:b]) + i // page]
+            bt[b, i // page] = p
+            if i >= first:
+                kc[p, :, i % page] = k[i]
+                if not latent:
+                    vc[p, :, i % page] = v[i]
+    q = torch.cat(qs)
+    tok_seq = torch.tensor([b for b in range(2) for _ in range(news[b])], dtype=torch.int32)
+    pos = torch.tensor([lens[b] - news[b] + i for b in range(2) for i in range(news[b])], dtype=torch.int32)
+    dev = [t.to(DEV) for t in (q, kc, bt, tok_seq, pos)]
+    vd = None if latent else vc.to(DEV)
+    opt = dict(softcap=cap, slopes=None if sl is None else sl.to(DEV), sinks=None if sk is None else sk.to(DEV),
+               value_dim=dv if latent else None, chunk=chunk)
+    run = lambda rows, **kw: kernels.attention_generic(dev[0][rows].contiguous(), dev[1], vd, dev[2], dev[3][rows].contiguous(),
+                                                       dev[4][rows].contiguous(), scale, window, **opt, **kw)
+    assert kernels.lib().xi_attention_f32_takes(nq, nkv, d, dv)
+    got = run(slice(None))
+    ref = torch.cat(want).reshape(q.shape[0], -1)
+    # scores of about 2 whose float32 sums of d products are off by about 2^-24 sqrt(d) of their size, weighed sums likewise
+    assert float((got.cpu().double() - ref).abs().max()) < 2e-5
+    for r in (0, 20, 36, 37, 77):
+        assert torch.equal(run(slice(r, r + 1))[0], got[r]), r
+    plain = run(slice(None), matrix=False)
+    assert float((plain.cpu().double() - ref).abs().max()) < 2e-5

@@ -891,7 +891,7 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                       scale: float, window: int = 0, out: Optional[torch.Tensor] = None,
                       v_grouped: bool = False, softcap: float = 0.0,
                       slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None,
-                      value_dim: Optional[int] = None, chunk: int = 0) -> torch.Tensor:
+                      value_dim: Optional[int] = None, chunk: int = 0, matrix: bool = True) -> torch.Tensor:
     """Causal paged GQA attention for any mix of tokens.  q [T, nq, d]; caches
     [pages, nkv, page_size, d] (the V pool's last size, the value head size, may differ);
     block_tables int32 [B, max_pages]; tok_seq / positions
@@ -937,6 +937,14 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         out = torch.empty((T, nq * dv), dtype=q.dtype, device=q.device)
     elif out.shape != (T, nq * dv) or out.dtype != q.dtype:
         raise KernelError("attention: out has the wrong shape or dtype")
+    # float32 at head sizes in steps of 16 up to 256: on the matrix cores (`matrix` False: the kernel for every size)
+    if (matrix and q.dtype == torch.float32 and nkk == nkv and not v_grouped and lib().xi_attention_f32_takes(nq, nkv, d, dv)
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache))):
+        _ok(lib().xi_attention_f32(
+            _p(q), _p(k_cache), _p(v_cache), _p(block_tables), int(block_tables.shape[1]), _p(tok_seq), _p(positions), _p(out),
+            ctypes.c_float(scale), int(window), int(page), T, nq, nkv, d, dv, ctypes.c_float(softcap), _p(slopes), _p(sinks),
+            int(v_cache is None), int(chunk), int(block_tables.shape[0]), _stream()))
+        return out
     _ok(lib().xi_attention_generic(
         _p(q), _p(k_cache), _p(v_cache), _code(q, "attention"), _p(block_tables),
         int(block_tables.shape[1]), _p(tok_seq), _p(positions), _p(out), ctypes.c_float(scale),
