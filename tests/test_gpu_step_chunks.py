@@ -1,0 +1,78 @@
+"""A selective state space's long portions on the matrix cores (`xi_step_chunks`) against float64 and beside the walk token by
+token: unequal requests, portions at the edges of a chunk of 64 tokens, columns of a packed projection, slots in no order,
+decays from none to all within a token."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _plain(q, k, v, raw, bias, rate_log, S, group_heads, q_scale, k_scale):
+    """One portion in float64; returns the results and the state behind it."""
+    H, T = raw.shape[1], q.shape[0]
+    dk = S.shape[1]
+    q, k = ((t.double().view(T, -1, dk) * s).repeat_interleave(group_heads, dim=1) for t, s in ((q, q_scale), (k, k_scale)))
+    v = v.double().view(T, H, -1)
+    d = torch.nn.functional.softplus(raw.double() + bias.double(), threshold=1e9)
+    a = torch.exp(-torch.exp(rate_log.double()) * d)
+    S = S.double().clone()
+    out = []
+    for t in range(T):
+        S = a[t][:, None, None] * S + k[t][:, :, None] * (d[t][:, None] * v[t])[:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+@pytest.mark.parametrize("H,G,dk,dv,rate", [(4, 1, 128, 64, -1.0), (6, 2, 32, 32, -6.0), (2, 2, 96, 96, 3.0), (3, 1, 64, 32, 0.5)])
+def test_portions_of_unequal_requests(H, G, dk, dv, rate, monkeypatch):
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(dk + dv)
+    steps = [[64, 1, 32, 200], [65, 31, 129, 1], [1, 63, 33, 128]]
+    B, slots = 4, [2, 0, 4, 3]
+    bias, rate_log = torch.randn(H, generator=g) - 1.0, torch.randn(H, generator=g) * 0.5 + rate
+    state0 = torch.randn(5, H, dk, dv, generator=g)
+    errors = {}
+    for matrix in (False, True):
+        monkeypatch.setattr(kernels, "STEP_MFMA", matrix)
+        g2 = torch.Generator().manual_seed(5)
+        state = state0.clone().to(DEV)
+        want = {b: state0[s] for b, s in enumerate(slots)}
+        worst = [0.0, 0.0]
+        for lens in steps:
+            T = sum(lens)
+            width = 2 * G * dk + H * dv
+            packed = torch.randn(T, width + 8 + H, generator=g2).to(torch.bfloat16)
+            dev = packed.to(DEV)
+            cols = lambda t: (t[:, :G * dk], t[:, G * dk:2 * G * dk], t[:, 2 * G * dk:width], t[:, width + 8:width + 8 + H])
+            if (width + 8 + H) % 8:          # rows of whole 16-byte pieces for q, k and v; the step sizes lie anywhere
+                pad = torch.zeros(T, -(width + 8 + H) % 8, dtype=torch.bfloat16)
+                dev = torch.cat([packed, pad], dim=1).to(DEV)
+            q, k, v, raw = cols(dev)
+            cu = [0]
+            for n in lens:
+                cu.append(cu[-1] + n)
+            o = kernels.linear_scan(q, k, v, state, torch.tensor(slots, device=DEV), torch.tensor(cu, dtype=torch.int32, device=DEV), H, dk,
+                                    dv, step=raw, step_bias=bias.to(DEV), decay_log=rate_log.to(DEV), groups=G, q_scale=0.7, k_scale=0.4,
+                                    q_lens=lens, plan_cache={})
+            for b in range(B):
+                part = [c[cu[b]:cu[b + 1]] for c in cols(packed)]
+                ref, want[b] = _plain(*part[:3], part[3], bias, rate_log, want[b], H // G, 0.7, 0.4)
+                worst[0] = max(worst[0], float((o[cu[b]:cu[b + 1]].cpu().double() - ref).norm() / ref.norm()))
+                worst[1] = max(worst[1], float((state[slots[b]].cpu().double() - want[b]).norm() / want[b].norm()))
+        untouched = [s for s in range(5) if s not in slots]
+        assert torch.equal(state[untouched].cpu(), state0[untouched])
+        errors[matrix] = worst
+    print(f"\n[step_chunks] dk={dk} dv={dv}: error of results and state against 64 bits: walk {errors[False]}, chunks {errors[True]}")
+    # three bfloat16 hold a float32 to 2^-24 of it, and both forms round float32 sums of at most 64 + dk terms
+    for w, c in zip(errors[False], errors[True]):
+        assert c < max(1.2 * w, 5e-7)
+
+
+def test_the_rule_takes_what_it_should(monkeypatch):
+    """Which portions go where, without a launch."""
+    from xinfer_amd import kernels
+    assert kernels.step_chunk_plan([1, 31, 32, 500, 1]) == ([0, 1, 4], [2, 3])
+    takes = kernels.lib().xi_step_chunks_takes
+    assert all(takes(dk, dv) for dk in (32, 64, 96, 128) for dv in (32, 64, 256))
+    assert not any(takes(*s) for s in ((16, 64), (160, 64), (48, 64), (128, 48), (128, 0), (0, 64)))

@@ -339,6 +339,50 @@ def _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, o
     return True
 
 
+STEP_MFMA = True                  # False: portions of a selective state space go through the walk token by token too
+STEP_FROM = 32                    # tokens of a portion from which it is walked in chunks on the matrix cores
+
+
+def step_chunk_plan(q_lens):
+    """The portions of a step for `xi_step_chunks`: the batch rows walked token by token, and those of STEP_FROM tokens and more."""
+    return ([b for b, n in enumerate(q_lens) if int(n) < STEP_FROM], [b for b, n in enumerate(q_lens) if int(n) >= STEP_FROM])
+
+
+def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale) -> bool:
+    """`linear_scan` for a step with long portions in bfloat16 under a step size a token and head: the long ones chunk by chunk on
+    the matrix cores, the others in one piece.  False: nothing was done (sizes, rows or lengths that it does not take)."""
+    q, k, v, qs, ks, vs, step, ss, step_bias, decay_log = (common[i] for i in (0, 1, 2, 3, 4, 5, 10, 11, 12, 13))
+    if (not STEP_MFMA or SCAN_CHUNK <= 0 or q.dtype != torch.bfloat16 or step is None or common[15] != dv or common[17]
+            or not lib().xi_step_chunks_takes(dk, dv) or qs % 8 or ks % 8 or vs % 8 or k_scale == 0.0
+            or any(t.data_ptr() % 16 for t in (q, k, v))):
+        return False
+    key = ("step_chunk_plan", STEP_FROM)
+    plan = plan_cache.get(key) if plan_cache is not None else None
+    if plan is None:
+        whole, long = step_chunk_plan(q_lens)
+        starts = [0]
+        for n in q_lens:
+            starts.append(starts[-1] + int(n))
+        rows = long + whole
+        L, W = len(long), len(whole)
+        i32 = torch.tensor([starts[b] for b in rows] + [starts[b + 1] for b in rows], dtype=torch.int32).to(q.device)
+        slots = state_slots.index_select(0, torch.tensor(rows, dtype=torch.int64).to(q.device))
+        plan = dict(L=L, W=W, first=i32[:L + W], last=i32[L + W:], slots=slots)
+        if plan_cache is not None:
+            plan_cache[key] = plan
+    L, W = plan["L"], plan["W"]
+    if not L:
+        return False
+    ll = ctypes.c_longlong
+    _ok(lib().xi_step_chunks(_p(q), ll(qs), _p(k), ll(ks), _p(v), ll(vs), _p(step), ll(ss), _p(step_bias), _p(decay_log), _p(state),
+                             ll(slot_stride), _p(plan["slots"]), _p(plan["first"]), _p(plan["last"]), L, _p(out), H, dk, dv,
+                             int(common[16]), ctypes.c_float(q_scale), ctypes.c_float(k_scale), _stream()))
+    if W:
+        _scan_launch(*common, state, slot_stride, plan["slots"][L:], state, slot_stride, plan["slots"][L:],
+                     plan["first"][L:].data_ptr(), plan["last"][L:].data_ptr(), out, None, W, H, dk, dv, q_scale, k_scale)
+    return True
+
+
 def _scan_launch(q, k, v, qs, ks, vs, z, z_bias, tau, head_decay, step, ss, step_bias, decay_log, gates, v_cols, group_heads, act,
                  state_in, in_stride, in_idx, state_out, out_stride, out_idx,
                  first, last, out, decay_out, items, H, dk, dv, q_scale, k_scale):
@@ -375,7 +419,8 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     of single tokens wants it): portions of two chunks and more (`SCAN_CHUNK`) are cut into chunks that are walked
     side by side in three launches (each chunk's own share from a zero state; the states the chunks start from,
     one after the other; the chunks' results), the others in one piece; in bfloat16 with a constant decay per head the long
-    ones go through the matrix cores (`xi_decay_chunks`, portions from DECAY_FROM tokens on).  `plan_cache`: a dict of the step in which
+    ones go through the matrix cores (`xi_decay_chunks`, portions from DECAY_FROM tokens on), and so they do with a step size a
+    token and head (`xi_step_chunks`, from STEP_FROM tokens on, one chunk after the other).  `plan_cache`: a dict of the step in which
     the index arrays of this cutting are kept for the next layer."""
     H, dk, dv = int(heads), int(key_dim), int(value_dim)
     T = q.shape[0]
@@ -436,6 +481,8 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     out = torch.empty((T, H, dv), dtype=torch.float32, device=q.device)
     slot_stride = int(state.stride(0)) if state.shape[0] > 1 else H * dk * dv
     common = (q, k, v, qs, ks, vs, z, z_bias, tau, head_decay, step, ss, step_bias, decay_log, gates, vc, H // G, int(bool(silu)))
+    if q_lens is not None and _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
+        return out
     if q_lens is not None and _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
         return out
     whole, long, chunks = scan_chunk_plan(q_lens) if q_lens is not None else (None, [], [])
