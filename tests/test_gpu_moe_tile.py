@@ -1,0 +1,71 @@
+"""The experts' products in tiles of many rows (`moe_experts_tiled`) against float64, and bit for bit beside the grouped form for
+few rows: experts with no row, one row, and rows at the edges of a tile; features and widths that end inside a tile."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _plain(x, gate_up, down, idx, wt, act, gated, weigh_input, E, add):
+    x, gate_up, down, wt = x.double(), gate_up.double(), down.double(), wt.double()
+    F = gate_up.shape[1] // 2 if gated else gate_up.shape[1]
+    f = {"silu": torch.nn.functional.silu, "relu2": lambda z: torch.relu(z) ** 2,
+         "gelu_tanh": lambda z: torch.nn.functional.gelu(z, approximate="tanh")}[act]
+    out = torch.zeros_like(x)
+    for r in range(idx.shape[1]):
+        for e in range(int(idx.max()) + 1):
+            rows = (idx[:, r] == e).nonzero()[:, 0]
+            if not len(rows):
+                continue
+            w = wt[rows, r, None]
+            h = x[rows] * w if weigh_input else x[rows]
+            if e >= E:
+                y = h
+            else:
+                u = h @ gate_up[e].T
+                u = f(u[:, :F]) * u[:, F:] if gated else f(u)
+                y = u @ down[e].T
+            out[rows] += y if weigh_input else y * w
+    return out if add is None else out + add.double()
+
+
+@pytest.mark.parametrize("H,F,act,gated,weigh,identity,shared", [
+    (64, 64, "silu", True, False, 2, True), (192, 320, "gelu_tanh", True, True, 0, False), (320, 192, "relu2", False, False, 0, True),
+    (512, 256, "silu", False, False, 1, False), (256, 576, "silu", True, False, 0, False)])
+def test_experts_in_tiles(H, F, act, gated, weigh, identity, shared):
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(H + F)
+    E, rows = 6, [0, 1, 127, 128, 129, 300]              # pairs an expert (the identity experts take some of the rest)
+    rb = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    gate_up, down = rb(E, (2 if gated else 1) * F, H) * H ** -0.5, rb(E, H, F) * F ** -0.5
+    pairs = [e for e, n in enumerate(rows) for _ in range(n)] + [E + i % max(1, identity) for i in range(40) if identity]
+    pairs += [5] * (len(pairs) % 2)
+    idx = torch.tensor(pairs)[torch.randperm(len(pairs), generator=g)].view(-1, 2).to(torch.int32)
+    T = idx.shape[0]
+    x, wt = rb(T, H), torch.rand(T, 2, generator=g) + 0.1
+    add = rb(T, H) if shared else None
+    dev = [t.to(DEV) for t in (x, gate_up, down, idx, wt)]
+    kw = dict(gated=gated, weigh_input=weigh, identity=identity, add=None if add is None else add.to(DEV))
+    ref = _plain(x, gate_up, down, idx.long(), wt, act, gated, weigh, E, add)
+    few = kernels.moe_experts(*dev, act, grouped=True, tile_rows=32, **kw)
+    for bm in (64, 128, 256):
+        got = kernels.moe_experts_tiled(*dev, act, tile_rows=bm, **kw)
+        # one rounding of the hidden rows to bfloat16 (2^-9 of each), averaged over F products
+        assert float((got.cpu().double() - ref).norm() / ref.norm()) < 2.0 ** -8
+        assert torch.equal(got, few), bm
+    assert torch.equal(kernels.moe_experts_tiled(*dev, act, **kw), few)
+
+
+def test_what_is_taken_and_refused():
+    from xinfer_amd import kernels
+    assert kernels.moe_tiled_takes(100, 2, 8, 128, 192, True)
+    assert not kernels.moe_tiled_takes(100, 2, 8, 128, 200, True) and not kernels.moe_tiled_takes(100, 2, 8, 136, 192, True)
+    assert not kernels.moe_tiled_takes(1 << 20, 2, 8, 4096, 6144, True)          # rows whose offsets pass 32 bits
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
+    idx = torch.zeros(3, 1, dtype=torch.int32, device=DEV)
+    wt = torch.ones(3, 1, device=DEV)
+    with pytest.raises(kernels.KernelError):
+        kernels.moe_experts_tiled(z(3, 96), z(2, 128, 96), z(2, 96, 64), idx, wt)
+    with pytest.raises(kernels.KernelError):
+        kernels.moe_experts_tiled(z(3, 64), z(2, 128, 64), z(2, 64, 64), idx, wt, tile_rows=32)

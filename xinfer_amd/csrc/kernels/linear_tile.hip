@@ -44,54 +44,22 @@
 //
 // Reference call site: candle matmul in /root/reference/src/models/layers/linear.rs:76-124
 // (vendor BLAS).
-#include "common.h"
+#include "tile_core.h"
 
 namespace xi {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 namespace tile {
 
 constexpr int kSliceK = 64;        // K is cut into slices in tiles of this many
 
-__device__ __forceinline__ void load_lds16(const void* base, unsigned lane_off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
-               : "memory", "m0");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-__device__ __forceinline__ bf16x8 lds8(const unsigned char* p) { return *reinterpret_cast<const bf16x8*>(p); }
-
-// BM rows of x by BN rows of w a workgroup, BK = 64 k a tile; WGM x WGN waves, each (BM / WGM) by
-// (BN / WGN).
-template <int BM, int BN, int BK, int WGM, int WGN, int S, bool PARTIAL>
+// BM rows of x by BN rows of w a workgroup; see Walk.
+template <int BM, int BN, int WGM, int WGN, int S, bool PARTIAL>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w, void* __restrict__ yv, int M, int N, int K, int tiles_m,
     int tiles_n, int slices, int k_tiles_all) {
-  static_assert(BK == 64, "tiles of 64 k: rows of 128 bytes");
-  constexpr int kRowBytes = BK * 2, kBK = BK;
-  constexpr int CPR = BK / 8;                                // 16-byte chunks of a row
-  constexpr int PS = BK == 64 ? 1 : 2;                       // rows that share a 256-byte phase differ in place: p >> PS
-  constexpr int RPL = 1024 / kRowBytes;                      // rows a wave-wide load brings
-  constexpr int KSTEPS = BK / 32;
-  constexpr int NWV = WGM * WGN;
-  constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16;      // 16 x 16 tiles of a wave
-  constexpr int WBYTES = BN * kRowBytes, XBYTES = BM * kRowBytes, STAGE = WBYTES + XBYTES;
-  constexpr int WI = WBYTES / 1024, XI = XBYTES / 1024;      // wave-wide loads of a tile: w, then x
-  static_assert((WI + XI) % NWV == 0, "every wave issues the same number of loads a tile");
-  constexpr int LPW = (WI + XI) / NWV;
-  static_assert(S * LPW < 64 && S >= 2, "the tiles in flight must fit the load counter");
-  static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0, "whole 16 x 16 tiles a wave");
+  using W = Walk<BM, BN, WGM, WGN, S>;
+  constexpr int TM = W::TM, TN = W::TN;
   extern __shared__ __align__(1024) unsigned char smem[];
-  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, j = lane >> 4;
   const int wm = wave % WGM, wn = wave / WGM;
 
@@ -108,115 +76,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
   // slice s of the K / 64 tiles: [s * tiles / slices, (s + 1) * tiles / slices), one tile at least
   const int kt_begin = (int)((long long)slice * k_tiles_all / slices);
   const int k_tiles = (int)((long long)(slice + 1) * k_tiles_all / slices) - kt_begin;
-  const size_t k0 = (size_t)kt_begin * BK;
+  const size_t k0 = (size_t)kt_begin * kSliceK;
 
-  // ---- what this lane brings of every tile: per load of its wave the byte offset of its chunk from
-  // the tile's first element of w (or x); rows past the end are read from the last row (nobody
-  // stores what they make)
-  unsigned ld_off[LPW];
-#pragma unroll
-  for (int t = 0; t < LPW; ++t) {
-    const int ii = wave + NWV * t;
-    const bool is_w = ii < WI;
-    const int p = RPL * (is_w ? ii : ii - WI) + lane / CPR;      // row within the operand's tile
-    const int ch = (lane % CPR) ^ ((p >> PS) & (CPR - 1));       // the chunk that belongs at this lane's place
-    int row = (is_w ? n0 : m0) + p;
-    const int last = (is_w ? N : M) - 1;
-    row = row > last ? last : row;
-    ld_off[t] = (unsigned)(((size_t)(row - (is_w ? n0 : m0)) * K) * 2 + ch * 16);
-  }
-  const bf16* wbase = w + (size_t)n0 * K + k0;
-  const bf16* xbase = x + (size_t)m0 * K + k0;
-
-  // the t-th of this wave's loads of tile kt, into stage st
-  auto fetch_one = [&](int kt, int st, int t) {
-    const int ii = wave + NWV * t;
-    // (which operand a wave's t-th load takes is the same in all its lanes: made a scalar by hand)
-    const unsigned long long a = (unsigned long long)(uintptr_t)((ii < WI ? wbase : xbase) + (size_t)kt * kBK);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
-    load_lds16(reinterpret_cast<const void*>((uintptr_t)(((unsigned long long)hi << 32) | lo)), ld_off[t],
-               __builtin_amdgcn_readfirstlane(lds0 + (unsigned)st * STAGE + (unsigned)ii * 1024u));
-  };
-  auto fetch = [&](int kt, int st) {
-#pragma unroll
-    for (int t = 0; t < LPW; ++t) fetch_one(kt, st, t);
-  };
-
-  // where this lane reads its operands within a stage: row r of a 16-row tile, chunk 4 ks + j at
-  // its permuted place (16 rows further on the permutation is the same)
-  unsigned rd[KSTEPS];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) rd[ks] = (unsigned)(r * kRowBytes + 16 * ((4 * ks + j) ^ ((r >> PS) & (CPR - 1))));
-  const unsigned w_rd = (unsigned)(wn * TN * 16) * kRowBytes;
-  const unsigned x_rd = WBYTES + (unsigned)(wm * TM * 16) * kRowBytes;
-
+  unsigned ld_off[W::LPW];
+  W::offsets(ld_off, [&](bool is_w, int p) {      // (rows past the end: the last row)
+    const int first = is_w ? n0 : m0, last = (is_w ? N : M) - 1;
+    const int row = first + p > last ? last : first + p;
+    return (unsigned)(((size_t)(row - first) * K) * 2);
+  });
   f32x4 acc[TN][TM];
-#pragma unroll
-  for (int a = 0; a < TN; ++a)
-#pragma unroll
-    for (int b = 0; b < TM; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto read = [&](const unsigned char* T, int ks, bf16x8 (&wa)[TN], bf16x8 (&xb)[TM]) {
-#pragma unroll
-    for (int a = 0; a < TN; ++a) wa[a] = lds8(T + w_rd + rd[ks] + a * 16 * kRowBytes);
-#pragma unroll
-    for (int b = 0; b < TM; ++b) xb[b] = lds8(T + x_rd + rd[ks] + b * 16 * kRowBytes);
-  };
-  auto multiply = [&](const bf16x8 (&wa)[TN], const bf16x8 (&xb)[TM]) {
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-      for (int b = 0; b < TM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[a], xb[b], acc[a][b], 0, 0, 0);
-  };
-
-  // The walk, one barrier a tile.  A tile's two 32-wide steps have their operands in two sets of
-  // registers; each set is read from LDS while the matrix cores work on the other: the second
-  // step's before the first step's products are issued, the next tile's first step's (behind the
-  // barrier that says the tile has landed) before the second step's products.  Tiles past the
-  // slice's last are asked for all the same (from the last one's place) and read too, so that the
-  // number of loads in flight and the code do not depend on where the walk is.
-  static_assert(KSTEPS == 2, "two sets of operand registers, one a step");
-#pragma unroll
-  for (int p = 0; p < S; ++p) fetch(p < k_tiles ? p : k_tiles - 1, p);
-  bf16x8 wa0[TN], xb0[TM], wa1[TN], xb1[TM];
-  wait_loads<(S - 1) * LPW>();       // this wave's loads of the first tile have landed
-  __syncthreads();                   // everybody's have
-  read(smem, 0, wa0, xb0);
-  int st = 0;
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    const unsigned char* T = smem + (size_t)st * STAGE;
-    read(T, 1, wa1, xb1);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(wa0, xb0);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_loads<(S - 2) * LPW>();     // this wave's loads of the next tile have landed, and its reads of this one
-    __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0): the operands above are in registers)
-    __syncthreads();                 // everybody's: the next tile is whole, and this tile's stage is free
-    const int filled = st;
-    const int nxt = kt + S < k_tiles ? kt + S : k_tiles - 1;
-    st = st + 1 == S ? 0 : st + 1;
-    read(smem + (size_t)st * STAGE, 0, wa0, xb0);
-    __builtin_amdgcn_sched_barrier(0);
-    // the second step's products with the loads of the tile S ahead between them: a wave that asks
-    // for all its loads at once waits until the load unit has taken them (it takes a compute unit's
-    // 48 to 64 KB a tile at about 55 bytes a clock) before it issues its first product
-    {
-      constexpr int PER = (TN * TM) / LPW;       // products between two loads
-#pragma unroll
-      for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) {
-          const int idx = a * TM + b;
-          if (idx % PER == 0 && idx / PER < LPW) {
-            __builtin_amdgcn_sched_barrier(0);
-            fetch_one(nxt, filled, idx / PER);
-          }
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa1[a], xb1[b], acc[a][b], 0, 0, 0);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  wait_loads<0>();     // the tiles asked for past the end are still on their way into LDS
+  W::run(w + (size_t)n0 * K + k0, x + (size_t)m0 * K + k0, ld_off, k_tiles, smem, acc);
 
   // ---- a lane holds features n .. n + 3 of row m of every 16 x 16 tile
   const int mw = m0 + wm * TM * 16 + r, nw = n0 + wn * TN * 16 + 4 * j;
@@ -275,24 +144,24 @@ int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, i
   const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   const long long total = (long long)tiles_m * tiles_n * slices;
   XI_CHECK(total <= 0x7fffffffLL, "linear_tile: too many workgroups");
-#define XI_TILE(BM, BN, BK, WGM, WGN, S, PARTIAL)                                                                 \
+#define XI_TILE(BM, BN, WGM, WGN, S, PARTIAL)                                                                 \
   do {                                                                                                            \
-    auto kern = tile::linear_tile_kernel<BM, BN, BK, WGM, WGN, S, PARTIAL>;                                        \
-    const size_t lds = (size_t)(S) * (BM + BN) * BK * 2;                                                          \
+    auto kern = tile::linear_tile_kernel<BM, BN, WGM, WGN, S, PARTIAL>;                                        \
+    const size_t lds = tile::Walk<BM, BN, WGM, WGN, S>::LDS;                                                          \
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);  \
     XI_CHECK(e == hipSuccess, "linear_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));         \
     kern<<<(unsigned)total, 64 * WGM * WGN, lds, stream>>>((const bf16*)x, (const bf16*)w, y, M, N, K, tiles_m,   \
-                                                           tiles_n, slices, K / BK);                   \
+                                                           tiles_n, slices, K / tile::kSliceK);                   \
   } while (0)
   if (shape == 0) {
-    if (partial) XI_TILE(128, 256, 64, 2, 4, 3, true);
-    else XI_TILE(128, 256, 64, 2, 4, 3, false);
+    if (partial) XI_TILE(128, 256, 2, 4, 3, true);
+    else XI_TILE(128, 256, 2, 4, 3, false);
   } else if (shape == 1) {
-    if (partial) XI_TILE(256, 128, 64, 4, 2, 3, true);
-    else XI_TILE(256, 128, 64, 4, 2, 3, false);
+    if (partial) XI_TILE(256, 128, 4, 2, 3, true);
+    else XI_TILE(256, 128, 4, 2, 3, false);
   } else {
-    if (partial) XI_TILE(256, 256, 64, 2, 4, 2, true);
-    else XI_TILE(256, 256, 64, 2, 4, 2, false);
+    if (partial) XI_TILE(256, 256, 2, 4, 2, true);
+    else XI_TILE(256, 256, 2, 4, 2, false);
   }
 #undef XI_TILE
   XI_LAUNCH_CHECK("linear_tile");

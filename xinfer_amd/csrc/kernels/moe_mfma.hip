@@ -17,7 +17,7 @@
 // Experts numbered E .. E + I - 1 are identity experts: they get slots behind the others' and no tiles.
 // A row's result depends on its own operands alone (the matrix cores keep rows apart), so it does not
 // matter which other rows share its tile.
-#include "common.h"
+#include "moe_act.h"
 
 namespace xi {
 
@@ -30,7 +30,8 @@ constexpr int kSortExperts = 1024;
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __restrict__ idx, int P, int E, int I, int BM,
                                                                 int* __restrict__ order, int* __restrict__ slot_of,
                                                                 int* __restrict__ tile_expert, int* __restrict__ tile_row0,
-                                                                int* __restrict__ tile_rows, int* __restrict__ n_tiles) {
+                                                                int* __restrict__ tile_rows, int* __restrict__ n_tiles,
+                                                                int* __restrict__ tile_first, int* __restrict__ tile_count) {
   __shared__ int count[kSortExperts], cursor[kSortExperts];
   const int A = E + I;
   for (int e = threadIdx.x; e < A; e += kSortThreads) count[e] = 0;
@@ -45,7 +46,12 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __res
     int at = 0, tiles = 0;
     for (int e = 0; e < A; ++e) {
       cursor[e] = at;
+      const int first = tiles;
       for (int r = 0; e < E && r < count[e]; r += BM) {
+        if (tile_first) {
+          tile_first[tiles] = first;
+          tile_count[tiles] = (count[e] + BM - 1) / BM;
+        }
         tile_expert[tiles] = e;
         tile_row0[tiles] = at + r;
         tile_rows[tiles] = count[e] - r < BM ? count[e] - r : BM;
@@ -63,13 +69,6 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __res
     order[slot] = p;
     slot_of[p] = slot;
   }
-}
-
-template <int ACT>
-__device__ __forceinline__ float moe_act_m(float z) {
-  if constexpr (ACT == 2) return z > 0.f ? z * z : 0.f;       // the square of relu
-  if constexpr (ACT == 0) return z / (1.f + __expf(-z));
-  else return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
 static __device__ __forceinline__ mbf16x8 mld8(const bf16* p) { return *reinterpret_cast<const mbf16x8*>(p); }
@@ -335,11 +334,14 @@ extern "C" {
 // Most tiles of up to `bm` rows that P pairs on E experts can make.
 int xi_moe_tiles_most(int P, int E, int bm) { return (P + bm - 1) / bm + E; }
 
-// idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P]; tile_* int32 [xi_moe_tiles_most]; n_tiles int32 [1].
+// idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P]; tile_* int32 [xi_moe_tiles_most]; n_tiles int32 [1];
+// tile_first, tile_count (both or neither): the first tile of a tile's expert and how many it has.
 int xi_moe_sort(const int* idx, int P, int E, int I, int bm, int* order, int* slot_of, int* tile_expert, int* tile_row0,
-                int* tile_rows, int* n_tiles, hipStream_t stream) {
-  XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && (bm == 32 || bm == 64 || bm == 128), "moe_sort: bad sizes pairs=%d experts=%d rows=%d", P, E, bm);
-  moe_sort_kernel<<<1, kSortThreads, 0, stream>>>(idx, P, E, I, bm, order, slot_of, tile_expert, tile_row0, tile_rows, n_tiles);
+                int* tile_rows, int* n_tiles, int* tile_first, int* tile_count, hipStream_t stream) {
+  XI_CHECK((tile_first == nullptr) == (tile_count == nullptr), "moe_sort: an operand is missing");
+  XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && (bm == 32 || bm == 64 || bm == 128 || bm == 256), "moe_sort: bad sizes pairs=%d experts=%d rows=%d", P, E, bm);
+  moe_sort_kernel<<<1, kSortThreads, 0, stream>>>(idx, P, E, I, bm, order, slot_of, tile_expert, tile_row0, tile_rows, n_tiles,
+                                                   tile_first, tile_count);
   XI_LAUNCH_CHECK("moe_sort");
   return 0;
 }

@@ -1,0 +1,163 @@
+// The walk of a bfloat16 tile product over K that the many-row kernels share (linear_tile.hip says what it is
+// and what it was measured against; moe_tile.hip takes the rows of x and w from other places): BM rows of
+// x by BN rows of w, tiles of 64 k brought into an LDS ring by loads that write LDS, two sets of operand
+// registers a wave.
+#pragma once
+#include "common.h"
+
+namespace xi {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+namespace tile {
+
+__device__ __forceinline__ void load_lds16(const void* base, unsigned lane_off, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+__device__ __forceinline__ bf16x8 lds8(const unsigned char* p) { return *reinterpret_cast<const bf16x8*>(p); }
+
+// BM rows of x by BN rows of w a workgroup, BK = 64 k a tile; WGM x WGN waves, each (BM / WGM) by (BN / WGN); a ring of S stages.
+template <int BM, int BN, int WGM, int WGN, int S>
+struct Walk {
+  static constexpr int BK = 64, kBK = BK;
+  static constexpr int kRowBytes = BK * 2;
+  static constexpr int CPR = BK / 8;                                // 16-byte chunks of a row
+  static constexpr int PS = 1;                                      // rows that share a 256-byte phase differ in place: p >> PS
+  static constexpr int RPL = 1024 / kRowBytes;                      // rows a wave-wide load brings
+  static constexpr int KSTEPS = BK / 32;
+  static constexpr int NWV = WGM * WGN;
+  static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16;      // 16 x 16 tiles of a wave
+  static constexpr int WBYTES = BN * kRowBytes, XBYTES = BM * kRowBytes, STAGE = WBYTES + XBYTES;
+  static constexpr int WI = WBYTES / 1024, XI = XBYTES / 1024;      // wave-wide loads of a tile: w, then x
+  static_assert((WI + XI) % NWV == 0, "every wave issues the same number of loads a tile");
+  static constexpr int LPW = (WI + XI) / NWV;
+  static constexpr int LDS = S * STAGE;
+  static_assert(S * LPW < 64 && S >= 2, "the tiles in flight must fit the load counter");
+  static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0, "whole 16 x 16 tiles a wave");
+
+  // What a lane brings of every tile: per load t of its wave the byte offset of its chunk from the operand's base.
+  // `offset(is_w, p)`: of row p of the tile (rows past the end: of any row; nobody stores what they make).
+  template <typename F>
+  static __device__ __forceinline__ void offsets(unsigned (&ld_off)[LPW], F offset) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int t = 0; t < LPW; ++t) {
+      const int ii = wave + NWV * t;
+      const bool is_w = ii < WI;
+      const int p = RPL * (is_w ? ii : ii - WI) + lane / CPR;      // row within the operand's tile
+      const int ch = (lane % CPR) ^ ((p >> PS) & (CPR - 1));       // the chunk that belongs at this lane's place
+      ld_off[t] = offset(is_w, p) + (unsigned)(ch * 16);
+    }
+  }
+
+  // acc (features of w down, rows of x across: a lane holds features 4 j .. 4 j + 3 of row r of a 16 x 16 tile) = the sums
+  // over k_tiles tiles of 64 k from wbase and xbase on.
+  static __device__ __forceinline__ void run(const bf16* wbase, const bf16* xbase, const unsigned (&ld_off)[LPW], int k_tiles,
+                                             unsigned char* smem, f32x4 (&acc)[TN][TM]) {
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, j = lane >> 4;
+    const int wm = wave % WGM, wn = wave / WGM;
+
+    // the t-th of this wave's loads of tile kt, into stage st
+    auto fetch_one = [&](int kt, int st, int t) {
+      const int ii = wave + NWV * t;
+      // (which operand a wave's t-th load takes is the same in all its lanes: made a scalar by hand)
+      const unsigned long long a = (unsigned long long)(uintptr_t)((ii < WI ? wbase : xbase) + (size_t)kt * kBK);
+      const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+      load_lds16(reinterpret_cast<const void*>((uintptr_t)(((unsigned long long)hi << 32) | lo)), ld_off[t],
+                 __builtin_amdgcn_readfirstlane(lds0 + (unsigned)st * STAGE + (unsigned)ii * 1024u));
+    };
+    auto fetch = [&](int kt, int st) {
+#pragma unroll
+      for (int t = 0; t < LPW; ++t) fetch_one(kt, st, t);
+    };
+
+    // where this lane reads its operands within a stage: row r of a 16-row tile, chunk 4 ks + j at
+    // its permuted place (16 rows further on the permutation is the same)
+    unsigned rd[KSTEPS];
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) rd[ks] = (unsigned)(r * kRowBytes + 16 * ((4 * ks + j) ^ ((r >> PS) & (CPR - 1))));
+    const unsigned w_rd = (unsigned)(wn * TN * 16) * kRowBytes;
+    const unsigned x_rd = WBYTES + (unsigned)(wm * TM * 16) * kRowBytes;
+
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+      for (int b = 0; b < TM; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    auto read = [&](const unsigned char* T, int ks, bf16x8 (&wa)[TN], bf16x8 (&xb)[TM]) {
+#pragma unroll
+      for (int a = 0; a < TN; ++a) wa[a] = lds8(T + w_rd + rd[ks] + a * 16 * kRowBytes);
+#pragma unroll
+      for (int b = 0; b < TM; ++b) xb[b] = lds8(T + x_rd + rd[ks] + b * 16 * kRowBytes);
+    };
+    auto multiply = [&](const bf16x8 (&wa)[TN], const bf16x8 (&xb)[TM]) {
+#pragma unroll
+      for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[a], xb[b], acc[a][b], 0, 0, 0);
+    };
+
+    // The walk, one barrier a tile.  A tile's two 32-wide steps have their operands in two sets of
+    // registers; each set is read from LDS while the matrix cores work on the other: the second
+    // step's before the first step's products are issued, the next tile's first step's (behind the
+    // barrier that says the tile has landed) before the second step's products.  Tiles past the
+    // slice's last are asked for all the same (from the last one's place) and read too, so that the
+    // number of loads in flight and the code do not depend on where the walk is.
+    static_assert(KSTEPS == 2, "two sets of operand registers, one a step");
+#pragma unroll
+    for (int p = 0; p < S; ++p) fetch(p < k_tiles ? p : k_tiles - 1, p);
+    bf16x8 wa0[TN], xb0[TM], wa1[TN], xb1[TM];
+    wait_loads<(S - 1) * LPW>();       // this wave's loads of the first tile have landed
+    __syncthreads();                   // everybody's have
+    read(smem, 0, wa0, xb0);
+    int st = 0;
+    for (int kt = 0; kt < k_tiles; ++kt) {
+      const unsigned char* T = smem + (size_t)st * STAGE;
+      read(T, 1, wa1, xb1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(wa0, xb0);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_loads<(S - 2) * LPW>();     // this wave's loads of the next tile have landed, and its reads of this one
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0): the operands above are in registers)
+      __syncthreads();                 // everybody's: the next tile is whole, and this tile's stage is free
+      const int filled = st;
+      const int nxt = kt + S < k_tiles ? kt + S : k_tiles - 1;
+      st = st + 1 == S ? 0 : st + 1;
+      read(smem + (size_t)st * STAGE, 0, wa0, xb0);
+      __builtin_amdgcn_sched_barrier(0);
+      // the second step's products with the loads of the tile S ahead between them: a wave that asks
+      // for all its loads at once waits until the load unit has taken them (it takes a compute unit's
+      // 48 to 64 KB a tile at about 55 bytes a clock) before it issues its first product
+      {
+        constexpr int PER = (TN * TM) / LPW;       // products between two loads
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+          for (int b = 0; b < TM; ++b) {
+            const int idx = a * TM + b;
+            if (idx % PER == 0 && idx / PER < LPW) {
+              __builtin_amdgcn_sched_barrier(0);
+              fetch_one(nxt, filled, idx / PER);
+            }
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa1[a], xb1[b], acc[a][b], 0, 0, 0);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wait_loads<0>();     // the tiles asked for past the end are still on their way into LDS
+  }
+};
+
+}  // namespace tile
+}  // namespace xi

@@ -759,7 +759,7 @@ def moe_experts_library(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     order, slot_of = ints[:P], ints[P:2 * P]
     _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), 128, _p(order), _p(slot_of), _p(ints[2 * P:2 * P + most]),
                           _p(ints[2 * P + most:2 * P + 2 * most]), _p(ints[2 * P + 2 * most:2 * P + 3 * most]),
-                          _p(ints[2 * P + 3 * most:]), _stream()))
+                          _p(ints[2 * P + 3 * most:]), None, None, _stream()))
     if weigh_input and not gated:
         raise KernelError("moe_experts_library: a weight on the input is built for gated experts")
     wt_in = wt.reshape(-1).contiguous() if weigh_input else None
@@ -779,6 +779,80 @@ def moe_experts_library(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
             torch.mm(mid, down[e].t(), out_dtype=torch.float32, out=y[at:at + n])
             at += n
     out = torch.empty((T, H), dtype=torch.float32, device=x.device)
+    _ok(lib().xi_moe_combine(_p(y), _p(slot_of), _p(wt), _p(out), T, H, top, _p(idx), E, _p(x if identity else None), _p(add), _stream()))
+    return out
+
+
+MOE_TILED = True          # False: the grouped form, a pair at a time, and the vendor library for steps of portions with many rows
+
+
+def moe_tiled_takes(T: int, top: int, E: int, H: int, F: int, gated: bool) -> bool:
+    """Whether `moe_experts_tiled` takes a step's sizes: both products in whole tiles of 64 k, experts' numbers as `moe_sort` has them."""
+    takes = lib().xi_moe_tile_takes
+    P = ctypes.c_longlong(T * top)
+    return E <= 1024 and bool(takes(ctypes.c_longlong(T), F, H, int(gated))) and bool(takes(P, H, F, 0))
+
+
+def moe_tile_rows(P: int, E: int, F: int, gated: bool) -> int:
+    """Rows of a tile of `moe_experts_tiled` for P pairs on E experts.  Measured on MI355X, width 4096, 8 experts of 6144, both
+    products and what stands around them (us, tiles of 64 | 128 rows): gated (two identity experts beside them) at 8 pairs an
+    expert 220 | 256, at 32 229 | 265, at 64 296 | 278, at 250 546 | 352; without a gate at 4 170 | 193, at 64 235 | 222;
+    width 2048, 16 experts of 4096 at 32 131 | 142, at 50 135 | 147, at 125 201 | 178.  128 | 256 rows: gated at 512 610 | 553, at
+    1,024 1,062 | 1,038, without a gate at 512 564 | 588, at 1,024 939 | 966."""
+    if P <= 56 * E:
+        return 64
+    wide = (P // 256 + E) * (2 * F // 256) >= 512          # workgroups of the larger tile that fill the chip twice
+    return 256 if gated and P >= 384 * E and wide else 128
+
+
+def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, idx: torch.Tensor, wt: torch.Tensor,
+                      act: str = "silu", gated: bool = True, weigh_input: bool = False, identity: int = 0,
+                      add: Optional[torch.Tensor] = None, tile_rows: Optional[int] = None) -> torch.Tensor:
+    """`moe_experts` in bfloat16 at sizes of `moe_tiled_takes`: the pairs sorted by expert on the device, each expert's rows
+    multiplied in tiles of `tile_rows` (64, 128 or 256; None: `moe_tile_rows`) by the walk of the dense many-row product, the
+    activation on the first product's float32 sums.  Nothing is read on the host.  From one token on it is ahead of the other
+    forms: 16 pairs on 8 gated experts of 6144 at width 4096 184 us where the grouped form takes 331 and a pair at a time 441,
+    2,048 tokens 553 where the vendor library's products an expert take 925."""
+    _dev(x, gate_up, down, idx, wt, add)
+    _moe_rows(x, add, identity, weigh_input)
+    acts = ACTIVATIONS if gated else UNGATED_ACTIVATIONS
+    if act not in acts:
+        raise KernelError(f"moe_experts_tiled: unknown activation {act!r}")
+    if weigh_input and not gated:
+        raise KernelError("moe_experts_tiled: a weight on the input is built for gated experts")
+    if gate_up.dim() != 3 or down.dim() != 3 or x.dim() != 2 or idx.dim() != 2:
+        raise KernelError("moe_experts_tiled: x [T, H], gate_up [E, 2F, H], down [E, H, F], idx [T, top]")
+    T, H = x.shape
+    E, F2, _ = gate_up.shape
+    F, top = (F2 // 2 if gated else F2), int(idx.shape[1])
+    if any(t.dtype != torch.bfloat16 for t in (x, gate_up, down)):
+        raise KernelError("moe_experts_tiled: operands must be bfloat16")
+    if gate_up.shape != (E, (2 if gated else 1) * F, H) or down.shape != (E, H, F) or idx.shape != (T, top) or wt.shape != (T, top):
+        raise KernelError("moe_experts_tiled: x [T, H], gate_up [E, 2F, H] (up alone: [E, F, H]), down [E, H, F], idx and weights [T, top]")
+    _want(idx, torch.int32, "moe_experts_tiled: idx")
+    _want(wt, torch.float32, "moe_experts_tiled: weights")
+    if not moe_tiled_takes(T, top, E, H, F, gated):
+        raise KernelError(f"moe_experts_tiled: {T} tokens, {E} experts, H={H} F={F} are not taken (sizes in 64s)")
+    P = T * top
+    bm = int(tile_rows) if tile_rows is not None else moe_tile_rows(P, E, F, gated)
+    if bm not in (64, 128, 256):
+        raise KernelError("moe_experts_tiled: tiles of 64, 128 or 256 rows")
+    most = int(lib().xi_moe_tiles_most(P, E, bm))
+    ints = torch.empty((2 * P + 5 * most + 1,), dtype=torch.int32, device=x.device)
+    at = [0, P, 2 * P] + [2 * P + i * most for i in range(1, 6)] + [2 * P + 5 * most + 1]
+    order, slot_of, t_e, t_r0, t_n, t_f, t_c, n_tiles = (ints[a:b] for a, b in zip(at, at[1:]))
+    _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
+                          _p(t_c), _stream()))
+    wt_in = wt.contiguous() if weigh_input else None
+    mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
+    _ok(lib().xi_moe_tile(_p(x), ctypes.c_longlong(T), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
+                          _p(t_c), most, _p(mid), F, H, bm, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
+    y = torch.empty((P, H), dtype=torch.float32, device=x.device)
+    _ok(lib().xi_moe_tile(_p(mid), ctypes.c_longlong(P), _p(order), top, _p(down), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
+                          _p(t_c), most, _p(y), H, F, bm, 0, 0, None, _stream()))
+    out = torch.empty((T, H), dtype=torch.float32, device=x.device)
+    if weigh_input:
+        wt = torch.ones_like(wt)
     _ok(lib().xi_moe_combine(_p(y), _p(slot_of), _p(wt), _p(out), T, H, top, _p(idx), E, _p(x if identity else None), _p(add), _stream()))
     return out
 
@@ -843,7 +917,7 @@ def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, idx:
         order, slot_of = ints[:P], ints[P:2 * P]
         t_e, t_r0, t_n, n_tiles = (ints[2 * P:2 * P + most], ints[2 * P + most:2 * P + 2 * most],
                                    ints[2 * P + 2 * most:2 * P + 3 * most], ints[2 * P + 3 * most:])
-        _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _stream()))
+        _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), None, None, _stream()))
         mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
         _ok(lib().xi_moe_group(_p(x), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), most, _p(mid),
                                F, H, bm, 1 if gated else 2, acts[act], _p(wt_in), _stream()))

@@ -162,15 +162,19 @@ class RoutedExperts(FeedForward):
         idx, wt = routed[0], routed[1]
         # the shared expert's result is added where the experts' are, unless a factor opens it
         add = self._shared(x) if self.shared and not opens else None
-        # a step that brings portions is never recorded: with many rows an expert it may read the experts' row
-        # counts on the host and hand each expert's rows to the vendor library, as the dense products of many rows go
-        if (ctx.max_q_len > 1 and x.dtype == torch.bfloat16 and self.LIBRARY
-                and x.shape[0] * self.top >= kernels.MOE_LIBRARY_ROWS * self.experts):
-            out = kernels.moe_experts_library(x, self.gate_up, self.down, idx, wt, self.activation, gated=self.gated,
-                                              weigh_input=self.weigh_input, identity=self.identity, add=add)
+        kw = dict(gated=self.gated, weigh_input=self.weigh_input, identity=self.identity, add=add)
+        T = x.shape[0]
+        # bfloat16 in sizes of 64: the tiled products, for single tokens as for portions; other sizes go to the vendor library,
+        # expert by expert, where a step of portions (which is never recorded: the experts' row counts are read on the host)
+        # brings many rows an expert, and to the grouped form or a pair at a time otherwise
+        if x.dtype == torch.bfloat16 and kernels.MOE_TILED and kernels.moe_tiled_takes(T, self.top, self.experts, self.hidden,
+                                                                                     self.inter, self.gated):
+            out = kernels.moe_experts_tiled(x, self.gate_up, self.down, idx, wt, self.activation, **kw)
+        elif (ctx.max_q_len > 1 and x.dtype == torch.bfloat16 and self.LIBRARY
+                and T * self.top >= kernels.MOE_LIBRARY_ROWS * self.experts):
+            out = kernels.moe_experts_library(x, self.gate_up, self.down, idx, wt, self.activation, **kw)
         else:
-            out = kernels.moe_experts(x, self.gate_up, self.down, idx, wt, self.activation, gated=self.gated,
-                                      weigh_input=self.weigh_input, identity=self.identity, add=add)
+            out = kernels.moe_experts(x, self.gate_up, self.down, idx, wt, self.activation, **kw)
         if opens:            # out (float32) += sigmoid(opening) * the shared expert's result
             out = kernels.gated_add_(out, self._shared(x), routed[2][:, 0])
         return out
