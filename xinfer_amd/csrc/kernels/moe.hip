@@ -31,47 +31,91 @@
 namespace xi {
 
 struct alignas(16) Bf8 { bf16 v[8]; };
-constexpr int kRouteWaves = 4;
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTop = 64;
 
-template <typename T>
-__global__ __launch_bounds__(kRouteWaves* kWave) void moe_route_kernel(const T* __restrict__ x,
-                                                                       const float* __restrict__ wr,
-                                                                       const float* __restrict__ br, int* __restrict__ idx,
-                                                                       float* __restrict__ wt, int H, int E, int top,
-                                                                       int all_scores, float* __restrict__ extra, int X,
-                                                                       const float* __restrict__ correction) {
-  __shared__ float z[kMaxExperts];
-  __shared__ float score[kMaxExperts];       // with a correction: the scores the weights are made of
-  __shared__ float denom_all[2];
-  __shared__ float chosen[kMaxTop];
-  const int t = blockIdx.x;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const T* xr = x + (size_t)t * H;
-  for (int e = wave; e < E + X; e += kRouteWaves) {
+// eight consecutive elements as float
+static __device__ __forceinline__ void route_load8(const float* p, float (&v)[8]) {
+  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+static __device__ __forceinline__ void route_load8(const bf16* p, float (&v)[8]) {
+  const Bf8 a = *reinterpret_cast<const Bf8*>(p);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = to_float(a.v[i]);
+}
+
+// A workgroup of `waves` waves takes TT tokens; a wave an output of the router at a time, for all of them, and then wave i
+// chooses for token i.  VEC: rows in whole pieces of eight: a lane takes eight k side by side, 512 k a round of the wave, eight
+// chains; else four chains of single numbers.  The order of a sum is fixed by H alone.
+// Measured on MI355X, width 4096, ten outputs: 8 tokens (sixteen waves, one token) 6.3 us against 25 with four waves and four
+// chains of single numbers, whose rounds waited for one another; 2,048 tokens (eight waves, four tokens: a row of the router is
+// read once for four) 16 us against 29.
+template <typename T, bool VEC, int TT>
+__global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ x, const float* __restrict__ wr,
+                                                         const float* __restrict__ br, int* __restrict__ idx,
+                                                         float* __restrict__ wt, int H, int E, int top, int all_scores,
+                                                         float* __restrict__ extra, int X, const float* __restrict__ correction,
+                                                         int n_tok) {
+  __shared__ float z_all[TT][kMaxExperts];
+  __shared__ float score_all[TT][kMaxExperts];       // with a correction: the scores the weights are made of
+  __shared__ float denom_every[TT][2];
+  __shared__ float chosen_all[TT][kMaxTop];
+  const int t0 = blockIdx.x * TT;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+  for (int e = wave; e < E + X; e += waves) {
     const float* w = wr + (size_t)e * H;
-    // four chains a lane, so that four rounds of loads are in flight; the order is fixed by H alone
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-    int k = lane;
-    for (; k + 3 * kWave < H; k += 4 * kWave) {
-      const float x0 = to_float(xr[k]), x1 = to_float(xr[k + kWave]), x2 = to_float(xr[k + 2 * kWave]),
-                  x3 = to_float(xr[k + 3 * kWave]);
-      const float w0 = w[k], w1 = w[k + kWave], w2 = w[k + 2 * kWave], w3 = w[k + 3 * kWave];
-      a0 = fmaf(x0, w0, a0);
-      a1 = fmaf(x1, w1, a1);
-      a2 = fmaf(x2, w2, a2);
-      a3 = fmaf(x3, w3, a3);
+    float acc[TT];
+    if (VEC) {
+      float a[TT][8];
+#pragma unroll
+      for (int u = 0; u < TT; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[u][i] = 0.f;
+#pragma unroll 4
+      for (int k = 8 * lane; k < H; k += 8 * kWave) {
+        float wv[8];
+        route_load8(w + k, wv);
+#pragma unroll
+        for (int u = 0; u < TT; ++u) {
+          float xv[8];
+          route_load8(x + (size_t)(t0 + u < n_tok ? t0 + u : n_tok - 1) * H + k, xv);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[u][i] = fmaf(xv[i], wv[i], a[u][i]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < TT; ++u)
+        acc[u] = ((a[u][0] + a[u][1]) + (a[u][2] + a[u][3])) + ((a[u][4] + a[u][5]) + (a[u][6] + a[u][7]));
+    } else {
+#pragma unroll
+      for (int u = 0; u < TT; ++u) {
+        const T* xr = x + (size_t)(t0 + u < n_tok ? t0 + u : n_tok - 1) * H;
+        float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+        int k = lane;
+        for (; k + 3 * kWave < H; k += 4 * kWave) {
+          a0 = fmaf(to_float(xr[k]), w[k], a0);
+          a1 = fmaf(to_float(xr[k + kWave]), w[k + kWave], a1);
+          a2 = fmaf(to_float(xr[k + 2 * kWave]), w[k + 2 * kWave], a2);
+          a3 = fmaf(to_float(xr[k + 3 * kWave]), w[k + 3 * kWave], a3);
+        }
+        for (; k < H; k += kWave) a0 = fmaf(to_float(xr[k]), w[k], a0);
+        acc[u] = (a0 + a1) + (a2 + a3);
+      }
     }
-    for (; k < H; k += kWave) a0 = fmaf(to_float(xr[k]), w[k], a0);
-    float acc = wave_sum((a0 + a1) + (a2 + a3));
-    if (lane == 0) {
-      if (e < E) z[e] = acc + (br ? br[e] : 0.f);
-      else extra[(size_t)t * X + (e - E)] = acc;
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+      const float sum = wave_sum(acc[u]);
+      if (lane == 0 && t0 + u < n_tok) {
+        if (e < E) z_all[u][e] = sum + (br ? br[e] : 0.f);
+        else extra[(size_t)(t0 + u) * X + (e - E)] = sum;
+      }
     }
   }
   __syncthreads();
-  if (wave != 0) return;
+  const int t = t0 + wave;
+  if (wave >= TT || t >= n_tok) return;
+  float *z = z_all[wave], *score = score_all[wave], *denom_all = denom_every[wave], *chosen = chosen_all[wave];
   if (all_scores == 1) {     // the softmax's maximum and denominator over every expert, in a fixed order
     float m = -INFINITY;
     for (int e = lane; e < E; e += kWave) m = fmaxf(m, z[e]);
@@ -256,14 +300,22 @@ int xi_moe_route(const void* x, int dtype, const float* wr, const float* br, int
   XI_CHECK(all_scores >= 0 && all_scores <= 2, "moe_route: unknown kind of scores %d", all_scores);
   XI_CHECK(top > 0 && top <= E && top <= kMaxTop, "moe_route: %d of %d experts cannot be chosen (at most %d)", top, E, kMaxTop);
   if (n_tok == 0) return 0;
-  if (dtype == kF32)
-    moe_route_kernel<float><<<n_tok, kRouteWaves * kWave, 0, stream>>>((const float*)x, wr, br, idx, wt, H, E, top, all_scores,
-                                                                       extra, X, correction);
-  else if (dtype == kBF16)
-    moe_route_kernel<bf16><<<n_tok, kRouteWaves * kWave, 0, stream>>>((const bf16*)x, wr, br, idx, wt, H, E, top, all_scores,
-                                                                      extra, X, correction);
+  const bool vec = H % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
+#define XI_ROUTE(TT_, VEC, TOK, WAVES)                                                                                      \
+  moe_route_kernel<TT_, VEC, TOK><<<(unsigned)((n_tok + TOK - 1) / TOK), WAVES * kWave, 0, stream>>>(                        \
+      (const TT_*)x, wr, br, idx, wt, H, E, top, all_scores, extra, X, correction, n_tok)
+#define XI_ROUTE_T(TT_)                                  \
+  do {                                                   \
+    if (!vec) XI_ROUTE(TT_, false, 1, 8);                \
+    else if (n_tok < 1024) XI_ROUTE(TT_, true, 1, 16);   \
+    else XI_ROUTE(TT_, true, 4, 8);                      \
+  } while (0)
+  if (dtype == kF32) XI_ROUTE_T(float);
+  else if (dtype == kBF16) XI_ROUTE_T(bf16);
   else
     XI_CHECK(false, "moe_route: unknown dtype %d", dtype);
+#undef XI_ROUTE_T
+#undef XI_ROUTE
   XI_LAUNCH_CHECK("moe_route");
   return 0;
 }
