@@ -33,7 +33,7 @@ def _plain(x, gate_up, down, idx, wt, act, gated, weigh_input, E, add):
 @pytest.mark.parametrize("H,F,act,gated,weigh,identity,shared", [
     (64, 64, "silu", True, False, 2, True), (192, 320, "gelu_tanh", True, True, 0, False), (320, 192, "relu2", False, False, 0, True),
     (512, 256, "silu", False, False, 1, False), (256, 576, "silu", True, False, 0, False)])
-def test_experts_in_tiles(H, F, act, gated, weigh, identity, shared):
+def test_experts_in_tiles(H, F, act, gated, weigh, identity, shared, monkeypatch):
     from xinfer_amd import kernels
     g = torch.Generator().manual_seed(H + F)
     E, rows = 6, [0, 1, 127, 128, 129, 300]              # pairs an expert (the identity experts take some of the rest)
@@ -55,6 +55,9 @@ def test_experts_in_tiles(H, F, act, gated, weigh, identity, shared):
         assert float((got.cpu().double() - ref).norm() / ref.norm()) < 2.0 ** -8
         assert torch.equal(got, few), bm
     assert torch.equal(kernels.moe_experts_tiled(*dev, act, **kw), few)
+    for pair in ((256, 128), (128, 256), (256, 64), (64, 128)):          # the products in tiles of their own
+        monkeypatch.setattr(kernels, "moe_tile_rows", lambda *a: pair)
+        assert torch.equal(kernels.moe_experts_tiled(*dev, act, **kw), few), pair
 
 
 def test_what_is_taken_and_refused():

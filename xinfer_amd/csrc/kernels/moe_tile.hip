@@ -26,7 +26,7 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
                                                           const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
                                                           const int* __restrict__ n_tiles, const int* __restrict__ tile_first,
                                                           const int* __restrict__ tile_count, void* __restrict__ out, int N, int K,
-                                                          int tiles_n, const float* __restrict__ in_wt) {
+                                                          int tiles_n, int parts, const float* __restrict__ in_wt) {
   constexpr bool GATED = FORM == 1, GATHER = FORM != 0;
   constexpr int WGM = 2, WGN = 4;
   using W = Walk<BM, BN, WGM, WGN, S>;
@@ -37,13 +37,15 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, j = lane >> 4;
   const int wm = wave % WGM, wn = wave / WGM;
-  const int total = *n_tiles * tiles_n, per_die = (total + 7) >> 3;
+  const int total = *n_tiles * parts * tiles_n, per_die = (total + 7) >> 3;
   const int in_die = blockIdx.x >> 3, place = (blockIdx.x & 7) * per_die + in_die;
   if (in_die >= per_die || place >= total) return;
-  // the places of an expert's tiles lie together: tile t's expert has places first * tiles_n .. (first + count) * tiles_n - 1
-  const int some = place / tiles_n, first = tile_first[some], count = tile_count[some];
-  const int q = place - first * tiles_n, tn_i = q / count, tile = first + (q - tn_i * count);
-  const int e = tile_expert[tile], row0 = tile_row0[tile], rows = tile_rows[tile];
+  // the places of an expert's tiles lie together: those of a tile's expert are first * parts * tiles_n and on
+  const int some = place / tiles_n / parts, first = tile_first[some] * parts, count = tile_count[some] * parts;
+  const int q = place - first * tiles_n, tn_i = q / count, piece = first + (q - tn_i * count), tile = piece / parts;
+  const int skip = (piece - tile * parts) * BM;                      // this part's rows of the tile
+  const int e = tile_expert[tile], row0 = tile_row0[tile] + skip, rows = tile_rows[tile] - skip;
+  if (rows <= 0) return;
   const int f0 = tn_i * (WGN * WF);                                  // the first feature
   unsigned ld_off[W::LPW];
   W::offsets(ld_off, [&](bool is_w, int p) {
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
 #pragma unroll
   for (int b = 0; b < TM; ++b) {
     const int m = (wm * TM + b) * 16 + r;
-    if (m >= rows) continue;
+    if (m >= rows) continue;                   // (rows may go on in the tile's next part: m < BM)
     const int slot = row0 + m;
     // a weight on the expert's INPUT: the products are linear, so it multiplies their sums before the activation
     const float wi = (GATHER && in_wt) ? in_wt[order[slot]] : 1.f;
@@ -102,11 +104,11 @@ int xi_moe_tile_takes(long long rows_x, int N, int K, int gated) {
 }
 
 // The operands of `xi_moe_group` (moe_mfma.hip) for tiles of bm = 64, 128 or 256 rows, with the tiles' `first` and `count` of `xi_moe_sort`;
-// rows_x: rows of A.
+// rows_x: rows of A.  parts: a tile of `xi_moe_sort` has parts * bm rows at most and is that many workgroups' (bm: of one).
 int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, const void* W, const int* tile_expert, const int* tile_row0,
                 const int* tile_rows, const int* n_tiles, const int* tile_first, const int* tile_count, int tiles_most, void* out, int N,
-                int K, int bm, int form, int act, const float* in_wt, hipStream_t stream) {
-  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && tiles_most > 0 && (bm == 64 || bm == 128 || bm == 256),
+                int K, int bm, int parts, int form, int act, const float* in_wt, hipStream_t stream) {
+  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && tiles_most > 0 && (bm == 64 || bm == 128 || bm == 256) && parts >= 1 && parts <= 4,
            "moe_tile: bad sizes N=%d K=%d top=%d tiles=%d rows=%d", N, K, top, tiles_most, bm);
   XI_CHECK(act >= 0 && act <= 2 && form >= 0 && form <= 2, "moe_tile: unknown activation %d or form %d", act, form);
   XI_CHECK(tile_first && tile_count && n_tiles && order, "moe_tile: an operand is missing");
@@ -114,7 +116,7 @@ int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, cons
   XI_CHECK(on16(A) && on16(W) && on16(out), "moe_tile: operands must start on 16 bytes");
   const int bn = bm == 64 ? 128 : 256, features = form == 1 ? bn / 2 : bn;
   const int tiles_n = (N + features - 1) / features;
-  const long long wgs = ((long long)tiles_most * tiles_n + 7) / 8 * 8;
+  const long long wgs = ((long long)tiles_most * parts * tiles_n + 7) / 8 * 8;
   XI_CHECK(wgs <= 0x7fffffffLL, "moe_tile: too many workgroups");
 #define XI_MT(BM, BN, S, FORM, ACT)                                                                                         \
   do {                                                                                                                      \
@@ -123,7 +125,7 @@ int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, cons
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);      \
     XI_CHECK(e == hipSuccess, "moe_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));                      \
     kern<<<(unsigned)wgs, 512, lds, stream>>>((const bf16*)A, order, top, (const bf16*)W, tile_expert, tile_row0, tile_rows, \
-                                              n_tiles, tile_first, tile_count, out, N, K, tiles_n, in_wt);                  \
+                                              n_tiles, tile_first, tile_count, out, N, K, tiles_n, parts, in_wt);           \
   } while (0)
 #define XI_MT_FORM(...)                                        \
   do {                                                         \

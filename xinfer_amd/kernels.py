@@ -793,23 +793,32 @@ def moe_tiled_takes(T: int, top: int, E: int, H: int, F: int, gated: bool) -> bo
     return E <= 1024 and bool(takes(ctypes.c_longlong(T), F, H, int(gated))) and bool(takes(P, H, F, 0))
 
 
-def moe_tile_rows(P: int, E: int, F: int, gated: bool) -> int:
-    """Rows of a tile of `moe_experts_tiled` for P pairs on E experts.  Measured on MI355X, width 4096, 8 experts of 6144, both
-    products and what stands around them (us, tiles of 64 | 128 rows): gated (two identity experts beside them) at 8 pairs an
-    expert 220 | 256, at 32 229 | 265, at 64 296 | 278, at 250 546 | 352; without a gate at 4 170 | 193, at 64 235 | 222;
-    width 2048, 16 experts of 4096 at 32 131 | 142, at 50 135 | 147, at 125 201 | 178.  128 | 256 rows: gated at 512 610 | 553, at
-    1,024 1,062 | 1,038, without a gate at 512 564 | 588, at 1,024 939 | 966."""
+MOE_TILE_RATE = {64: 0.55, 128: 0.80, 256: 1.0}      # products a second of a workgroup's tile, by its rows, of the largest's
+
+
+@functools.lru_cache(maxsize=1024)
+def moe_tile_rows(P: int, E: int, F: int, H: int, gated: bool):
+    """Rows of a workgroup's tile in the two products of `moe_experts_tiled` for P pairs on E experts: tiles of 64 rows up to
+    56 pairs an expert; beyond, the fewest rounds of 256 workgroups by the time of one, with half a tile past an expert's
+    rows on average.  Measured on MI355X, width 4096, 8 experts of 6144, both products and what stands around them
+    (us, tiles of 64 | 128 rows): gated (two identity experts beside them) at 8 pairs an expert 220 | 256, at 32 229 | 265, at 64
+    296 | 278, at 250 546 | 352; without a gate at 4 170 | 193, at 64 235 | 222; width 2048, 16 experts of 4096 at 32 131 | 142,
+    at 50 135 | 147, at 125 201 | 178.  128 | 256 rows, equal loads: gated at 512 610 | 553, at 1,024 1,062 | 1,038, without a gate at 512
+    564 | 588, at 1,024 939 | 966: tiles of 256 rows and 256 features are the faster ones where their rounds come out even."""
     if P <= 56 * E:
-        return 64
-    wide = (P // 256 + E) * (2 * F // 256) >= 512          # workgroups of the larger tile that fill the chip twice
-    return 256 if gated and P >= 384 * E and wide else 128
+        return 64, 64
+
+    def best(rows_w):
+        cost = {bm: -(-int((P / bm + 0.5 * E) * -(-rows_w // 256)) // 256) * bm / MOE_TILE_RATE[bm] for bm in (128, 256)}
+        return min(cost, key=lambda bm: (cost[bm], bm))
+    return best(2 * F if gated else F), best(H)
 
 
 def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, idx: torch.Tensor, wt: torch.Tensor,
                       act: str = "silu", gated: bool = True, weigh_input: bool = False, identity: int = 0,
                       add: Optional[torch.Tensor] = None, tile_rows: Optional[int] = None) -> torch.Tensor:
     """`moe_experts` in bfloat16 at sizes of `moe_tiled_takes`: the pairs sorted by expert on the device, each expert's rows
-    multiplied in tiles of `tile_rows` (64, 128 or 256; None: `moe_tile_rows`) by the walk of the dense many-row product, the
+    multiplied in tiles of `tile_rows` (64, 128 or 256; None: `moe_tile_rows`, one for each product) by the walk of the dense many-row product, the
     activation on the first product's float32 sums.  Nothing is read on the host.  From one token on it is ahead of the other
     forms: 16 pairs on 8 gated experts of 6144 at width 4096 184 us where the grouped form takes 331 and a pair at a time 441,
     2,048 tokens 553 where the vendor library's products an expert take 925."""
@@ -834,9 +843,10 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     if not moe_tiled_takes(T, top, E, H, F, gated):
         raise KernelError(f"moe_experts_tiled: {T} tokens, {E} experts, H={H} F={F} are not taken (sizes in 64s)")
     P = T * top
-    bm = int(tile_rows) if tile_rows is not None else moe_tile_rows(P, E, F, gated)
-    if bm not in (64, 128, 256):
+    bm1, bm2 = (int(tile_rows),) * 2 if tile_rows is not None else moe_tile_rows(P, E, F, H, gated)
+    if bm1 not in (64, 128, 256):
         raise KernelError("moe_experts_tiled: tiles of 64, 128 or 256 rows")
+    bm = max(bm1, bm2)                   # the tiles of the sort; a product whose workgroups take fewer rows cuts them
     most = int(lib().xi_moe_tiles_most(P, E, bm))
     ints = torch.empty((2 * P + 5 * most + 1,), dtype=torch.int32, device=x.device)
     at = [0, P, 2 * P] + [2 * P + i * most for i in range(1, 6)] + [2 * P + 5 * most + 1]
@@ -846,10 +856,10 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     wt_in = wt.contiguous() if weigh_input else None
     mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
     _ok(lib().xi_moe_tile(_p(x), ctypes.c_longlong(T), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
-                          _p(t_c), most, _p(mid), F, H, bm, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
+                          _p(t_c), most, _p(mid), F, H, bm1, bm // bm1, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
     y = torch.empty((P, H), dtype=torch.float32, device=x.device)
     _ok(lib().xi_moe_tile(_p(mid), ctypes.c_longlong(P), _p(order), top, _p(down), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
-                          _p(t_c), most, _p(y), H, F, bm, 0, 0, None, _stream()))
+                          _p(t_c), most, _p(y), H, F, bm2, bm // bm2, 0, 0, None, _stream()))
     out = torch.empty((T, H), dtype=torch.float32, device=x.device)
     if weigh_input:
         wt = torch.ones_like(wt)
