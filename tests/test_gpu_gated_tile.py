@@ -1,0 +1,55 @@
+"""The feed-forward's first product with its activation in tiles of many rows (`linear_gated_tile`) against float64, and the
+rule that chooses it (CPU)."""
+import pytest
+import torch
+
+from xinfer_amd import kernels
+
+DEV = "cuda:0"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K,act", [
+    (65, 320, 128, "silu"), (1, 4, 64, "gelu_tanh"), (257, 132, 192, "gelu_tanh"), (300, 12288, 64, "silu"),
+    (700, 17408, 128, "silu"), (2048, 5000, 64, "gelu_tanh"),      # 256 tiles and a rest, cut in halves (152: not), quarters
+    (1024, 9000, 64, "silu"), (1100, 7168, 64, "gelu_tanh")])
+def test_gated_product_in_tiles(M, F, K, act):
+    g = torch.Generator().manual_seed(M + F)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16), (torch.randn(2 * F, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    z = (x.to(DEV).double() @ w.to(DEV).double().t()).cpu()
+    a, b = z[:, :F], z[:, F:]
+    ref = (torch.nn.functional.silu(a) if act == "silu" else torch.nn.functional.gelu(a, approximate="tanh")) * b
+    got = [kernels.linear_gated_tile(x.to(DEV), w.to(DEV), act, shape).cpu() for shape in (0, 1, 2)]
+    # one rounding to bfloat16 (8 significant bits, neighbours 2^-7 of a power of two apart: at most 2^-8 of an element); the float32 sums and the activation's exponential add up to
+    # (K + 20) 2^-24 of the terms' absolute values, which are below 8 here for sums of K products of unit variance
+    bound = 2.0 ** -8 * ref.abs() + 8 * (K + 20) * 2.0 ** -24 * (1 + b.abs() + a.abs())
+    assert bool(((got[0].double() - ref).abs() <= bound).all())
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+class _Rows:
+    """An operand's type, sizes, order and place, all that the rule looks at."""
+    dtype = torch.bfloat16
+
+    def __init__(self, *shape, start=0, contiguous=True, dtype=torch.bfloat16):
+        self.shape, self.start, self.contiguous, self.dtype = shape, start, contiguous, dtype
+
+    dim = lambda self: len(self.shape)
+    data_ptr = lambda self: self.start
+    is_contiguous = lambda self: self.contiguous
+
+
+@pytest.mark.parametrize("M,F,K,shape", [
+    (64, 3072, 1024, None), (65, 3072, 1024, 0), (320, 3072, 1024, 0), (321, 3072, 1024, 1), (1280, 3072, 1024, 1),
+    (1281, 3072, 1024, 2), (128, 8192, 2048, 0), (129, 8192, 2048, None), (512, 8192, 2048, 1), (513, 8192, 2048, None),
+    (897, 8192, 2048, 2), (4096, 12288, 4096, None), (512, 17408, 5120, None), (513, 17408, 5120, None),
+    (700, 17408, 5120, 2), (2048, 25600, 5120, 2), (2049, 25600, 5120, 2), (256, 3074, 1024, None), (256, 3072, 1000, None)])
+def test_gated_tile_rule(M, F, K, shape):
+    """Where the tiled product is taken, and never an operand that it does not take."""
+    x, w = _Rows(M, K), _Rows(2 * F, K)
+    assert kernels.gated_tile_shape(x, w) == shape
+    for other in (_Rows(M, K, start=8), _Rows(M, K, contiguous=False), _Rows(M, K, dtype=torch.float32), _Rows(1, M, K),
+                  _Rows(M, K + 64)):
+        assert kernels.gated_tile_shape(other, w) is None
+    for other in (_Rows(2 * F, K, start=8), _Rows(2 * F, K, dtype=torch.float32), _Rows(2 * F + 1, K)):
+        assert kernels.gated_tile_shape(x, other) is None

@@ -44,6 +44,7 @@
 //
 // Reference call site: candle matmul in /root/reference/src/models/layers/linear.rs:76-124
 // (vendor BLAS).
+#include "moe_act.h"
 #include "tile_core.h"
 
 namespace xi {
@@ -115,6 +116,85 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
   }
 }
 
+// The feed-forward's first product with its activation (in place of a product of 2 N features, a pass that reads them again and
+// writes half, and their two launches): w [2 N, K] = [gate; up], y bfloat16 [M, N] = act(gate) * up of the
+// float32 sums, one rounding.  A workgroup owns BM rows of x and BN / 2 features; a wave's rows of w are gate rows and the up
+// rows of the same features (as in moe_tile.hip).  Bound by the walk, as above, and by how evenly the tiles fill rounds of 256
+// workgroups; measured at N=17408, K=5120 against the library and the activation's pass: 1,024 rows 313 us (1.17 PFLOP/s) / 411,
+// 2,048 rows 583 / 626; at N=3072, K=1024: 256 rows in tiles of 64 by 64 9.5 / 16.9, 1,024 in 128 by 128 19.0 / 23.1, 2,048 in
+// 256 by 128 28.7 / 35.2.
+template <int BM, int BN, int S, int ACT>
+__device__ __forceinline__ void gated_tile(const bf16* x, const bf16* w, bf16* y, int M, int N, int K, int m0, int f0, unsigned char* smem) {
+  constexpr int WGM = 2, WGN = 4;
+  using W = Walk<BM, BN, WGM, WGN, S>;
+  constexpr int TM = W::TM, TN = W::TN, TF = TN / 2, WF = 16 * TF;
+  static_assert(TN % 2 == 0, "half of a wave's rows of w are gate rows");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, j = lane >> 4;
+  const int wm = wave % WGM, wn = wave / WGM;
+  unsigned ld_off[W::LPW];
+  W::offsets(ld_off, [&](bool is_w, int p) {
+    int row;
+    if (is_w) {
+      int f = f0 + WF * (p / (2 * WF)) + p % WF;
+      f = f < N ? f : N - 1;
+      row = (p & WF) ? N + f : f;
+    } else {
+      row = m0 + p < M ? m0 + p : M - 1;
+    }
+    return (unsigned)((size_t)row * K * 2);
+  });
+  f32x4 acc[TN][TM];
+  W::run(w, x, ld_off, K / kSliceK, smem, acc);
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+#pragma unroll
+  for (int b = 0; b < TM; ++b) {
+    const int m = m0 + (wm * TM + b) * 16 + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int a = 0; a < TF; ++a) {
+      const int n = f0 + WF * wn + 16 * a + 4 * j;
+      if (n >= N) continue;                    // (N is a multiple of 4)
+      bf16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (__bf16)(moe_act_m<ACT>(acc[a][b][i]) * acc[TF + a][b][i]);
+      *reinterpret_cast<bf16x4*>(y + (size_t)m * N + n) = o;
+    }
+  }
+}
+
+// Tiles of BM rows by BN / 2 features, the rows innermost.  Workgroup numbers of one die get consecutive places: its L2 holds the
+// rows of w they share.
+template <int BM, int BN, int S, int ACT>
+__global__ __launch_bounds__(512, 1) void gated_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                            bf16* __restrict__ y, int M, int N, int K, int tiles_m) {
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const int total = gridDim.x, q8 = total >> 3, r8 = total & 7, die = blockIdx.x & 7;
+  const int place = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
+  const int tn_i = place / tiles_m;
+  gated_tile<BM, BN, S, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * BM, tn_i * (BN / 2), smem);
+}
+
+// Tiles of 256 rows by 128 features, of which the last ones, a round of workgroups that would leave half of the compute units or
+// more idle, are cut into `parts` (2: halves of the rows; 4: and of the features).  `whole`: the tiles in front of those.
+// N=17408, K=5120, 2,048 rows (4.25 rounds): 665 us uncut, 583 cut; N=25600 (6.25 rounds): 962 and 846.
+template <int ACT>
+__global__ __launch_bounds__(512, 1) void gated_tile_rest_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                                 bf16* __restrict__ y, int M, int N, int K, int tiles_m, int whole,
+                                                                 int parts) {
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b < whole) {                             // (a multiple of 256)
+    const int place = (b & 7) * (whole >> 3) + (b >> 3), tn_i = place / tiles_m;
+    gated_tile<256, 256, 2, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * 256, tn_i * 128, smem);
+    return;
+  }
+  const int piece = b - whole, place = whole + piece / parts, part = piece % parts, tn_i = place / tiles_m;
+  const int m0 = (place - tn_i * tiles_m) * 256 + 128 * (part & 1), f0 = tn_i * 128 + 64 * (part >> 1);
+  if (m0 >= M || f0 >= N) return;
+  if (parts == 2) gated_tile<128, 256, 3, ACT>(x, w, y, M, N, K, m0, f0, smem);
+  else gated_tile<128, 128, 4, ACT>(x, w, y, M, N, K, m0, f0, smem);
+}
 
 }  // namespace tile
 }  // namespace xi
@@ -165,6 +245,53 @@ int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, i
   }
 #undef XI_TILE
   XI_LAUNCH_CHECK("linear_tile");
+  return 0;
+}
+
+// Whether the gated product takes a shape: K in whole tiles of 64, N in fours, offsets within x and w in 32 bits.
+int xi_linear_gated_tile_takes(long long M, int N, int K) {
+  return M > 0 && N > 0 && N % 4 == 0 && K > 0 && K % tile::kSliceK == 0 && M * K * 2 < (1LL << 32) && 4LL * N * K < (1LL << 32);
+}
+
+// x [M, K], w [2 N, K] = [gate; up], y [M, N] bfloat16 = act(gate) * up; act: 0 silu, 1 gelu (tanh form).  shape 0: 64 rows
+// by 64 features a workgroup; 1: 128 by 128; 2: 256 by 128, the last tiles cut where they would be a round of a few workgroups.
+int xi_linear_gated_tile(const void* x, const void* w, void* y, int M, int N, int K, int act, int shape, hipStream_t stream) {
+  XI_CHECK(xi_linear_gated_tile_takes(M, N, K), "linear_gated_tile: M=%d N=%d K=%d is not taken", M, N, K);
+  XI_CHECK((act == 0 || act == 1) && shape >= 0 && shape <= 2, "linear_gated_tile: unknown activation %d or shape %d", act, shape);
+  auto on16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  XI_CHECK(on16(x) && on16(w) && (reinterpret_cast<uintptr_t>(y) & 7) == 0, "linear_gated_tile: operands must start on 16 bytes");
+  const int bm = shape == 0 ? 64 : shape == 1 ? 128 : 256, features = shape == 0 ? 64 : 128;
+  const int tiles_m = (M + bm - 1) / bm;
+  const long long tiles = (long long)tiles_m * ((N + features - 1) / features);
+  XI_CHECK(tiles <= 0x3fffffffLL, "linear_gated_tile: too many workgroups");
+#define XI_GT_LAUNCH(KERN, LDS, WGS, ...)                                                                                    \
+  do {                                                                                                                       \
+    auto kern = KERN;                                                                                                        \
+    const size_t lds = LDS;                                                                                                  \
+    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);       \
+    XI_CHECK(e == hipSuccess, "linear_gated_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));              \
+    kern<<<(unsigned)(WGS), 512, lds, stream>>>((const bf16*)x, (const bf16*)w, (bf16*)y, M, N, K, __VA_ARGS__);             \
+  } while (0)
+#define XI_GT(BM, BN, S)                                                                                                     \
+  do {                                                                                                                       \
+    constexpr size_t bytes = tile::Walk<BM, BN, 2, 4, S>::LDS;                                                               \
+    if (act == 0) XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, 0>), bytes, tiles, tiles_m);                              \
+    else XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, 1>), bytes, tiles, tiles_m);                                       \
+  } while (0)
+  const long long whole = tiles / 256 * 256, rest = tiles - whole;
+  if (shape == 0) XI_GT(64, 128, 6);
+  else if (shape == 1) XI_GT(128, 256, 3);
+  else if (whole == 0 || rest == 0 || rest > 128) XI_GT(256, 256, 2);
+  else {
+    const int parts = rest <= 64 ? 4 : 2;
+    constexpr size_t bytes = tile::Walk<128, 256, 2, 4, 3>::LDS;       // the most of the three walks
+    static_assert(bytes >= tile::Walk<256, 256, 2, 4, 2>::LDS && bytes >= tile::Walk<128, 128, 2, 4, 4>::LDS, "");
+    if (act == 0) XI_GT_LAUNCH(tile::gated_tile_rest_kernel<0>, bytes, whole + rest * parts, tiles_m, (int)whole, parts);
+    else XI_GT_LAUNCH(tile::gated_tile_rest_kernel<1>, bytes, whole + rest * parts, tiles_m, (int)whole, parts);
+  }
+#undef XI_GT
+#undef XI_GT_LAUNCH
+  XI_LAUNCH_CHECK("linear_gated_tile");
   return 0;
 }
 

@@ -126,7 +126,9 @@ struct Walk {
       const unsigned char* T = smem + (size_t)st * STAGE;
       read(T, 1, wa1, xb1);
       __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);   // (a wave with products to issue goes before one that reads: 1 to 3%)
       multiply(wa0, xb0);
+      __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       wait_loads<(S - 2) * LPW>();     // this wave's loads of the next tile have landed, and its reads of this one
       __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0): the operands above are in registers)
@@ -140,7 +142,8 @@ struct Walk {
       // for all its loads at once waits until the load unit has taken them (it takes a compute unit's
       // 48 to 64 KB a tile at about 55 bytes a clock) before it issues its first product
       {
-        constexpr int PER = (TN * TM) / LPW;       // products between two loads
+        constexpr int PER = (TN * TM) / LPW > 0 ? (TN * TM) / LPW : 1;       // products between two loads
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int a = 0; a < TN; ++a)
 #pragma unroll
@@ -152,6 +155,8 @@ struct Walk {
             }
             acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa1[a], xb1[b], acc[a][b], 0, 0, 0);
           }
+        static_assert(TN * TM >= LPW, "a place for every load between the products");
+        __builtin_amdgcn_s_setprio(0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }

@@ -1753,10 +1753,60 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
     return y
 
 
+def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
+    """The tile shape in which act(x @ gate^T) * (x @ up^T) goes to `linear_gated_tile`, None: the library's product and a
+    kernel for the activation (which also stay for operands that the tiled kernel does not take).  Measured on MI355X
+    against those two, x M rows, w [2 F, K], us:
+      K <= 2048 (K <= 1024 in brackets): the smallest tile whose workgroups are one round of the 256 compute units (for 128
+      rows from half a round on, for 256 rows from 7/8 on [any]), and 256 rows beyond a round.  F=3072 K=1024: M=65 8.7 against 12.1,
+      256 9.5 / 16.9, 320 15.5 / 18.0, 512 17.5 / 19.1, 1024 19.0 / 23.1, 1500 28.0 / 37.0, 2048 28.7 / 35.2, 4096 48.8 / 63.4;
+      F=6144 K=2048: 128 18.2 / 21.5, 512 33.1 / 35.3, 1400 75 / 94, 2048 93 / 104, 4096 175 / 174; F=8192 K=2048: 128 19.9 / 23.5,
+      512 34.9 / 40.5, 1024 58 / 64, 2048 112 / 117.  What those rules leave out is level or behind (F=6144 M=700 53 / 44).
+      2048 < K <= 4096: the library's best sizes (F=12288 K=4096: 700 137 / 151, 900 187 / 158, 2048 313 / 303, 4096 662 / 608).
+      K > 4096, more than 512 rows of which four fifths of the last row of tiles' are there: F=17408 K=5120: 700 262 / 271,
+      1024 313 / 411, 1500 449 / 537, 2048 583 / 626, 4096 1160 / 1275; F=25600 K=5120: 700 353 / 408, 1024 447 / 516,
+      1727 757 / 883, 2048 846 / 891, 4096 1692 / 1766; left out: 513 329 / 290, 770 422 / 370."""
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] \
+            or w.shape[0] % 2 or x.shape[0] <= MID_GATED_UP_TO:
+        return None
+    M, K, F = x.shape[0], x.shape[1], w.shape[0] // 2
+    tiles = lambda rows, features: -(-M // rows) * -(-F // features)
+    shape = None
+    if K > 4096:
+        shape = 2 if M > 512 and 5 * M >= 4 * 256 * -(-M // 256) else None
+    elif K <= 2048:
+        if tiles(64, 64) <= COMPUTE_UNITS:
+            shape = 0
+        elif tiles(128, 128) <= COMPUTE_UNITS:
+            shape = 1 if K <= 1024 or 2 * tiles(128, 128) > COMPUTE_UNITS else None
+        elif K <= 1024 or 8 * tiles(256, 128) >= 7 * COMPUTE_UNITS:
+            shape = 2
+    if shape is None or not (x.is_contiguous() and w.is_contiguous()) or x.data_ptr() % 16 or w.data_ptr() % 16 \
+            or not lib().xi_linear_gated_tile_takes(M, F, K):
+        return None
+    return shape
+
+
+def linear_gated_tile(x: torch.Tensor, w: torch.Tensor, act: str = "silu", shape: int = 0) -> torch.Tensor:
+    """act(x @ gate^T) * (x @ up^T) in bfloat16, [M, N] for w [2 N, K] = [gate; up], in the many-row tiled kernel.  `shape`: 0
+    64 rows by 64 features a workgroup, 1 128 by 128, 2 256 by 128 (`gated_tile_shape` chooses); the value of an element does
+    not depend on it."""
+    _dev(x, w)
+    _want(x, torch.bfloat16, "linear_gated_tile: x")
+    _want(w, torch.bfloat16, "linear_gated_tile: w")
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or w.shape[0] % 2 or act not in ACTIVATIONS:
+        raise KernelError(f"linear_gated_tile: x {tuple(x.shape)}, w {tuple(w.shape)} = [gate; up] and {act!r} do not go together")
+    M, K = x.shape
+    N = w.shape[0] // 2
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _ok(lib().xi_linear_gated_tile(_p(x), _p(w), _p(y), M, N, K, ACTIVATIONS[act], int(shape), _stream()))
+    return y
+
+
 MID_GATED_ROWS = 128      # most rows of the gated form of the tiled product
 MID_GATED_FEATURES = 0    # features a workgroup of it owns; 0: chosen from N (the fewest workgroups that are a multiple of 256)
 MID_GATED_UP_TO = 64      # it is used up to this many rows (more: its reads of x from L2 outweigh the library's
-                          # weakness); measured on MI355X at the gate/up sizes of Qwen3-8B, 14B and 32B, it is
+                          # weakness; `gated_tile_shape`); measured on MI355X at the gate/up sizes of Qwen3-8B, 14B and 32B, it is
 MID_GATED_FROM = 2        # ahead of the streaming kernel from this many rows on, and from the first row where
 MID_GATED_BIG = 300 << 20  # the weight has this many bytes (the streaming kernel falls behind on large weights)
 

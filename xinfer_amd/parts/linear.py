@@ -7,7 +7,9 @@ BLAS (/root/reference/src/models/layers/linear.rs:76-124).  Here:
   bfloat16 : the hand-written kernels for few rows (decode), the vendor library
              (hipBLASLt through torch) for many rows, as the reference uses a library;
              narrow outputs at 129 to 1,024 rows in the hand-written many-row tiled kernel over
-             slices of K where the caller takes partial sums (`kernels.tile_split_plan`).
+             slices of K where the caller takes partial sums (`kernels.tile_split_plan`), and
+             the gated form of more than 64 rows in that kernel's tiles with the activation in
+             them where it is ahead (`kernels.gated_tile_shape`).
 A weight that the checkpoint stores in 32 bits stays in 32 bits; activations are then
 widened for this product.
 """
@@ -56,6 +58,10 @@ class Linear:
         if gated:
             if x.dtype == torch.bfloat16 and x.dim() == 2 and kernels.gated_uses_mid(x.shape[0], w):
                 return kernels.linear_mid_gated(x, w, act=act)        # gate, up and act*mul in one pass
+            if out_dtype in (None, torch.bfloat16) and act in kernels.ACTIVATIONS:
+                shape = kernels.gated_tile_shape(x, w)
+                if shape is not None:
+                    return kernels.linear_gated_tile(x, w, act, shape)    # the same in tiles of many rows
             if act != "silu":
                 return None                                           # the streaming kernel's gated form applies silu
             if (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
