@@ -22,20 +22,20 @@
 // v_mfma_f32_16x16x32_bf16 tiles per 32-wide k step: A = 16 rows of w, B = 16 rows of x, so that a
 // lane holds four consecutive features of one row of the result.  The operands of a tile's two
 // steps live in two sets of registers, each read from LDS while the matrix cores work on the other
-// set, and the loads of the tile S ahead are issued one at a time between the products: a wave that
+// set, and both these reads and the loads of the tile S ahead are issued one at a time between the products: a wave that
 // asks for all its loads at once waits until the load unit has taken them before it issues its
 // first product (5 to 10% of the kernel's time).
 //
 // Measured on MI355X (random operands, the clock under load about 1.8 GHz): 2,048 rows by
 // N = 4096, K = 12288 in 172 us (1.2 PFLOP/s; the library 174), K = 4096 in 68 us (the library 64);
-// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 108 us (1.27; the library 94); the matrix cores are
+// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 102 us (1.35; the library 94); the matrix cores are
 // busy 63% of the time, LDS serves the tiles' 48 to 64 KB of writes and 128 to 192 KB of reads a
 // tile and is what the kernel waits for (without the barrier or without the wait for the loads it
 // is no faster).  Where it is ahead of the library is the narrow output at few rows, whose tiles
 // leave most of the chip idle unless K is cut: 256 rows of N = 4096, K = 12288 in 30 us against 41.
 // Not kept: tiles of 32 k with two workgroups a compute unit (0.85 PFLOP/s against 0.95 at 4,096
 // cubed); the tiles going memory -> registers -> LDS (0.83); four waves of twice the tile each
-// (0.80); the operands of one step only in registers (the second step's reads then wait: -8%).
+// (0.80, and 7% behind with the reads between the products); the operands of one step only in registers (the second step's reads then wait: -8%).
 //
 // Workgroups go round the chip's eight dies; consecutive workgroup numbers of one die are mapped
 // to tiles that share rows of w, then of x, so that a die's L2 holds what its workgroups share.

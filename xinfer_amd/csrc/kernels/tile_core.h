@@ -3,6 +3,8 @@
 // x by BN rows of w, tiles of 64 k brought into an LDS ring by loads that write LDS, two sets of operand
 // registers a wave.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace xi {
@@ -21,6 +23,15 @@ template <int N>
 __device__ __forceinline__ void wait_loads() {
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// f(0), f(1), .. f(N - 1) with the number as a constant
+template <int I, int N, typename F>
+__device__ __forceinline__ void steps(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    steps<I + 1, N>(f);
+  }
 }
 
 __device__ __forceinline__ bf16x8 lds8(const unsigned char* p) { return *reinterpret_cast<const bf16x8*>(p); }
@@ -101,19 +112,43 @@ struct Walk {
 #pragma unroll
       for (int b = 0; b < TM; ++b) xb[b] = lds8(T + x_rd + rd[ks] + b * 16 * kRowBytes);
     };
-    auto multiply = [&](const bf16x8 (&wa)[TN], const bf16x8 (&xb)[TM]) {
-#pragma unroll
-      for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[a], xb[b], acc[a][b], 0, 0, 0);
+    constexpr int NM = TN * TM, READS = TN + TM;
+    // A step's products, wa x xb, with the reads of the next step's operands between them, in the order in which its products
+    // want them and done by three quarters of these, and `load(i)` before product i.  (A wave with products to issue goes
+    // before one that waits to: setprio, 1 to 3%.)
+    auto step = [&](const bf16x8 (&wa)[TN], const bf16x8 (&xb)[TM], const unsigned char* T, int ks, bf16x8 (&wn_)[TN], bf16x8 (&xn_)[TM],
+                    auto load) {
+      __builtin_amdgcn_s_setprio(1);
+      steps<0, NM>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        constexpr int SPAN = NM * 3 / 4;
+        steps<0, READS>([&](auto oc) {
+          constexpr int o = decltype(oc)::value;
+          if constexpr (o * SPAN / READS == i) {
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (o == 0) wn_[0] = lds8(T + w_rd + rd[ks]);
+            else if constexpr (o <= TM) xn_[o - 1] = lds8(T + x_rd + rd[ks] + (o - 1) * 16 * kRowBytes);
+            else wn_[o - TM] = lds8(T + w_rd + rd[ks] + (o - TM) * 16 * kRowBytes);
+          }
+        });
+        load(ic);
+        acc[i / TM][i % TM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i / TM], xb[i % TM], acc[i / TM][i % TM], 0, 0, 0);
+      });
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
     };
 
     // The walk, one barrier a tile.  A tile's two 32-wide steps have their operands in two sets of
-    // registers; each set is read from LDS while the matrix cores work on the other: the second
-    // step's before the first step's products are issued, the next tile's first step's (behind the
-    // barrier that says the tile has landed) before the second step's products.  Tiles past the
-    // slice's last are asked for all the same (from the last one's place) and read too, so that the
-    // number of loads in flight and the code do not depend on where the walk is.
+    // registers; each set is read from LDS between the products of the other: the second step's
+    // between the first step's, the next tile's first step's (behind the barrier that says the tile
+    // has landed) between the second step's, and there too the loads of the tile S ahead.  One at a
+    // time: eight waves that leave the barrier and ask for a whole set at once keep LDS busy for
+    // half a step while the matrix cores have nothing (tiles of 256 by 256, 3,000 x 5120 x 17408:
+    // 428 us so, 414 one at a time; 2,048 x 12288 x 4096 gated 334 and 320), and a wave that asks
+    // for all its loads at once waits until the load unit has taken them (it takes a compute unit's
+    // 48 to 64 KB a tile at about 55 bytes a clock).  Tiles past the slice's last are asked for all
+    // the same (from the last one's place) and read too, so that the number of loads in flight and
+    // the code do not depend on where the walk is.
     static_assert(KSTEPS == 2, "two sets of operand registers, one a step");
 #pragma unroll
     for (int p = 0; p < S; ++p) fetch(p < k_tiles ? p : k_tiles - 1, p);
@@ -124,41 +159,22 @@ struct Walk {
     int st = 0;
     for (int kt = 0; kt < k_tiles; ++kt) {
       const unsigned char* T = smem + (size_t)st * STAGE;
-      read(T, 1, wa1, xb1);
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(1);   // (a wave with products to issue goes before one that reads: 1 to 3%)
-      multiply(wa0, xb0);
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_sched_barrier(0);
+      step(wa0, xb0, T, 1, wa1, xb1, [](auto) {});
       wait_loads<(S - 2) * LPW>();     // this wave's loads of the next tile have landed, and its reads of this one
       __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0): the operands above are in registers)
       __syncthreads();                 // everybody's: the next tile is whole, and this tile's stage is free
       const int filled = st;
       const int nxt = kt + S < k_tiles ? kt + S : k_tiles - 1;
       st = st + 1 == S ? 0 : st + 1;
-      read(smem + (size_t)st * STAGE, 0, wa0, xb0);
       __builtin_amdgcn_sched_barrier(0);
-      // the second step's products with the loads of the tile S ahead between them: a wave that asks
-      // for all its loads at once waits until the load unit has taken them (it takes a compute unit's
-      // 48 to 64 KB a tile at about 55 bytes a clock) before it issues its first product
-      {
-        constexpr int PER = (TN * TM) / LPW > 0 ? (TN * TM) / LPW : 1;       // products between two loads
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-          for (int b = 0; b < TM; ++b) {
-            const int idx = a * TM + b;
-            if (idx % PER == 0 && idx / PER < LPW) {
-              __builtin_amdgcn_sched_barrier(0);
-              fetch_one(nxt, filled, idx / PER);
-            }
-            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa1[a], xb1[b], acc[a][b], 0, 0, 0);
+      step(wa1, xb1, smem + (size_t)st * STAGE, 0, wa0, xb0, [&](auto ic) {
+        steps<0, LPW>([&](auto tc) {
+          if constexpr (decltype(tc)::value * NM / LPW == decltype(ic)::value) {
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_one(nxt, filled, decltype(tc)::value);
           }
-        static_assert(TN * TM >= LPW, "a place for every load between the products");
-        __builtin_amdgcn_s_setprio(0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+        });
+      });
     }
     wait_loads<0>();     // the tiles asked for past the end are still on their way into LDS
   }
