@@ -1,5 +1,5 @@
-"""The feed-forward's first product with its activation in tiles of many rows (`linear_gated_tile`) against float64, and the
-rule that chooses it (CPU)."""
+"""The feed-forward's first product with its activation in tiles of many rows (`linear_gated_tile`) and the product of a long K in the
+lowest tiles that are one round (`linear_tall`) against float64, and the rules that choose them (CPU)."""
 import pytest
 import torch
 
@@ -53,3 +53,31 @@ def test_gated_tile_rule(M, F, K, shape):
         assert kernels.gated_tile_shape(other, w) is None
     for other in (_Rows(2 * F, K, start=8), _Rows(2 * F, K, dtype=torch.float32), _Rows(2 * F + 1, K)):
         assert kernels.gated_tile_shape(x, other) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(97, 260, 64), (1, 4, 128), (333, 516, 192), (1000, 1028, 320), (673, 300, 64)])
+def test_product_in_tall_tiles(M, N, K):
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV), torch.randn(N, K, generator=g).to(torch.bfloat16).to(DEV)
+    ref = x.double() @ w.double().t()
+    got = [kernels.linear_tall(x, w, rows) for rows in kernels.TALL_SHAPES]
+    # one rounding to bfloat16, 2^-8 of an element at most, and K float32 roundings of sums of terms of unit variance (below 8 sqrt(K))
+    assert bool(((got[0].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * 8 * K ** 0.5).all())
+    assert all(torch.equal(got[0], y) for y in got[1:])
+    assert torch.equal(got[0], kernels.linear_tile(x, w, shape=2))
+
+
+@pytest.mark.parametrize("M,N,K,rows", [
+    (1024, 5120, 17408, None), (1025, 5120, 17408, 96), (1152, 5120, 17408, 96), (1153, 5120, 25600, 128), (1536, 5120, 17408, 128),
+    (1537, 5120, 17408, 160), (1760, 5120, 25600, 160), (1761, 5120, 17408, None), (2304, 5120, 17408, None), (2305, 5120, 17408, 224),
+    (2688, 5120, 17408, 224), (2689, 5120, 17408, None), (2400, 4612, 17408, 224), (2400, 4608, 17408, None), (1500, 8192, 28672, None), (1280, 8192, 28672, 160),
+    (1100, 4096, 16384, None), (1100, 5120, 16320, None), (1100, 5122, 17408, None), (1100, 5120, 17400, None)])
+def test_tall_tile_rule(M, N, K, rows):
+    """Where the product is taken (never more than a round of 256 workgroups), and never an operand that it does not take."""
+    x, w = _Rows(M, K), _Rows(N, K)
+    assert kernels.tall_tile_rows(x, w) == rows
+    for other in (_Rows(M, K, start=8), _Rows(M, K, contiguous=False), _Rows(M, K, dtype=torch.float32), _Rows(1, M, K),
+                  _Rows(M, K + 64)):
+        assert kernels.tall_tile_rows(other, w) is None
+    assert kernels.tall_tile_rows(x, _Rows(N, K, start=8)) is None

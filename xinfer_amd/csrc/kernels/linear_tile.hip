@@ -33,7 +33,13 @@
 // tile and is what the kernel waits for (without the barrier or without the wait for the loads it
 // is no faster).  Where it is ahead of the library is the narrow output at few rows, whose tiles
 // leave most of the chip idle unless K is cut: 256 rows of N = 4096, K = 12288 in 30 us against 41.
-// Not kept: tiles of 32 k with two workgroups a compute unit (0.85 PFLOP/s against 0.95 at 4,096
+// A long K whose output is less than a round of such tiles (down projections of 1,025 to 2,688 rows) goes in the lowest tiles that
+// still are one round, 96 to 224 rows by 256 features: 1,727 rows of N = 5120, K = 17408 in 11 x 20 tiles of 160 rows 255 us
+// (1.2 PFLOP/s, its loads into LDS at 57 GB/s a compute unit, which bounds tiles up to that height), the library 473; 256 rows 401;
+// four slices of 128 rows 309 and the reader's four float32 parts.
+// Not kept: the tiles' k shared out evenly over the compute units, whoever comes last at a tile adding up its parts (345 us there:
+// workgroups at different places of K share nothing in L2, and the parts go through memory); v_mfma_f32_32x32x16_bf16 (4,096 cubed 114
+// us); a ring of five stages of 32 k (113); tiles of 32 k with two workgroups a compute unit (0.85 PFLOP/s against 0.95 at 4,096
 // cubed); the tiles going memory -> registers -> LDS (0.83); four waves of twice the tile each
 // (0.80, and 7% behind with the reads between the products); the operands of one step only in registers (the second step's reads then wait: -8%).
 //
@@ -67,8 +73,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
   // ---- which tile and slice: workgroup numbers b, b + 8, b + 16, .. run on one die; they get
   // consecutive places in the order (slice, tile of features, tile of rows)
   const int total = tiles_m * tiles_n * slices;
-  int place = blockIdx.x;
-  if (total % 8 == 0) place = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
+  const int q8 = total >> 3, r8 = total & 7, die = blockIdx.x & 7;
+  const int place = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
   const int per_slice = tiles_m * tiles_n;
   const int slice = place / per_slice;
   const int in_slice = place - slice * per_slice;
@@ -212,15 +218,16 @@ int xi_linear_tile_takes(int M, int N, int K, int slices) {
 // float32 [slices, M, N], the sums over the slices of K: slice s takes the tiles of 64 k from
 // s * (K / 64) / slices up to (s + 1) * (K / 64) / slices (whole numbers: the slices differ by a tile
 // at most).  shape 0: tiles of 128 rows by 256
-// features; 1: 256 rows by 128 features; 2: 256 by 256.
+// features; 1: 256 rows by 128 features; 2: 256 by 256; without slices also 4, 5, 6: 96, 160 and 224 rows by 256 features.
 int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, int slices, int partial, int shape,
                    hipStream_t stream) {
   XI_CHECK(xi_linear_tile_takes(M, N, K, slices), "linear_tile: M=%d N=%d K=%d in %d slices is not taken (K in tiles of "
            "64, a tile a slice at least, N a multiple of 4)", M, N, K, slices);
   XI_CHECK(partial || slices == 1, "linear_tile: %d slices need the float32 partial sums", slices);
-  XI_CHECK(shape >= 0 && shape <= 2, "linear_tile: unknown tile shape %d", shape);
+  XI_CHECK((shape >= 0 && shape <= 2) || (shape >= 4 && shape <= 6 && !partial), "linear_tile: unknown tile shape %d", shape);
   XI_CHECK((size_t)K * 2 * 256 < ((size_t)1 << 32), "linear_tile: K=%d is too long for 32-bit offsets within a tile", K);
-  const int bm = shape == 0 ? 128 : 256, bn = shape == 1 ? 128 : 256;
+  static const int heights[7] = {128, 256, 256, 0, 96, 160, 224};
+  const int bm = heights[shape], bn = shape == 1 ? 128 : 256;
   const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   const long long total = (long long)tiles_m * tiles_n * slices;
   XI_CHECK(total <= 0x7fffffffLL, "linear_tile: too many workgroups");
@@ -239,18 +246,20 @@ int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, i
   } else if (shape == 1) {
     if (partial) XI_TILE(256, 128, 4, 2, 3, true);
     else XI_TILE(256, 128, 4, 2, 3, false);
-  } else {
+  } else if (shape == 2) {
     if (partial) XI_TILE(256, 256, 2, 4, 2, true);
     else XI_TILE(256, 256, 2, 4, 2, false);
-  }
+  } else if (shape == 4) XI_TILE(96, 256, 2, 4, 3, false);
+  else if (shape == 5) XI_TILE(160, 256, 2, 4, 3, false);
+  else XI_TILE(224, 256, 2, 4, 2, false);
 #undef XI_TILE
   XI_LAUNCH_CHECK("linear_tile");
   return 0;
 }
 
 // Whether the gated product takes a shape: K in whole tiles of 64, N in fours, offsets within x and w in 32 bits.
-int xi_linear_gated_tile_takes(long long M, int N, int K) {
-  return M > 0 && N > 0 && N % 4 == 0 && K > 0 && K % tile::kSliceK == 0 && M * K * 2 < (1LL << 32) && 4LL * N * K < (1LL << 32);
+int xi_linear_gated_tile_takes(int M, int N, int K) {
+  return M > 0 && N > 0 && N % 4 == 0 && K > 0 && K % tile::kSliceK == 0 && 2LL * M * K < (1LL << 32) && 4LL * N * K < (1LL << 32);
 }
 
 // x [M, K], w [2 N, K] = [gate; up], y [M, N] bfloat16 = act(gate) * up; act: 0 silu, 1 gelu (tanh form).  shape 0: 64 rows

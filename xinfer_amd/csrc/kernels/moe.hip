@@ -22,10 +22,9 @@
 //   gets weights of 1).
 //
 // Every sum runs in an order fixed by the sizes alone (lanes stride over k, then the wave's
-// butterfly), so a token's result does not depend on the batch it is in.  The grouped
-// matrix-core products for many tokens are in moe_mfma.hip; this file is the float32 path and
-// what decode steps of few tokens use (a pair reads its expert's weights once: the least traffic
-// there is when every pair has another expert).
+// butterfly), so a token's result does not depend on the batch it is in.  The matrix-core products
+// are in moe_tile.hip (bfloat16, sizes in 64s) and moe_mfma.hip (other bfloat16 sizes with many pairs);
+// the pair-at-a-time products here are the float32 path and what is left of bfloat16.
 #include "common.h"
 
 namespace xi {

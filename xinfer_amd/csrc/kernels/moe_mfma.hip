@@ -1,6 +1,8 @@
 // Routed experts for many tokens on the gfx950 matrix cores (bfloat16): the (token, chosen expert)
 // pairs are put in the order of their experts on the device, and each expert's rows go through its
 // weights in tiles, so a weight is read once per tile of up to 128 rows instead of once per pair.
+// The sort and the combine serve moe_tile.hip too, whose products take the sizes that are multiples of 64;
+// the group products here serve the others.
 //
 //   moe_sort      pairs [T * top] -> `order` (slot -> pair), `slot_of` (pair -> slot), and the list of
 //                 tiles (expert, first slot, rows); one workgroup, nothing read on the host

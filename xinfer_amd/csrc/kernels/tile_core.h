@@ -49,11 +49,16 @@ struct Walk {
   static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16;      // 16 x 16 tiles of a wave
   static constexpr int WBYTES = BN * kRowBytes, XBYTES = BM * kRowBytes, STAGE = WBYTES + XBYTES;
   static constexpr int WI = WBYTES / 1024, XI = XBYTES / 1024;      // wave-wide loads of a tile: w, then x
-  static_assert((WI + XI) % NWV == 0, "every wave issues the same number of loads a tile");
-  static constexpr int LPW = (WI + XI) / NWV;
+  // every wave issues the same number of loads a tile (where they do not come out even, the last few bring the last chunk again)
+  static constexpr int LPW = (WI + XI + NWV - 1) / NWV;
   static constexpr int LDS = S * STAGE;
-  static_assert(S * LPW < 64 && S >= 2, "the tiles in flight must fit the load counter");
+  static_assert(S * LPW < 64 && S >= 2 && LDS <= 160 * 1024, "the tiles in flight must fit the load counter");
   static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0, "whole 16 x 16 tiles a wave");
+
+  static __device__ __forceinline__ int load_number(int wave, int t) {
+    const int ii = wave + NWV * t;
+    return (WI + XI) % NWV == 0 || ii < WI + XI ? ii : WI + XI - 1;
+  }
 
   // What a lane brings of every tile: per load t of its wave the byte offset of its chunk from the operand's base.
   // `offset(is_w, p)`: of row p of the tile (rows past the end: of any row; nobody stores what they make).
@@ -62,7 +67,7 @@ struct Walk {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int t = 0; t < LPW; ++t) {
-      const int ii = wave + NWV * t;
+      const int ii = load_number(wave, t);
       const bool is_w = ii < WI;
       const int p = RPL * (is_w ? ii : ii - WI) + lane / CPR;      // row within the operand's tile
       const int ch = (lane % CPR) ^ ((p >> PS) & (CPR - 1));       // the chunk that belongs at this lane's place
@@ -81,7 +86,7 @@ struct Walk {
 
     // the t-th of this wave's loads of tile kt, into stage st
     auto fetch_one = [&](int kt, int st, int t) {
-      const int ii = wave + NWV * t;
+      const int ii = load_number(wave, t);
       // (which operand a wave's t-th load takes is the same in all its lanes: made a scalar by hand)
       const unsigned long long a = (unsigned long long)(uintptr_t)((ii < WI ? wbase : xbase) + (size_t)kt * kBK);
       const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
@@ -121,7 +126,7 @@ struct Walk {
       __builtin_amdgcn_s_setprio(1);
       steps<0, NM>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        constexpr int SPAN = NM * 3 / 4;
+        constexpr int SPAN = NM * 3 / 4;      // (a half or all of them: level to 5% behind)
         steps<0, READS>([&](auto oc) {
           constexpr int o = decltype(oc)::value;
           if constexpr (o * SPAN / READS == i) {

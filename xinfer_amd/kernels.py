@@ -783,7 +783,6 @@ def moe_experts_library(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     return out
 
 
-MOE_TILED = True          # False: the grouped form, a pair at a time, and the vendor library for steps of portions with many rows
 
 
 def moe_tiled_takes(T: int, top: int, E: int, H: int, F: int, gated: bool) -> bool:
@@ -1743,6 +1742,8 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
     partial = bool(partial) or slices > 1
     if not linear_tile_takes(M, N, K, slices):
         raise KernelError(f"linear_tile: M={M} N={N} K={K} in {slices} slices is not taken")
+    if shape not in (None, 0, 1, 2):
+        raise KernelError(f"linear_tile: unknown tile shape {shape}")
     if shape is None:
         shape = 1 if -(-M // 256) * -(-N // 128) < -(-M // 128) * -(-N // 256) else 0
     if partial:
@@ -1750,6 +1751,50 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
     else:
         y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _ok(lib().xi_linear_tile(_p(x), _p(w), _p(y), M, N, K, int(slices), int(partial), int(shape), _stream()))
+    return y
+
+
+TALL_SHAPES = {96: 4, 128: 0, 160: 5, 224: 6}         # rows of a tile of 256 features, by `shape` of xi_linear_tile
+TALL_K = 16384            # least K of a product that goes in the lowest tiles that are one round
+
+
+def tall_tile_rows(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
+    """The rows of a tile in which x [M, K] @ w [N, K]^T goes to `linear_tall`, None: not there.  The lowest of `TALL_SHAPES` whose
+    tiles of 256 features are one round of the compute units.  For K of 16,384 and more and N above 4,608, where the library has
+    kernels at half the matrix cores' rate beside its good ones.  Measured on MI355X, us, library / this kernel:
+      N=5120 K=17408, rows 1025 271/209, 1280 294/220, 1536 352/224, 1727 475/252 (160 rows a tile), 2400 544/364 (224), 2688 596/375;
+      K=25600: 1025 412/311, 1536 509/332, 1727 682/395, 2400 774/575, 2688 830/594; N=6144 K=20480: 1025 394/236, 1280 421/266,
+      1400 303/311, 1600 307/325.
+    Not there: 1,761 to 2,304 rows (K=17408: 1790 251/266, 2048 276/365) and more than 2,688 (3072 359/414); K=13824 (1100 152/162,
+    1600 200/210); N=4096 K=16384 (1100 165/181, 1536 181/198).  Up to 1,024 rows `tile_split_plan`'s slices are ahead."""
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        return None
+    M, K, N = x.shape[0], x.shape[1], w.shape[0]
+    if K < TALL_K or N <= 4608 or not (1024 < M <= 1760 or 2304 < M <= 2688):
+        return None
+    for rows in TALL_SHAPES:
+        if -(-M // rows) * -(-N // 256) <= COMPUTE_UNITS:
+            break
+    else:
+        return None
+    if (rows == 224) != (M > 2304) or not (x.is_contiguous() and w.is_contiguous()) or x.data_ptr() % 16 or w.data_ptr() % 16 \
+            or not linear_tile_takes(M, N, K) or K * 512 >= 1 << 32:
+        return None
+    return rows
+
+
+def linear_tall(x: torch.Tensor, w: torch.Tensor, rows: int) -> torch.Tensor:
+    """bfloat16 x [M, K] @ w [N, K]^T, [M, N] bfloat16, in the many-row tiled kernel's tiles of `rows` (`TALL_SHAPES`) by 256; the
+    value of an element does not depend on `rows`."""
+    _dev(x, w)
+    _want(x, torch.bfloat16, "linear_tall: x")
+    _want(w, torch.bfloat16, "linear_tall: w")
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or rows not in TALL_SHAPES:
+        raise KernelError(f"linear_tall: x {tuple(x.shape)} and w {tuple(w.shape)} in tiles of {rows} rows do not go together")
+    M, K = x.shape
+    N = w.shape[0]
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _ok(lib().xi_linear_tile(_p(x), _p(w), _p(y), M, N, K, 1, 0, TALL_SHAPES[rows], _stream()))
     return y
 
 
@@ -1990,7 +2035,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     """bfloat16 x @ w.T with float32 accumulation, rounded once to `out_dtype` (bfloat16 or
     float32).  Up to `skinny_rows` rows (decode): the hand-written streaming kernel, which with
     `allow_split` may answer with float32 partial sums [slices, M, N] for a narrow output.  More
-    rows: the vendor library (hipBLASLt through torch), which the reference's engine also
+    rows: where K is long and the output narrow `linear_tall`, else the vendor library (hipBLASLt through torch), which the reference's engine also
     uses for its matrix products."""
     _dev(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
@@ -2017,6 +2062,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
         return linear_skinny(x, w, out_dtype, allow_split=allow_split)
     if out_dtype == torch.float32:
         return torch.mm(x, w.t(), out_dtype=torch.float32)
+    rows = tall_tile_rows(x, w)
+    if rows is not None:
+        return linear_tall(x, w, rows)
     return torch.nn.functional.linear(x, w)
 
 

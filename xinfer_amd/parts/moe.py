@@ -167,8 +167,7 @@ class RoutedExperts(FeedForward):
         # bfloat16 in sizes of 64: the tiled products, for single tokens as for portions; other sizes go to the vendor library,
         # expert by expert, where a step of portions (which is never recorded: the experts' row counts are read on the host)
         # brings many rows an expert, and to the grouped form or a pair at a time otherwise
-        if x.dtype == torch.bfloat16 and kernels.MOE_TILED and kernels.moe_tiled_takes(T, self.top, self.experts, self.hidden,
-                                                                                     self.inter, self.gated):
+        if x.dtype == torch.bfloat16 and kernels.moe_tiled_takes(T, self.top, self.experts, self.hidden, self.inter, self.gated):
             out = kernels.moe_experts_tiled(x, self.gate_up, self.down, idx, wt, self.activation, **kw)
         elif (ctx.max_q_len > 1 and x.dtype == torch.bfloat16 and self.LIBRARY
                 and T * self.top >= kernels.MOE_LIBRARY_ROWS * self.experts):
