@@ -42,7 +42,7 @@ class _Rows:
 @pytest.mark.parametrize("M,F,K,shape", [
     (64, 3072, 1024, None), (65, 3072, 1024, 0), (320, 3072, 1024, 0), (321, 3072, 1024, 1), (1280, 3072, 1024, 1),
     (1281, 3072, 1024, 2), (128, 8192, 2048, 0), (129, 8192, 2048, None), (512, 8192, 2048, 1), (513, 8192, 2048, None),
-    (897, 8192, 2048, 2), (4096, 12288, 4096, None), (512, 17408, 5120, None), (513, 17408, 5120, None),
+    (897, 8192, 2048, 2), (4096, 12288, 4096, None), (511, 17408, 5120, None), (512, 17408, 5120, 2), (513, 17408, 5120, None),
     (700, 17408, 5120, 2), (2048, 25600, 5120, 2), (2049, 25600, 5120, 2), (256, 3074, 1024, None), (256, 3072, 1000, None)])
 def test_gated_tile_rule(M, F, K, shape):
     """Where the tiled product is taken, and never an operand that it does not take."""

@@ -28,7 +28,7 @@
 //
 // Measured on MI355X (random operands, the clock under load about 1.8 GHz): 2,048 rows by
 // N = 4096, K = 12288 in 172 us (1.2 PFLOP/s; the library 174), K = 4096 in 68 us (the library 64);
-// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 102 us (1.35; the library 94); the matrix cores are
+// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 102 us (1.35; the library 92); the matrix cores are
 // busy 63% of the time, LDS serves the tiles' 48 to 64 KB of writes and 128 to 192 KB of reads a
 // tile and is what the kernel waits for (without the barrier or without the wait for the loads it
 // is no faster).  Where it is ahead of the library is the narrow output at few rows, whose tiles
@@ -126,9 +126,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
 // writes half, and their two launches): w [2 N, K] = [gate; up], y bfloat16 [M, N] = act(gate) * up of the
 // float32 sums, one rounding.  A workgroup owns BM rows of x and BN / 2 features; a wave's rows of w are gate rows and the up
 // rows of the same features (as in moe_tile.hip).  Bound by the walk, as above, and by how evenly the tiles fill rounds of 256
-// workgroups; measured at N=17408, K=5120 against the library and the activation's pass: 1,024 rows 313 us (1.17 PFLOP/s) / 411,
-// 2,048 rows 583 / 626; at N=3072, K=1024: 256 rows in tiles of 64 by 64 9.5 / 16.9, 1,024 in 128 by 128 19.0 / 23.1, 2,048 in
-// 256 by 128 28.7 / 35.2.
+// workgroups; measured at N=17408, K=5120 against the library and the activation's pass: 1,024 rows 301 us (1.21 PFLOP/s) / 408,
+// 2,048 rows 563 / 619; at N=3072, K=1024: 256 rows in tiles of 64 by 64 9.3 / 16.9, 1,024 in 128 by 128 17.3 / 22.8, 2,048 in
+// 256 by 128 27.5 / 35.2.
 template <int BM, int BN, int S, int ACT>
 __device__ __forceinline__ void gated_tile(const bf16* x, const bf16* w, bf16* y, int M, int N, int K, int m0, int f0, unsigned char* smem) {
   constexpr int WGM = 2, WGN = 4;
@@ -183,7 +183,8 @@ __global__ __launch_bounds__(512, 1) void gated_tile_kernel(const bf16* __restri
 
 // Tiles of 256 rows by 128 features, of which the last ones, a round of workgroups that would leave half of the compute units or
 // more idle, are cut into `parts` (2: halves of the rows; 4: and of the features).  `whole`: the tiles in front of those.
-// N=17408, K=5120, 2,048 rows (4.25 rounds): 665 us uncut, 583 cut; N=25600 (6.25 rounds): 962 and 846.
+// N=17408, K=5120, 2,048 rows (4.25 rounds): 665 us uncut, 583 cut (563 with the walk as it is now); N=25600 (6.25 rounds): 962
+// and 846 (819).
 template <int ACT>
 __global__ __launch_bounds__(512, 1) void gated_tile_rest_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                  bf16* __restrict__ y, int M, int N, int K, int tiles_m, int whole,

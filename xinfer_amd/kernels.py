@@ -1802,15 +1802,16 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     """The tile shape in which act(x @ gate^T) * (x @ up^T) goes to `linear_gated_tile`, None: the library's product and a
     kernel for the activation (which also stay for operands that the tiled kernel does not take).  Measured on MI355X
     against those two, x M rows, w [2 F, K], us:
-      K <= 2048 (K <= 1024 in brackets): the smallest tile whose workgroups are one round of the 256 compute units (for 128
-      rows from half a round on, for 256 rows from 7/8 on [any]), and 256 rows beyond a round.  F=3072 K=1024: M=65 8.7 against 12.1,
-      256 9.5 / 16.9, 320 15.5 / 18.0, 512 17.5 / 19.1, 1024 19.0 / 23.1, 1500 28.0 / 37.0, 2048 28.7 / 35.2, 4096 48.8 / 63.4;
-      F=6144 K=2048: 128 18.2 / 21.5, 512 33.1 / 35.3, 1400 75 / 94, 2048 93 / 104, 4096 175 / 174; F=8192 K=2048: 128 19.9 / 23.5,
-      512 34.9 / 40.5, 1024 58 / 64, 2048 112 / 117.  What those rules leave out is level or behind (F=6144 M=700 53 / 44).
-      2048 < K <= 4096: the library's best sizes (F=12288 K=4096: 700 137 / 151, 900 187 / 158, 2048 313 / 303, 4096 662 / 608).
-      K > 4096, more than 512 rows of which four fifths of the last row of tiles' are there: F=17408 K=5120: 700 262 / 271,
-      1024 313 / 411, 1500 449 / 537, 2048 583 / 626, 4096 1160 / 1275; F=25600 K=5120: 700 353 / 408, 1024 447 / 516,
-      1727 757 / 883, 2048 846 / 891, 4096 1692 / 1766; left out: 513 329 / 290, 770 422 / 370."""
+      K <= 2048: the smallest tile whose workgroups are one round of the 256 compute units (K > 1024: for 128 rows from half a
+      round on, for 256 rows from 7/8 on), and 256 rows beyond a round.  F=3072 K=1024: M=65 8.7 against 12.1, 256 9.3 / 16.9,
+      384 15.7 / 17.8, 512 15.9 / 19.1, 1024 17.3 / 22.8, 1500 26.4 / 36.8, 2048 27.5 / 35.2, 4096 47.3 / 63.3; F=8192 K=2048: 128
+      19.7 / 23.3, 512 34.4 / 40.5, 1024 56.5 / 64.0, 2048 112 / 118, 4096 219 / 229.  What is left out is level or behind (M=256
+      32.8 / 33.1, 700 52.5 / 51.4; F=6144 K=2048 M=700 53 / 44).
+      2048 < K <= 4096: not taken, the library's best sizes (F=12288 K=4096: M=512 103 / 91, 700 135 / 150, 900 173 / 165,
+      2048 301 / 298, 4096 625 / 595).
+      K > 4096, 512 rows and more of which four fifths of the last row of tiles' are there: F=17408 K=5120: 512 184 / 193, 700
+      254 / 275, 1024 301 / 408, 1500 433 / 531, 2048 563 / 619, 4096 1098 / 1265; F=25600 K=5120: 512 262 / 287, 700 345 / 402,
+      1024 434 / 511, 1727 731 / 877, 2048 819 / 885, 4096 1609 / 1756; left out: 384 182 / 173 and 257 / 208, 770 422 / 370."""
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] \
             or w.shape[0] % 2 or x.shape[0] <= MID_GATED_UP_TO:
         return None
@@ -1818,7 +1819,7 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     tiles = lambda rows, features: -(-M // rows) * -(-F // features)
     shape = None
     if K > 4096:
-        shape = 2 if M > 512 and 5 * M >= 4 * 256 * -(-M // 256) else None
+        shape = 2 if M >= 512 and 5 * M >= 4 * 256 * -(-M // 256) else None
     elif K <= 2048:
         if tiles(64, 64) <= COMPUTE_UNITS:
             shape = 0
