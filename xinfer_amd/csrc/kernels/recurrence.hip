@@ -24,7 +24,7 @@
 //
 // `linear_scan_kernel`: one workgroup per (item, head, 64 value columns) walks the item's tokens in order,
 // from a state it is told to start from, and may leave the new state somewhere.  Lane l owns value column l
-// of the tile, wave w the key channels w RPT .. (w + 1) RPT - 1 (read from LDS four at a time; channels past
+// of the tile (or columns l and l + 64), wave w the key channels w RPT .. (w + 1) RPT - 1 (read from LDS four at a time; channels past
 // the head's are zeros there, so the inner loop has no bounds); a thread keeps its RPT state elements in
 // registers for the whole walk.  A token costs one barrier: q, k and the decay of the next token are fetched while this
 // one is worked on.  An item is a request's tokens of this step (from the state in its slot, back into it:
@@ -58,7 +58,10 @@ __device__ __forceinline__ float decay_of(float z, float inv_tau) {
 // ONE: a token's decay is one number for all of a head's channels (a constant per head, or from a step size): every
 // thread makes it itself and keeps it in a register, and the decays' row in LDS is neither written nor read.
 // ACT: q, k and v pass silu.
-template <typename T, int RPT, bool ONE, bool ACT>
+// COLS: value columns a lane owns, 64 apart.  A token's operands are the same numbers in all lanes, read from LDS by every wave,
+// and these reads bound a walk with many workgroups: two columns a lane read them once for both.
+// RES: there are results; without them q is neither fetched nor multiplied.
+template <typename T, int RPT, bool ONE, bool ACT, int COLS, bool RES>
 __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     const T* __restrict__ q, long long q_stride, const T* __restrict__ k, long long k_stride, const T* __restrict__ v,
     long long v_stride, const float* __restrict__ z, const float* __restrict__ z_bias, float inv_tau,
@@ -69,22 +72,26 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     const int* __restrict__ first, const int* __restrict__ last, float* __restrict__ out, float* __restrict__ decay_out,
     int H, int dk, int dv, float q_scale, float k_scale) {
   __shared__ __attribute__((aligned(16))) float qs[2][kScanWaves * 64], ks[2][kScanWaves * 64], as[2][kScanWaves * 64];
-  __shared__ float part[2][kScanWaves][kScanCols];
+  __shared__ float part[2][kScanWaves][COLS * kScanCols];
   __shared__ float npart[2][kScanWaves];
-  const int b = blockIdx.x, h = blockIdx.y, j = blockIdx.z * kScanCols + (threadIdx.x & 63);
+  const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * (COLS * kScanCols) + (threadIdx.x & 63);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t0 = first[b], t1 = last[b];
   if (t1 <= t0) return;
   const bool ones = v_cols < dv;            // the state's last column is the keys' own sum
-  const bool col = j < v_cols;
+  bool col[COLS];
+#pragma unroll
+  for (int e = 0; e < COLS; ++e) col[e] = j0 + kScanCols * e < v_cols;
   const long long from = in_idx ? in_idx[b] : -1, to = out_idx ? out_idx[b] : -1;      // negative: from zeros / kept nowhere
   const float* S = state_in + (size_t)(from < 0 ? 0 : from) * in_stride + (size_t)h * dk * dv;
-  float s[RPT];
+  float s[COLS][RPT];
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int i = wave * RPT + r;
-    s[r] = (from >= 0 && col && i < dk) ? S[(size_t)i * dv + j] : 0.f;
-  }
+  for (int e = 0; e < COLS; ++e)
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const int i = wave * RPT + r;
+      s[e][r] = (from >= 0 && col[e] && i < dk) ? S[(size_t)i * dv + j0 + kScanCols * e] : 0.f;
+    }
   float all_decays = 1.f;               // of channel c, over the item's tokens
   const int c = threadIdx.x;            // the channel this thread fetches for the workgroup
   float nc = (ones && from >= 0 && c < dk) ? S[(size_t)c * dv + v_cols] : 0.f;
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
   };
   auto fetch = [&](int t, float dt, float& fq, float& fk, float& fa) {      // (channels past the head's stay zero)
     if (c < dk) {
-      fq = read(q[(size_t)t * q_stride + qk0 + c]) * q_scale;
+      if (RES) fq = read(q[(size_t)t * q_stride + qk0 + c]) * q_scale;
       fk = read(k[(size_t)t * k_stride + qk0 + c]) * k_scale;
       if (!ONE) fa = decay_of(z[((size_t)t * H + h) * dk + c] + zb, inv_tau);
     }
@@ -116,9 +123,11 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
   fetch(t0, dt, fq, fk, fa);
   // the token's value is asked for a token ahead as well: no step of the walk waits for memory
   // (a column past the value rows' own reads 1)
-  auto value_of = [&](int t) { return j < v_cols ? read(v[(size_t)t * v_stride + h * v_cols + j]) : 1.f; };
-  float v_next = col ? value_of(t0) * dt : 0.f;
-  qs[0][c] = fq;
+  auto value_of = [&](int t, int j) { return j < v_cols ? read(v[(size_t)t * v_stride + h * v_cols + j]) : 1.f; };
+  float v_next[COLS];
+#pragma unroll
+  for (int e = 0; e < COLS; ++e) v_next[e] = col[e] ? value_of(t0, j0 + kScanCols * e) * dt : 0.f;
+  if (RES) qs[0][c] = fq;
   ks[0][c] = fk;
   if (!ONE) as[0][c] = fa;
   __syncthreads();
@@ -126,53 +135,72 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     const int cur = (t - t0) & 1;
     all_decays *= fa;
     const float a_now = fa;
-    const float vj = v_next;
+    float vj[COLS];
+#pragma unroll
+    for (int e = 0; e < COLS; ++e) vj[e] = v_next[e];
     if (ones) {                          // (this token's k and q are in LDS since the last barrier)
       nc = fmaf(a_now, nc, dt * ks[cur][c]);
-      const float nq = wave_sum(nc * qs[cur][c]);
-      if (out && lane == 0) npart[cur][wave] = nq;
+      if (RES) {
+        const float nq = wave_sum(nc * qs[cur][c]);
+        if (lane == 0) npart[cur][wave] = nq;
+      }
     }
     if (t + 1 < t1) {
       dt = step_of(t + 1);
       fetch(t + 1, dt, fq, fk, fa);
-      if (col) v_next = value_of(t + 1) * dt;
+#pragma unroll
+      for (int e = 0; e < COLS; ++e)
+        if (col[e]) v_next[e] = value_of(t + 1, j0 + kScanCols * e) * dt;
     }
-    float acc = 0.f;
+    float acc[COLS] = {};
     const float4* a4 = reinterpret_cast<const float4*>(&as[cur][wave * RPT]);
     const float4* k4 = reinterpret_cast<const float4*>(&ks[cur][wave * RPT]);
     const float4* q4 = reinterpret_cast<const float4*>(&qs[cur][wave * RPT]);
 #pragma unroll
     for (int r = 0; r < RPT; r += 4) {
       const float4 av = ONE ? make_float4(a_now, a_now, a_now, a_now) : a4[r / 4];
-      const float4 kv = k4[r / 4], qv = q4[r / 4];
-      s[r] = fmaf(av.x, s[r], kv.x * vj);
-      s[r + 1] = fmaf(av.y, s[r + 1], kv.y * vj);
-      s[r + 2] = fmaf(av.z, s[r + 2], kv.z * vj);
-      s[r + 3] = fmaf(av.w, s[r + 3], kv.w * vj);
-      acc = fmaf(s[r], qv.x, acc);
-      acc = fmaf(s[r + 1], qv.y, acc);
-      acc = fmaf(s[r + 2], qv.z, acc);
-      acc = fmaf(s[r + 3], qv.w, acc);
+      const float4 kv = k4[r / 4], qv = RES ? q4[r / 4] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) {
+        s[e][r] = fmaf(av.x, s[e][r], kv.x * vj[e]);
+        s[e][r + 1] = fmaf(av.y, s[e][r + 1], kv.y * vj[e]);
+        s[e][r + 2] = fmaf(av.z, s[e][r + 2], kv.z * vj[e]);
+        s[e][r + 3] = fmaf(av.w, s[e][r + 3], kv.w * vj[e]);
+        if (RES) {
+          acc[e] = fmaf(s[e][r], qv.x, acc[e]);
+          acc[e] = fmaf(s[e][r + 1], qv.y, acc[e]);
+          acc[e] = fmaf(s[e][r + 2], qv.z, acc[e]);
+          acc[e] = fmaf(s[e][r + 3], qv.w, acc[e]);
+        }
+      }
     }
-    if (out) part[cur][wave][lane] = acc;
+    if (RES) {
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) part[cur][wave][lane + kScanCols * e] = acc[e];
+    }
     if (t + 1 < t1) {
-      qs[cur ^ 1][c] = fq;
+      if (RES) qs[cur ^ 1][c] = fq;
       ks[cur ^ 1][c] = fk;
       if (!ONE) as[cur ^ 1][c] = fa;
     }
     __syncthreads();
-    if (out && wave == 0 && col)
-      out[((size_t)t * H + h) * dv + j] = (part[cur][0][lane] + part[cur][1][lane]) + (part[cur][2][lane] + part[cur][3][lane]);
-    if (out && ones && blockIdx.z == 0 && threadIdx.x == 0)
+    if (RES && wave < COLS) {
+      const int at = lane + kScanCols * wave, j = j0 + kScanCols * wave;
+      if (j < v_cols)
+        out[((size_t)t * H + h) * dv + j] = (part[cur][0][at] + part[cur][1][at]) + (part[cur][2][at] + part[cur][3][at]);
+    }
+    if (RES && ones && blockIdx.z == 0 && threadIdx.x == 0)
       out[((size_t)t * H + h) * dv + v_cols] = (npart[cur][0] + npart[cur][1]) + (npart[cur][2] + npart[cur][3]);
   }
   if (to >= 0) {
     float* D = state_out + (size_t)to * out_stride + (size_t)h * dk * dv;
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int i = wave * RPT + r;
-      if (col && i < dk) D[(size_t)i * dv + j] = s[r];
-    }
+    for (int e = 0; e < COLS; ++e)
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        const int i = wave * RPT + r;
+        if (col[e] && i < dk) D[(size_t)i * dv + j0 + kScanCols * e] = s[e][r];
+      }
     if (ones && blockIdx.z == 0 && c < dk) D[(size_t)c * dv + v_cols] = nc;
   }
   if (decay_out && blockIdx.z == 0 && c < dk) decay_out[((size_t)b * H + h) * dk + c] = all_decays;
@@ -324,19 +352,32 @@ int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k
   XI_CHECK(act == 0 || (act == 1 && z == nullptr), "linear_scan: activation %d (silu comes with one decay a head and token)", act);
   XI_CHECK(first && last, "linear_scan: the items' token ranges are missing");
   if (n_items == 0) return 0;
-  dim3 grid((unsigned)n_items, (unsigned)H, (unsigned)((v_cols + kScanCols - 1) / kScanCols));
+  const int rpt = (dk + kScanWaves - 1) / kScanWaves;
+  // two columns a lane for chunks (which never walk from and to the same states) where that still leaves two rounds of workgroups:
+  // 8 heads of 128 by 256 over 2,048 tokens, all three launches, 344 us with one column and 229 with two and no results in the first
+  // (z); half a round either way 184 / 173.  A walk in one piece is bound by its states' bytes (200 single tokens 83 / 85).
+  const bool two = state_in != state_out && rpt <= 32 && v_cols > kScanCols &&
+                   (long long)n_items * H * ((v_cols + 2 * kScanCols - 1) / (2 * kScanCols)) >= 2 * 256;
+  const int cols = two ? 2 * kScanCols : kScanCols;
+  dim3 grid((unsigned)n_items, (unsigned)H, (unsigned)((v_cols + cols - 1) / cols));
   XI_CHECK(grid.y <= 65535u && grid.z <= 65535u, "linear_scan: too many heads or value columns");
   const float inv_tau = z ? 1.f / tau : 0.f;
-  const int rpt = (dk + kScanWaves - 1) / kScanWaves;
 #define XI_SCAN_ARGS(TT)                                                                                                      \
       (const TT*)q, q_stride, (const TT*)k, k_stride, (const TT*)v, v_stride, z, z_bias, inv_tau, head_decay, (const TT*)step,    \
       step_stride, step_bias, decay_log, gates, v_cols, group_heads, state_in, in_stride,                                                    \
       in_idx, state_out, out_stride, out_idx, first, last, out, decay_out, H, dk, dv, q_scale, k_scale
-#define XI_SCAN(TT, R)                                                                                                        \
+#define XI_SCAN_F(TT, R, COLS, RES)                                                                                           \
   do {                                                                                                                        \
-    if (z) linear_scan_kernel<TT, R, false, false><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));                \
-    else if (act) linear_scan_kernel<TT, R, true, true><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));           \
-    else linear_scan_kernel<TT, R, true, false><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));                   \
+    if (z) linear_scan_kernel<TT, R, false, false, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));     \
+    else if (act) linear_scan_kernel<TT, R, true, true, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT)); \
+    else linear_scan_kernel<TT, R, true, false, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));        \
+  } while (0)
+#define XI_SCAN(TT, R)                          \
+  do {                                          \
+    if (two && out) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), true);  \
+    else if (two) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), false);   \
+    else if (out) XI_SCAN_F(TT, R, 1, true);    \
+    else XI_SCAN_F(TT, R, 1, false);            \
   } while (0)
 #define XI_SCAN_T(TT)            \
   do {                           \
@@ -350,6 +391,7 @@ int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k
   else XI_CHECK(false, "linear_scan: unknown dtype %d", dtype);
 #undef XI_SCAN_T
 #undef XI_SCAN
+#undef XI_SCAN_F
 #undef XI_SCAN_ARGS
   XI_LAUNCH_CHECK("linear_scan");
   return 0;
