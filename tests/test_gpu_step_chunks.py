@@ -14,7 +14,8 @@ def _plain(q, k, v, raw, bias, rate_log, S, group_heads, q_scale, k_scale):
     dk = S.shape[1]
     q, k = ((t.double().view(T, -1, dk) * s).repeat_interleave(group_heads, dim=1) for t, s in ((q, q_scale), (k, k_scale)))
     v = v.double().view(T, H, -1)
-    d = torch.nn.functional.softplus(raw.double() + bias.double(), threshold=1e9)
+    x = raw.double() + bias.double()
+    d = torch.logaddexp(x, torch.zeros_like(x))
     a = torch.exp(-torch.exp(rate_log.double()) * d)
     S = S.double().clone()
     out = []
@@ -67,6 +68,42 @@ def test_portions_of_unequal_requests(H, G, dk, dv, rate, monkeypatch):
     # three bfloat16 hold a float32 to 2^-24 of it, and both forms round float32 sums of at most 64 + dk terms
     for w, c in zip(errors[False], errors[True]):
         assert c < max(1.2 * w, 5e-7)
+
+
+def _portion(seed, T, H, dk, dv, device=DEV):
+    """One request's operands (one group) as `_plain` takes them, and as `linear_scan` does."""
+    g = torch.Generator().manual_seed(seed)
+    rb = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    q, k, v, raw = rb(T, dk), rb(T, dk), rb(T, H * dv), rb(T, H)
+    bias, rate_log = torch.randn(H, generator=g) - 1.0, torch.randn(H, generator=g) * 0.5 - 1.0
+    return q, k, v, raw, bias, rate_log, torch.randn(1, H, dk, dv, generator=g)
+
+
+def _walk(monkeypatch, matrix, q, k, v, raw, bias, rate_log, state):
+    from xinfer_amd import kernels
+    monkeypatch.setattr(kernels, "STEP_MFMA", matrix)
+    T, (_, H, dk, dv) = q.shape[0], state.shape
+    st = state.to(DEV)
+    o = kernels.linear_scan(q.to(DEV), k.to(DEV), v.to(DEV), st, torch.zeros(1, dtype=torch.int64, device=DEV),
+                            torch.tensor([0, T], dtype=torch.int32, device=DEV), H, dk, dv, step=raw.to(DEV), step_bias=bias.to(DEV),
+                            decay_log=rate_log.to(DEV), groups=1, q_lens=[T])
+    return o.cpu(), st[0].cpu()
+
+
+@pytest.mark.parametrize("at", [0, 41, 63, 64])
+@pytest.mark.parametrize("size", [3e4, 1e9, 1e20])
+def test_a_token_that_forgets_everything(at, size, monkeypatch):
+    """A step size that leaves nothing of the state: the decays of the tokens behind it keep their digits."""
+    x = _portion(int(size) % 1000 + at, 150, 3, 64, 64)
+    x[3][at, 1] = size
+    ref, state = _plain(*x[:6], x[6][0], 3, 1.0, 1.0)
+    size, state_size = _plain(x[0].abs(), x[1].abs(), x[2].abs(), *x[3:6], x[6][0].abs(), 3, 1.0, 1.0)       # of the terms, all added up
+    # dk + 64 roundings of sums of the terms, and the decays' exponents in float32, up to 2^5 where what they scale still counts
+    bound = (64 + 64 + 32) * 2.0 ** -24
+    for matrix in (False, True):
+        o, st = _walk(monkeypatch, matrix, *x)
+        assert float(((o.double() - ref).abs() / size).max()) < bound, matrix
+        assert float(((st.double() - state).abs() / state_size).max()) < bound, matrix
 
 
 def test_the_rule_takes_what_it_should(monkeypatch):

@@ -141,7 +141,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
     const float x = nraw + bias;
     const float d = there ? fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))) : 0.f;
     const float la = rate * d;
-    double L = there ? (double)(la < -1e30f ? -1e30f : la) * 1.4426950408889634 : 0.0;      // base 2 from here on
+    // (e^-10000 is 0 in float32: a token that forgets everything still does, and the sums keep the later tokens' digits)
+    double L = there ? (double)(la < -1e4f ? -1e4f : la) * 1.4426950408889634 : 0.0;      // base 2 from here on
 #pragma unroll
     for (int off = 1; off < kTok; off <<= 1) {
       const double up = __shfl_up(L, off, kWave);
