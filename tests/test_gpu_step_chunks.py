@@ -106,6 +106,35 @@ def test_a_token_that_forgets_everything(at, size, monkeypatch):
         assert float(((st.double() - state).abs() / state_size).max()) < bound, matrix
 
 
+INF, NAN = float("inf"), float("nan")
+
+
+@pytest.mark.parametrize("what,values", [("v", (INF, NAN, 1e34, -1e30)), ("k", (INF, NAN, 1e34)), ("q", (-INF, NAN, 1e36)),
+                                         ("raw", (INF, NAN, 1e34, -INF)), ("state", (INF, NAN, 3.395e38))])
+@pytest.mark.parametrize("dk,dv,at", [(64, 64, 41), (128, 32, 64), (32, 32, 127), (96, 32, 0)])
+def test_values_without_a_bound(what, values, dk, dv, at, monkeypatch):
+    """An infinite, undefined or very large value in the operands: the same results are finite, infinite and undefined as where the
+    walk goes token by token, none of them in front of the value, and the finite ones agree."""
+    T, H = 150, 2
+    for value in values:
+        x = _portion(at + dk, T, H, dk, dv)
+        if what == "state":
+            x[6][0, 1, 3, 5] = value
+        else:
+            x[("q", "k", "v", "raw").index(what)][at, 1] = value
+        (wo, ws), (co, cs) = _walk(monkeypatch, False, *x), _walk(monkeypatch, True, *x)
+        before = 0 if what == "state" else at
+        assert bool(co[:before].isfinite().all()), value
+        for w, c in ((wo, co), (ws, cs)):
+            assert torch.equal(w.isnan(), c.isnan()) and torch.equal(w.isinf(), c.isinf()), value
+            assert torch.equal(w[w.isinf()], c[w.isinf()]), value
+            fine = w.isfinite()
+            # two float32 sums of dk + 64 terms in different orders; a sum in front of which a large term has decayed again
+            # keeps that term's rounding, so the error is taken against the largest of the column's finite values
+            most = torch.where(fine, w, 0.0).abs().amax(dim=0, keepdim=True)
+            assert float(torch.where(fine, (w - c).abs() / most.clamp(min=1.0), torch.zeros(())).max()) < (dk + 64) * 2.0 ** -23, value
+
+
 def test_the_rule_takes_what_it_should(monkeypatch):
     """Which portions go where, without a launch."""
     from xinfer_amd import kernels

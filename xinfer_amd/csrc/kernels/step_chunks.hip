@@ -17,11 +17,16 @@
 // between them.  Relative error of the results against 64 bits over portions of 32 to 200 tokens: 1.6e-7 to 2.3e-7, the walk
 // 1.6e-7 to 9.8e-7 (tests/test_gpu_step_chunks.py).
 //
-// Measured on MI355X, us against the walk in three launches: 128 heads of 128 by 64 over 2,048 tokens 125 (1,180), over
-// 8,192 500 (4,560), 32 heads over 2,048 119 (338), three portions of 1,974 tokens together 175 (1,186); a portion of 32 tokens
-// of 32 heads 22 (44), which is why it starts there (STEP_FROM).  A chunk takes 3.9 us: three barriers, about 370 KB of operand
+// A chunk with an infinite or undefined operand, a step size of 2^33 and more, or scores, decayed values or a state's results of 2^64
+// and more is walked token by token instead (from the operands in LDS and the state in front of it): a masked score times a value
+// without a bound is undefined and would reach the tokens in front of that value, and so are three bfloat16 that add up to an
+// infinite number.  Below these sizes the chunk's numbers stay in float32's range wherever the walk's do.
+//
+// Measured on MI355X, us against the walk in three launches: 128 heads of 128 by 64 over 2,048 tokens 131 (1,051), over
+// 8,192 517 (4,016), 32 heads over 2,048 124 (289), three portions of 1,974 tokens together 181 (1,040); a portion of 32 tokens
+// of 32 heads 22 (43), which is why it starts there (STEP_FROM).  A chunk takes 4.0 us: three barriers, about 370 KB of operand
 // reads from LDS a workgroup and the vector instructions of the splits, with two waves a SIMD; its 38 matrix instructions a
-// wave are a sixth of it.
+// wave are a sixth of it, and looking for what has no bound 4% (as sums of absolute values; as comparisons 8%).
 #include "common.h"
 
 namespace xi {
@@ -73,6 +78,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
   __bf16* ss = ps + 3 * kTok * kRow;                         // [3][kCols][QR]: the state, a column a row
   double* Ls2 = reinterpret_cast<double*>(ss + 3 * kCols * QR);     // [2][kTok]: this chunk's and the next one's
   float* ds2 = reinterpret_cast<float*>(Ls2 + 2 * kTok);     // [2][kTok]
+  int* large = reinterpret_cast<int*>(ds2 + 2 * kTok);       // [2]: this chunk, the next one is walked token by token
+  float* part = reinterpret_cast<float*>(wt);                // [DK / 16][kTok][kCols], in the place of wt, ps and ss: the walk's results
   const int p = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * kCols;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, j = lane >> 4;
@@ -88,6 +95,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int i = 0; i < 4; ++i) st[b][i] = owns ? S[(size_t)(16 * wave + 4 * j + i) * A.dv + col0 + 16 * b + r] : 0.f;
+  if (tid < 2) large[tid] = 0;
+  __syncthreads();
   auto keep_state = [&] {
     if (!owns) return;
 #pragma unroll
@@ -107,10 +116,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
   };
   keep_state();
   // the tiles above the diagonal that are read beside one on it are zeros and stay so
-  for (int i = tid; i < 3 * kTok * 16; i += 64 * kWaves) {
-    const int row = (i >> 4) % kTok, at = row < 16 ? 16 : row >= 32 && row < 48 ? 48 : -1;
-    if (at >= 0) ps[(i >> 4) * kRow + at + (i & 15)] = (__bf16)0.f;
-  }
+  auto clear_above = [&] {
+    for (int i = tid; i < 3 * kTok * 16; i += 64 * kWaves) {
+      const int row = (i >> 4) % kTok, at = row < 16 ? 16 : row >= 32 && row < 48 ? 48 : -1;
+      if (at >= 0) ps[(i >> 4) * kRow + at + (i & 15)] = (__bf16)0.f;
+    }
+  };
+  clear_above();
   // what a thread brings of a chunk: q by rows; k and v a token a lane, so that their 2-byte stores by channel lie side by side
   typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
   u32x4 nq[KI], nk[KI], nv = {0u, 0u, 0u, 0u};
@@ -148,6 +160,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
       const double up = __shfl_up(L, off, kWave);
       if (lane >= off) L += up;
     }
+    if (there && !(x < 0x1p33f)) large[buf] = 1;
     Ls2[buf * kTok + lane] = L;                // (tokens past the chunk's end: the last one's)
     ds2[buf * kTok + lane] = d;
   };
@@ -186,12 +199,15 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
     if (t0 + kTok < t_end) ask(t0 + kTok);
     // ---- the decayed values, the scores with their decays, and what the state gives
     const double all = Ls[kTok - 1];
+    float sizes = 0.f;                         // of what this lane has seen of the chunk, added up: undefined if one of them is
     if (vwave >= 0) {
       const float w = pow2(all - Ls[lane]) * ds[lane] * A.k_scale;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         __bf16 x[3];
-        split3(w * (float)half(cv, e), x[0], x[1], x[2]);
+        const float wv = w * (float)half(cv, e);
+        sizes += fabsf(wv);                    // (a decay of 0 times a value without a bound is undefined)
+        split3(wv, x[0], x[1], x[2]);
 #pragma unroll
         for (int s = 0; s < 3; ++s) wt[(s * kCols + 8 * vwave + e) * kRow + lane] = x[s];
       }
@@ -205,6 +221,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
       for (int s = 0; s < DKS; ++s)
         sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ld8(ks + (16 * kt_ + r) * QR + 32 * s + 8 * j),
                                                      ld8(qs + (16 * qt_ + r) * QR + 32 * s + 8 * j), sc, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sizes += fabsf(sc[i]);       // (a q or k without a bound is in a score on the diagonal)
       const int qi = 16 * qt_ + r, k0 = 16 * kt_ + 4 * j;
       const double lq = Ls[qi];
       bf16x4 x[3];
@@ -235,8 +253,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
     }
     f32x4 o = (os[2] + os[1]) + os[0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] *= pow2(Ls[16 * rt + 4 * j + i]) * (A.scale / A.k_scale);
+    for (int i = 0; i < 4; ++i) {
+      sizes += fabsf(o[i]);                    // (so is what a state without a bound gives)
+      o[i] *= pow2(Ls[16 * rt + 4 * j + i]) * (A.scale / A.k_scale);
+    }
+    if (!(sizes < 0x1p64f)) large[buf] = 1;
     __syncthreads();
+    const int walk = large[buf];
     // ---- the results, and the state behind the chunk
 #pragma unroll
     for (int s = 0; s < kTok / 32; ++s) {
@@ -251,6 +274,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
       const int tok = 16 * rt + 4 * j + i;
       if (tok < n) A.out[((size_t)(t0 + tok) * A.H + h) * A.dv + col0 + 16 * ct + r] = o[i];
     }
+    const f32x4 front[2] = {st[0], st[1]};
     if (owns) {
       const float f = pow2(all);
 #pragma unroll
@@ -264,6 +288,46 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
           for (int x = 2; x >= 0; --x)
             st[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, ld8(wt + (x * kCols + 16 * b + r) * kRow + 32 * s + 8 * j), st[b], 0, 0, 0);
       }
+    }
+    if (walk) {
+      __syncthreads();
+      st[0] = front[0];
+      st[1] = front[1];
+      if (owns) {
+        const float q_scale = A.scale / A.k_scale;
+        for (int t = 0; t < n; ++t) {
+          const float d = ds[t], a = expf(rate * d);
+          float acc[2] = {0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int at = t * QR + 16 * wave + 4 * j + i;
+            const float kv = (float)ks[at] * A.k_scale, qv = (float)qs[at] * q_scale;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+              st[b][i] = fmaf(a, st[b][i], kv * ((float)vt[(16 * b + r) * kRow + t] * d));
+              acc[b] = fmaf(st[b][i], qv, acc[b]);
+            }
+          }
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            acc[b] += lane_xor<16>(acc[b]);
+            acc[b] += lane_xor<32>(acc[b]);
+            if (j == 0) part[(wave * kTok + t) * kCols + 16 * b + r] = acc[b];
+          }
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {            // (over what this thread has stored above)
+        const int tok = 16 * rt + 4 * j + i;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < DK / 16; ++w) sum += part[(w * kTok + tok) * kCols + 16 * ct + r];
+        if (tok < n) A.out[((size_t)(t0 + tok) * A.H + h) * A.dv + col0 + 16 * ct + r] = sum;
+      }
+      __syncthreads();
+      if (tid == 0) large[buf] = 0;
+      clear_above();
     }
     keep_state();
     __syncthreads();                           // (the next chunk overwrites k, v and the decayed values)
@@ -309,7 +373,7 @@ int xi_step_chunks(const void* q, long long q_stride, const void* k, long long k
   do {                                                                                                                       \
     const size_t qr = 32 * DKS + 8;                                                                                          \
     const size_t lds = 2 * (2 * step::kTok * qr + (32 * DKS + 4 * step::kCols + 3 * step::kTok) * step::kRow + 3 * step::kCols * qr) + \
-                       2 * step::kTok * 12;                                                                                   \
+                       2 * step::kTok * 12 + 8;                                                                               \
     const hipError_t e = hipFuncSetAttribute((const void*)step::step_chunks_kernel<DKS>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                              (int)lds);                                                                      \
     XI_CHECK(e == hipSuccess, "step_chunks: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));                    \
