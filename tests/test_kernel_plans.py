@@ -48,3 +48,16 @@ def test_decode_mixed_lengths_take_whole_sequences_where_there_are_many():
     assert kernels.decode_keys_per_workgroup(1536, 2048, False) == 2176
     assert kernels.decode_keys_per_workgroup(2048, 3072, False) == 2048
     assert kernels.decode_keys_per_workgroup(2048, 16384, False) == 2048
+
+
+def test_float32_attention_sets_one_limit_a_kernel():
+    """The dynamic LDS that the kernel of a class of head sizes is allowed: one number for the class, enough for all of it, so that
+    two engines with different heads do not lower it between each other's setting and launch."""
+    limit = kernels.lib().xi_attention_f32_lds
+    sizes = [(d, dv) for d in range(16, 257, 16) for dv in range(16, 257, 16)]
+    kinds = {}
+    for d, dv in sizes:
+        kinds.setdefault(next(m for m in (64, 128, 256) if max(d, dv) <= m), set()).add(limit(d, dv))
+        need = 4 * (8 * (16 * dv + 32) + 16 * (d + 4))          # eight waves' sums of 16 rows, their maxima and totals, the queries
+        assert need <= limit(d, dv) <= 160 * 1024
+    assert all(len(v) == 1 for v in kinds.values())

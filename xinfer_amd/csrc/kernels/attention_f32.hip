@@ -37,6 +37,9 @@ namespace attn_f32 {
 typedef __attribute__((ext_vector_type(4))) float f4;
 constexpr int kWaves = 8, kBlock = 16;
 
+// Bytes of LDS for `rows` (token, head) rows of heads of d and dv.
+constexpr size_t lds_bytes(int rows, int d, int dv) { return ((size_t)kWaves * (rows * dv + 2 * 16) + 16 * (d + 4)) * sizeof(float); }
+
 // DT: 16-dim tiles that the registers have room for (head sizes up to 16 DT)
 template <int DT>
 __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
@@ -256,6 +259,12 @@ int xi_attention_f32_takes(int nq, int nkv, int d, int dv) {
   return nkv > 0 && nq % nkv == 0 && d > 0 && d % 16 == 0 && d <= 256 && dv > 0 && dv % 16 == 0 && dv <= 256;
 }
 
+// The limit that is set on the dynamic LDS of the kernel for these head sizes: what its widest heads take.
+int xi_attention_f32_lds(int d, int dv) {
+  const int most = (d > dv ? d : dv) <= 64 ? 64 : (d > dv ? d : dv) <= 128 ? 128 : 256;
+  return (int)attn_f32::lds_bytes(16, most, most);
+}
+
 // The operands of `xi_attention_generic` in float32 with as many key heads as value heads; K and V rows of whole 16-byte pieces.
 // n_seqs: rows of block_tables.  Tiles of several tokens where the step brings several of a request on average; single tokens
 // have a workgroup each.
@@ -275,13 +284,13 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
   const int tile = (long long)n_seqs * 4 <= n_tok ? 16 / heads : 1;
   dim3 grid((unsigned)((n_tok + tile - 1) / tile), (unsigned)nkv, (unsigned)((nq / nkv + 15) / 16));
   XI_CHECK(grid.z <= 65535u, "attention_f32: too many heads (%d)", nq);
-  const size_t lds = ((size_t)attn_f32::kWaves * (tile * heads * dv + 2 * 16) + 16 * (d + 4)) * sizeof(float);
+  const size_t lds = attn_f32::lds_bytes(tile * heads, d, dv);
   const int most = d > dv ? d : dv;
 #define XI_AF(DT)                                                                                                             \
   do {                                                                                                                        \
-    if (lds > 65536) {                                                                                                        \
+    if (lds > 65536) {     /* always the most this kernel may want: another thread's launch may lie between */                \
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32::attention_f32_kernel<DT>),              \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                         \
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, xi_attention_f32_lds(d, dv));      \
       XI_CHECK(e == hipSuccess, "attention_f32: %s", hipGetErrorString(e));                                                   \
     }                                                                                                                         \
     attn_f32::attention_f32_kernel<DT><<<grid, 64 * attn_f32::kWaves, lds, stream>>>(                                         \
