@@ -43,7 +43,14 @@ class _Rows:
     (64, 3072, 1024, None), (65, 3072, 1024, 0), (320, 3072, 1024, 0), (321, 3072, 1024, 1), (1280, 3072, 1024, 1),
     (1281, 3072, 1024, 2), (128, 8192, 2048, 0), (129, 8192, 2048, None), (512, 8192, 2048, 1), (513, 8192, 2048, None),
     (897, 8192, 2048, 2), (4096, 12288, 4096, None), (511, 17408, 5120, None), (512, 17408, 5120, 2), (513, 17408, 5120, None),
-    (700, 17408, 5120, 2), (2048, 25600, 5120, 2), (2049, 25600, 5120, 2), (256, 3074, 1024, None), (256, 3072, 1000, None)])
+    (700, 17408, 5120, 2), (2048, 25600, 5120, 2), (2049, 25600, 5120, 2), (256, 3074, 1024, None), (256, 3072, 1000, None),
+    # too few workgroups: the library's smaller tiles fill the chip
+    (512, 64, 5120, None), (512, 1536, 5120, None), (2048, 2048, 7168, None), (4096, 64, 8192, None), (65, 64, 2048, None),
+    (128, 512, 2048, None), (128, 1024, 1088, None), (256, 768, 2048, 0), (65, 64, 1024, 0),
+    # the last round: cut, or too much of it, or the library's even rounds at other K
+    (1024, 10240, 4608, 2), (1024, 10304, 4608, None), (1024, 12288, 5120, None), (1024, 12288, 4608, None), (1230, 8192, 4160, 2),
+    (2048, 8192, 8192, None), (2048, 8192, 6144, None), (2048, 8192, 5120, 2), (2048, 17408, 6144, 2), (2048, 25600, 6144, None),
+    (640, 12288, 5120, None), (4096, 8192, 5120, None), (1024, 6144, 5120, None), (1280, 5120, 5120, 2)])
 def test_gated_tile_rule(M, F, K, shape):
     """Where the tiled product is taken, and never an operand that it does not take."""
     x, w = _Rows(M, K), _Rows(2 * F, K)

@@ -1802,16 +1802,24 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     """The tile shape in which act(x @ gate^T) * (x @ up^T) goes to `linear_gated_tile`, None: the library's product and a
     kernel for the activation (which also stay for operands that the tiled kernel does not take).  Measured on MI355X
     against those two, x M rows, w [2 F, K], us:
-      K <= 2048: the smallest tile whose workgroups are one round of the 256 compute units (K > 1024: for 128 rows from half a
-      round on, for 256 rows from 7/8 on), and 256 rows beyond a round.  F=3072 K=1024: M=65 8.7 against 12.1, 256 9.3 / 16.9,
-      384 15.7 / 17.8, 512 15.9 / 19.1, 1024 17.3 / 22.8, 1500 26.4 / 36.8, 2048 27.5 / 35.2, 4096 47.3 / 63.3; F=8192 K=2048: 128
-      19.7 / 23.3, 512 34.4 / 40.5, 1024 56.5 / 64.0, 2048 112 / 118, 4096 219 / 229.  What is left out is level or behind (M=256
-      32.8 / 33.1, 700 52.5 / 51.4; F=6144 K=2048 M=700 53 / 44).
-      2048 < K <= 4096: not taken, the library's best sizes (F=12288 K=4096: M=512 103 / 91, 700 135 / 150, 900 173 / 165,
-      2048 301 / 298, 4096 625 / 595).
-      K > 4096, 512 rows and more of which four fifths of the last row of tiles' are there: F=17408 K=5120: 512 184 / 193, 700
-      254 / 275, 1024 301 / 408, 1500 433 / 531, 2048 563 / 619, 4096 1098 / 1265; F=25600 K=5120: 512 262 / 287, 700 345 / 402,
-      1024 434 / 511, 1727 731 / 877, 2048 819 / 885, 4096 1609 / 1756; left out: 384 182 / 173 and 257 / 208, 770 422 / 370."""
+      K <= 2048: the smallest tile whose workgroups are one round of the 256 compute units (K > 1024: 48 workgroups at least, for
+      128 rows from half a round on, for 256 rows from 7/8 on), and 256 rows beyond a round.  F=3072 K=1024: M=65 8.7 against 12.1, 256
+      9.3 / 16.9, 384 15.7 / 17.8, 512 15.9 / 19.1, 1024 17.3 / 22.8, 1500 26.4 / 36.8, 2048 27.5 / 35.2, 4096 47.3 / 63.3; F=8192
+      K=2048: 128 19.7 / 23.3, 512 34.4 / 40.5, 1024 56.5 / 64.0, 2048 112 / 118, 4096 219 / 229; F=64 K=1024 M=65 8.6 / 8.9.  What is
+      left out is level or behind (M=256 32.8 / 33.1, 700 52.5 / 51.4; F=6144 K=2048 M=700 53 / 44; 2 to 32 workgroups of K=2048: F=64
+      M=65 12.1 / 9.1, M=1024 12.6 / 11.7, F=512 M=65 12.5 / 10.0, F=1024 M=128 13.2 / 12.5; 48: F=1536 M=65 13.2 / 13.1).
+      2048 < K <= 4096: not taken.  The library has its best sizes there (F=12288 K=4096: M=512 103 / 91, 900 173 / 165, 2048 301 / 298,
+      4096 625 / 595) and others (700 135 / 150, 1500 239 / 264, 3000 469 / 599), and no rule for them is built.
+      4096 < K <= 6144, 512 rows and more, 8/9 of the rows of the tiles there: up to four rounds of 256 workgroups and a rest of up to
+      64, which is cut (see the kernel) and for which the library has a whole round: K=4608 F=8192: 1230 155 / 163, F=10240: 1024 158
+      / 176, K=6144 F=17408: 2048 670 / 674; the median of 299 sizes 7% ahead, none behind.
+      K = 5120 besides, where the library's even rounds come to 1.17 PFLOP/s (1.28 to 1.35 at every other K measured from 4,160 to
+      8,192, in steps of 64 next to it; the tiles 1.20 to 1.25 at all of them): from 3/4 of a round on but for 65 to 143 workgroups
+      behind a first round, and for even rounds beyond three.  F=17408: 512 184 / 193, 700 254 / 275, 1024 301 / 408, 1500 433 / 531,
+      2048 563 / 619, 4096 1098 / 1265; F=25600: 512 262 / 287, 700 345 / 402, 1024 434 / 511, 1727 731 / 877, 2048 819 / 885, 4096 1609
+      / 1756; the median of 655 sizes 7% ahead, 7 behind by more than 2% (F=5504: 2500 248 / 234).
+      Left out: F=64 K=5120 M=512 87 / 17, F=1536 94 / 31, F=2048 K=7168 M=2048 162 / 107, F=12288 K=5120 M=1024 233 / 220, K=4608 M=1280 239 / 222,
+      F=8192 K=8192 M=4096 855 / 731, F=17408 K=5120 M=384 182 / 173, 770 422 / 370."""
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] \
             or w.shape[0] % 2 or x.shape[0] <= MID_GATED_UP_TO:
         return None
@@ -1819,10 +1827,14 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     tiles = lambda rows, features: -(-M // rows) * -(-F // features)
     shape = None
     if K > 4096:
-        shape = 2 if M >= 512 and 5 * M >= 4 * 256 * -(-M // 256) else None
+        full, rest = divmod(tiles(256, 128), COMPUTE_UNITS)
+        cut = 1 <= full <= 4 and 0 < 4 * rest <= COMPUTE_UNITS
+        if K == 5120 and not cut:
+            cut = (4 * rest > 3 * COMPUTE_UNITS if full == 0 else not 65 <= rest <= 143 if full == 1 else rest > 0 or full <= 3)
+        shape = 2 if cut and K <= 6144 and M >= 512 and 9 * M >= 8 * 256 * -(-M // 256) else None
     elif K <= 2048:
         if tiles(64, 64) <= COMPUTE_UNITS:
-            shape = 0
+            shape = 0 if K <= 1024 or tiles(64, 64) >= 48 else None
         elif tiles(128, 128) <= COMPUTE_UNITS:
             shape = 1 if K <= 1024 or 2 * tiles(128, 128) > COMPUTE_UNITS else None
         elif K <= 1024 or 8 * tiles(256, 128) >= 7 * COMPUTE_UNITS:
