@@ -78,7 +78,11 @@ def test_product_in_tall_tiles(M, N, K):
 @pytest.mark.parametrize("M,N,K,rows", [
     (1024, 5120, 17408, None), (1025, 5120, 17408, 96), (1152, 5120, 17408, 96), (1153, 5120, 25600, 128), (1536, 5120, 17408, 128),
     (1537, 5120, 17408, 160), (1760, 5120, 25600, 160), (1761, 5120, 17408, None), (2304, 5120, 17408, None), (2305, 5120, 17408, 224),
-    (2688, 5120, 17408, 224), (2689, 5120, 17408, None), (2400, 4612, 17408, 224), (2400, 4608, 17408, None), (1500, 8192, 28672, None), (1280, 8192, 28672, 160),
+    (2688, 5120, 17408, 224), (2689, 5120, 17408, None), (2400, 4868, 17408, 224), (2400, 4864, 17408, None), (1500, 8192, 28672, None),
+    # where the library is ahead or was not measured: other widths, and few rows at some K
+    (2400, 4612, 17408, None), (1280, 8192, 28672, None), (1400, 6144, 20480, None), (1600, 6144, 20480, None), (1600, 5124, 17408, None),
+    (1300, 5120, 16384, None), (1300, 5120, 16448, 128), (1300, 5120, 30720, 128), (1300, 5120, 30784, None), (1100, 5120, 18432, None), (1200, 5120, 18432, 128), (1100, 5120, 17920, 96),
+    (1100, 5120, 18944, 96),
     (1100, 4096, 16384, None), (1100, 5120, 16320, None), (1100, 5122, 17408, None), (1100, 5120, 17400, None)])
 def test_tall_tile_rule(M, N, K, rows):
     """Where the product is taken (never more than a round of 256 workgroups), and never an operand that it does not take."""

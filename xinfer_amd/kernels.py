@@ -1755,22 +1755,27 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
 
 
 TALL_SHAPES = {96: 4, 128: 0, 160: 5, 224: 6}         # rows of a tile of 256 features, by `shape` of xi_linear_tile
-TALL_K = 16384            # least K of a product that goes in the lowest tiles that are one round
+TALL_K = (16448, 30720)   # least and most K of a product that goes in the lowest tiles that are one round
 
 
 def tall_tile_rows(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     """The rows of a tile in which x [M, K] @ w [N, K]^T goes to `linear_tall`, None: not there.  The lowest of `TALL_SHAPES` whose
-    tiles of 256 features are one round of the compute units.  For K of 16,384 and more and N above 4,608, where the library has
-    kernels at half the matrix cores' rate beside its good ones.  Measured on MI355X, us, library / this kernel:
-      N=5120 K=17408, rows 1025 271/209, 1280 294/220, 1536 352/224, 1727 475/252 (160 rows a tile), 2400 544/364 (224), 2688 596/375;
-      K=25600: 1025 412/311, 1536 509/332, 1727 682/395, 2400 774/575, 2688 830/594; N=6144 K=20480: 1025 394/236, 1280 421/266,
-      1400 303/311, 1600 307/325.
+    tiles of 256 features are one round of the compute units.  For K of 16,448 to 30,720 and 20 tiles of features (N of 4,865
+    to 5,120), for which the library has kernels at half the matrix cores' rate beside its good ones.  Measured on MI355X, us,
+    library / this kernel: N=5120 K=17408, rows 1025 271/209, 1280 294/220, 1536 352/224, 1727 475/252 (160 rows a tile), 2400 544/364
+    (224), 2688 596/375; K=25600: 1025 412/311, 1536 509/332, 1727 682/395, 2400 774/575, 2688 830/594; N=4872 and 5000 within 6% of
+    these, 20 K from 16,448 to 30,720 all ahead (1.04 to 1.9 times) but for up to 1,152 rows at K of 18,176 to 18,688 (1025 194/225).
     Not there: 1,761 to 2,304 rows (K=17408: 1790 251/266, 2048 276/365) and more than 2,688 (3072 359/414); K=13824 (1100 152/162,
-    1600 200/210); N=4096 K=16384 (1100 165/181, 1536 181/198).  Up to 1,024 rows `tile_split_plan`'s slices are ahead."""
+    1600 200/210), K=16384 (1025 180/192, 1536 212/214, 1600 444/233); one tile of features less or more, where the library's good
+    kernels lie at other rows (N=4740 K=17408: 1600 226/233, 2400 309/367; N=5248: 2600 348/393; N=6144 K=20480: 1400 303/311, 1600
+    307/325; N=8192 K=28672: 1152 432/472).
+    Up to 1,024 rows `tile_split_plan`'s slices are ahead."""
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         return None
     M, K, N = x.shape[0], x.shape[1], w.shape[0]
-    if K < TALL_K or N <= 4608 or not (1024 < M <= 1760 or 2304 < M <= 2688):
+    if not TALL_K[0] <= K <= TALL_K[1] or not 4864 < N <= 5120 or not (1024 < M <= 1760 or 2304 < M <= 2688):
+        return None
+    if M <= 1152 and 17920 < K < 18944:
         return None
     for rows in TALL_SHAPES:
         if -(-M // rows) * -(-N // 256) <= COMPUTE_UNITS:
