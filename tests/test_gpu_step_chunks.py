@@ -135,6 +135,18 @@ def test_values_without_a_bound(what, values, dk, dv, at, monkeypatch):
             assert float(torch.where(fine, (w - c).abs() / most.clamp(min=1.0), torch.zeros(())).max()) < (dk + 64) * 2.0 ** -23, value
 
 
+def test_short_portions_bring_no_plan_to_the_device(monkeypatch):
+    """A step whose portions are all walked token by token copies nothing for the chunks' sake."""
+    from xinfer_amd import kernels
+    x = _portion(1, 40, 2, 32, 32)
+    q, k, v, raw, bias, rate_log, state = (t.to(DEV) for t in x)
+    kept = {}
+    st = state.expand(3, -1, -1, -1).contiguous()
+    kernels.linear_scan(q, k, v, st, torch.arange(3, device=DEV), torch.tensor([0, 31, 32, 40], dtype=torch.int32, device=DEV), 2, 32, 32,
+                        step=raw, step_bias=bias, decay_log=rate_log, groups=1, q_lens=[31, 1, 8], plan_cache=kept)
+    assert not [k for plan in kept.values() for k, t in plan.items() if torch.is_tensor(t)]
+
+
 def test_the_rule_takes_what_it_should(monkeypatch):
     """Which portions go where, without a launch."""
     from xinfer_amd import kernels

@@ -360,14 +360,16 @@ def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, ou
     plan = plan_cache.get(key) if plan_cache is not None else None
     if plan is None:
         whole, long = step_chunk_plan(q_lens)
-        starts = [0]
-        for n in q_lens:
-            starts.append(starts[-1] + int(n))
-        rows = long + whole
-        L, W = len(long), len(whole)
-        i32 = torch.tensor([starts[b] for b in rows] + [starts[b + 1] for b in rows], dtype=torch.int32).to(q.device)
-        slots = state_slots.index_select(0, torch.tensor(rows, dtype=torch.int64).to(q.device))
-        plan = dict(L=L, W=W, first=i32[:L + W], last=i32[L + W:], slots=slots)
+        plan = dict(L=len(long), W=len(whole))
+        if long:                 # (a step of short portions wants none of these on the device)
+            starts = [0]
+            for n in q_lens:
+                starts.append(starts[-1] + int(n))
+            rows = long + whole
+            L, W = len(long), len(whole)
+            i32 = torch.tensor([starts[b] for b in rows] + [starts[b + 1] for b in rows], dtype=torch.int32).to(q.device)
+            slots = state_slots.index_select(0, torch.tensor(rows, dtype=torch.int64).to(q.device))
+            plan.update(first=i32[:L + W], last=i32[L + W:], slots=slots)
         if plan_cache is not None:
             plan_cache[key] = plan
     L, W = plan["L"], plan["W"]
