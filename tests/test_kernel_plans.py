@@ -61,3 +61,30 @@ def test_float32_attention_sets_one_limit_a_kernel():
         need = 4 * (8 * (16 * dv + 32) + 16 * (d + 4))          # eight waves' sums of 16 rows, their maxima and totals, the queries
         assert need <= limit(d, dv) <= 160 * 1024
     assert all(len(v) == 1 for v in kinds.values())
+
+
+@pytest.mark.parametrize("lens,H,dk,dv,walk", [
+    ([2048], 1, 128, 64, False), ([2304], 1, 128, 64, False), ([3072], 1, 128, 64, True), ([8192], 8, 128, 64, True),
+    ([4096], 8, 128, 64, True), ([8192], 16, 128, 64, False), ([8192], 128, 128, 64, False), ([3000, 3000], 8, 128, 64, False),
+    ([8192], 1, 32, 32, True), ([2816], 1, 32, 32, False), ([4096, 64, 300], 8, 128, 64, False), ([1] * 60, 8, 64, 64, False)])
+def test_few_heads_walk_a_long_portion_side_by_side(lens, H, dk, dv, walk, monkeypatch):
+    import torch
+    assert kernels.step_walk_ahead(lens, H, dk, dv) == walk
+    # the route that `linear_scan` takes, without a launch
+    taken = []
+    monkeypatch.setattr(kernels, "_stream", lambda: 0)
+    monkeypatch.setattr(kernels, "_ok", lambda rc: None)
+
+    class Lib:
+        xi_step_chunks_takes = staticmethod(lambda dk, dv: 1)
+
+        def __getattr__(self, name):
+            return lambda *a: taken.append(name)
+
+    monkeypatch.setattr(kernels, "lib", lambda: Lib())
+    T = sum(lens)
+    t = torch.empty(1, dtype=torch.bfloat16)
+    common = (t, t, t, 8, 8, 8, None, None, 1.0, None, t, H, t, t, None, dv, H, 0)
+    done = kernels._step_chunks(common, t, H * dk * dv, torch.arange(len(lens)), lens, {}, t, H, dk, dv, 1.0, 1.0)
+    assert done == (not walk and max(lens) >= kernels.STEP_FROM)
+    assert taken[:1] == (["xi_step_chunks"] if done else [])

@@ -341,11 +341,25 @@ def _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, o
 
 STEP_MFMA = True                  # False: portions of a selective state space go through the walk token by token too
 STEP_FROM = 32                    # tokens of a portion from which it is walked in chunks on the matrix cores
+STEP_CHAIN = 2048                 # tokens of a portion up to which that is ahead whatever the heads
 
 
 def step_chunk_plan(q_lens):
     """The portions of a step for `xi_step_chunks`: the batch rows walked token by token, and those of STEP_FROM tokens and more."""
     return ([b for b, n in enumerate(q_lens) if int(n) < STEP_FROM], [b for b, n in enumerate(q_lens) if int(n) >= STEP_FROM])
+
+
+def step_walk_ahead(q_lens, H: int, dk: int, dv: int) -> bool:
+    """Whether the three launches over chunks side by side are ahead of `xi_step_chunks` for a step: a portion's chunks are a chain
+    there, 4.0 us each at dk = 128, however few workgroups walk (heads by 32 value columns by portions).  Both sides' time as measured on
+    MI355X (810 steps of 1 to 48 such workgroups, dk 32 to 128, 1,536 to 8,192 tokens; of the two the slower one by more than 5% for 11
+    of them, 15% at most).  Us, walk / chunks, dk = 128 and dv = 64: 1 head 2,048 tokens 143 / 118, 3,072 149 / 175, 8,192 174 / 470; 8
+    heads 2,048 156 / 120, 4,096 191 / 235, 8,192 333 / 474; 16 heads 4,096 314 / 242, 8,192 543 / 474; two portions of 3,000 of 8 heads 227
+    / 175."""
+    lens = [int(n) for n in q_lens]
+    chain = max(lens) * (0.0345 + 0.00017 * dk)
+    one_by_one = max((n for n in lens if n < 2 * SCAN_CHUNK), default=0)          # a launch of its own, token by token
+    return chain > 107 + 0.15 * dk + (0.0011 + 0.000013 * dk) * sum(lens) * H * -(-dv // 64) + 1.1 * one_by_one
 
 
 def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale) -> bool:
@@ -355,6 +369,8 @@ def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, ou
     if (not STEP_MFMA or SCAN_CHUNK <= 0 or q.dtype != torch.bfloat16 or step is None or common[15] != dv or common[17]
             or not lib().xi_step_chunks_takes(dk, dv) or qs % 8 or ks % 8 or vs % 8 or k_scale == 0.0
             or any(t.data_ptr() % 16 for t in (q, k, v))):
+        return False
+    if max(q_lens, default=0) > STEP_CHAIN and step_walk_ahead(q_lens, H, dk, dv):
         return False
     key = ("step_chunk_plan", STEP_FROM)
     plan = plan_cache.get(key) if plan_cache is not None else None
@@ -422,7 +438,8 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     side by side in three launches (each chunk's own share from a zero state; the states the chunks start from,
     one after the other; the chunks' results), the others in one piece; in bfloat16 with a constant decay per head the long
     ones go through the matrix cores (`xi_decay_chunks`, portions from DECAY_FROM tokens on), and so they do with a step size a
-    token and head (`xi_step_chunks`, from STEP_FROM tokens on, one chunk after the other).  `plan_cache`: a dict of the step in which
+    token and head (`xi_step_chunks`, from STEP_FROM tokens on, one chunk after the other, but for long portions of few heads:
+    `step_walk_ahead`).  `plan_cache`: a dict of the step in which
     the index arrays of this cutting are kept for the next layer."""
     H, dk, dv = int(heads), int(key_dim), int(value_dim)
     T = q.shape[0]
