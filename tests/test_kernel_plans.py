@@ -88,3 +88,23 @@ def test_few_heads_walk_a_long_portion_side_by_side(lens, H, dk, dv, walk, monke
     done = kernels._step_chunks(common, t, H * dk * dv, torch.arange(len(lens)), lens, {}, t, H, dk, dv, 1.0, 1.0)
     assert done == (not walk and max(lens) >= kernels.STEP_FROM)
     assert taken[:1] == (["xi_step_chunks"] if done else [])
+
+
+@pytest.mark.parametrize("bm", [32, 64, 128, 256])
+def test_most_tiles_of_routed_experts(bm):
+    """The largest number of tiles that any sharing out of the pairs makes, and no more."""
+    most = kernels.lib().xi_moe_tiles_most
+    for P in (1, 2, 7, 31, 32, 33, 64, 65, 200, 257, 1000, 4097):
+        for E in (1, 2, 3, 8, 100, 1024):
+            # one pair for every expert that gets any, bm more for as many tiles as the rest gives, the remainder anywhere
+            n = min(P, E)
+            counts = [1] * n
+            full, rest = divmod(P - n, bm)
+            for i in range(full):
+                counts[i % n] += bm
+            assert sum(-(-c // bm) for c in counts) == most(P, E, bm)
+            counts[0] += rest
+            assert sum(-(-c // bm) for c in counts) == most(P, E, bm)
+            even = [P // n + (i < P % n) for i in range(n)]
+            assert sum(-(-c // bm) for c in even) <= most(P, E, bm)
+            assert -(-P // bm) <= most(P, E, bm)

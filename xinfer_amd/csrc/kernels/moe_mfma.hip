@@ -333,8 +333,12 @@ using namespace xi;
 
 extern "C" {
 
-// Most tiles of up to `bm` rows that P pairs on E experts can make.
-int xi_moe_tiles_most(int P, int E, int bm) { return (P + bm - 1) / bm + E; }
+// Most tiles of up to `bm` rows that P pairs on E experts can make: an expert with pairs has one, and one more for every bm pairs
+// beyond its first.  (The grids are sized by it: few pairs on many experts launch a workgroup a pair at most.)
+int xi_moe_tiles_most(int P, int E, int bm) {
+  const int taken = P < E ? P : E;
+  return taken + (P - taken) / bm;
+}
 
 // idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P]; tile_* int32 [xi_moe_tiles_most]; n_tiles int32 [1];
 // tile_first, tile_count (both or neither): the first tile of a tile's expert and how many it has.
