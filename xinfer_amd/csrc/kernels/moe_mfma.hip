@@ -34,7 +34,8 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __res
                                                                 int* __restrict__ tile_expert, int* __restrict__ tile_row0,
                                                                 int* __restrict__ tile_rows, int* __restrict__ n_tiles,
                                                                 int* __restrict__ tile_first, int* __restrict__ tile_count) {
-  __shared__ int count[kSortExperts], cursor[kSortExperts];
+  static_assert(kSortThreads >= kSortExperts, "an expert a thread");
+  __shared__ int count[kSortExperts], cursor[kSortExperts], wave_pairs[kSortThreads / kWave], wave_tiles[kSortThreads / kWave];
   const int A = E + I;
   for (int e = threadIdx.x; e < A; e += kSortThreads) count[e] = 0;
   __syncthreads();
@@ -44,24 +45,45 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __res
     atomicAdd(&count[e], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, tiles = 0;
-    for (int e = 0; e < A; ++e) {
-      cursor[e] = at;
-      const int first = tiles;
-      for (int r = 0; e < E && r < count[e]; r += BM) {
-        if (tile_first) {
-          tile_first[tiles] = first;
-          tile_count[tiles] = (count[e] + BM - 1) / BM;
-        }
-        tile_expert[tiles] = e;
-        tile_row0[tiles] = at + r;
-        tile_rows[tiles] = count[e] - r < BM ? count[e] - r : BM;
-        ++tiles;
+  // an expert a thread: its first slot and tile are the sums of those in front of it, along the wave and then over the waves
+  // (one thread going through them took 55 ns each: 56 of 75 us at 1,024 experts and one token)
+  const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
+  const int pairs = e < A ? count[e] : 0, tiles = e < E ? (pairs + BM - 1) / BM : 0;
+  int at = pairs, first = tiles;
+  if (wave * kWave < A) {
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int a = __shfl_up(at, o, kWave), f = __shfl_up(first, o, kWave);
+      if (lane >= o) {
+        at += a;
+        first += f;
       }
-      at += count[e];
     }
-    *n_tiles = tiles;
+  }
+  if (A > kWave) {
+    if (lane == 63) {
+      wave_pairs[wave] = at;
+      wave_tiles[wave] = first;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave && wave * kWave < A; ++w) {
+      at += wave_pairs[w];
+      first += wave_tiles[w];
+    }
+  }
+  if (e == A - 1) *n_tiles = first;
+  at -= pairs;
+  first -= tiles;
+  if (e < A) cursor[e] = at;
+  for (int i = 0; i < tiles; ++i) {
+    const int r = i * BM;
+    if (tile_first) {
+      tile_first[first + i] = first;
+      tile_count[first + i] = tiles;
+    }
+    tile_expert[first + i] = e;
+    tile_row0[first + i] = at + r;
+    tile_rows[first + i] = pairs - r < BM ? pairs - r : BM;
   }
   __syncthreads();
   for (int p = threadIdx.x; p < P; p += kSortThreads) {
