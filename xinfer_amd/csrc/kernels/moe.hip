@@ -46,10 +46,14 @@ static __device__ __forceinline__ void route_load8(const bf16* p, float (&v)[8])
 
 // A workgroup of `waves` waves takes TT tokens; a wave an output of the router at a time, for all of them, and then wave i
 // chooses for token i.  VEC: rows in whole pieces of eight: a lane takes eight k side by side, 512 k a round of the wave, eight
-// chains; else four chains of single numbers.  The order of a sum is fixed by H alone.
-// Measured on MI355X, width 4096, ten outputs: 8 tokens (sixteen waves, one token) 6.3 us against 25 with four waves and four
-// chains of single numbers, whose rounds waited for one another; 2,048 tokens (eight waves, four tokens: a row of the router is
-// read once for four) 16 us against 29.
+// chains; else four chains of single numbers.  The order of a sum is fixed by H (and the rows' alignment), the same for every TT
+// and number of waves.
+// Bound by its rounds of loads where there are few tokens, by the router's rows from L2 where there are many.  Measured on MI355X, us,
+// against one token and four waves with chains of single numbers, which was here before: bfloat16, width 4096, 16 outputs: 1 token
+// (sixteen waves, one token) 7.3 / 12.8, 384 11.2 / 14.5, 768 (eight waves, two tokens) 13.3 / 17.9, 2,048 (eight waves, four tokens) 18.5
+// / 38.7; 256 outputs, 1,024: 170 / 303.  float32, 16 outputs: 1,024 (two tokens) 17.2 / 24.3, four 25.4; 256 outputs, 8,192: two 1,885, four
+// 1,753 / 3,409.  Width 512, 10 outputs, float32, 8,192: two tokens and four waves 16.2 / 18.9, eight waves 19.5, four tokens 21.4.  Width 256, 8
+// outputs, 8,192: 15.0 as it was, and 14 to 32 with vectors.
 template <typename T, bool VEC, int TT>
 __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ x, const float* __restrict__ wr,
                                                          const float* __restrict__ br, int* __restrict__ idx,
@@ -299,15 +303,25 @@ int xi_moe_route(const void* x, int dtype, const float* wr, const float* br, int
   XI_CHECK(all_scores >= 0 && all_scores <= 2, "moe_route: unknown kind of scores %d", all_scores);
   XI_CHECK(top > 0 && top <= E && top <= kMaxTop, "moe_route: %d of %d experts cannot be chosen (at most %d)", top, E, kMaxTop);
   if (n_tok == 0) return 0;
-  const bool vec = H % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
+  // Up to 512 k less than half of the lanes have a vector's piece: single numbers there, as for rows in other places.
+  const bool vec = H >= 512 && H % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
+  // Few tokens: sixteen waves for one, as many outputs at a time as there can be.  From where these fill the chip on, two tokens a
+  // workgroup, and four where a row of the router is long and read by many: see the kernel.
+  const int outputs = E + X;
+  const bool few = n_tok < (outputs <= 32 && H <= 4096 ? 640 : 900);
+  const bool four = H >= 1024 && (dtype == kBF16 ? n_tok >= 1024 : n_tok >= 2048 && outputs >= 32);
 #define XI_ROUTE(TT_, VEC, TOK, WAVES)                                                                                      \
   moe_route_kernel<TT_, VEC, TOK><<<(unsigned)((n_tok + TOK - 1) / TOK), WAVES * kWave, 0, stream>>>(                        \
       (const TT_*)x, wr, br, idx, wt, H, E, top, all_scores, extra, X, correction, n_tok)
 #define XI_ROUTE_T(TT_)                                  \
   do {                                                   \
-    if (!vec) XI_ROUTE(TT_, false, 1, 8);                \
-    else if (n_tok < 1024) XI_ROUTE(TT_, true, 1, 16);   \
-    else XI_ROUTE(TT_, true, 4, 8);                      \
+    if (!vec && n_tok < 640 && outputs <= 16) XI_ROUTE(TT_, false, 1, 8); \
+    else if (!vec && n_tok < 640) XI_ROUTE(TT_, false, 1, 16); \
+    else if (!vec) XI_ROUTE(TT_, false, 1, 4);           \
+    else if (few) XI_ROUTE(TT_, true, 1, 16);            \
+    else if (four) XI_ROUTE(TT_, true, 4, 8);            \
+    else if (H < 1024 && n_tok >= 4096) XI_ROUTE(TT_, true, 2, 4); \
+    else XI_ROUTE(TT_, true, 2, 8);                      \
   } while (0)
   if (dtype == kF32) XI_ROUTE_T(float);
   else if (dtype == kBF16) XI_ROUTE_T(bf16);
