@@ -8,11 +8,28 @@ from xinfer_amd import kernels
 DEV = "cuda:0"
 
 
+def _last_round(M, F):
+    """How the kernel of 256 rows by 128 features takes the tiles behind the last whole round of 256: 1 uncut, 2 in halves of the rows, 4."""
+    tiles = -(-M // 256) * -(-F // 128)
+    rest = tiles % 256
+    return 1 if tiles < 256 or rest == 0 or rest > 128 else 4 if rest <= 64 else 2
+
+
+def test_every_last_round_is_among_the_sizes():
+    """Uncut, halves and quarters all run below, halves and quarters with a last tile of rows that ends in its first half too."""
+    marks = [m for m in test_gated_product_in_tiles.pytestmark if m.name == "parametrize"]
+    sizes = [(M, F) for M, F, _, _ in marks[0].args[1]]
+    assert {_last_round(*s) for s in sizes} == {1, 2, 4}
+    assert {_last_round(M, F) for M, F in sizes if 0 < M % 256 <= 128 and M > 256} >= {2, 4}
+    assert {_last_round(M, F) for M, F in sizes if M % 256 > 128} >= {2}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,F,K,act", [
     (65, 320, 128, "silu"), (1, 4, 64, "gelu_tanh"), (257, 132, 192, "gelu_tanh"), (300, 12288, 64, "silu"),
-    (700, 17408, 128, "silu"), (2048, 5000, 64, "gelu_tanh"),      # 256 tiles and a rest, cut in halves (152: not), quarters
-    (1024, 9000, 64, "silu"), (1100, 7168, 64, "gelu_tanh")])
+    (700, 17408, 128, "silu"), (2048, 5000, 64, "gelu_tanh"),
+    (1024, 9000, 64, "silu"), (1100, 7168, 64, "gelu_tanh"),
+    (2048, 6144, 64, "silu"), (1800, 5300, 128, "gelu_tanh"), (1992, 5300, 64, "silu"), (1800, 4604, 64, "silu")])
 def test_gated_product_in_tiles(M, F, K, act):
     g = torch.Generator().manual_seed(M + F)
     x, w = torch.randn(M, K, generator=g).to(torch.bfloat16), (torch.randn(2 * F, K, generator=g) * K ** -0.5).to(torch.bfloat16)
