@@ -29,3 +29,65 @@ def test_two_columns_a_lane(H, dk, dv, dtype):
     for a in range(0, dv, 64):
         part, own = walk(a, min(dv, a + 64))       # up to 64 columns: one a lane
         assert torch.equal(whole[..., a:a + 64], part) and torch.equal(st[..., a:a + 64], own)
+
+
+def _plain(q, k, v, decay, weight, S, q_scale):
+    """One request in float64, from the state S [H, dk, dv]: decay, weight [T, H]; v [T, H, dv]."""
+    S, out = S.double().clone(), []
+    for t in range(q.shape[0]):
+        S = decay[t][:, None, None] * S + k[t][:, :, None] * (weight[t][:, None] * v[t])[:, None, :]
+        out.append((S * (q[t] * q_scale)[:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+@pytest.mark.parametrize("how,dtype", [("gates", torch.bfloat16), ("gates", torch.float32), ("silu", torch.float32), ("step", torch.float32)])
+@pytest.mark.parametrize("H,dk,vc", [(16, 64, 129), (11, 100, 200)])
+def test_other_decays_with_two_columns_a_lane(how, dtype, H, dk, vc):
+    """Ready-made gates beside the keys' own sum (a state's last column), one decay a head under silu, and a step size: enough chunks
+    that a lane has two columns, against float64 and against walks of up to 64 columns."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(dk + vc)
+    lens = [1130, 2, 901]
+    T = sum(lens)
+    cu = torch.tensor([0, 1130, 1132, T], dtype=torch.int32, device=DEV)
+    chunks = len(kernels.scan_chunk_plan(lens)[2])
+    assert chunks * H * -(-vc // 128) >= 512           # xi_linear_scan's rule: two rounds of workgroups with two columns a lane
+    ones = how == "gates"
+    q, k = (torch.randn(T, H * dk, generator=g).to(dtype) for _ in range(2))
+    v = torch.randn(T, H, vc, generator=g).to(dtype)
+    state = torch.randn(3, H, dk, vc + ones, generator=g)
+    step, bias, rate = torch.randn(T, H, generator=g).to(dtype), torch.randn(H, generator=g) - 1.0, torch.randn(H, generator=g) * 0.5 - 1.0
+    gates = torch.stack([torch.rand(T, H, generator=g) * 0.3 + 0.7, torch.rand(T, H, generator=g)], dim=2)
+    head = torch.rand(H, generator=g) * 0.3 + 0.7
+    d = lambda t: t.to(DEV)
+    kw = {"gates": dict(gates=d(gates)), "silu": dict(head_decay=d(head), silu=True),
+          "step": dict(step=d(step), step_bias=d(bias), decay_log=d(rate))}[how]
+
+    def walk(a, b):
+        cols = list(range(a, b)) + ([vc] if ones else [])
+        st = d(state[..., cols].contiguous())
+        o = kernels.linear_scan(d(q), d(k), d(v[..., a:b].reshape(T, -1).contiguous()), st, torch.arange(3, device=DEV), cu, H, dk, len(cols),
+                                q_scale=dk ** -0.5, q_lens=lens, **({**kw, "value_cols": b - a} if ones else kw))
+        return o.view(T, H, -1).cpu(), st.cpu()
+
+    whole, st = walk(0, vc)
+    for a in range(0, vc, 64):
+        b = min(vc, a + 64)
+        part, own = walk(a, b)
+        assert torch.equal(whole[..., a:b], part[..., :b - a]) and torch.equal(st[..., a:b], own[..., :b - a])
+        assert torch.equal(whole[..., vc:], part[..., b - a:]) and torch.equal(st[..., vc:], own[..., b - a:])
+
+    x = step.double() + bias.double()
+    size = torch.logaddexp(x, torch.zeros_like(x))
+    decay = {"gates": gates[..., 0].double(), "silu": head.double().expand(T, H), "step": torch.exp(-torch.exp(rate.double()) * size)}[how]
+    weight = {"gates": gates[..., 1].double(), "silu": torch.ones(T, H, dtype=torch.float64), "step": size}[how]
+    act = torch.nn.functional.silu if how == "silu" else lambda t: t
+    qd, kd = act(q.double()).view(T, H, dk), act(k.double()).view(T, H, dk)
+    vd = torch.cat([act(v.double()), torch.ones(T, H, 1, dtype=torch.float64)], dim=2) if ones else act(v.double())
+    for i, (a, b) in enumerate(((0, 1130), (1130, 1132), (1132, T))):
+        ref, s = _plain(qd[a:b], kd[a:b], vd[a:b], decay[a:b], weight[a:b], state[i], dk ** -0.5)
+        sizes, s_sizes = _plain(qd[a:b].abs(), kd[a:b].abs(), vd[a:b].abs(), decay[a:b], weight[a:b], state[i].abs(), dk ** -0.5)
+        # float32 sums of dk products of a state that holds about 1 / (1 - decay) tokens' terms, each a few roundings old
+        bound = (dk + 64) * 2.0 ** -23
+        assert float(((whole[a:b].double() - ref).abs() / sizes).max()) < bound
+        assert float(((st[i].double() - s).abs() / s_sizes).max()) < bound
