@@ -121,3 +121,27 @@ def test_attention(nq, nkv, d, dv, page, window, chunk, cap, slopes, sinks, late
         assert torch.equal(run(slice(r, r + 1))[0], got[r]), r
     plain = run(slice(None), matrix=False)
     assert float((plain.cpu().double() - ref).abs().max()) < 2e-5
+
+
+def test_attention_keys_without_weight():
+    """Scores of -inf through whole blocks of keys, at the request's start and further on: no weight for these keys, and
+    results undefined only for a token that has no other key."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(5)
+    L, nq, nkv, d = 300, 4, 2, 64
+    q, k, v = torch.randn(L, nq, d, generator=g), torch.randn(L, nkv, d, generator=g), torch.randn(L, nkv, d, generator=g)
+    q[..., 0] = q[..., 0].abs() + 0.1
+    off = torch.zeros(L, dtype=torch.bool)
+    off[:20] = off[128:160] = True           # wave 0's first block and the second one of waves 0 and 1; a part of wave 1's first
+    k[off, :, 0] = float("-inf")
+    want = _plain_attention(q.double(), k.double(), v.double(), d ** -0.5, 0, 0, 0.0, None, None)
+    pages = lambda x: torch.nn.functional.pad(x, (0, 0, 0, 0, 0, 4)).view(-1, 16, nkv, x.shape[2]).transpose(1, 2).contiguous().to(DEV)
+    bt = torch.arange(19, dtype=torch.int32, device=DEV)[None]
+    pos = torch.arange(L, dtype=torch.int32, device=DEV)
+    for rows in (slice(0, L), slice(20, 21), slice(130, 131), slice(170, 171)):
+        got = kernels.attention_generic(q[rows].contiguous().to(DEV), pages(k), pages(v), bt, torch.zeros_like(pos[rows]), pos[rows].contiguous(),
+                                        d ** -0.5).cpu().double().view(-1, nq, d)
+        has = torch.arange(L)[rows] >= 20
+        assert bool(got[~has].isnan().all())
+        # as in `test_attention`
+        assert float((got[has] - want[rows][has]).abs().max()) < 2e-5, rows

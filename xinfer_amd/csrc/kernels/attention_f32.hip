@@ -155,15 +155,16 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
       most = fmaxf(most, lane_xor<32>(most));
       const bool any = own && (b + 1) * kBlock > lo && b * kBlock <= pos;       // (a block that a row does not see leaves it as it is)
       const float m_new = any ? fmaxf(m, most) : m;
+      const float top = m_new == -INFINITY ? 0.f : m_new;         // (scores of -inf alone so far: weights of 0)
       float sum = 0.f;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        s[v] = sees[v] ? expf(s[v] - m_new) : 0.f;
+        s[v] = sees[v] ? expf(s[v] - top) : 0.f;
         sum += s[v];
       }
       sum += lane_xor<16>(sum);
       sum += lane_xor<32>(sum);
-      const float corr = any ? expf(m - m_new) : 1.f;             // exp(-inf) = 0 on the first block
+      const float corr = any ? expf(m - top) : 1.f;               // exp(-inf) = 0 on the first block
       l = l * corr + sum;
       m = m_new;
 #pragma unroll
