@@ -105,3 +105,19 @@ def test_what_is_taken_and_refused():
         kernels.moe_experts_tiled(z(3, 96), z(2, 128, 96), z(2, 96, 64), idx, wt)
     with pytest.raises(kernels.KernelError):
         kernels.moe_experts_tiled(z(3, 64), z(2, 128, 64), z(2, 64, 64), idx, wt, tile_rows=32)
+
+
+@pytest.mark.parametrize("T", [3, 200])
+def test_rows_off_16_bytes(T):
+    """Rows may start on any element, as in the other forms."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(T)
+    E, H, F = 3, 128, 64
+    rb = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    gate_up, down, x = (rb(E, 2 * F, H) * H ** -0.5).to(DEV), (rb(E, H, F) * F ** -0.5).to(DEV), rb(T, H).to(DEV)
+    idx = torch.randint(0, E + 1, (T, 2), generator=g).to(torch.int32).to(DEV)           # (one identity expert)
+    wt = torch.rand(T, 2, generator=g).to(DEV)
+    flat = torch.zeros(T * H + 1, dtype=torch.bfloat16, device=DEV)
+    flat[1:] = x.reshape(-1)
+    got = kernels.moe_experts_tiled(flat[1:].view(T, H), gate_up, down, idx, wt, identity=1)
+    assert torch.equal(got, kernels.moe_experts_tiled(x, gate_up, down, idx, wt, identity=1))

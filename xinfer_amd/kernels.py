@@ -860,6 +860,7 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     _want(wt, torch.float32, "moe_experts_tiled: weights")
     if not moe_tiled_takes(T, top, E, H, F, gated):
         raise KernelError(f"moe_experts_tiled: {T} tokens, {E} experts, H={H} F={F} are not taken (sizes in 64s)")
+    rows = x if x.data_ptr() % 16 == 0 else x.clone()          # (the products want them on 16 bytes)
     P = T * top
     bm1, bm2 = (int(tile_rows),) * 2 if tile_rows is not None else moe_tile_rows(P, E, F, H, gated)
     if bm1 not in (64, 128, 256):
@@ -873,7 +874,7 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
                           _p(t_c), _stream()))
     wt_in = wt.contiguous() if weigh_input else None
     mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
-    _ok(lib().xi_moe_tile(_p(x), ctypes.c_longlong(T), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
+    _ok(lib().xi_moe_tile(_p(rows), ctypes.c_longlong(T), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
                           _p(t_c), most, _p(mid), F, H, bm1, bm // bm1, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
     y = torch.empty((P, H), dtype=torch.float32, device=x.device)
     _ok(lib().xi_moe_tile(_p(mid), ctypes.c_longlong(P), _p(order), top, _p(down), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
@@ -881,7 +882,7 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     out = torch.empty((T, H), dtype=torch.float32, device=x.device)
     if weigh_input:
         wt = torch.ones_like(wt)
-    _ok(lib().xi_moe_combine(_p(y), _p(slot_of), _p(wt), _p(out), T, H, top, _p(idx), E, _p(x if identity else None), _p(add), _stream()))
+    _ok(lib().xi_moe_combine(_p(y), _p(slot_of), _p(wt), _p(out), T, H, top, _p(idx), E, _p(rows if identity else None), _p(add), _stream()))
     return out
 
 
