@@ -1,7 +1,7 @@
 // Paged causal GQA attention, one workgroup per (token, query head), float32 math.
-// It serves every case (prompt portions, decode tokens, windows, any head size) and is
-// the attention of the 32-bit path; the bfloat16 path uses it where no faster kernel
-// applies.  Keys of a token at position p are the cached positions lo..p of its own
+// It serves every case (prompt portions, decode tokens, windows, any head size); either
+// path uses it where no faster kernel applies (float32: head sizes that attention_f32.hip
+// does not take, or key heads of another number than the value heads).  Keys of a token at position p are the cached positions lo..p of its own
 // request, lo = max(0, p - window + 1) (with chunks of size c also not before the chunk's first position, p - p mod c), read through the request's block table.  K is
 // [page, kv_head, offset, d]; V is [page, kv_head, offset, dv] or, with v_grouped,
 // [page, kv_head, offset / 8, dv, 8]; the value head size dv may differ from d.

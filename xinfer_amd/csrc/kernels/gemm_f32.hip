@@ -11,10 +11,14 @@
 //
 //   few rows  (M <= 64)  a workgroup owns 16 or 32 features and all rows, its eight waves a chunk
 //             each; operands go straight from memory into registers, 16 bytes a lane, some steps
-//             ahead; the chunks meet in LDS.  Bound by the weights' bytes.
+//             ahead; the chunks meet in LDS.  Bound by the weights' bytes
+//             beside x, which every tile of features reads again: 3.4 (N = 6144, K = 4096) to 5.3 TB/s
+//             (N = 151936) of weights at 8 rows.
 //   tile      a workgroup of four waves owns BM rows by BN features; tiles of 32 k go through
-//             registers into two LDS buffers, one barrier a tile.  Bound by the matrix cores
-//             (157 TFLOP/s).
+//             registers into two LDS buffers, one barrier a tile.  The matrix cores (157 TFLOP/s)
+//             are busy 67 to 71% of the time in tiles of 64 x 64 and 56% in those of 32 x 64; a
+//             step's operands are read together in front of its products, and half of the 36 to
+//             48% of the time that LDS is active is bank conflicts.
 //
 // Reference call site: candle matmul, /root/reference/src/models/layers/linear.rs:76-124.
 #include "common.h"
