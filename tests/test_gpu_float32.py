@@ -145,3 +145,35 @@ def test_attention_keys_without_weight():
         assert bool(got[~has].isnan().all())
         # as in `test_attention`
         assert float((got[has] - want[rows][has]).abs().max()) < 2e-5, rows
+
+
+@pytest.mark.parametrize("nq,nkv,d", [(3, 3, 32), (4, 2, 144), (20, 1, 64)])
+def test_attention_tiles_are_one(nq, nkv, d):
+    """Single tokens and portions side by side: the same bits for every number of tokens a workgroup, tiles where requests meet among
+    them, and a request's infinite values stay its own."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d)
+    lens, news = [70, 1, 290, 33, 61, 200], [1, 1, 1, 20, 61, 15]
+    mp, page = 10, 32
+    kc, vc = (torch.randn(6 * mp, nkv, page, d, generator=g).to(DEV) for _ in range(2))
+    bt = torch.randperm(6 * mp, generator=g).to(torch.int32).view(6, mp).to(DEV)
+    q = torch.randn(sum(news), nq, d, generator=g).to(DEV)
+    seq = torch.tensor([b for b in range(6) for _ in range(news[b])], dtype=torch.int32)
+    pos = torch.tensor([lens[b] - news[b] + i for b in range(6) for i in range(news[b])], dtype=torch.int32)
+    run = lambda **kw: kernels.attention_generic(q, kc, vc, bt, seq.to(DEV), pos.to(DEV), d ** -0.5, **kw).cpu()
+    most = 16 // min(16, nq // nkv)
+    want = run(tile=1)
+    assert float((want - run(matrix=False)).abs().max()) < 2e-5           # as in `test_attention`
+    for tile in range(0, most + 1):
+        for lead in (0, 3):
+            assert torch.equal(run(tile=tile, lead=lead), want), (tile, lead)
+    vc[bt[4].long()] = float("inf")
+    vc[bt[2, 1].long()] = float("nan")
+    own = (seq == 4) | (seq == 2)
+    for tile in {1, most // 2 or 1, most}:
+        for lead in (0, 3):
+            assert torch.equal(run(tile=tile, lead=lead)[~own], want[~own]), (tile, lead)
+    with pytest.raises(kernels.KernelError):
+        run(tile=most + 1)
+    with pytest.raises(kernels.KernelError):
+        run(lead=q.shape[0] + 1)

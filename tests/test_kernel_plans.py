@@ -108,3 +108,24 @@ def test_most_tiles_of_routed_experts(bm):
             even = [P // n + (i < P % n) for i in range(n)]
             assert sum(-(-c // bm) for c in even) <= most(P, E, bm)
             assert -(-P // bm) <= most(P, E, bm)
+
+
+def test_float32_attention_tiles():
+    """Tokens a workgroup: the fewest that make one round of workgroups, at most 16 (token, head) rows, one for single tokens."""
+    from xinfer_amd import kernels
+    tile = kernels.lib().xi_attention_f32_tile
+    assert [tile(n, 1, 16, 16) for n in (1, 16, 17, 20, 64, 128, 240, 256, 257, 2048)] == [1, 1, 2, 2, 4, 8, 15, 16, 16, 16]
+    assert [tile(n, 1, 32, 8) for n in (20, 32, 33, 64, 2048)] == [1, 1, 2, 2, 4]
+    assert tile(2048, 1, 40, 1) == 1 and tile(4000, 1, 12, 4) == 5
+    assert tile(64, 64, 16, 16) == 1 and tile(64, 17, 16, 16) == 1 and tile(64, 16, 16, 16) == 4
+
+
+def test_leading_singles():
+    from types import SimpleNamespace
+    import torch
+    from xinfer_amd import kernels
+    f, b = torch.zeros(1), torch.zeros(1, dtype=torch.bfloat16)
+    ctx = lambda cu, most: SimpleNamespace(cu_q_host=cu, max_q_len=most, scratch={})
+    assert kernels.leading_singles(f, ctx([0, 1, 2, 9, 10], 7)) == 2
+    assert kernels.leading_singles(f, ctx([0, 7, 8], 7)) == 0
+    assert kernels.leading_singles(f, ctx((), 1)) == 0 and kernels.leading_singles(b, ctx([0, 1, 9], 8)) == 0

@@ -28,7 +28,9 @@
 // A value that a token does not see never reaches it, not even with a weight of 0 (an infinite or
 // undefined one would): in a block that some token of the tile does not see in full, each token's
 // product is made by itself, with the nearest key that it sees in the place of one that it does not,
-// and only its own columns keep it.  What no token of the tile sees is not read.
+// and only its own columns keep it.  What no token of the tile sees is not read.  Where requests meet in a
+// tile, a block that all of one's tokens see in full is one product, which their columns keep (16 heads of
+// 128, 300 tokens and one behind contexts of 2,000: 260 us, 592 with a product a token there).
 #include "common.h"
 
 namespace xi {
@@ -45,14 +47,15 @@ template <int DT>
 __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_pages, const int* __restrict__ tok_seq, const int* __restrict__ positions,
-    float* __restrict__ out, float scale, int window, int page_size, int n_tok, int tile_tokens, int nq, int nkv, int d, int dv,
+    float* __restrict__ out, float scale, int window, int page_size, int n_tok, int lead, int tile_tokens, int nq, int nkv, int d, int dv,
     float softcap, const float* __restrict__ slopes, const float* __restrict__ sinks, int values_in_keys, int chunk) {
   constexpr int DG = (DT + 3) / 4;                  // groups of 64 value dims
   extern __shared__ float lds[];                    // m and l [kWaves][16] each, then q [16][d + 4], then [kWaves][rows][dv]
   float *m_s = lds, *l_s = lds + kWaves * 16, *q_s = lds + 2 * kWaves * 16, *acc_s = q_s + 16 * (d + 4);
   const int group = nq / nkv, kvh = blockIdx.y, hb = blockIdx.z * 16;
   const int heads = group - hb < 16 ? group - hb : 16;
-  const int t0 = blockIdx.x * tile_tokens, t1 = t0 + tile_tokens < n_tok ? t0 + tile_tokens : n_tok;
+  const int bx = blockIdx.x, t0 = bx < lead ? bx : lead + (bx - lead) * tile_tokens;
+  const int t1 = bx < lead ? t0 + 1 : t0 + tile_tokens < n_tok ? t0 + tile_tokens : n_tok;
   const int rows = (t1 - t0) * heads;               // row: token by token, its heads side by side
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, j = lane >> 4;
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
     int row = b <= last ? row_of(b) : 0, row_next = 0;
     if (b <= last) ask_k(row);
     for (; b <= last; b += kWaves) {
-      const bool whole = one && b * kBlock >= lo_most && b * kBlock + kBlock - 1 <= pos_least;
+      const bool full = b * kBlock >= lo_most && b * kBlock + kBlock - 1 <= pos_least, whole = one && full;
       const bool more = b + kWaves <= last;
       if (more) row_next = row_of(b + kWaves);
       if (kEarly && whole) {
@@ -183,7 +186,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
             }
         }
       } else {
-        for (int x = ta; x < tb; ++x) {
+        const int per = full ? tb - ta : 1;
+        for (int x = ta; x < tb; x += per) {     // (beside another request's tokens: one product for all of this one's)
           const int px = positions[x], lx = first_seen(px);
           if ((b + 1) * kBlock <= lx || b * kBlock > px) continue;
           const int key = b * kBlock + (lane & (kBlock - 1));
@@ -207,7 +211,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
 #pragma unroll
           for (int g = 0; g < DG; ++g)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[g][e] = t == x ? ox[g][e] : o[g][e];
+            for (int e = 0; e < 4; ++e) o[g][e] = (unsigned)(t - x) < (unsigned)per ? ox[g][e] : o[g][e];
         }
       }
       row = row_next;
@@ -266,13 +270,27 @@ int xi_attention_f32_lds(int d, int dv) {
   return (int)attn_f32::lds_bytes(16, most, most);
 }
 
+// Tokens a workgroup for `rest` tokens of `seqs` requests: one where a request brings fewer than four on average, else the fewest with
+// which the workgroups are one round of the compute units, at most 16 (token, head) rows: what a tile saves are reads of keys, what it
+// costs are the blocks on its diagonal, a product a token.  Measured, us, 16 heads of 128, tokens a workgroup 1 | 2 | 4 | 8 | 16 (one lane
+// a key): a prompt of 20: 14.0 | 10.0 | 12.5 | 18.7 | 30.5 (13.1); of 128: 64 | 41 | 28 | 21 | 33 (57); of 2,048: 4,435 | 2,313 | 1,313 | 809
+// | 569 (3,781); 300 tokens behind 1,700: 1,119 | 603 | 323 | 214 | 170 (1,293).
+int xi_attention_f32_tile(int rest, int seqs, int nq, int nkv) {
+  const int heads = nq / nkv < 16 ? nq / nkv : 16, most = 16 / heads;
+  const long long a_token = (long long)nkv * ((nq / nkv + 15) / 16);
+  int tile = 1;
+  if ((long long)seqs * 4 <= rest)
+    while (tile < most && ((long long)rest + tile - 1) / tile * a_token > 256) ++tile;
+  return tile;
+}
+
 // The operands of `xi_attention_generic` in float32 with as many key heads as value heads; K and V rows of whole 16-byte pieces.
-// n_seqs: rows of block_tables.  Tiles of several tokens where the step brings several of a request on average; single tokens
-// have a workgroup each.
+// n_seqs: rows of block_tables; lead: tokens at the front that have a workgroup each (single tokens of `lead` requests, which would
+// be walked one after the other in a tile: 30 at 4,000 keys in front of a prompt of 512, 16 heads of 128, 440 us, 3,059 in tiles).  tile: tokens a workgroup of the others (a token's bits do not depend on it), 0: chosen.
 int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, int max_pages,
                      const int* tok_seq, const int* positions, float* out, float scale, int window, int page_size, int n_tok, int nq,
                      int nkv, int d, int dv, float softcap, const float* slopes, const float* sinks, int values_in_keys, int chunk,
-                     int n_seqs, hipStream_t stream) {
+                     int n_seqs, int lead, int tile, hipStream_t stream) {
   XI_CHECK(n_tok >= 0 && nq > 0 && page_size > 0 && max_pages > 0, "attention_f32: bad sizes T=%d nq=%d page=%d max_pages=%d", n_tok, nq,
            page_size, max_pages);
   XI_CHECK(xi_attention_f32_takes(nq, nkv, d, dv) && nkv <= 65535, "attention_f32: %d heads of %d and %d on %d kv heads", nq, d, dv, nkv);
@@ -282,8 +300,11 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
   XI_CHECK(on16(q) && on16(k_cache) && (values_in_keys || on16(v_cache)), "attention_f32: operands must start on 16 bytes");
   if (n_tok == 0) return 0;
   const int heads = nq / nkv < 16 ? nq / nkv : 16;
-  const int tile = (long long)n_seqs * 4 <= n_tok ? 16 / heads : 1;
-  dim3 grid((unsigned)((n_tok + tile - 1) / tile), (unsigned)nkv, (unsigned)((nq / nkv + 15) / 16));
+  const int most_tokens = 16 / heads;
+  XI_CHECK(lead >= 0 && lead <= n_tok && tile >= 0 && tile <= most_tokens, "attention_f32: %d tokens a workgroup, %d of %d alone", tile, lead, n_tok);
+  const int rest = n_tok - lead;
+  if (tile == 0) tile = xi_attention_f32_tile((int)rest, n_seqs - lead, nq, nkv);
+  dim3 grid((unsigned)(lead + (rest + tile - 1) / tile), (unsigned)nkv, (unsigned)((nq / nkv + 15) / 16));
   XI_CHECK(grid.z <= 65535u, "attention_f32: too many heads (%d)", nq);
   const size_t lds = attn_f32::lds_bytes(tile * heads, d, dv);
   const int most = d > dv ? d : dv;
@@ -295,7 +316,7 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
       XI_CHECK(e == hipSuccess, "attention_f32: %s", hipGetErrorString(e));                                                   \
     }                                                                                                                         \
     attn_f32::attention_f32_kernel<DT><<<grid, 64 * attn_f32::kWaves, lds, stream>>>(                                         \
-        q, k_cache, v_cache, block_tables, max_pages, tok_seq, positions, out, scale, window, page_size, n_tok, tile, nq, nkv, d, dv, softcap, \
+        q, k_cache, v_cache, block_tables, max_pages, tok_seq, positions, out, scale, window, page_size, n_tok, lead, tile, nq, nkv, d, dv, softcap, \
         slopes, sinks, values_in_keys, chunk);                                                                                \
   } while (0)
   if (most <= 64) XI_AF(4);

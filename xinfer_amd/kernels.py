@@ -1041,7 +1041,8 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                       scale: float, window: int = 0, out: Optional[torch.Tensor] = None,
                       v_grouped: bool = False, softcap: float = 0.0,
                       slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None,
-                      value_dim: Optional[int] = None, chunk: int = 0, matrix: bool = True) -> torch.Tensor:
+                      value_dim: Optional[int] = None, chunk: int = 0, matrix: bool = True, lead: int = 0,
+                      tile: int = 0) -> torch.Tensor:
     """Causal paged GQA attention for any mix of tokens.  q [T, nq, d]; caches
     [pages, nkv, page_size, d] (the V pool's last size, the value head size, may differ);
     block_tables int32 [B, max_pages]; tok_seq / positions
@@ -1087,13 +1088,14 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         out = torch.empty((T, nq * dv), dtype=q.dtype, device=q.device)
     elif out.shape != (T, nq * dv) or out.dtype != q.dtype:
         raise KernelError("attention: out has the wrong shape or dtype")
-    # float32 at head sizes in steps of 16 up to 256: on the matrix cores (`matrix` False: the kernel for every size)
+    # float32 at head sizes in steps of 16 up to 256: on the matrix cores (`matrix` False: the kernel for every size); the first
+    # `lead` tokens, each of another request, with a workgroup each, the others `tile` a workgroup (0: chosen there)
     if (matrix and q.dtype == torch.float32 and nkk == nkv and not v_grouped and lib().xi_attention_f32_takes(nq, nkv, d, dv)
             and all(t is None or t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache))):
         _ok(lib().xi_attention_f32(
             _p(q), _p(k_cache), _p(v_cache), _p(block_tables), int(block_tables.shape[1]), _p(tok_seq), _p(positions), _p(out),
             ctypes.c_float(scale), int(window), int(page), T, nq, nkv, d, dv, ctypes.c_float(softcap), _p(slopes), _p(sinks),
-            int(v_cache is None), int(chunk), int(block_tables.shape[0]), _stream()))
+            int(v_cache is None), int(chunk), int(block_tables.shape[0]), int(lead), int(tile), _stream()))
         return out
     _ok(lib().xi_attention_generic(
         _p(q), _p(k_cache), _p(v_cache), _code(q, "attention"), _p(block_tables),
@@ -1476,6 +1478,19 @@ def attention_decode_packed_bf16(qkv, q_weight, k_weight, eps, cos, sin, rotary_
     return out
 
 
+def leading_singles(q: torch.Tensor, ctx) -> int:
+    """Sequences at the head of a float32 step of portions that bring one token (the scheduler puts the decoding requests first)."""
+    if q.dtype != torch.float32 or ctx.max_q_len <= 1:
+        return 0
+    lead = ctx.scratch.get("leading_singles")
+    if lead is None:
+        lead, cu = 0, ctx.cu_q_host
+        while lead + 1 < len(cu) and cu[lead + 1] - cu[lead] == 1:
+            lead += 1
+        ctx.scratch["leading_singles"] = lead
+    return lead
+
+
 def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx, group: int,
               scale: float, window: int = 0, v_grouped: bool = False, softcap: float = 0.0,
               slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None,
@@ -1493,7 +1508,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx
     bt = ctx.block_tables[group]
     if v_cache is None:
         return attention_generic(q, k_cache, None, bt, ctx.tok_seq, ctx.positions, scale, window, softcap=softcap,
-                                 slopes=slopes, sinks=sinks, value_dim=value_dim, chunk=chunk)
+                                 slopes=slopes, sinks=sinks, value_dim=value_dim, chunk=chunk, lead=leading_singles(q, ctx))
     if chunk > 0 or softcap > 0 or slopes is not None or sinks is not None or v_cache.shape[3] != d or nkk != nkv:
         dv = int(v_cache.shape[3])
         # the most keys a single token sees, and up to a tile before them
@@ -1564,7 +1579,8 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx
             return attention_biased_bf16(q, k_cache, v_cache, bt, tiles, ctx.cu_q, ctx.ctx_lens, scale, window,
                                          softcap=softcap, slopes=slopes, small=small, split_keys=split, span=span, sinks=sinks, chunk=chunk)
         return attention_generic(q, k_cache, v_cache, bt, ctx.tok_seq, ctx.positions, scale, window,
-                                 v_grouped=v_grouped, softcap=softcap, slopes=slopes, sinks=sinks, chunk=chunk)
+                                 v_grouped=v_grouped, softcap=softcap, slopes=slopes, sinks=sinks, chunk=chunk,
+                                 lead=leading_singles(q, ctx))
     if q.dtype == torch.bfloat16 and v_grouped and mfma_attention_supported(nq, nkv, d, page):
         g = nq // nkv
         if ctx.max_q_len == 1 and decode_attention_takes(nq, nkv, d):
@@ -1602,7 +1618,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx
         return attention_prefill_bf16(q, k_cache, v_cache, bt, tiles, ctx.cu_q, ctx.ctx_lens, scale, window,
                                       out=out, small=small)
     return attention_generic(q, k_cache, v_cache, bt, ctx.tok_seq, ctx.positions, scale, window,
-                             v_grouped=v_grouped)
+                             v_grouped=v_grouped, lead=leading_singles(q, ctx))
 
 
 SKINNY_MAX_ROWS = 64      # most rows the streaming kernel takes
