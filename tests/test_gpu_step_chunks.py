@@ -147,6 +147,27 @@ def test_short_portions_bring_no_plan_to_the_device(monkeypatch):
     assert not [k for plan in kept.values() for k, t in plan.items() if torch.is_tensor(t)]
 
 
+def test_steps_of_both_kinds_make_no_arrays():
+    """Rows of either kind between those of the other are passed over: the bits of each portion by itself, and nothing copied for it."""
+    from xinfer_amd import kernels
+    H, dk, dv = 2, 64, 32
+    for lens in ([40], [64, 90], [1, 1, 40, 70], [70, 3, 1], [5, 33, 1, 64, 31, 200, 2], [64, 1, 64]):
+        x = _portion(len(lens), sum(lens), H, dk, dv)
+        q, k, v, raw, bias, rate_log, state = (t.to(DEV) for t in x)
+        B = len(lens)
+        slots = torch.arange(B, device=DEV).flip(0)
+        cu = [sum(lens[:i]) for i in range(B + 1)]
+        run = lambda st, sl, a, b, n, kept: kernels.linear_scan(
+            q[a:b], k[a:b], v[a:b], st, sl, torch.tensor([sum(n[:i]) for i in range(len(n) + 1)], dtype=torch.int32, device=DEV), H, dk, dv,
+            step=raw[a:b], step_bias=bias, decay_log=rate_log, groups=1, q_lens=n, plan_cache=kept)
+        both, single, kept = state.repeat(B, 1, 1, 1), state.repeat(B, 1, 1, 1), {}
+        got = run(both, slots, 0, cu[B], lens, kept)
+        for i in range(B):
+            assert torch.equal(got[cu[i]:cu[i + 1]], run(single, slots[i:i + 1].contiguous(), cu[i], cu[i + 1], lens[i:i + 1], {})), (lens, i)
+        assert torch.equal(both, single), lens
+        assert not [k for plan in kept.values() for k, t in plan.items() if torch.is_tensor(t)]
+
+
 def test_the_rule_takes_what_it_should(monkeypatch):
     """Which portions go where, without a launch."""
     from xinfer_amd import kernels

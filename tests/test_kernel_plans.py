@@ -85,7 +85,8 @@ def test_few_heads_walk_a_long_portion_side_by_side(lens, H, dk, dv, walk, monke
     T = sum(lens)
     t = torch.empty(1, dtype=torch.bfloat16)
     common = (t, t, t, 8, 8, 8, None, None, 1.0, None, t, H, t, t, None, dv, H, 0)
-    done = kernels._step_chunks(common, t, H * dk * dv, torch.arange(len(lens)), lens, {}, t, H, dk, dv, 1.0, 1.0)
+    cu_q = torch.zeros(len(lens) + 1, dtype=torch.int32)
+    done = kernels._step_chunks(common, t, H * dk * dv, torch.arange(len(lens)), cu_q, lens, {}, t, H, dk, dv, 1.0, 1.0)
     assert done == (not walk and max(lens) >= kernels.STEP_FROM)
     assert taken[:1] == (["xi_step_chunks"] if done else [])
 

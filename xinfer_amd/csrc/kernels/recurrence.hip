@@ -70,14 +70,14 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     int group_heads, const float* __restrict__ state_in, long long in_stride, const long long* __restrict__ in_idx,
     float* __restrict__ state_out, long long out_stride, const long long* __restrict__ out_idx,
     const int* __restrict__ first, const int* __restrict__ last, float* __restrict__ out, float* __restrict__ decay_out,
-    int H, int dk, int dv, float q_scale, float k_scale) {
+    int H, int dk, int dv, float q_scale, float k_scale, int skip_from) {
   __shared__ __attribute__((aligned(16))) float qs[2][kScanWaves * 64], ks[2][kScanWaves * 64], as[2][kScanWaves * 64];
   __shared__ float part[2][kScanWaves][COLS * kScanCols];
   __shared__ float npart[2][kScanWaves];
   const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * (COLS * kScanCols) + (threadIdx.x & 63);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t0 = first[b], t1 = last[b];
-  if (t1 <= t0) return;
+  if (t1 <= t0 || t1 - t0 >= skip_from) return;
   const bool ones = v_cols < dv;            // the state's last column is the keys' own sum
   bool col[COLS];
 #pragma unroll
@@ -337,7 +337,8 @@ int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k
                    int group_heads, const float* state_in,
                    long long in_stride, const long long* in_idx, float* state_out, long long out_stride,
                    const long long* out_idx, const int* first, const int* last, float* out, float* decay_out, int n_items, int H,
-                   int dk, int dv, float q_scale, float k_scale, int act, hipStream_t stream) {
+                   int dk, int dv, float q_scale, float k_scale, int act, int skip_from, hipStream_t stream) {
+  if (skip_from <= 0) skip_from = 0x7fffffff;
   XI_CHECK(n_items >= 0 && H > 0 && dk > 0 && dv > 0, "linear_scan: bad sizes items=%d H=%d dk=%d dv=%d", n_items, H, dk, dv);
   XI_CHECK(dk <= kScanWaves * 64, "linear_scan: key heads of up to %d channels, not %d", kScanWaves * 64, dk);
   XI_CHECK((z != nullptr) + (head_decay != nullptr) + (step != nullptr) + (gates != nullptr) == 1,
@@ -365,7 +366,7 @@ int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k
 #define XI_SCAN_ARGS(TT)                                                                                                      \
       (const TT*)q, q_stride, (const TT*)k, k_stride, (const TT*)v, v_stride, z, z_bias, inv_tau, head_decay, (const TT*)step,    \
       step_stride, step_bias, decay_log, gates, v_cols, group_heads, state_in, in_stride,                                                    \
-      in_idx, state_out, out_stride, out_idx, first, last, out, decay_out, H, dk, dv, q_scale, k_scale
+      in_idx, state_out, out_stride, out_idx, first, last, out, decay_out, H, dk, dv, q_scale, k_scale, skip_from
 #define XI_SCAN_F(TT, R, COLS, RES)                                                                                           \
   do {                                                                                                                        \
     if (z) linear_scan_kernel<TT, R, false, false, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));     \

@@ -48,7 +48,7 @@ struct Args {
   const long long* slots;
   const int *first, *last;
   float* out;
-  int H, dv, group_heads;
+  int H, dv, group_heads, least;
   float scale, k_scale;                        // q_scale * k_scale; k_scale
 };
 
@@ -84,6 +84,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void step_chunks_kernel(const Args 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, j = lane >> 4;
   const int t_end = A.last[p];
+  if (t_end - A.first[p] < A.least) return;    // (walked token by token, by another launch)
   const int qk0 = (h / A.group_heads) * DK;
   const float bias = A.bias[h], rate = -expf(A.rate_log[h]);
   float* S = A.state + (size_t)A.slots[p] * A.slot_stride + (size_t)h * DK * A.dv;
@@ -352,11 +353,12 @@ int xi_step_chunks_takes(int dk, int dv) { return dk > 0 && dk <= 128 && dk % 32
 
 // q, k [T, .] with (H / group_heads) dk columns, v [T, .] with H dv, raw [T, .] with H, bfloat16 rows `*_stride` elements apart;
 // bias, rate_log float32 [H]; portion p: tokens first[p] .. last[p] - 1, its request's state at state + slots[p] * slot_stride
-// ([H, dk, dv] float32, read and left behind the portion); out float32 [T, H, dv].
+// ([H, dk, dv] float32, read and left behind the portion); out float32 [T, H, dv].  Portions of fewer than `least` tokens are
+// left alone.
 int xi_step_chunks(const void* q, long long q_stride, const void* k, long long k_stride, const void* v, long long v_stride,
                    const void* raw, long long raw_stride, const float* bias, const float* rate_log, float* state, long long slot_stride,
                    const long long* slots, const int* first, const int* last, int n_portions, float* out, int H, int dk, int dv,
-                   int group_heads, float q_scale, float k_scale, hipStream_t stream) {
+                   int group_heads, int least, float q_scale, float k_scale, hipStream_t stream) {
   XI_CHECK(xi_step_chunks_takes(dk, dv) && H > 0 && H <= 65535 && group_heads > 0 && H % group_heads == 0 && dv / step::kCols <= 65535,
            "step_chunks: %d heads of %d by %d in groups of %d are not taken", H, dk, dv, group_heads);
   XI_CHECK(q_stride % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 &&
@@ -367,7 +369,7 @@ int xi_step_chunks(const void* q, long long q_stride, const void* k, long long k
   XI_CHECK(k_scale != 0.f, "step_chunks: keys with a factor of 0");
   if (n_portions == 0) return 0;
   const step::Args A{(const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)raw, q_stride, k_stride, v_stride, raw_stride, bias,
-                     rate_log, state, slot_stride, slots, first, last, out, H, dv, group_heads, q_scale * k_scale, k_scale};
+                     rate_log, state, slot_stride, slots, first, last, out, H, dv, group_heads, least, q_scale * k_scale, k_scale};
   const dim3 grid((unsigned)n_portions, (unsigned)H, (unsigned)(dv / step::kCols));
 #define XI_SC(DKS)                                                                                                           \
   do {                                                                                                                       \

@@ -362,7 +362,7 @@ def step_walk_ahead(q_lens, H: int, dk: int, dv: int) -> bool:
     return chain > 107 + 0.15 * dk + (0.0011 + 0.000013 * dk) * sum(lens) * H * -(-dv // 64) + 1.1 * one_by_one
 
 
-def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale) -> bool:
+def _step_chunks(common, state, slot_stride, state_slots, cu_q, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale) -> bool:
     """`linear_scan` for a step with long portions in bfloat16 under a step size a token and head: the long ones chunk by chunk on
     the matrix cores, the others in one piece.  False: nothing was done (sizes, rows or lengths that it does not take)."""
     q, k, v, qs, ks, vs, step, ss, step_bias, decay_log = (common[i] for i in (0, 1, 2, 3, 4, 5, 10, 11, 12, 13))
@@ -374,43 +374,36 @@ def _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, ou
         return False
     key = ("step_chunk_plan", STEP_FROM)
     plan = plan_cache.get(key) if plan_cache is not None else None
-    if plan is None:
-        whole, long = step_chunk_plan(q_lens)
-        plan = dict(L=len(long), W=len(whole))
-        if long:                 # (a step of short portions wants none of these on the device)
-            starts = [0]
-            for n in q_lens:
-                starts.append(starts[-1] + int(n))
-            rows = long + whole
-            L, W = len(long), len(whole)
-            i32 = torch.tensor([starts[b] for b in rows] + [starts[b + 1] for b in rows], dtype=torch.int32).to(q.device)
-            slots = state_slots.index_select(0, torch.tensor(rows, dtype=torch.int64).to(q.device))
-            plan.update(first=i32[:L + W], last=i32[L + W:], slots=slots)
+    if plan is None:     # from the first to the last row of either kind, straight from the step's own arrays: rows of the other kind between
+        whole, long = step_chunk_plan(q_lens)          # them are passed over (arrays of their own are copied to a device that works)
+        plan = dict(long=(long[0], long[-1] - long[0] + 1) if long else None, whole=(whole[0], whole[-1] - whole[0] + 1) if whole else None)
         if plan_cache is not None:
             plan_cache[key] = plan
-    L, W = plan["L"], plan["W"]
-    if not L:
+    if plan["long"] is None:
         return False
-    ll = ctypes.c_longlong
+    ll, (b0, n) = ctypes.c_longlong, plan["long"]
+    at, slots = (lambda b: cu_q.data_ptr() + 4 * b), (lambda b: ctypes.c_void_p(state_slots.data_ptr() + 8 * b))
     _ok(lib().xi_step_chunks(_p(q), ll(qs), _p(k), ll(ks), _p(v), ll(vs), _p(step), ll(ss), _p(step_bias), _p(decay_log), _p(state),
-                             ll(slot_stride), _p(plan["slots"]), _p(plan["first"]), _p(plan["last"]), L, _p(out), H, dk, dv,
-                             int(common[16]), ctypes.c_float(q_scale), ctypes.c_float(k_scale), _stream()))
-    if W:
-        _scan_launch(*common, state, slot_stride, plan["slots"][L:], state, slot_stride, plan["slots"][L:],
-                     plan["first"][L:].data_ptr(), plan["last"][L:].data_ptr(), out, None, W, H, dk, dv, q_scale, k_scale)
+                             ll(slot_stride), slots(b0), ctypes.c_void_p(at(b0)), ctypes.c_void_p(at(b0 + 1)), n, _p(out), H, dk, dv,
+                             int(common[16]), STEP_FROM, ctypes.c_float(q_scale), ctypes.c_float(k_scale), _stream()))
+    if plan["whole"]:
+        b0, n = plan["whole"]
+        own = state_slots[b0:b0 + n]
+        _scan_launch(*common, state, slot_stride, own, state, slot_stride, own, at(b0), at(b0 + 1), out, None, n, H, dk, dv,
+                     q_scale, k_scale, STEP_FROM)
     return True
 
 
 def _scan_launch(q, k, v, qs, ks, vs, z, z_bias, tau, head_decay, step, ss, step_bias, decay_log, gates, v_cols, group_heads, act,
                  state_in, in_stride, in_idx, state_out, out_stride, out_idx,
-                 first, last, out, decay_out, items, H, dk, dv, q_scale, k_scale):
+                 first, last, out, decay_out, items, H, dk, dv, q_scale, k_scale, skip_from=0):
     _ok(lib().xi_linear_scan(_p(q), ctypes.c_longlong(qs), _p(k), ctypes.c_longlong(ks), _p(v), ctypes.c_longlong(vs),
                              _code(q, "linear_scan"), _p(z), _p(z_bias), ctypes.c_float(tau), _p(head_decay),
                              _p(step), ctypes.c_longlong(ss), _p(step_bias), _p(decay_log), _p(gates), int(v_cols),
                              int(group_heads), _p(state_in),
                              ctypes.c_longlong(in_stride), _p(in_idx), _p(state_out), ctypes.c_longlong(out_stride),
                              _p(out_idx), ctypes.c_void_p(first), ctypes.c_void_p(last), _p(out), _p(decay_out), int(items),
-                             H, dk, dv, ctypes.c_float(q_scale), ctypes.c_float(k_scale), int(act), _stream()))
+                             H, dk, dv, ctypes.c_float(q_scale), ctypes.c_float(k_scale), int(act), int(skip_from), _stream()))
 
 
 def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor,
@@ -500,7 +493,7 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     out = torch.empty((T, H, dv), dtype=torch.float32, device=q.device)
     slot_stride = int(state.stride(0)) if state.shape[0] > 1 else H * dk * dv
     common = (q, k, v, qs, ks, vs, z, z_bias, tau, head_decay, step, ss, step_bias, decay_log, gates, vc, H // G, int(bool(silu)))
-    if q_lens is not None and _step_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
+    if q_lens is not None and _step_chunks(common, state, slot_stride, state_slots, cu_q, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
         return out
     if q_lens is not None and _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
         return out
