@@ -366,21 +366,21 @@ def _step_chunks(common, state, slot_stride, state_slots, cu_q, q_lens, plan_cac
     """`linear_scan` for a step with long portions in bfloat16 under a step size a token and head: the long ones chunk by chunk on
     the matrix cores, the others in one piece.  False: nothing was done (sizes, rows or lengths that it does not take)."""
     q, k, v, qs, ks, vs, step, ss, step_bias, decay_log = (common[i] for i in (0, 1, 2, 3, 4, 5, 10, 11, 12, 13))
-    if (not STEP_MFMA or SCAN_CHUNK <= 0 or q.dtype != torch.bfloat16 or step is None or common[15] != dv or common[17]
+    if step is None or max(q_lens, default=0) < STEP_FROM:
+        return False
+    if (not STEP_MFMA or SCAN_CHUNK <= 0 or q.dtype != torch.bfloat16 or common[15] != dv or common[17]
             or not lib().xi_step_chunks_takes(dk, dv) or qs % 8 or ks % 8 or vs % 8 or k_scale == 0.0
             or any(t.data_ptr() % 16 for t in (q, k, v))):
         return False
-    if max(q_lens, default=0) > STEP_CHAIN and step_walk_ahead(q_lens, H, dk, dv):
+    if max(q_lens) > STEP_CHAIN and step_walk_ahead(q_lens, H, dk, dv):
         return False
     key = ("step_chunk_plan", STEP_FROM)
     plan = plan_cache.get(key) if plan_cache is not None else None
     if plan is None:     # from the first to the last row of either kind, straight from the step's own arrays: rows of the other kind between
         whole, long = step_chunk_plan(q_lens)          # them are passed over (arrays of their own are copied to a device that works)
-        plan = dict(long=(long[0], long[-1] - long[0] + 1) if long else None, whole=(whole[0], whole[-1] - whole[0] + 1) if whole else None)
+        plan = dict(long=(long[0], long[-1] - long[0] + 1), whole=(whole[0], whole[-1] - whole[0] + 1) if whole else None)
         if plan_cache is not None:
             plan_cache[key] = plan
-    if plan["long"] is None:
-        return False
     ll, (b0, n) = ctypes.c_longlong, plan["long"]
     at, slots = (lambda b: cu_q.data_ptr() + 4 * b), (lambda b: ctypes.c_void_p(state_slots.data_ptr() + 8 * b))
     _ok(lib().xi_step_chunks(_p(q), ll(qs), _p(k), ll(ks), _p(v), ll(vs), _p(step), ll(ss), _p(step_bias), _p(decay_log), _p(state),
@@ -797,6 +797,7 @@ def moe_experts_library(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
 
 
 
+@functools.lru_cache(maxsize=4096)
 def moe_tiled_takes(T: int, top: int, E: int, H: int, F: int, gated: bool) -> bool:
     """Whether `moe_experts_tiled` takes a step's sizes: both products in whole tiles of 64 k, experts' numbers as `moe_sort` has them."""
     takes = lib().xi_moe_tile_takes
@@ -861,21 +862,22 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     bm = max(bm1, bm2)                   # the tiles of the sort; a product whose workgroups take fewer rows cuts them
     most = int(lib().xi_moe_tiles_most(P, E, bm))
     ints = torch.empty((2 * P + 5 * most + 1,), dtype=torch.int32, device=x.device)
-    at = [0, P, 2 * P] + [2 * P + i * most for i in range(1, 6)] + [2 * P + 5 * most + 1]
-    order, slot_of, t_e, t_r0, t_n, t_f, t_c, n_tiles = (ints[a:b] for a, b in zip(at, at[1:]))
-    _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
-                          _p(t_c), _stream()))
+    at = ints.data_ptr()                 # (addresses, not slices: eight of these cost the host 10 us)
+    order, slot_of, n_tiles = ctypes.c_void_p(at), ctypes.c_void_p(at + 4 * P), ctypes.c_void_p(at + 4 * (2 * P + 5 * most))
+    t_e, t_r0, t_n, t_f, t_c = (ctypes.c_void_p(at + 4 * (2 * P + i * most)) for i in range(5))
+    _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, order, slot_of, t_e, t_r0, t_n, n_tiles, t_f,
+                          t_c, _stream()))
     wt_in = wt.contiguous() if weigh_input else None
     mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
-    _ok(lib().xi_moe_tile(_p(rows), ctypes.c_longlong(T), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
-                          _p(t_c), most, _p(mid), F, H, bm1, bm // bm1, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
+    _ok(lib().xi_moe_tile(_p(rows), ctypes.c_longlong(T), order, top, _p(gate_up), t_e, t_r0, t_n, n_tiles, t_f,
+                          t_c, most, _p(mid), F, H, bm1, bm // bm1, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
     y = torch.empty((P, H), dtype=torch.float32, device=x.device)
-    _ok(lib().xi_moe_tile(_p(mid), ctypes.c_longlong(P), _p(order), top, _p(down), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _p(t_f),
-                          _p(t_c), most, _p(y), H, F, bm2, bm // bm2, 0, 0, None, _stream()))
+    _ok(lib().xi_moe_tile(_p(mid), ctypes.c_longlong(P), order, top, _p(down), t_e, t_r0, t_n, n_tiles, t_f,
+                          t_c, most, _p(y), H, F, bm2, bm // bm2, 0, 0, None, _stream()))
     out = torch.empty((T, H), dtype=torch.float32, device=x.device)
     if weigh_input:
         wt = torch.ones_like(wt)
-    _ok(lib().xi_moe_combine(_p(y), _p(slot_of), _p(wt), _p(out), T, H, top, _p(idx), E, _p(rows if identity else None), _p(add), _stream()))
+    _ok(lib().xi_moe_combine(_p(y), slot_of, _p(wt), _p(out), T, H, top, _p(idx), E, _p(rows if identity else None), _p(add), _stream()))
     return out
 
 
