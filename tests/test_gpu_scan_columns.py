@@ -93,11 +93,37 @@ def test_other_decays_with_two_columns_a_lane(how, dtype, H, dk, vc):
         assert float(((st[i].double() - s).abs() / s_sizes).max()) < bound
 
 
-@pytest.mark.parametrize("H,dk,dv,lens", [(2, 100, 70, [300, 5, 130]), (8, 64, 96, [1030, 127, 1]), (1, 128, 256, [129, 64])])
-def test_short_chunks(H, dk, dv, lens):
-    """Chunks of a quarter and a half of the usual tokens, last ones of one and two tokens, beside portions in one piece, against float64."""
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,dk,dv", [(8, 128, 256), (2, 100, 70)])
+def test_a_portion_alone_and_beside_others(H, dk, dv, dtype):
+    """What a request gets, and the state left in its slot, do not depend on the other portions of the step: the same bits."""
     from xinfer_amd import kernels
-    assert kernels.scan_chunk_for(lens, H) < kernels.SCAN_CHUNK
+    g = torch.Generator().manual_seed(H + dk)
+    lens = [300, 2, 129, 1030, 64, 2300]
+    T, B = sum(lens), len(lens)
+    q, k, v = (torch.randn(T, H * n, generator=g).to(dtype).to(DEV) for n in (dk, dk, dv))
+    z, state = (torch.randn(T, H * dk, generator=g) + 1.5).to(DEV), torch.randn(B, H, dk, dv, generator=g).to(DEV)
+    first = [sum(lens[:b]) for b in range(B)]
+
+    def walk(rows):
+        at = torch.cat([torch.arange(first[b], first[b] + lens[b]) for b in rows]).to(DEV)
+        own = [lens[b] for b in rows]
+        cu = torch.tensor([sum(own[:i]) for i in range(len(own) + 1)], dtype=torch.int32, device=DEV)
+        st = state[rows].clone()
+        o = kernels.linear_scan(q[at], k[at], v[at], st, torch.arange(len(rows), device=DEV), cu, H, dk, dv, z=z[at], tau=8.0,
+                                q_scale=dk ** -0.5, q_lens=own)
+        return dict(zip(rows, zip(o.split(own), st)))
+
+    everyone = walk(list(range(B)))
+    for rows in [[b] for b in range(B)] + [[2, 0], [3, 1, 0]]:
+        for b, (o, s) in walk(rows).items():
+            assert torch.equal(o, everyone[b][0]) and torch.equal(s, everyone[b][1]), (rows, lens[b])
+
+
+@pytest.mark.parametrize("H,dk,dv,lens", [(2, 100, 70, [300, 5, 130]), (8, 64, 96, [1030, 127, 1]), (1, 128, 256, [129, 64])])
+def test_last_chunks_of_a_few_tokens(H, dk, dv, lens):
+    """Last chunks of one and two tokens and more, beside portions in one piece, against float64."""
+    from xinfer_amd import kernels
     g = torch.Generator().manual_seed(H + dk)
     T, B = sum(lens), len(lens)
     q, k, v = (torch.randn(T, H * n, generator=g).to(torch.bfloat16) for n in (dk, dk, dv))

@@ -111,16 +111,6 @@ def test_most_tiles_of_routed_experts(bm):
             assert -(-P // bm) <= most(P, E, bm)
 
 
-def test_chunks_of_a_walk_follow_from_the_pairs():
-    """A quarter of a chunk's tokens, a half or all of them by the (chunk, head) pairs; shorter portions count for nothing and stay whole."""
-    chunk = kernels.scan_chunk_for
-    assert [chunk([n], 8) for n in (127, 128, 1023, 1024, 2047, 2048, 9000)] == [16, 16, 16, 32, 32, 64, 64]
-    assert chunk([1000, 1048], 8) == 64 and chunk([1000, 1047, 127, 1], 8) == 32 and chunk([64] * 500, 8) == 16
-    whole, long, chunks = kernels.scan_chunk_plan([1, 130, 64, 127, 300], 16, 64)
-    assert whole == [0, 2, 3] and long == [(1, 0, 9), (4, 9, 19)]
-    assert chunks[:9] == [(16 * i, 16) for i in range(8)] + [(128, 2)] and chunks[-1] == (288, 12)
-
-
 def test_float32_attention_tiles():
     """Tokens a workgroup: the fewest that make one round of workgroups, at most 16 (token, head) rows, one for single tokens."""
     from xinfer_amd import kernels

@@ -266,25 +266,12 @@ def _columns(t: torch.Tensor, width: int, what: str):
 
 
 SCAN_CHUNK = 64           # tokens of a chunk of a long portion (see `linear_scan`); 0: every portion is walked in one piece
-SCAN_BUSY = 256           # (chunk, head) pairs of a step under which its chunks are shorter
 SCAN_CHUNKS_MOST = 512    # chunks of a step at most (their states are kept side by side): longer steps get longer chunks
 
 
-def scan_chunk_for(q_lens, heads: int) -> int:
-    """Tokens of a chunk of `linear_scan`: SCAN_CHUNK, or a half or a quarter of it where a step makes few (chunk, head) pairs: a chunk
-    then is a chain of tokens with hardly another beside it on its compute unit.  Measured on MI355X, us, all three launches, chunks of
-    64 | 32 | 16 (decay a channel, heads of 128 by 256): 8 heads, 300 tokens 137 | 91 | 67, 800 161 | 163 | 147, 1,974 251 | 247 | 323, 2,048
-    217 | 252 | 356; 4 heads, 300 134 | 80 | 62, 1,974 173 | 184 | 158, 4,000 353 | 274 | 365; 4 heads of 64 by 128, 800 115 | 69 | 54, 2,048
-    124 | 94 | 96.  Of the heads and lengths alone: a value column's bits do not depend on how many there are."""
-    if SCAN_CHUNK < 64:
-        return SCAN_CHUNK
-    pairs = sum(int(n) for n in q_lens if int(n) >= 2 * SCAN_CHUNK) // SCAN_CHUNK * heads
-    return SCAN_CHUNK // 4 if pairs < SCAN_BUSY // 2 else SCAN_CHUNK // 2 if pairs < SCAN_BUSY else SCAN_CHUNK
-
-
-def scan_chunk_plan(q_lens, chunk: Optional[int] = None, least: int = 0):
+def scan_chunk_plan(q_lens, chunk: Optional[int] = None):
     """How a step's portions are walked by `linear_scan`: (whole, long, chunks) with `whole` the batch rows walked in
-    one piece (single tokens and portions of less than two chunks, or than two of `least`) and, for the others, `long` = [(row, first chunk,
+    one piece (single tokens and portions of less than two chunks) and, for the others, `long` = [(row, first chunk,
     number of chunks)] and `chunks` = [(first token within the portion, tokens)] in the order of their numbers."""
     chunk = SCAN_CHUNK if chunk is None else int(chunk)
     total = sum(int(n) for n in q_lens)
@@ -293,7 +280,7 @@ def scan_chunk_plan(q_lens, chunk: Optional[int] = None, least: int = 0):
     whole, long, chunks = [], [], []
     for b, n in enumerate(q_lens):
         n = int(n)
-        if chunk <= 0 or n < 2 * max(chunk, least):
+        if chunk <= 0 or n < 2 * chunk:
             whole.append(b)
             continue
         count = -(-n // chunk)
@@ -455,7 +442,7 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     state float32 [slots, H, dk, dv] (slots may be strided); state_slots int64 [B]; cu_q int32 [B + 1].
     Returns o float32 [T, H, dv].
     `q_lens` (the host's copy of the portions' lengths; None: nothing of the step is read on the host, as a step
-    of single tokens wants it): portions of two chunks and more (`SCAN_CHUNK`) are cut into chunks (`scan_chunk_for`) that are walked
+    of single tokens wants it): portions of two chunks and more (`SCAN_CHUNK`) are cut into chunks that are walked
     side by side in three launches (each chunk's own share from a zero state; the states the chunks start from,
     one after the other; the chunks' results), the others in one piece; in bfloat16 with a constant decay per head the long
     ones go through the matrix cores (`xi_decay_chunks`, portions from DECAY_FROM tokens on), and so they do with a step size a
@@ -525,15 +512,12 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
         return out
     if q_lens is not None and _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, out, H, dk, dv, q_scale, k_scale):
         return out
-    whole, long, chunks = None, [], []
-    if q_lens is not None:
-        chunk = scan_chunk_for(q_lens, H)
-        whole, long, chunks = scan_chunk_plan(q_lens, chunk, SCAN_CHUNK)
+    whole, long, chunks = scan_chunk_plan(q_lens) if q_lens is not None else (None, [], [])
     if not long:            # every request in one piece, straight from the step's own arrays
         _scan_launch(*common, state, slot_stride, state_slots, state, slot_stride, state_slots, cu_q.data_ptr(),
                      cu_q.data_ptr() + 4, out, None, B, H, dk, dv, q_scale, k_scale)
         return out
-    key = ("linear_scan_plan", SCAN_CHUNK, chunk)
+    key = ("linear_scan_plan", SCAN_CHUNK)
     plan = plan_cache.get(key) if plan_cache is not None else None
     if plan is None:             # the same for every layer of the step: made once
         starts = [0]
