@@ -123,7 +123,7 @@ def test_tiles_of_the_plan(E, I, P, highs):
         t = tiles.tolist()
         n, many = t[5 * most], t[5 * most + 1]
         assert 0 <= n <= most and t[5 * most + 2] == -1
-        assert many == (2 * n > 3 * sum(c > 0 for c in counts[:E]))
+        assert bool(many) == (2 * n > 3 * sum(c > 0 for c in counts[:E])) and many <= 2
         e, row0, rows, first, count = (t[i * most:i * most + n] for i in range(5))
         assert max(rows, default=0) <= (high or 256)
         at = i = 0
@@ -134,6 +134,22 @@ def test_tiles_of_the_plan(E, I, P, highs):
             assert all(rows[j] == rows[i] for j in mine[:-1]) and all(0 < rows[j] <= rows[i] for j in mine)
             assert all(first[j] == i and count[j] == len(mine) for j in mine)
             at, i = at + counts[x], i + len(mine)
+
+
+@pytest.mark.parametrize("counts,orders", [([1024] * 8, (2, 2)), ([1000] * 16, (2, 2)), ([700, 130] * 4, (1, 1)), ([128] * 8, (0, 0)),
+                                           ([0, 512, 0, 512] * 300, (2, 2)), ([2000] + [60] * 8, (1, 1))])
+def test_orders_of_the_tiles(counts, orders):
+    """Tiles of about one height go an expert after the other, unequal ones the same columns of all experts to every die, single ones in turn."""
+    from xinfer_amd import kernels
+    counts = counts[:1024]
+    E, P = len(counts), sum(counts)
+    dev = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32)[torch.randperm(P, generator=torch.Generator().manual_seed(0))].to(DEV)
+    (h1, m1, c1), (h2, m2, c2) = (kernels._moe_tiles(P, E, 0, n, False) for n in (6144, 4096))
+    order, slot_of = (torch.empty(P, dtype=torch.int32, device=DEV) for _ in range(2))
+    lists = [torch.empty(5 * m + 2, dtype=torch.int32, device=DEV) for m in (m1, m2)]
+    p = kernels._p
+    kernels._ok(kernels.lib().xi_moe_plan(p(dev), P, E, 0, h1, h2, c1, c2, p(order), p(slot_of), p(lists[0]), p(lists[1]), m1, m2, kernels._stream()))
+    assert tuple(int(t[5 * m + 1]) for t, m in zip(lists, (m1, m2))) == orders
 
 
 @pytest.mark.parametrize("E,I", [(1, 0), (63, 2), (64, 0), (65, 1), (1000, 24), (1024, 0)])

@@ -12,9 +12,10 @@
 // holds it; how high tiles may be is chosen on the device from the counts, for each product by its rounds of workgroups.
 // (Tiles of one height for all, chosen from the average: 410 pairs an expert filled two of 256 to 80%, and 490 in four of
 // 128 ran at 0.8 of the larger ones' rate.)  Both products and what stands around them, us, one height | this: 8 gated experts
-// of 6144 at width 4096, 39 to 761 pairs each 582 | 538, 163 to 622 592 | 585, 410 587 | 541, 130 to 399 490 | 398, 326 to 1,244
-// 993 | 970, 512 580 | 580, 1,024 1,045 | 1,068 (even and a multiple of 256: the one place where the order over the dies costs);
-// without a gate 130 to 634 521 | 462, 260 to 1,268 928 | 841.  What is left: rows past an expert's in the tiles (7%), the last
+// of 6144 at width 4096, 39 to 761 pairs each 584 | 539, 163 to 622 595 | 576, 410 596 | 552, 78 to 1,522 989 | 969, 512 584 | 570, 1,024
+// 1,061 | 1,060; without a gate 130 to 634 519 | 457, 260 to 1,268 932 | 838, 1,536 1,116 | 1,161; 16 of 4096 at 2048, 512 each 302 | 290, 1,024 539 |
+// 548, 156 to 3,044 919 | 983 (192 rows where 256 are ahead: the one load of 125 with more than 5% lost); 8 of 1536 at 1024, 1,024 each
+// 113 | 104, 512 55 | 57.  What is left: rows past an expert's in the tiles (7%), the last
 // round of workgroups, and 1 PFLOP/s in between where the dense walk has 1.3.
 //
 // A workgroup owns a tile and BN rows of w; the number of tiles is known on the device alone, and the grid is the most
@@ -37,36 +38,47 @@ __device__ __forceinline__ int lowest(int rows) { return rows <= 64 ? 64 : rows 
 // a round's time, in rows: 1.95 us for 64 k of 256 rows, and what a tile costs beyond its products
 __device__ __forceinline__ int tile_time(int high) { return high + 16; }
 
+// ceil(n / d), n and d > 0, of up to 2^22: the float quotient is one off at most (the compiler's division is three times as many instructions).
+__device__ __forceinline__ int share(int n, int d) {
+  const int m = n + d - 1;
+  int q = (int)((float)m * __builtin_amdgcn_rcpf((float)d));
+  const int left = m - q * d;
+  q += left >= d ? 1 : left < 0 ? -1 : 0;
+  return q;
+}
+
 // The pairs in the order of their experts, and the tiles of the two products: of product i up to high[i] rows (0: chosen here), an expert's all
-// of one height but the last.
+// of one height but the last.  One workgroup, so a chain of dependent instructions: a wave a height, and divisions by a float's reciprocal (2,048
+// pairs on 8 experts 8.8 us with all heights in every thread, 6.6 so; the sort alone, whose tiles were of one height, 4.3).
 __global__ __launch_bounds__(kSortThreads) void moe_plan_kernel(const int* __restrict__ idx, int P, int E, int I, int high1, int high2,
                                                                 int columns1, int columns2, int* __restrict__ order,
                                                                 int* __restrict__ slot_of, int* __restrict__ tiles1,
                                                                 int* __restrict__ tiles2, int most1, int most2) {
   __shared__ int count[kSortExperts], cursor[kSortExperts], across[3][kSortThreads / kWave];
-  __shared__ int total[kHeights][2];
-  const int A = E + I, e = threadIdx.x, lane = e & 63;
-  if (e < 2 * kHeights) total[e >> 1][e & 1] = 0;
+  __shared__ float tiles_of[kHeights], time_of[kHeights];      // of every height: the tiles, and the mean time of one
+  const int A = E + I, e = threadIdx.x, lane = e & 63, wave = e >> 6;
   moe_count_pairs(idx, P, A, count);
   const int pairs = e < A ? count[e] : 0, routed = e < E ? pairs : 0;
   int high[2] = {high1, high2};
+  bool even[2] = {false, false};       // the tiles take about as long as the highest ones would
   if (high1 == 0 || high2 == 0) {
-    // tiles and their time for every height, over the experts
-    if ((e & ~63) < E) {
-#pragma unroll
-      for (int h = 0; h < kHeights; ++h) {
-        int t = (routed + height(h) - 1) / height(h);
-        int cost = t ? t * tile_time(lowest((routed + t - 1) / t)) : 0;
-        t += lane_xor<32>(t), cost += lane_xor<32>(cost);
-        t += lane_xor<16>(t), cost += lane_xor<16>(cost);
-        t += lane_xor<8>(t), cost += lane_xor<8>(cost);
-        t += lane_xor<4>(t), cost += lane_xor<4>(cost);
-        t += lane_xor<2>(t), cost += lane_xor<2>(cost);
-        t += lane_xor<1>(t), cost += lane_xor<1>(cost);
-        if (lane == 0) {
-          atomicAdd(&total[h][0], t);
-          atomicAdd(&total[h][1], cost);
-        }
+    for (int h = wave; h < kHeights; h += blockDim.x >> 6) {
+      const int up_to = h == 0 ? height(0) : h == 1 ? height(1) : h == 2 ? height(2) : h == 3 ? height(3) : height(4);
+      int t = 0, cost = 0;
+      for (int x = lane; x < E; x += kWave) {
+        const int n = share(count[x], up_to);
+        t += n;
+        cost += n ? n * tile_time(lowest(share(count[x], n))) : 0;
+      }
+      t += lane_xor<32>(t), cost += lane_xor<32>(cost);
+      t += lane_xor<16>(t), cost += lane_xor<16>(cost);
+      t += lane_xor<8>(t), cost += lane_xor<8>(cost);
+      t += lane_xor<4>(t), cost += lane_xor<4>(cost);
+      t += lane_xor<2>(t), cost += lane_xor<2>(cost);
+      t += lane_xor<1>(t), cost += lane_xor<1>(cost);
+      if (lane == 0) {
+        tiles_of[h] = (float)t;
+        time_of[h] = t ? (float)cost * __builtin_amdgcn_rcpf((float)t) : 0.f;
       }
     }
     __syncthreads();
@@ -74,32 +86,32 @@ __global__ __launch_bounds__(kSortThreads) void moe_plan_kernel(const int* __res
     for (int i = 0; i < 2; ++i) {
       if (high[i]) continue;
       float least = 0.f;
-      const int columns = i ? columns2 : columns1;
+      const float columns = (float)(i ? columns2 : columns1) * (1.f / kUnits);
 #pragma unroll
       for (int h = 0; h < kHeights; ++h) {
-        const float t = (float)total[h][0], rounds = ceilf(t * (float)columns * (1.f / kUnits));
-        const float cost = t > 0.f ? rounds * (float)total[h][1] / t : 0.f;
+        const float cost = ceilf(tiles_of[h] * columns) * time_of[h];
         if (h == 0 || cost < least) {
           least = cost;
           high[i] = height(h);
+          even[i] = time_of[h] >= 0.97f * (float)tile_time(height(h));
         }
       }
     }
   }
-  const int n1 = (routed + high[0] - 1) / high[0], n2 = (routed + high[1] - 1) / high[1];
+  const int n1 = routed ? share(routed, high[0]) : 0, n2 = routed ? share(routed, high[1]) : 0;
   int before[3] = {pairs, n1, n2};
   moe_sums_before(before, A, across);
   const int busy = __syncthreads_count(routed > 0);
   if (e == A - 1) {
     tiles1[5 * most1] = before[1] + n1;
     tiles2[5 * most2] = before[2] + n2;
-    tiles1[5 * most1 + 1] = 2 * (before[1] + n1) > 3 * busy;
-    tiles2[5 * most2 + 1] = 2 * (before[2] + n2) > 3 * busy;
+    tiles1[5 * most1 + 1] = 2 * (before[1] + n1) > 3 * busy ? 1 + even[0] : 0;
+    tiles2[5 * most2 + 1] = 2 * (before[2] + n2) > 3 * busy ? 1 + even[1] : 0;
   }
   if (e < A) cursor[e] = before[0];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int n = i ? n2 : n1, rows = n ? (routed + n - 1) / n : 0, most = i ? most2 : most1;
+    const int n = i ? n2 : n1, rows = n ? share(routed, n) : 0, most = i ? most2 : most1;
     int* to = (i ? tiles2 : tiles1) + before[1 + i];
     for (int t = 0; t < n; ++t) {
       to[t] = e;
@@ -188,15 +200,19 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
     column = q / count;
     tile = first + (q - column * count);
   };
-  if constexpr (LOW) {                 // consecutive places a die
+  const int order_of = LOW ? 2 : tiles[5 * most + 1];
+  if (order_of == 2) {
+    // Consecutive places a die, an expert after the other: a die's L2 holds an expert's rows and the rows of w that its tiles share.  For
+    // tiles that take about as long as each other (within 3%, the list says): 16 experts of 4096 at width 2048, 1,024 rows each 577 us the other way,
+    // 547 so, 2,048 each 1,139 and 1,075; 8 gated ones of 1536 at width 1024, 1,024 each 114 and 108.
     const int total = n_tiles * columns, per_die = (total + 7) >> 3, place = die * per_die + in_die;
     if (in_die >= per_die || place >= total) return;
     find(place, columns);
   } else {
-    // Every die gets the same columns of all experts, so that their heights come out even over the dies; columns that do not
-    // share out go round in tiles, and so do all where few experts have a second tile to share w with (64 rows an expert
-    // 290 us in that order, 310 an expert after the other; 1,024 rows 1,138 and 1,073).
-    const int whole = tiles[5 * most + 1] ? columns >> 3 : 0, rest = columns - 8 * whole;
+    // Tiles of unequal height: every die gets the same columns of all experts, so that the heights come out even over the dies; columns that do
+    // not share out go round in tiles, and so do all where few experts have a second tile to share w with (64 rows an expert
+    // 290 us in that order, 310 an expert after the other).
+    const int whole = order_of == 1 ? columns >> 3 : 0, rest = columns - 8 * whole;
     if (in_die < whole * n_tiles) {
       find(in_die, whole);
       column += die * whole;
@@ -241,7 +257,7 @@ int xi_moe_tile_takes(long long rows_x, int N, int K, int gated) {
 
 // idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P] and the tiles of the two products, int32
 // [5 most + 2] each: expert, first slot and rows of each, the first tile of its expert and how many that has, how many there are in all, and
-// whether that is more than one and a half an expert with any.  high: most rows of a tile, 0: chosen from the counts on the
+// their order over the dies: 0 up to one and a half an expert with any, 2 where they are of about one height, 1 otherwise.  high: most rows of a tile, 0: chosen from the counts on the
 // device, of 128 to 256, for that many columns of workgroups; most: xi_moe_tiles_most for high or for 128.
 int xi_moe_plan(const int* idx, int P, int E, int I, int high1, int high2, int columns1, int columns2, int* order, int* slot_of, int* tiles1,
                 int* tiles2, int most1, int most2, hipStream_t stream) {
