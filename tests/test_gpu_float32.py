@@ -74,6 +74,45 @@ def test_product_parts(M, N, K):
         assert torch.equal(again.nan_to_num(1.5, 2.5, 3.5), z.nan_to_num(1.5, 2.5, 3.5)), f
 
 
+# tiles of 32 and of 64 rows for short K: edges of tiles, one step, an odd number of steps, rows that are not on 16 bytes
+@pytest.mark.parametrize("M,N,K", [(3, 5, 16), (33, 70, 3), (700, 1024, 100), (1300, 301, 256), (4097, 4096, 16), (10007, 130, 96), (20000, 129, 1024),
+                                   (70001, 65, 33), (5000, 300, 2080)])
+def test_short_products(M, N, K):
+    from xinfer_amd import kernels
+    assert kernels.gemm_f32_form(M, N, K) == 5
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, w, base = (torch.randn(s, generator=g, device=DEV) for s in ((M, K), (N, K), (M, N)))
+    y = kernels.gemm_tn(x, w)
+    for f in (2, 3, 4):
+        assert torch.equal(kernels.gemm_tn(x, w, form=f), y), f
+    size = x.double().abs() @ w.double().abs().T
+    assert float(((y.double() - x.double() @ w.double().T).abs() / size).max()) < (-(-K // 256) + 5) * 2.0 ** -23       # as above
+    assert torch.equal(kernels.gemm_tn(x, w, out=base.clone(), accumulate=True), base + y)
+    flat = torch.zeros(M * K + 1, device=DEV)
+    flat[1:] = x.reshape(-1)
+    assert torch.equal(kernels.gemm_tn(flat[1:].view(M, K), w), y)
+    x[M // 2, K - 1], x[M - 1, 0], w[N - 1, 0] = float("inf"), float("nan"), 3.0
+    z, want = kernels.gemm_tn(x, w), x.double() @ w.double().T
+    assert torch.equal(z.isnan(), want.isnan()) and torch.equal(z.isposinf(), want.isposinf()) and torch.equal(z.isneginf(), want.isneginf())
+    others = torch.arange(M, device=DEV)[(torch.arange(M, device=DEV) != M // 2) & (torch.arange(M, device=DEV) != M - 1)]
+    assert torch.equal(z[others][:, :N - 1], y[others][:, :N - 1])
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 16, 4096), (10007, 16, 1024), (4096, 128, 1024), ((1 << 24) + 5, 3, 4)])
+def test_many_rows_of_few_features(M, N, K):
+    """The kernel for few rows over many blocks of rows, on all dies; more rows than its workgroups make a launch."""
+    from xinfer_amd import kernels
+    assert kernels.gemm_f32_form(M, N, K) < 2 or M > 1 << 20
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    y = kernels.gemm_tn(x, w)
+    size = x.double().abs() @ w.double().abs().T
+    assert float(((y.double() - x.double() @ w.double().T).abs() / size).max()) < (-(-K // 256) + 5) * 2.0 ** -23
+    if M < 1 << 20:
+        assert torch.equal(kernels.gemm_tn(x, w, form=2), y)
+    assert torch.equal(kernels.gemm_tn(x[-50:], w), y[-50:])
+
+
 def test_product_form_refused():
     from xinfer_amd import kernels
     x, w = torch.zeros(65, 32, device=DEV), torch.zeros(8, 32, device=DEV)

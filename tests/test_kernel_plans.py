@@ -130,3 +130,15 @@ def test_leading_singles():
     assert kernels.leading_singles(f, ctx([0, 1, 2, 9, 10], 7)) == 2
     assert kernels.leading_singles(f, ctx([0, 7, 8], 7)) == 0
     assert kernels.leading_singles(f, ctx((), 1)) == 0 and kernels.leading_singles(b, ctx([0, 1, 9], 8)) == 0
+
+
+def test_float32_product_forms():
+    """Tiles for short K and narrow outputs of many rows, the kernel for few rows, and the cut tiles, by size; every launch within 2^32 threads."""
+    from xinfer_amd import kernels
+    form = kernels.gemm_f32_form
+    assert form(1 << 20, 16, 128) == 5 and form(1 << 29, 16, 4096) == 5 and form(2048, 1024, 16) == 5
+    assert form(8, 4096, 4096) == 0 and form(8, 24576, 4096) == 1 and form(4096, 16, 4096) == 0
+    assert form(200, 4096, 4096) == 2 and form(562, 151936, 4096) == 3 and form(562, 4096, 4096) == 4
+    assert form(8, 151936, 4096) == 1 and form(32, 24576, 4096) == 1          # wide outputs of few rows: bound by the weights
+    scratch = lambda M, N, K: int(kernels.lib().xi_gemm_f32_scratch(M, N, K, -1))
+    assert scratch(1 << 20, 16, 128) == 0 and scratch(562, 4096, 4096) == 6 * 4096 * 562 and scratch(100_000, 4096, 4096) == 6 * 4096 * 2048

@@ -1123,10 +1123,21 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return out
 
 
-def gemm_f32_form(M: int, N: int) -> int:
-    """The form in which `gemm_tn` makes a float32 product of M rows and N features: 0, 1 the kernel for few rows with up to 16 or
-    up to 48 features a workgroup; 2, 3, 4 tiles of 64, 96 and 80 to 128 rows by 128 features.  All give the same bits."""
-    return int(lib().xi_gemm_f32_form(int(M), int(N)))
+def gemm_f32_form(M: int, N: int, K: int = 4096) -> int:
+    """The form in which `gemm_tn` makes a float32 product of M rows, N features and K: 0, 1 the kernel for few rows with up to 16 or
+    up to 48 features a workgroup; 2, 3, 4 tiles of 64, 96 and 80 to 128 rows by 128 features; 5 tiles of 64 by 64 for narrow outputs of many
+    rows and for short K.  All give the same bits."""
+    return int(lib().xi_gemm_f32_form(int(M), int(N), int(K)))
+
+
+_NO_BYTES = (0, ctypes.c_void_p(0), ctypes.c_longlong(0))
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_f32_scratch(M: int, N: int, K: int, form: int):
+    """Bytes for x in the parts that the tiles multiply, with what `xi_gemm_tn` is given where there are none."""
+    nbytes = int(lib().xi_gemm_f32_scratch(M, N, K, form))
+    return (nbytes, None, ctypes.c_longlong(nbytes)) if nbytes else _NO_BYTES
 
 
 def gemm_tn(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
@@ -1147,12 +1158,12 @@ def gemm_tn(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
         out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
     elif out.shape != (M, N) or (out_dtype is not None and out.dtype != out_dtype):
         raise KernelError("gemm: out has the wrong shape or dtype")
-    cut, nbytes = None, 0
-    if x.dtype == torch.float32:            # x in the parts that the tiles multiply
-        nbytes = int(lib().xi_gemm_f32_scratch(M, N, K, int(form)))
-        cut = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
+    nbytes, cut, size = _gemm_f32_scratch(M, N, K, int(form)) if x.dtype == torch.float32 else _NO_BYTES
+    if nbytes:
+        scratch = torch.empty((nbytes,), dtype=torch.uint8, device=x.device)
+        cut = _p(scratch)
     _ok(lib().xi_gemm_tn(_p(x), _p(w), _p(out), M, N, K, _code(x, "gemm"), _code(out, "gemm"),
-                         int(bool(accumulate)), int(form), _p(cut), ctypes.c_longlong(nbytes), _stream()))
+                         int(bool(accumulate)), int(form), cut, size, _stream()))
     return out
 
 
