@@ -74,6 +74,48 @@ def test_product_parts(M, N, K):
         assert torch.equal(again.nan_to_num(1.5, 2.5, 3.5), z.nan_to_num(1.5, 2.5, 3.5)), f
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 70, 40), (40, 70, 700), (64, 300, 2100)])
+def test_results_made_again(M, N, K):
+    """Operands near the largest float32, whose parts pass it, beside results that do not: finite, the same bits in every form, and other
+    results untouched."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) * 1e-3
+    y = kernels.gemm_tn(x.to(DEV), w.to(DEV))
+    big = torch.rand(M, generator=g) < 0.3
+    big[0], big[1] = True, False
+    at = torch.randint(0, K, (M,), generator=g)
+    x[torch.arange(M)[big], at[big]] = 3.4e38          # (rounded to bfloat16: no bound)
+    got = [kernels.gemm_tn(x.to(DEV), w.to(DEV), form=f) for f in (-1, 0, 1, 2, 3, 4)]
+    assert all(torch.equal(v, got[0]) for v in got)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # (chains of up to K / 8 + 4 sums of the eight chunks, and theirs: 2^-24 of the sum of the sizes each)
+    assert bool(got[0].isfinite().all()) and float(((got[0].cpu().double() - want).abs() / size).max()) < (K / 8 + 8) * 2.0 ** -24
+    assert torch.equal(got[0][~big.to(DEV)], y[~big.to(DEV)])
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 4096, 4096), (562, 4096, 4096)])
+def test_results_without_a_bound_in_bounded_time(M, N, K):
+    """A NaN in every row: a few times a product's time (an element at a time was 40 to 80 times)."""
+    from xinfer_amd import kernels
+
+    def time(x):
+        for _ in range(2):
+            kernels.gemm_tn(x, w)
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            kernels.gemm_tn(x, w)
+        b.record()
+        torch.cuda.synchronize()
+        return a.elapsed_time(b)
+
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    plain = time(x)
+    x[:, 5] = float("nan")
+    assert bool(kernels.gemm_tn(x, w).isnan().all()) and time(x) < 20 * plain
+
+
 # tiles of 32 and of 64 rows for short K: edges of tiles, one step, an odd number of steps, rows that are not on 16 bytes
 @pytest.mark.parametrize("M,N,K", [(3, 5, 16), (33, 70, 3), (700, 1024, 100), (1300, 301, 256), (4097, 4096, 16), (10007, 130, 96), (20000, 129, 1024),
                                    (70001, 65, 33), (5000, 300, 2080)])
