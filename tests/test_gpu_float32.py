@@ -74,6 +74,19 @@ def test_product_parts(M, N, K):
         assert torch.equal(again.nan_to_num(1.5, 2.5, 3.5), z.nan_to_num(1.5, 2.5, 3.5)), f
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 70, 40), (30, 300, 700), (200, 640, 512), (700, 300, 100)])
+@pytest.mark.parametrize("x_size,w_size", [(-100, 0), (-116, 0), (0, -124), (-126, 20), (-136, 30), (-70, -60), (100, -110), (-125, 103), (110, -20)])
+def test_small_and_large_operands(M, N, K, x_size, w_size):
+    """Operands down to the smallest float32 keep their digits, beside others of any size."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(M + x_size)
+    x, w = torch.randn(M, K, generator=g) * 2.0 ** (x_size / 2) * 2.0 ** (x_size / 2), torch.randn(N, K, generator=g) * 2.0 ** w_size
+    y, size = kernels.gemm_tn(x.to(DEV), w.to(DEV)).cpu().double(), x.double().abs() @ w.double().abs().T
+    # as above, half of the smallest float32 for the result; from 2^104 on a result is a float32 sum of up to K / 8 + 4 products a chunk
+    bound = size * ((-(-K // 256) + 5) * 2.0 ** -23 if x_size < 104 else (K / 8 + 12) * 2.0 ** -24) + 2.0 ** -149
+    assert bool(((y - x.double() @ w.double().T).abs() < bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(5, 70, 40), (40, 70, 700), (64, 300, 2100)])
 def test_results_made_again(M, N, K):
     """Operands near the largest float32, whose parts pass it, beside results that do not: finite, the same bits in every form, and other

@@ -143,3 +143,27 @@ def test_float32_product_forms():
     assert form(8, 151936, 4096) == 1 and form(32, 24576, 4096) == 1          # wide outputs of few rows: bound by the weights
     scratch = lambda M, N, K: int(kernels.lib().xi_gemm_f32_scratch(M, N, K, -1))
     assert scratch(1 << 20, 16, 128) == 0 and scratch(562, 4096, 4096) == 6 * 4096 * 562 and scratch(100_000, 4096, 4096) == 6 * 4096 * 2048
+
+
+def test_three_parts_of_a_float32():
+    """2^24 of any float32 up to 2^104 is the sum of three bfloat16, none of them subnormal, and what the six products of two numbers leave out is at most
+    2^-24 + 2^-34 of theirs."""
+    import torch
+    g = torch.Generator().manual_seed(0)
+    worst = torch.tensor([float.fromhex(h) for h in ("0x1.00ff8p+0", "0x1.01p+0", "0x1.fffffep+0", "0x1.00fffep+0", "0x1p-149", "0x1.fffffep-127", "0x1.fcp+103")])
+    x = torch.cat([worst, -worst, torch.randn(1 << 20, generator=g), torch.randn(1 << 20, generator=g) * 2.0 ** -110 * 2.0 ** -16])
+
+    def parts(x):
+        rest, out = x * 2.0 ** 24, []
+        for _ in range(3):
+            out.append(rest.to(torch.bfloat16))
+            rest = rest - out[-1].float()
+        assert bool((rest == 0).all())
+        return [p.double() for p in out]
+
+    hi, mid, lo = parts(x)
+    assert torch.equal(hi + mid + lo, x.double() * 2.0 ** 24)
+    assert all(bool(((p == 0) | (p.abs() >= 2.0 ** -126)).all()) for p in (hi, mid, lo))
+    perm = torch.cat([torch.arange(len(worst)), len(worst) + torch.randperm(len(x) - len(worst), generator=g)])
+    out = mid * lo[perm] + lo * mid[perm] + lo * lo[perm]
+    assert bool((out.abs() <= (2.0 ** -24 + 2.0 ** -34) * (x.double() * x.double()[perm]).abs() * 2.0 ** 48).all())
