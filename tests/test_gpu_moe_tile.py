@@ -153,7 +153,7 @@ def test_orders_of_the_tiles(counts, orders):
 
 
 @pytest.mark.parametrize("E,I", [(1, 0), (63, 2), (64, 0), (65, 1), (1000, 24), (1024, 0)])
-@pytest.mark.parametrize("P,bm", [(1, 64), (130, 32), (3000, 256), (5000, 128)])
+@pytest.mark.parametrize("P,bm", [(1, 64), (130, 32), (3000, 64), (5000, 128)])
 def test_pairs_in_the_order_of_their_experts(E, I, P, bm):
     """The sort for one expert to the most there are: every pair in one slot, experts in order, tiles as they follow from the counts."""
     from xinfer_amd import kernels
@@ -161,28 +161,25 @@ def test_pairs_in_the_order_of_their_experts(E, I, P, bm):
     idx = (torch.rand(P, generator=g) ** 3 * (E + I)).to(torch.int32)             # uneven, some experts without a pair
     most = kernels.lib().xi_moe_tiles_most(P, E, bm)
     order, slot_of = (torch.full((P,), -1, dtype=torch.int32, device=DEV) for _ in range(2))
-    lists = [torch.full((most + 1,), -1, dtype=torch.int32, device=DEV) for _ in range(5)]
+    lists = [torch.full((most + 1,), -1, dtype=torch.int32, device=DEV) for _ in range(3)]
     n_tiles = torch.zeros(1, dtype=torch.int32, device=DEV)
     dev = idx.to(DEV)
     p = kernels._p
-    for first_and_count in (True, False):
-        kernels._ok(kernels.lib().xi_moe_sort(p(dev), P, E, I, bm, p(order), p(slot_of), p(lists[0]), p(lists[1]), p(lists[2]), p(n_tiles),
-                                              *((p(lists[3]), p(lists[4])) if first_and_count else (None, None)), kernels._stream()))
-        want, at = [[], [], [], [], []], 0
-        for e in range(E + I):
-            c = int((idx == e).sum())
-            first, count = len(want[0]), -(-c // bm)
-            for r in range(0, c if e < E else 0, bm):
-                for w, v in zip(want, (e, at + r, min(bm, c - r), first, count)):
-                    w.append(v)
-            at += c
-        n = len(want[0])
-        assert n == int(n_tiles) <= most
-        for got, w in zip(lists, want):
-            assert got[:n].tolist() == w and got[most].item() == -1
-        o = order.cpu().long()
-        assert sorted(o.tolist()) == list(range(P)) and bool((idx[o][1:] >= idx[o][:-1]).all())
-        assert bool((slot_of.cpu().long()[o] == torch.arange(P)).all())
+    kernels._ok(kernels.lib().xi_moe_sort(p(dev), P, E, I, bm, p(order), p(slot_of), p(lists[0]), p(lists[1]), p(lists[2]), p(n_tiles), kernels._stream()))
+    want, at = [[], [], []], 0
+    for e in range(E + I):
+        c = int((idx == e).sum())
+        for r in range(0, c if e < E else 0, bm):
+            for w, v in zip(want, (e, at + r, min(bm, c - r))):
+                w.append(v)
+        at += c
+    n = len(want[0])
+    assert n == int(n_tiles) <= most
+    for got, w in zip(lists, want):
+        assert got[:n].tolist() == w and got[most].item() == -1
+    o = order.cpu().long()
+    assert sorted(o.tolist()) == list(range(P)) and bool((idx[o][1:] >= idx[o][:-1]).all())
+    assert bool((slot_of.cpu().long()[o] == torch.arange(P)).all())
 
 
 def test_what_is_taken_and_refused():

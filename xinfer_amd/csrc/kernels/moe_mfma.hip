@@ -30,8 +30,7 @@ typedef __attribute__((ext_vector_type(4))) float mf32x4;
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __restrict__ idx, int P, int E, int I, int BM,
                                                                 int* __restrict__ order, int* __restrict__ slot_of,
                                                                 int* __restrict__ tile_expert, int* __restrict__ tile_row0,
-                                                                int* __restrict__ tile_rows, int* __restrict__ n_tiles,
-                                                                int* __restrict__ tile_first, int* __restrict__ tile_count) {
+                                                                int* __restrict__ tile_rows, int* __restrict__ n_tiles) {
   __shared__ int count[kSortExperts], cursor[kSortExperts], across[2][kSortThreads / kWave];
   const int A = E + I, e = threadIdx.x;
   moe_count_pairs(idx, P, A, count);
@@ -43,10 +42,6 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(const int* __res
   if (e < A) cursor[e] = at;
   for (int i = 0; i < tiles; ++i) {
     const int r = i * BM;
-    if (tile_first) {
-      tile_first[first + i] = first;
-      tile_count[first + i] = tiles;
-    }
     tile_expert[first + i] = e;
     tile_row0[first + i] = at + r;
     tile_rows[first + i] = pairs - r < BM ? pairs - r : BM;
@@ -324,14 +319,11 @@ int xi_moe_tiles_most(int P, int E, int bm) {
   return taken + (P - taken) / bm;
 }
 
-// idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P]; tile_* int32 [xi_moe_tiles_most]; n_tiles int32 [1];
-// tile_first, tile_count (both or neither): the first tile of a tile's expert and how many it has.
+// idx int32 [P] (expert of every pair; E .. E + I - 1: identity experts) -> order, slot_of int32 [P]; tile_* int32 [xi_moe_tiles_most]; n_tiles int32 [1].
 int xi_moe_sort(const int* idx, int P, int E, int I, int bm, int* order, int* slot_of, int* tile_expert, int* tile_row0,
-                int* tile_rows, int* n_tiles, int* tile_first, int* tile_count, hipStream_t stream) {
-  XI_CHECK((tile_first == nullptr) == (tile_count == nullptr), "moe_sort: an operand is missing");
-  XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && (bm == 32 || bm == 64 || bm == 128 || bm == 256), "moe_sort: bad sizes pairs=%d experts=%d rows=%d", P, E, bm);
-  moe_sort_kernel<<<1, moe_sort_threads(P, E + I), 0, stream>>>(idx, P, E, I, bm, order, slot_of, tile_expert, tile_row0, tile_rows, n_tiles,
-                                                   tile_first, tile_count);
+                int* tile_rows, int* n_tiles, hipStream_t stream) {
+  XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && (bm == 32 || bm == 64 || bm == 128), "moe_sort: bad sizes pairs=%d experts=%d rows=%d", P, E, bm);
+  moe_sort_kernel<<<1, moe_sort_threads(P, E + I), 0, stream>>>(idx, P, E, I, bm, order, slot_of, tile_expert, tile_row0, tile_rows, n_tiles);
   XI_LAUNCH_CHECK("moe_sort");
   return 0;
 }

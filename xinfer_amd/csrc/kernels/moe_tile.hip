@@ -261,7 +261,7 @@ int xi_moe_tile_takes(long long rows_x, int N, int K, int gated) {
 // device, of 128 to 256, for that many columns of workgroups; most: xi_moe_tiles_most for high or for 128.
 int xi_moe_plan(const int* idx, int P, int E, int I, int high1, int high2, int columns1, int columns2, int* order, int* slot_of, int* tiles1,
                 int* tiles2, int most1, int most2, hipStream_t stream) {
-  auto fits = [](int h) { return h == 0 || h == 64 || (h >= 128 && h <= 256 && h % 32 == 0); };
+  auto fits = [](int h) { return h == 0 || h == 64 || h == 128 || h == 256; };
   XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && fits(high1) && fits(high2) && columns1 > 0 && columns2 > 0,
            "moe_plan: bad sizes pairs=%d experts=%d rows=%d, %d", P, E, high1, high2);
   XI_CHECK(most1 >= xi_moe_tiles_most(P, E, high1 ? high1 : 128) && most2 >= xi_moe_tiles_most(P, E, high2 ? high2 : 128),
@@ -281,7 +281,7 @@ int xi_moe_tile_columns(int N, int high, int gated) {
 // The operands of `xi_moe_group` (moe_mfma.hip) for the tiles of `xi_moe_plan` with this `high`; rows_x: rows of A.
 int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, const void* W, const int* tiles, int most, void* out,
                 int N, int K, int high, int form, int act, const float* in_wt, hipStream_t stream) {
-  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && most > 0 && (high == 0 || high == 64 || (high >= 128 && high <= 256)),
+  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && most > 0 && (high == 0 || high == 64 || high == 128 || high == 256),
            "moe_tile: bad sizes N=%d K=%d top=%d tiles=%d rows=%d", N, K, top, most, high);
   XI_CHECK(act >= 0 && act <= 2 && form >= 0 && form <= 2, "moe_tile: unknown activation %d or form %d", act, form);
   XI_CHECK(tiles && order, "moe_tile: an operand is missing");

@@ -786,7 +786,7 @@ def moe_experts_library(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     order, slot_of = ints[:P], ints[P:2 * P]
     _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), 128, _p(order), _p(slot_of), _p(ints[2 * P:2 * P + most]),
                           _p(ints[2 * P + most:2 * P + 2 * most]), _p(ints[2 * P + 2 * most:2 * P + 3 * most]),
-                          _p(ints[2 * P + 3 * most:]), None, None, _stream()))
+                          _p(ints[2 * P + 3 * most:]), _stream()))
     if weigh_input and not gated:
         raise KernelError("moe_experts_library: a weight on the input is built for gated experts")
     wt_in = wt.reshape(-1).contiguous() if weigh_input else None
@@ -964,7 +964,7 @@ def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, idx:
         order, slot_of = ints[:P], ints[P:2 * P]
         t_e, t_r0, t_n, n_tiles = (ints[2 * P:2 * P + most], ints[2 * P + most:2 * P + 2 * most],
                                    ints[2 * P + 2 * most:2 * P + 3 * most], ints[2 * P + 3 * most:])
-        _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), None, None, _stream()))
+        _ok(lib().xi_moe_sort(_p(idx), P, E, int(identity), bm, _p(order), _p(slot_of), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), _stream()))
         mid = torch.empty((P, F), dtype=torch.bfloat16, device=x.device)
         _ok(lib().xi_moe_group(_p(x), _p(order), top, _p(gate_up), _p(t_e), _p(t_r0), _p(t_n), _p(n_tiles), most, _p(mid),
                                F, H, bm, 1 if gated else 2, acts[act], _p(wt_in), _stream()))
