@@ -141,6 +141,8 @@ def test_float32_product_forms():
     assert form(200, 4096, 4096) == 2 and form(562, 151936, 4096) == 3 and form(562, 4096, 4096) == 4
     assert form(40000, 4096, 256) == 5 and form(2048, 4096, 256) == 4         # 2,048 rows at a time leave gaps
     assert form(8, 151936, 4096) == 1 and form(32, 24576, 4096) == 1          # wide outputs of few rows: bound by the weights
+    # ... at K = 1024 too, where a workgroup's start counts once and not for every tile it walks; and weights from memory behind tiles for short K
+    assert form(1, 151936, 1024) == 0 and form(8, 151936, 1024) == 1 and form(100, 6144, 1024) == 1 and form(600, 1024, 3072) == 1
     scratch = lambda M, N, K: int(kernels.lib().xi_gemm_f32_scratch(M, N, K, -1))
     assert scratch(1 << 20, 16, 128) == 0 and scratch(562, 4096, 4096) == 6 * 4096 * 562 and scratch(100_000, 4096, 4096) == 6 * 4096 * 2048
 
