@@ -109,3 +109,23 @@ def test_tall_tile_rule(M, N, K, rows):
                   _Rows(M, K + 64)):
         assert kernels.tall_tile_rows(other, w) is None
     assert kernels.tall_tile_rows(x, _Rows(N, K, start=8)) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k_tiles", [1, 2, 3, 4, 5, 6, 7])
+def test_rings_of_unequal_depth(k_tiles):
+    """Every walk at fewer tiles of k than its rings have stages, and at their first turns: whole numbers of which every partial sum is exact in float32."""
+    M, N, K = 260, 520, 64 * k_tiles
+    g = torch.Generator().manual_seed(k_tiles)
+    x, w = (torch.randint(-4, 5, (n, K), generator=g).to(torch.bfloat16).to(DEV) for n in (M, N))
+    ref = x.double() @ w.double().t()
+    for shape in (0, 1, 2):
+        assert torch.equal(kernels.linear_tile(x, w, partial=True, shape=shape)[0].double(), ref)
+    for rows in kernels.TALL_SHAPES:
+        assert torch.equal(kernels.linear_tall(x, w, rows), ref.float().to(torch.bfloat16))
+    # the gated walks' sums are the same, the first shape's among them: one result for all
+    got = [kernels.linear_gated_tile(x, w, "silu", shape) for shape in (0, 1, 2)]
+    a, b = ref[:, :N // 2], ref[:, N // 2:]
+    want = torch.nn.functional.silu(a) * b
+    assert bool(((got[0].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * (1 + (a * b).abs())).all())
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

@@ -11,8 +11,8 @@
 //
 // Tiles of 64 k reach LDS through loads that write LDS themselves (`global_load_lds_dwordx4`:
 // every lane asks for one 16-byte chunk, a wave's 64 chunks land in 1 KB of consecutive LDS, no
-// register holds a tile), into a ring of S stages (3, or 2 for the tile of 256 by 256: 160 KB of
-// LDS); a tile is waited for with a count, not by draining the queue, and one barrier a tile orders
+// register holds a tile), into rings of two or three stages of x and three or more of w (160 KB of
+// LDS: tile_core.h); a tile is waited for with a count, not by draining the queue, and one barrier a tile orders
 // the stage's reuse.  Rows of 128 bytes cannot be padded then, so the 16-byte chunks of row p are
 // permuted: chunk c sits at place c ^ ((p >> 1) & 7), and the 16 lanes that read an operand together
 // (16 rows, one chunk each) fall into 16 different 16-byte groups of the 64 banks (the counters
@@ -28,13 +28,13 @@
 //
 // Measured on MI355X (random operands, the clock under load about 1.8 GHz): 2,048 rows by
 // N = 4096, K = 12288 in 172 us (1.2 PFLOP/s; the library 174), K = 4096 in 68 us (the library 64);
-// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 102 us (1.35; the library 92); the matrix cores are
+// 4,096 x 4,096 x 4,096 in tiles of 256 by 256 102 us (1.35; the library 92), operands in a cache: the matrix cores are
 // busy 63% of the time, LDS serves the tiles' 48 to 64 KB of writes and 128 to 192 KB of reads a
-// tile and is what the kernel waits for (without the barrier or without the wait for the loads it
-// is no faster).  Where it is ahead of the library is the narrow output at few rows, whose tiles
+// tile (without the barrier or without the wait for the loads it is no faster).  With weights from memory, as in a model, what
+// bounds it is how long they have been asked for when they are wanted (tile_core.h).  Where it is ahead of the library is the narrow output at few rows, whose tiles
 // leave most of the chip idle unless K is cut: 256 rows of N = 4096, K = 12288 in 30 us against 41.
 // A long K whose output is less than a round of such tiles (down projections of 1,025 to 2,688 rows) goes in the lowest tiles that
-// still are one round, 96 to 224 rows by 256 features: 1,727 rows of N = 5120, K = 17408 in 11 x 20 tiles of 160 rows 255 us
+// still are one round, 96 to 224 rows by 256 features: 1,727 rows of N = 5120, K = 17408 in 11 x 20 tiles of 160 rows 255 to 261 us
 // (1.2 PFLOP/s, its loads into LDS at 57 GB/s a compute unit, which bounds tiles up to that height), the library 473; 256 rows 401;
 // four slices of 128 rows 309 and the reader's four float32 parts.
 // Not kept: the tiles' k shared out evenly over the compute units, whoever comes last at a tile adding up its parts (345 us there:
@@ -59,11 +59,11 @@ namespace tile {
 constexpr int kSliceK = 64;        // K is cut into slices in tiles of this many
 
 // BM rows of x by BN rows of w a workgroup; see Walk.
-template <int BM, int BN, int WGM, int WGN, int S, bool PARTIAL>
+template <int BM, int BN, int WGM, int WGN, int S, int SW, bool PARTIAL>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w, void* __restrict__ yv, int M, int N, int K, int tiles_m,
     int tiles_n, int slices, int k_tiles_all) {
-  using W = Walk<BM, BN, WGM, WGN, S>;
+  using W = Walk<BM, BN, WGM, WGN, S, SW>;
   constexpr int TM = W::TM, TN = W::TN;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -126,13 +126,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void linear_tile_kernel(
 // writes half, and their two launches): w [2 N, K] = [gate; up], y bfloat16 [M, N] = act(gate) * up of the
 // float32 sums, one rounding.  A workgroup owns BM rows of x and BN / 2 features; a wave's rows of w are gate rows and the up
 // rows of the same features (as in moe_tile.hip).  Bound by the walk, as above, and by how evenly the tiles fill rounds of 256
-// workgroups; measured at N=17408, K=5120 against the library and the activation's pass: 1,024 rows 301 us (1.21 PFLOP/s) / 408,
-// 2,048 rows 563 / 619; at N=3072, K=1024: 256 rows in tiles of 64 by 64 9.3 / 16.9, 1,024 in 128 by 128 17.3 / 22.8, 2,048 in
+// workgroups; measured at N=17408, K=5120 against the library and the activation's pass: 1,024 rows 288 us (1.27 PFLOP/s) / 408,
+// 2,048 rows 537 / 619; at N=3072, K=1024: 256 rows in tiles of 64 by 64 9.3 / 16.9, 1,024 in 128 by 128 17.3 / 22.8, 2,048 in
 // 256 by 128 27.5 / 35.2.
-template <int BM, int BN, int S, int ACT>
+template <int BM, int BN, int S, int SW, int ACT>
 __device__ __forceinline__ void gated_tile(const bf16* x, const bf16* w, bf16* y, int M, int N, int K, int m0, int f0, unsigned char* smem) {
   constexpr int WGM = 2, WGN = 4;
-  using W = Walk<BM, BN, WGM, WGN, S>;
+  using W = Walk<BM, BN, WGM, WGN, S, SW>;
   constexpr int TM = W::TM, TN = W::TN, TF = TN / 2, WF = 16 * TF;
   static_assert(TN % 2 == 0, "half of a wave's rows of w are gate rows");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -171,20 +171,20 @@ __device__ __forceinline__ void gated_tile(const bf16* x, const bf16* w, bf16* y
 
 // Tiles of BM rows by BN / 2 features, the rows innermost.  Workgroup numbers of one die get consecutive places: its L2 holds the
 // rows of w they share.
-template <int BM, int BN, int S, int ACT>
+template <int BM, int BN, int S, int SW, int ACT>
 __global__ __launch_bounds__(512, 1) void gated_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                             bf16* __restrict__ y, int M, int N, int K, int tiles_m) {
   extern __shared__ __align__(1024) unsigned char smem[];
   const int total = gridDim.x, q8 = total >> 3, r8 = total & 7, die = blockIdx.x & 7;
   const int place = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
   const int tn_i = place / tiles_m;
-  gated_tile<BM, BN, S, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * BM, tn_i * (BN / 2), smem);
+  gated_tile<BM, BN, S, SW, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * BM, tn_i * (BN / 2), smem);
 }
 
 // Tiles of 256 rows by 128 features, of which the last ones, a round of workgroups that would leave half of the compute units or
 // more idle, are cut into `parts` (2: halves of the rows; 4: and of the features).  `whole`: the tiles in front of those.
 // N=17408, K=5120, 2,048 rows (4.25 rounds): 665 us uncut, 583 cut (563 with the walk as it is now); N=25600 (6.25 rounds): 962
-// and 846 (819).
+// and 846 (819); with three stages of w 537 and 779.
 template <int ACT>
 __global__ __launch_bounds__(512, 1) void gated_tile_rest_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                  bf16* __restrict__ y, int M, int N, int K, int tiles_m, int whole,
@@ -193,14 +193,14 @@ __global__ __launch_bounds__(512, 1) void gated_tile_rest_kernel(const bf16* __r
   const int b = blockIdx.x;
   if (b < whole) {                             // (a multiple of 256)
     const int place = (b & 7) * (whole >> 3) + (b >> 3), tn_i = place / tiles_m;
-    gated_tile<256, 256, 2, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * 256, tn_i * 128, smem);
+    gated_tile<256, 256, 2, 3, ACT>(x, w, y, M, N, K, (place - tn_i * tiles_m) * 256, tn_i * 128, smem);
     return;
   }
   const int piece = b - whole, place = whole + piece / parts, part = piece % parts, tn_i = place / tiles_m;
   const int m0 = (place - tn_i * tiles_m) * 256 + 128 * (part & 1), f0 = tn_i * 128 + 64 * (part >> 1);
   if (m0 >= M || f0 >= N) return;
-  if (parts == 2) gated_tile<128, 256, 3, ACT>(x, w, y, M, N, K, m0, f0, smem);
-  else gated_tile<128, 128, 4, ACT>(x, w, y, M, N, K, m0, f0, smem);
+  if (parts == 2) gated_tile<128, 256, 3, 3, ACT>(x, w, y, M, N, K, m0, f0, smem);
+  else gated_tile<128, 128, 4, 5, ACT>(x, w, y, M, N, K, m0, f0, smem);
 }
 
 }  // namespace tile
@@ -232,27 +232,27 @@ int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, i
   const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   const long long total = (long long)tiles_m * tiles_n * slices;
   XI_CHECK(total <= 0x7fffffffLL, "linear_tile: too many workgroups");
-#define XI_TILE(BM, BN, WGM, WGN, S, PARTIAL)                                                                 \
+#define XI_TILE(BM, BN, WGM, WGN, S, SW, PARTIAL)                                                             \
   do {                                                                                                            \
-    auto kern = tile::linear_tile_kernel<BM, BN, WGM, WGN, S, PARTIAL>;                                        \
-    const size_t lds = tile::Walk<BM, BN, WGM, WGN, S>::LDS;                                                          \
+    auto kern = tile::linear_tile_kernel<BM, BN, WGM, WGN, S, SW, PARTIAL>;                                    \
+    const size_t lds = tile::Walk<BM, BN, WGM, WGN, S, SW>::LDS;                                                      \
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);  \
     XI_CHECK(e == hipSuccess, "linear_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));         \
     kern<<<(unsigned)total, 64 * WGM * WGN, lds, stream>>>((const bf16*)x, (const bf16*)w, y, M, N, K, tiles_m,   \
                                                            tiles_n, slices, K / tile::kSliceK);                   \
   } while (0)
   if (shape == 0) {
-    if (partial) XI_TILE(128, 256, 2, 4, 3, true);
-    else XI_TILE(128, 256, 2, 4, 3, false);
+    if (partial) XI_TILE(128, 256, 2, 4, 3, 3, true);
+    else XI_TILE(128, 256, 2, 4, 3, 3, false);
   } else if (shape == 1) {
-    if (partial) XI_TILE(256, 128, 4, 2, 3, true);
-    else XI_TILE(256, 128, 4, 2, 3, false);
+    if (partial) XI_TILE(256, 128, 4, 2, 3, 4, true);
+    else XI_TILE(256, 128, 4, 2, 3, 4, false);
   } else if (shape == 2) {
-    if (partial) XI_TILE(256, 256, 2, 4, 2, true);
-    else XI_TILE(256, 256, 2, 4, 2, false);
-  } else if (shape == 4) XI_TILE(96, 256, 2, 4, 3, false);
-  else if (shape == 5) XI_TILE(160, 256, 2, 4, 3, false);
-  else XI_TILE(224, 256, 2, 4, 2, false);
+    if (partial) XI_TILE(256, 256, 2, 4, 2, 3, true);
+    else XI_TILE(256, 256, 2, 4, 2, 3, false);
+  } else if (shape == 4) XI_TILE(96, 256, 2, 4, 3, 3, false);
+  else if (shape == 5) XI_TILE(160, 256, 2, 4, 3, 3, false);
+  else XI_TILE(224, 256, 2, 4, 2, 3, false);
 #undef XI_TILE
   XI_LAUNCH_CHECK("linear_tile");
   return 0;
@@ -282,20 +282,20 @@ int xi_linear_gated_tile(const void* x, const void* w, void* y, int M, int N, in
     XI_CHECK(e == hipSuccess, "linear_gated_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));              \
     kern<<<(unsigned)(WGS), 512, lds, stream>>>((const bf16*)x, (const bf16*)w, (bf16*)y, M, N, K, __VA_ARGS__);             \
   } while (0)
-#define XI_GT(BM, BN, S)                                                                                                     \
+#define XI_GT(BM, BN, S, SW)                                                                                                  \
   do {                                                                                                                       \
-    constexpr size_t bytes = tile::Walk<BM, BN, 2, 4, S>::LDS;                                                               \
-    if (act == 0) XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, 0>), bytes, tiles, tiles_m);                              \
-    else XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, 1>), bytes, tiles, tiles_m);                                       \
+    constexpr size_t bytes = tile::Walk<BM, BN, 2, 4, S, SW>::LDS;                                                           \
+    if (act == 0) XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, SW, 0>), bytes, tiles, tiles_m);                              \
+    else XI_GT_LAUNCH((tile::gated_tile_kernel<BM, BN, S, SW, 1>), bytes, tiles, tiles_m);                                       \
   } while (0)
   const long long whole = tiles / 256 * 256, rest = tiles - whole;
-  if (shape == 0) XI_GT(64, 128, 6);
-  else if (shape == 1) XI_GT(128, 256, 3);
-  else if (whole == 0 || rest == 0 || rest > 128) XI_GT(256, 256, 2);
+  if (shape == 0) XI_GT(64, 128, 6, 6);
+  else if (shape == 1) XI_GT(128, 256, 3, 3);
+  else if (whole == 0 || rest == 0 || rest > 128) XI_GT(256, 256, 2, 3);
   else {
     const int parts = rest <= 64 ? 4 : 2;
-    constexpr size_t bytes = tile::Walk<128, 256, 2, 4, 3>::LDS;       // the most of the three walks
-    static_assert(bytes >= tile::Walk<256, 256, 2, 4, 2>::LDS && bytes >= tile::Walk<128, 128, 2, 4, 4>::LDS, "");
+    constexpr size_t bytes = tile::Walk<256, 256, 2, 4, 2, 3>::LDS;       // the most of the three walks
+    static_assert(bytes >= tile::Walk<128, 256, 2, 4, 3>::LDS && bytes >= tile::Walk<128, 128, 2, 4, 4, 5>::LDS, "");
     if (act == 0) XI_GT_LAUNCH(tile::gated_tile_rest_kernel<0>, bytes, whole + rest * parts, tiles_m, (int)whole, parts);
     else XI_GT_LAUNCH(tile::gated_tile_rest_kernel<1>, bytes, whole + rest * parts, tiles_m, (int)whole, parts);
   }

@@ -15,8 +15,9 @@
 // of 6144 at width 4096, 39 to 761 pairs each 584 | 539, 163 to 622 595 | 576, 410 596 | 552, 78 to 1,522 989 | 969, 512 584 | 570, 1,024
 // 1,061 | 1,060; without a gate 130 to 634 519 | 457, 260 to 1,268 932 | 838, 1,536 1,116 | 1,161; 16 of 4096 at 2048, 512 each 302 | 290, 1,024 539 |
 // 548, 156 to 3,044 919 | 983 (192 rows where 256 are ahead: the one load of 125 with more than 5% lost); 8 of 1536 at 1024, 1,024 each
-// 113 | 104, 512 55 | 57.  What is left: rows past an expert's in the tiles (7%), the last
-// round of workgroups, and 1 PFLOP/s in between where the dense walk has 1.3.
+// 113 | 104, 512 55 | 57.  (All of these with two stages of w in flight; with three 1 to 10% less: tile_core.h.)  What is left: rows past an expert's in
+// the tiles (7%), the last round of workgroups, and 1.1 PFLOP/s in between where the dense walk has 1.4: a tile's w is shared by the few
+// tiles of its expert.
 //
 // A workgroup owns a tile and BN rows of w; the number of tiles is known on the device alone, and the grid is the most
 // there can be.  Nothing is read on the host.  (As many workgroups as compute units, each taking its die's next tile by a counter:
@@ -131,14 +132,14 @@ __global__ __launch_bounds__(kSortThreads) void moe_plan_kernel(const int* __res
   moe_place_pairs(idx, P, A, cursor, order, slot_of);
 }
 
-// One tile: BM rows of x by BN rows of w (gated: BN / 2 features), a ring of S stages.
-template <int BM, int BN, int S, int FORM, int ACT>
+// One tile: BM rows of x by BN rows of w (gated: BN / 2 features), rings of S and SW stages.
+template <int BM, int BN, int S, int SW, int FORM, int ACT>
 __device__ __forceinline__ void moe_one_tile(const bf16* __restrict__ x, const int* __restrict__ order, int top,
                                              const bf16* __restrict__ w, int e, int row0, int rows, int tn_i, void* __restrict__ out,
                                              int N, int K, const float* __restrict__ in_wt, unsigned char* smem) {
   constexpr bool GATED = FORM == 1, GATHER = FORM != 0;
   constexpr int WGM = 2, WGN = 4;
-  using W = Walk<BM, BN, WGM, WGN, S>;
+  using W = Walk<BM, BN, WGM, WGN, S, SW>;
   constexpr int TM = W::TM, TN = W::TN;
   constexpr int TF = GATED ? TN / 2 : TN, WF = 16 * TF;            // 16-feature tiles of a wave, and its features
   static_assert(TN % 2 == 0, "half of a wave's rows of w are gate rows");
@@ -232,16 +233,16 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
     }
   }
   const int e = tiles[tile], row0 = tiles[most + tile], rows = tiles[2 * most + tile];
-#define XI_ONE(BM, BN, S) moe_one_tile<BM, BN, S, FORM, ACT>(x, order, top, w, e, row0, rows, column, out, N, K, in_wt, smem)
+#define XI_ONE(BM, BN, S, SW) moe_one_tile<BM, BN, S, SW, FORM, ACT>(x, order, top, w, e, row0, rows, column, out, N, K, in_wt, smem)
   if constexpr (LOW) {
-    XI_ONE(64, 128, 6);
+    XI_ONE(64, 128, 6, 6);
   } else {
-    if (rows > 224) XI_ONE(256, 256, 2);
-    else if (rows > 192) XI_ONE(224, 256, 2);
-    else if (rows > 160) XI_ONE(192, 256, 2);
-    else if (rows > 128) XI_ONE(160, 256, 3);
-    else if (rows > 64) XI_ONE(128, 256, 3);
-    else XI_ONE(64, 256, 3);
+    if (rows > 224) XI_ONE(256, 256, 2, 3);
+    else if (rows > 192) XI_ONE(224, 256, 2, 3);
+    else if (rows > 160) XI_ONE(192, 256, 2, 3);
+    else if (rows > 128) XI_ONE(160, 256, 3, 3);
+    else if (rows > 64) XI_ONE(128, 256, 3, 3);
+    else XI_ONE(64, 256, 3, 4);
   }
 #undef XI_ONE
 }
@@ -302,7 +303,7 @@ int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, cons
 #define XI_MT(LOW, FORM, ACT)                                                                                               \
   do {                                                                                                                      \
     auto kern = tile::moe_tile_kernel<LOW, FORM, ACT>;                                                                      \
-    const size_t lds = LOW ? tile::Walk<64, 128, 2, 4, 6>::LDS : tile::Walk<160, 256, 2, 4, 3>::LDS;                        \
+    const size_t lds = LOW ? tile::Walk<64, 128, 2, 4, 6>::LDS : tile::Walk<256, 256, 2, 4, 2, 3>::LDS;                        \
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);      \
     XI_CHECK(e == hipSuccess, "moe_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));                      \
     kern<<<wgs, 512, lds, stream>>>((const bf16*)A, order, top, (const bf16*)W, tiles, most, out, N, K, columns, in_wt); \
