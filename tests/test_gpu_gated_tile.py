@@ -129,3 +129,18 @@ def test_rings_of_unequal_depth(k_tiles):
     want = torch.nn.functional.silu(a) * b
     assert bool(((got[0].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * (1 + (a * b).abs())).all())
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("M,F,K,shape", [
+    # a round of 128 rows by 128 features, from 3/4 (K up to 4,096) or 7/8 (up to 6,144) of one on
+    (128, 14336, 4096, None), (129, 12288, 4096, 1), (129, 12160, 4096, None), (256, 16384, 4096, 1), (256, 16512, 4096, None), (512, 6144, 2304, 1),
+    (512, 7168, 5120, 1), (512, 7040, 5120, None), (512, 8192, 6144, 1), (512, 8192, 6208, None),
+    # 256 rows: 0.74 of the rounds' room, whole rounds and one of which the last tiles are cut
+    (256, 24576, 2112, None), (379, 16384, 4096, 2), (378, 16384, 4096, None), (700, 12288, 4096, 2), (800, 12288, 4096, None), (2048, 12288, 4096, 2),
+    (3584, 12288, 4096, 2), (3585, 12288, 4096, None), (2048, 64, 4096, None), (2048, 2048, 4096, 1),
+    (769, 17408, 5120, None), (848, 17408, 5120, None), (849, 17408, 5120, 2), (768, 12288, 5120, 2)])
+def test_gated_tile_rule_by_rounds(M, F, K, shape):
+    x, w = _Rows(M, K), _Rows(2 * F, K)
+    assert kernels.gated_tile_shape(x, w) == shape
+    for other in (_Rows(M, K, start=8), _Rows(M, K, contiguous=False), _Rows(M, K, dtype=torch.float32), _Rows(M, K + 64)):
+        assert kernels.gated_tile_shape(other, w) is None

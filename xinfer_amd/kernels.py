@@ -1872,6 +1872,13 @@ def linear_tall(x: torch.Tensor, w: torch.Tensor, rows: int) -> torch.Tensor:
     return y
 
 
+def _tile_room(full: int, rest: int) -> float:
+    """Rows times features that the time of `full` rounds of tiles of 256 by 128 and `rest` more has room for: less than a round takes one, and the
+    last ones behind whole rounds, which are cut (see the kernel), 0.38 of one up to 64 and 0.6 up to 128."""
+    last = 0.0 if rest == 0 else 1.0 if full == 0 or 2 * rest > COMPUTE_UNITS else 0.38 if 4 * rest <= COMPUTE_UNITS else 0.6
+    return (full + last) * COMPUTE_UNITS * 256 * 128
+
+
 def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     """The tile shape in which act(x @ gate^T) * (x @ up^T) goes to `linear_gated_tile`, None: the library's product and a
     kernel for the activation (which also stay for operands that the tiled kernel does not take).  Measured on MI355X
@@ -1882,8 +1889,11 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
       K=2048: 128 19.7 / 23.3, 512 34.4 / 40.5, 1024 56.5 / 64.0, 2048 112 / 118, 4096 219 / 229; F=64 K=1024 M=65 8.6 / 8.9.  What is
       left out is level or behind (M=256 32.8 / 33.1, 700 52.5 / 51.4; F=6144 K=2048 M=700 53 / 44; 2 to 32 workgroups of K=2048: F=64
       M=65 12.1 / 9.1, M=1024 12.6 / 11.7, F=512 M=65 12.5 / 10.0, F=1024 M=128 13.2 / 12.5; 48: F=1536 M=65 13.2 / 13.1).
-      2048 < K <= 4096: not taken.  The library has its best sizes there (F=12288 K=4096: M=512 103 / 91, 900 173 / 165, 2048 301 / 298,
-      4096 625 / 595) and others (700 135 / 150, 1500 239 / 264, 3000 469 / 599), and no rule for them is built.
+      2048 < K <= 4096: 128 rows where their workgroups are 3/4 of a round to one; otherwise 256 rows, of 257 to 3,584, where 0.74 of the rounds'
+      room is rows and features (`_tile_room`).  F=12288 K=4096: M=200 62 / 68, 400 90 / 94, 700 129 / 163, 1024 175 / 180, 1400 225 / 259, 2048 296 /
+      302, 3000 436 / 597; F=6144: 400 52 / 60, 1400 127 / 153, 2048 153 / 180; K=2304 F=11008: 512 54 / 66, 1024 104 / 139; of 461 sizes, F of 1,536 to
+      14,336, 12% ahead in the median and up to 4% behind (F=14336: M=129 K=4096 66 / 63, 2049 398 / 388).  Left out: emptier rounds (F=12288 K=4096: 300 87 /
+      77, 800 161 / 152), and more rows, where the library has its best sizes (4096 600 / 589).
       4096 < K <= 6144, 512 rows and more, 8/9 of the rows of the tiles there: up to four rounds of 256 workgroups and a rest of up to
       64, which is cut (see the kernel) and for which the library has a whole round: K=4608 F=8192: 1230 155 / 163, F=10240: 1024 158
       / 176, K=6144 F=17408: 2048 670 / 674; the median of 299 sizes 7% ahead, none behind.
@@ -1891,7 +1901,11 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
       8,192, in steps of 64 next to it; the tiles 1.20 to 1.25 at all of them): from 3/4 of a round on but for 65 to 143 workgroups
       behind a first round, and for even rounds beyond three.  F=17408: 512 184 / 193, 700 254 / 275, 1024 301 / 408, 1500 433 / 531,
       2048 563 / 619, 4096 1098 / 1265; F=25600: 512 262 / 287, 700 345 / 402, 1024 434 / 511, 1727 731 / 877, 2048 819 / 885, 4096 1609
-      / 1756; the median of 655 sizes 7% ahead, 7 behind by more than 2% (F=5504: 2500 248 / 234).
+      / 1756; the median of 655 sizes 7% ahead, 7 behind by more than 2% (F=5504: 2500 248 / 234).  (With three stages of w in flight they take 5 to 8%
+      less than these figures.)
+      4096 < K <= 6144 besides: 128 rows where their workgroups are 7/8 of a round to one (F=8192 K=5120: 400 75 / 88, 512 83 / 92; K=6144 F=6144: 600
+      106 / 118), and from 769 rows on also fewer rows than 8/9 of the tiles' where 0.74 of the rounds' room is filled (F=17408 K=5120: 900
+      267 / 410); 30 sizes, 13% ahead in the median, none behind.
       Left out: F=64 K=5120 M=512 87 / 17, F=1536 94 / 31, F=2048 K=7168 M=2048 162 / 107, F=12288 K=5120 M=1024 233 / 220, K=4608 M=1280 239 / 222,
       F=8192 K=8192 M=4096 855 / 731, F=17408 K=5120 M=384 182 / 173, 770 422 / 370."""
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] \
@@ -1900,12 +1914,21 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     M, K, F = x.shape[0], x.shape[1], w.shape[0] // 2
     tiles = lambda rows, features: -(-M // rows) * -(-F // features)
     shape = None
+    low = tiles(128, 128)
     if K > 4096:
         full, rest = divmod(tiles(256, 128), COMPUTE_UNITS)
         cut = 1 <= full <= 4 and 0 < 4 * rest <= COMPUTE_UNITS
         if K == 5120 and not cut:
             cut = (4 * rest > 3 * COMPUTE_UNITS if full == 0 else not 65 <= rest <= 143 if full == 1 else rest > 0 or full <= 3)
-        shape = 2 if cut and K <= 6144 and M >= 512 and 9 * M >= 8 * 256 * -(-M // 256) else None
+        if K <= 6144 and M > 128 and 7 * COMPUTE_UNITS <= 8 * low <= 8 * COMPUTE_UNITS:
+            shape = 1
+        elif cut and K <= 6144 and M >= 512 and (9 * M >= 8 * 256 * -(-M // 256) or (M > 768 and M * F >= 0.74 * _tile_room(full, rest))):
+            shape = 2
+    elif K > 2048:
+        if M > 128 and 3 * COMPUTE_UNITS <= 4 * low <= 4 * COMPUTE_UNITS:
+            shape = 1
+        elif 256 < M <= 3584 and M * F >= 0.74 * _tile_room(*divmod(tiles(256, 128), COMPUTE_UNITS)):
+            shape = 2
     elif K <= 2048:
         if tiles(64, 64) <= COMPUTE_UNITS:
             shape = 0 if K <= 1024 or tiles(64, 64) >= 48 else None
