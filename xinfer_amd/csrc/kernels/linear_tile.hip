@@ -43,6 +43,13 @@
 // cubed); the tiles going memory -> registers -> LDS (0.83); four waves of twice the tile each
 // (0.80, and 7% behind with the reads between the products); the operands of one step only in registers (the second step's reads then wait: -8%).
 //
+// Products of a few MB at up to 1,024 rows (and any of one round of them: `kernels.small_tile_plan`) go in tiles of 64 x 64, 64 x 128 or 128 x 128 with
+// rings of four to eight stages: a workgroup has 96 to 128 KB on their way from its first clocks on, which for 512 k of 64 x 64 is all it
+// will need, and the time is a kernel's start, one way to memory and the results' way out.  With slices of K the reader adds partial sums.
+// Rows, N, K, us, weights from memory, the library | the tiles for 128 rows a block (linear_mid) | this: 256, 1024, 2048 8.4 | 15.6 | 5.8 (four
+// slices of 64 x 64), 256, 1024, 3072 9.7 | 16.6 | 7.3, 256, 4096, 1024 12.0 | 17.1 | 8.1 (whole), 512, 2048, 4096 21.7 | - | 15.8 (20.1 in six slices of
+// 256 x 256), 1024, 1024, 1024 8.9 | - | 6.9, 128, 1024, 2048 8.5 | 8.1 | 4.7, 64, 1024, 1024 8.5 | 5.0 | 4.3.
+//
 // Workgroups go round the chip's eight dies; consecutive workgroup numbers of one die are mapped
 // to tiles that share rows of w, then of x, so that a die's L2 holds what its workgroups share.
 // The value of an output element depends on (K, the slices) alone: never on M, on the tile shape or
@@ -219,16 +226,17 @@ int xi_linear_tile_takes(int M, int N, int K, int slices) {
 // float32 [slices, M, N], the sums over the slices of K: slice s takes the tiles of 64 k from
 // s * (K / 64) / slices up to (s + 1) * (K / 64) / slices (whole numbers: the slices differ by a tile
 // at most).  shape 0: tiles of 128 rows by 256
-// features; 1: 256 rows by 128 features; 2: 256 by 256; without slices also 4, 5, 6: 96, 160 and 224 rows by 256 features.
+// features; 1: 256 rows by 128 features; 2: 256 by 256; 7, 8, 9: 64 by 64, 64 by 128, 128 by 128; without slices also 4,
+// 5, 6: 96, 160 and 224 rows by 256 features.
 int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, int slices, int partial, int shape,
                    hipStream_t stream) {
   XI_CHECK(xi_linear_tile_takes(M, N, K, slices), "linear_tile: M=%d N=%d K=%d in %d slices is not taken (K in tiles of "
            "64, a tile a slice at least, N a multiple of 4)", M, N, K, slices);
   XI_CHECK(partial || slices == 1, "linear_tile: %d slices need the float32 partial sums", slices);
-  XI_CHECK((shape >= 0 && shape <= 2) || (shape >= 4 && shape <= 6 && !partial), "linear_tile: unknown tile shape %d", shape);
+  XI_CHECK((shape >= 0 && shape <= 2) || (shape >= 4 && shape <= 6 && !partial) || (shape >= 7 && shape <= 9), "linear_tile: unknown tile shape %d", shape);
   XI_CHECK((size_t)K * 2 * 256 < ((size_t)1 << 32), "linear_tile: K=%d is too long for 32-bit offsets within a tile", K);
-  static const int heights[7] = {128, 256, 256, 0, 96, 160, 224};
-  const int bm = heights[shape], bn = shape == 1 ? 128 : 256;
+  static const int heights[10] = {128, 256, 256, 0, 96, 160, 224, 64, 64, 128}, widths[10] = {256, 128, 256, 0, 256, 256, 256, 64, 128, 128};
+  const int bm = heights[shape], bn = widths[shape];
   const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   const long long total = (long long)tiles_m * tiles_n * slices;
   XI_CHECK(total <= 0x7fffffffLL, "linear_tile: too many workgroups");
@@ -252,7 +260,17 @@ int xi_linear_tile(const void* x, const void* w, void* y, int M, int N, int K, i
     else XI_TILE(256, 256, 2, 4, 2, 3, false);
   } else if (shape == 4) XI_TILE(96, 256, 2, 4, 3, 3, false);
   else if (shape == 5) XI_TILE(160, 256, 2, 4, 3, 3, false);
-  else XI_TILE(224, 256, 2, 4, 2, 3, false);
+  else if (shape == 6) XI_TILE(224, 256, 2, 4, 2, 3, false);
+  else if (shape == 7) {
+    if (partial) XI_TILE(64, 64, 2, 4, 8, 8, true);
+    else XI_TILE(64, 64, 2, 4, 8, 8, false);
+  } else if (shape == 8) {
+    if (partial) XI_TILE(64, 128, 2, 4, 6, 6, true);
+    else XI_TILE(64, 128, 2, 4, 6, 6, false);
+  } else {
+    if (partial) XI_TILE(128, 128, 2, 4, 4, 5, true);
+    else XI_TILE(128, 128, 2, 4, 4, 5, false);
+  }
 #undef XI_TILE
   XI_LAUNCH_CHECK("linear_tile");
   return 0;

@@ -1790,6 +1790,56 @@ def tile_split_plan(M: int, N: int, K: int):
     return (best[1], best[2]) if best is not None else (1, 0)
 
 
+SMALL_TILE_ROWS = 2048        # rows up to which the low tiles were measured
+SMALL_TILE_SLICES = 12
+SMALL_TILES = (               # shape of `linear_tile`, rows, features; us: a kernel's start, a tile of 64 k alone and what the others of a round add to
+    (7, 64, 64, 2.72, 0.239, 0.073, 0.270, 0.0),           # it, a MB of results, a round of workgroups
+    (8, 64, 128, 2.64, 0.376, 0.086, 0.130, 1.08),
+    (9, 128, 128, 3.31, 0.448, 0.164, 0.254, 0.0))
+
+
+@functools.lru_cache(maxsize=4096)
+def small_tile_plan(M: int, N: int, K: int, split: bool):
+    """(shape of `linear_tile`, slices of K) of x [M, K] @ w [N, K]^T in one round of low tiles, None: not there.  `split`: the caller takes float32
+    partial sums.
+
+    The least of `SMALL_TILES`' times and the reader's of the partial sums (6 TB/s), by a fit to 4,100 measured times on MI355X with weights from memory
+    (1% of them more than 20 to 35% off).  What it stands against, with 38 weights of 256 to 10,240 features by 512 to 25,600 and 17 to 2,048 rows:
+      up to 128 rows, split, weights under 16 MB: `linear_mid`.  17 to 64 rows 12% ahead in the median, 2% behind at most, 65 to 128 35%, never
+      behind; a step of 20, 61 and 128 requests at Qwen3-0.6B sizes 1,333, 1,635 and 2,483 us with linear_mid, 1,303, 1,569 and 2,232 so.  (Larger
+      weights are 0 to 15% ahead alone and level to 3% behind in a step: 20 requests of 8 layers at 8B sizes 1,083 for 1,117.  Under 1,024 features
+      linear_mid stays: tests pin its bits there.)
+      where `tile_split_plan` cuts K, narrow ones: N up to 1,024, and up to 2,048 to 512 rows (256 rows, K=6144 15.1 for 18.5, 512 rows 21.5 for
+      24.1, with half the partial sums and less; 768 rows, K=8192 40.2 for 32.4).  (Wider ones are 5 to 20% ahead alone up to 256 rows, 2% of a step
+      at 8B sizes; tests pin the slices there.)
+      129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
+      otherwise, from 65 rows on: the library, where the time is below what that takes at its better sizes (8 us; 6 us and 0.7, 0.85 or 1.25 PFLOP/s up
+      to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
+    if not 17 <= M <= SMALL_TILE_ROWS or N % 4 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)) or (M < 65 and not split):
+        return None
+    k_tiles, best = K // 64, None
+    for shape, rows, features, start, alone, more, out, full in SMALL_TILES:
+        tiles = -(-M // rows) * -(-N // features)
+        for slices in range(1, SMALL_TILE_SLICES + 1 if split else 2):
+            share = tiles * slices / COMPUTE_UNITS
+            if share > 1 or (slices > 1 and k_tiles // slices < 4):
+                break
+            written = M * N * (4e-6 * slices if slices > 1 else 2e-6)
+            cost = start + -(-k_tiles // slices) * (alone + more * share) + out * written + full * share
+            if slices > 1:
+                cost += M * N * (4 * slices - 2) / 6e6
+            if best is None or cost < best[0]:
+                best = (cost, shape, slices)
+    if best is None:
+        return None
+    if split and tile_split_plan(M, N, K)[0] > 1:
+        return best[1:] if N <= 1024 or (N <= 2048 and M <= 512) else None
+    if split and M <= 256:
+        return best[1:]
+    library = max(8.0, 6 + 2e-9 * M * N * K / (0.7 if M <= 512 else 0.85 if M <= 1024 else 1.25))
+    return best[1:] if best[0] < library else None
+
+
 def linear_tile_takes(M: int, N: int, K: int, slices: int = 1) -> bool:
     """Whether the many-row tiled product takes a shape: K in whole tiles of 64, a tile a slice at least, N in fours."""
     return bool(lib().xi_linear_tile_takes(int(M), int(N), int(K), int(slices)))
@@ -1800,7 +1850,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
     """bfloat16 x [M, K] @ w [N, K]^T on the matrix cores for many rows: bfloat16 [M, N], or with
     `partial` (needed for more than one slice) float32 partial sums [slices, M, N] over slices of K
     (whole tiles of 64, equal but for one tile).  `shape` 0: workgroup tiles of 128 rows by 256 features, 1: 256 by 128; None: the
-    one that makes fewer tiles (128 by 256 at equal numbers); 2: 256 by 256."""
+    one that makes fewer tiles (128 by 256 at equal numbers); 2: 256 by 256; 7, 8, 9: 64 by 64, 64 by 128, 128 by 128."""
     _dev(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError("linear_tile: operands must be bfloat16")
@@ -1811,7 +1861,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, slices: int = 1, partial: bool
     partial = bool(partial) or slices > 1
     if not linear_tile_takes(M, N, K, slices):
         raise KernelError(f"linear_tile: M={M} N={N} K={K} in {slices} slices is not taken")
-    if shape not in (None, 0, 1, 2):
+    if shape not in (None, 0, 1, 2, 7, 8, 9):
         raise KernelError(f"linear_tile: unknown tile shape {shape}")
     if shape is None:
         shape = 1 if -(-M // 256) * -(-N // 128) < -(-M // 128) * -(-N // 256) else 0
@@ -2154,6 +2204,10 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     if out_dtype == torch.float32 and MID_WIDE_FROM <= x.shape[0] <= MID_GATED_ROWS \
             and linear_mid_slices(w.shape[0], w.shape[1]) == 1:
         return linear_mid(x, w)[0]           # a wide output in float32 (the head): one slice is the result
+    if out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15:
+        small = small_tile_plan(x.shape[0], w.shape[0], x.shape[1], bool(allow_split))
+        if small is not None:
+            return linear_tile(x, w, small[1], shape=small[0])
     if allow_split and MID_BLOCK < x.shape[0] <= TILE_SPLIT_ROWS:
         slices, shape = tile_split_plan(x.shape[0], w.shape[0], w.shape[1])
         if slices > 1:

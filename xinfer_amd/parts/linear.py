@@ -6,7 +6,8 @@ BLAS (/root/reference/src/models/layers/linear.rs:76-124).  Here:
              an output element does not depend on the batch it was computed in;
   bfloat16 : the hand-written kernels for few rows (decode), the vendor library
              (hipBLASLt through torch) for many rows, as the reference uses a library;
-             narrow outputs at 129 to 1,024 rows in the hand-written many-row tiled kernel over
+             products of one round of low tiles from 17 rows on in the hand-written many-row tiled
+             kernel (`kernels.small_tile_plan`), narrow outputs at 129 to 1,024 rows in it over
              slices of K where the caller takes partial sums (`kernels.tile_split_plan`), and
              the gated form of more than 64 rows in that kernel's tiles with the activation in
              them where it is ahead (`kernels.gated_tile_shape`).
