@@ -143,3 +143,32 @@ def test_last_chunks_of_a_few_tokens(H, dk, dv, lens):
             ref, most = ((x * y[..., None]).sum(1) * dk ** -0.5 for x, y in ((S, qd[t]), (size, qd[t].abs())))
             assert float(((o[t] - ref).abs() / most).max()) < bound
         assert float(((st[b].cpu().double() - S).abs() / size).max()) < bound
+
+
+@pytest.mark.parametrize("kind", ["z", "head", "step", "gates"])
+@pytest.mark.parametrize("H,dk,dv,dtype", [(3, 256, 40, torch.bfloat16), (4, 100, 130, torch.float32), (5, 64, 64, torch.bfloat16), (2, 24, 70, torch.float32)])
+def test_tokens_fetched_together(H, dk, dv, dtype, kind):
+    """Portions that end anywhere in a group of tokens give the bits of their tokens one at a time, results and states."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(dk)
+    lens = [1, 2, 3, 5, 8, 17, 31]
+    T, B = sum(lens), len(lens)
+    vc = dv - 1 if kind == "gates" else dv
+    starts = [sum(lens[:b]) for b in range(B + 1)]
+    q, k = (torch.randn(T, H * dk, generator=g).to(dtype).to(DEV) for _ in range(2))
+    v = torch.randn(T, H * vc, generator=g).to(dtype).to(DEV)
+    rows = {"z": dict(z=torch.randn(T, H * dk, generator=g).to(DEV)), "head": {}, "step": dict(step=torch.randn(T, H, generator=g).to(dtype).to(DEV)),
+            "gates": dict(gates=torch.rand(T, H, 2, generator=g).to(DEV))}[kind]
+    fixed = {"z": dict(z_bias=torch.randn(H * dk, generator=g).to(DEV), tau=4.0), "head": dict(head_decay=torch.rand(H, generator=g).to(DEV)),
+             "step": dict(step_bias=torch.randn(H, generator=g).to(DEV), decay_log=torch.randn(H, generator=g).to(DEV)), "gates": {}}[kind]
+    state = torch.randn(B, H, dk, dv, generator=g).to(DEV)
+    st, one = state.clone(), state.clone()
+    cu = torch.tensor(starts, dtype=torch.int32, device=DEV)
+    out = kernels.linear_scan(q, k, v, st, torch.arange(B, device=DEV), cu, H, dk, dv, value_cols=vc, **rows, **fixed)
+    for t in range(max(lens)):
+        live = [b for b in range(B) if t < lens[b]]
+        at = torch.tensor([starts[b] + t for b in live], device=DEV)
+        o = kernels.linear_scan(q[at], k[at], v[at], one, torch.tensor(live, device=DEV), torch.arange(len(live) + 1, dtype=torch.int32, device=DEV), H, dk, dv,
+                                value_cols=vc, **{n: r[at] for n, r in rows.items()}, **fixed)
+        assert torch.equal(out[at], o), t
+    assert torch.equal(st, one)

@@ -26,8 +26,9 @@
 // from a state it is told to start from, and may leave the new state somewhere.  Lane l owns value column l
 // of the tile (or columns l and l + 64), wave w the key channels w RPT .. (w + 1) RPT - 1 (read from LDS four at a time; channels past
 // the head's are zeros there, so the inner loop has no bounds); a thread keeps its RPT state elements in
-// registers for the whole walk.  A token costs one barrier: q, k and the decay of the next token are fetched while this
-// one is worked on.  An item is a request's tokens of this step (from the state in its slot, back into it:
+// registers for the whole walk.  q, k and the decays of the next few tokens are fetched while these are worked on, with one
+// barrier for all of them (a token at a time, the walk waited for memory at every token: 8 heads of 128 by 256 over 1,974 tokens
+// in chunks of 64 254 -> 182 us, 100 tokens in one piece 108 -> 74, of which the instructions are 100 and 60).  An item is a request's tokens of this step (from the state in its slot, back into it:
 // steps of single tokens and short portions; what a token gets then does not depend on how the prompt was
 // cut, bit for bit), or one chunk of a long portion:
 //
@@ -47,6 +48,9 @@ namespace xi {
 
 constexpr int kScanWaves = 4;
 constexpr int kScanCols = 64;
+// tokens of a group by a thread's channels.  2, 4 and 8 tokens, us, all of a portion's launches: 8 heads of 128 by 256, 1,974 tokens 182 | 187 | 245 (254
+// with one), a mixed step's 300 173 | 185 | 186 (280), 4 heads of 64 by 128, 90 tokens 55 | 43 | 41 (81), of 24 by 40, 200 tokens 97 | 74 | 64 (173).
+constexpr int together(int rpt) { return rpt <= 8 ? 8 : rpt <= 16 ? 4 : 2; }
 
 __device__ __forceinline__ float decay_of(float z, float inv_tau) {
   // sigmoid(z)^(1/tau) = exp(-softplus(-z) / tau); softplus(x) = max(x, 0) + log1p(exp(-|x|))
@@ -61,7 +65,9 @@ __device__ __forceinline__ float decay_of(float z, float inv_tau) {
 // COLS: value columns a lane owns, 64 apart.  A token's operands are the same numbers in all lanes, read from LDS by every wave,
 // and these reads bound a walk with many workgroups: two columns a lane read them once for both.
 // RES: there are results; without them q is neither fetched nor multiplied.
-template <typename T, int RPT, bool ONE, bool ACT, int COLS, bool RES>
+// U: tokens that are fetched together, while the U before them are worked on, with one barrier for all of them: a walk of U = 1 over a portion waits
+// for memory once a token.  U = 1 for steps of single tokens.
+template <typename T, int RPT, bool ONE, bool ACT, int COLS, bool RES, int U>
 __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     const T* __restrict__ q, long long q_stride, const T* __restrict__ k, long long k_stride, const T* __restrict__ v,
     long long v_stride, const float* __restrict__ z, const float* __restrict__ z_bias, float inv_tau,
@@ -71,9 +77,12 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
     float* __restrict__ state_out, long long out_stride, const long long* __restrict__ out_idx,
     const int* __restrict__ first, const int* __restrict__ last, float* __restrict__ out, float* __restrict__ decay_out,
     int H, int dk, int dv, float q_scale, float k_scale, int skip_from) {
-  __shared__ __attribute__((aligned(16))) float qs[2][kScanWaves * 64], ks[2][kScanWaves * 64], as[2][kScanWaves * 64];
-  __shared__ float part[2][kScanWaves][COLS * kScanCols];
-  __shared__ float npart[2][kScanWaves];
+  constexpr int CH = kScanWaves * RPT;                       // channels with room, zeros past the head's
+  constexpr int SIDE = kScanWaves * kWave / CH;              // tokens whose channels the threads fetch side by side
+  constexpr int FU = (U + SIDE - 1) / SIDE;                  // tokens of a group that a thread fetches a channel of
+  __shared__ __attribute__((aligned(16))) float qs[2][U][RES ? CH : 4], ks[2][U][CH], as[2][U][ONE ? 4 : CH];
+  __shared__ float part[2][U][kScanWaves][COLS * kScanCols];
+  __shared__ float npart[2][U][kScanWaves];
   const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * (COLS * kScanCols) + (threadIdx.x & 63);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t0 = first[b], t1 = last[b];
@@ -92,105 +101,137 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
       const int i = wave * RPT + r;
       s[e][r] = (from >= 0 && col[e] && i < dk) ? S[(size_t)i * dv + j0 + kScanCols * e] : 0.f;
     }
-  float all_decays = 1.f;               // of channel c, over the item's tokens
-  const int c = threadIdx.x;            // the channel this thread fetches for the workgroup
-  float nc = (ones && from >= 0 && c < dk) ? S[(size_t)c * dv + v_cols] : 0.f;
+  float all_decays = 1.f;               // of channel `own`, over the item's tokens
+  const int own = threadIdx.x;
+  float nc = (ones && from >= 0 && own < dk) ? S[(size_t)own * dv + v_cols] : 0.f;
+  const int c = threadIdx.x % CH, side = threadIdx.x / CH;      // the channel this thread fetches for the workgroup, of tokens side, side + SIDE, ..
   const float hd = head_decay ? head_decay[h] : 0.f;
   const float zb = (z_bias && c < dk) ? z_bias[h * dk + c] : 0.f;
   const int qk0 = (h / group_heads) * dk;       // the head's set of q and k columns
   const float sb = step ? step_bias[h] : 0.f, rate = step ? -expf(decay_log[h]) : 0.f;
-  // the token's step size (1 where the decay has another source): every thread makes its own copy
-  auto step_of = [&](int t) {
-    if (gates) return gates[((size_t)t * H + h) * 2 + 1];
-    if (!step) return 1.f;
-    const float x = to_float(step[(size_t)t * step_stride + h]) + sb;
-    return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
-  };
   auto read = [&](T x) {
     const float f = to_float(x);
     return ACT ? f / (1.f + expf(-f)) : f;
   };
-  auto fetch = [&](int t, float dt, float& fq, float& fk, float& fa) {      // (channels past the head's stay zero)
-    if (c < dk) {
-      if (RES) fq = read(q[(size_t)t * q_stride + qk0 + c]) * q_scale;
-      fk = read(k[(size_t)t * k_stride + qk0 + c]) * k_scale;
-      if (!ONE) fa = decay_of(z[((size_t)t * H + h) * dk + c] + zb, inv_tau);
+  // tokens t .. t + U - 1 as they come from memory
+  T rq[FU], rk[FU], rv[U][COLS];
+  float rz[FU], keep[U], take[U];             // keep, take: ready-made gates, or the step size's raw value in `take`
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < FU; ++i) {
+      const int u = side + SIDE * i;
+      if (u >= U || t + u >= t1 || c >= dk) continue;
+      const size_t row = (size_t)(t + u);
+      if (RES) rq[i] = q[row * q_stride + qk0 + c];
+      rk[i] = k[row * k_stride + qk0 + c];
+      if (!ONE) rz[i] = z[(row * H + h) * dk + c];
     }
-    if (ONE) fa = gates ? gates[((size_t)t * H + h) * 2] : step ? expf(rate * dt) : hd;
-  };
-  float fq = 0.f, fk = 0.f, fa = 0.f;
-  float dt = step_of(t0);
-  fetch(t0, dt, fq, fk, fa);
-  // the token's value is asked for a token ahead as well: no step of the walk waits for memory
-  // (a column past the value rows' own reads 1)
-  auto value_of = [&](int t, int j) { return j < v_cols ? read(v[(size_t)t * v_stride + h * v_cols + j]) : 1.f; };
-  float v_next[COLS];
 #pragma unroll
-  for (int e = 0; e < COLS; ++e) v_next[e] = col[e] ? value_of(t0, j0 + kScanCols * e) * dt : 0.f;
-  if (RES) qs[0][c] = fq;
-  ks[0][c] = fk;
-  if (!ONE) as[0][c] = fa;
-  __syncthreads();
-  for (int t = t0; t < t1; ++t) {
-    const int cur = (t - t0) & 1;
-    all_decays *= fa;
-    const float a_now = fa;
-    float vj[COLS];
-#pragma unroll
-    for (int e = 0; e < COLS; ++e) vj[e] = v_next[e];
-    if (ones) {                          // (this token's k and q are in LDS since the last barrier)
-      nc = fmaf(a_now, nc, dt * ks[cur][c]);
-      if (RES) {
-        const float nq = wave_sum(nc * qs[cur][c]);
-        if (lane == 0) npart[cur][wave] = nq;
+    for (int u = 0; u < U; ++u) {
+      if (t + u >= t1) continue;
+      const size_t row = (size_t)(t + u);
+      if (ONE && gates) {
+        keep[u] = gates[(row * H + h) * 2];
+        take[u] = gates[(row * H + h) * 2 + 1];
+      } else if (ONE && step) {
+        take[u] = to_float(step[row * step_stride + h]);
       }
-    }
-    if (t + 1 < t1) {
-      dt = step_of(t + 1);
-      fetch(t + 1, dt, fq, fk, fa);
 #pragma unroll
       for (int e = 0; e < COLS; ++e)
-        if (col[e]) v_next[e] = value_of(t + 1, j0 + kScanCols * e) * dt;
+        if (col[e]) rv[u][e] = v[row * v_stride + h * v_cols + j0 + kScanCols * e];
     }
-    float acc[COLS] = {};
-    const float4* a4 = reinterpret_cast<const float4*>(&as[cur][wave * RPT]);
-    const float4* k4 = reinterpret_cast<const float4*>(&ks[cur][wave * RPT]);
-    const float4* q4 = reinterpret_cast<const float4*>(&qs[cur][wave * RPT]);
+  };
+  // the same as the walk uses them: q, k and the channels' decays in LDS (channels past the head's are zeros); every thread makes its own copy of the token's
+  // step size (1 where the decay has another source) and of a decay that is one number a head
+  float vj[U][COLS], dt[U], a_one[U];
+  auto put = [&](int buf, int t) {
 #pragma unroll
-    for (int r = 0; r < RPT; r += 4) {
-      const float4 av = ONE ? make_float4(a_now, a_now, a_now, a_now) : a4[r / 4];
-      const float4 kv = k4[r / 4], qv = RES ? q4[r / 4] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < FU; ++i) {
+      const int u = side + SIDE * i;
+      if (u >= U || t + u >= t1) continue;
+      if (RES) qs[buf][u][c] = c < dk ? read(rq[i]) * q_scale : 0.f;
+      ks[buf][u][c] = c < dk ? read(rk[i]) * k_scale : 0.f;
+      if (!ONE) as[buf][u][c] = c < dk ? decay_of(rz[i] + zb, inv_tau) : 0.f;
+    }
 #pragma unroll
-      for (int e = 0; e < COLS; ++e) {
-        s[e][r] = fmaf(av.x, s[e][r], kv.x * vj[e]);
-        s[e][r + 1] = fmaf(av.y, s[e][r + 1], kv.y * vj[e]);
-        s[e][r + 2] = fmaf(av.z, s[e][r + 2], kv.z * vj[e]);
-        s[e][r + 3] = fmaf(av.w, s[e][r + 3], kv.w * vj[e]);
+    for (int u = 0; u < U; ++u) {
+      if (t + u >= t1) continue;
+      dt[u] = 1.f;
+      a_one[u] = hd;
+      if (ONE && gates) {
+        dt[u] = take[u];
+        a_one[u] = keep[u];
+      } else if (ONE && step) {
+        const float x = take[u] + sb;
+        dt[u] = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
+        a_one[u] = expf(rate * dt[u]);
+      }
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) vj[u][e] = col[e] ? read(rv[u][e]) * dt[u] : 0.f;
+    }
+  };
+  fetch(t0);
+  put(0, t0);
+  __syncthreads();
+  int cur = 0;
+  for (int t = t0; t < t1; t += U, cur ^= 1) {
+    const bool more = t + U < t1;
+    if (more) fetch(t + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (t + u >= t1) break;
+      const float a_own = ONE ? a_one[u] : own < dk ? as[cur][u][own] : 0.f;
+      all_decays *= a_own;
+      if (ones) {
+        const float k_own = own < dk ? ks[cur][u][own] : 0.f;
+        nc = fmaf(a_own, nc, dt[u] * k_own);
         if (RES) {
-          acc[e] = fmaf(s[e][r], qv.x, acc[e]);
-          acc[e] = fmaf(s[e][r + 1], qv.y, acc[e]);
-          acc[e] = fmaf(s[e][r + 2], qv.z, acc[e]);
-          acc[e] = fmaf(s[e][r + 3], qv.w, acc[e]);
+          const float q_own = own < dk ? qs[cur][u][own] : 0.f;
+          const float nq = wave_sum(nc * q_own);
+          if (lane == 0) npart[cur][u][wave] = nq;
         }
       }
+      float acc[COLS] = {};
+      const float4* a4 = reinterpret_cast<const float4*>(&as[cur][u][ONE ? 0 : wave * RPT]);
+      const float4* k4 = reinterpret_cast<const float4*>(&ks[cur][u][wave * RPT]);
+      const float4* q4 = reinterpret_cast<const float4*>(&qs[cur][u][RES ? wave * RPT : 0]);
+#pragma unroll
+      for (int r = 0; r < RPT; r += 4) {
+        const float4 av = ONE ? make_float4(a_one[u], a_one[u], a_one[u], a_one[u]) : a4[r / 4];
+        const float4 kv = k4[r / 4], qv = RES ? q4[r / 4] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int e = 0; e < COLS; ++e) {
+          s[e][r] = fmaf(av.x, s[e][r], kv.x * vj[u][e]);
+          s[e][r + 1] = fmaf(av.y, s[e][r + 1], kv.y * vj[u][e]);
+          s[e][r + 2] = fmaf(av.z, s[e][r + 2], kv.z * vj[u][e]);
+          s[e][r + 3] = fmaf(av.w, s[e][r + 3], kv.w * vj[u][e]);
+          if (RES) {
+            acc[e] = fmaf(s[e][r], qv.x, acc[e]);
+            acc[e] = fmaf(s[e][r + 1], qv.y, acc[e]);
+            acc[e] = fmaf(s[e][r + 2], qv.z, acc[e]);
+            acc[e] = fmaf(s[e][r + 3], qv.w, acc[e]);
+          }
+        }
+      }
+      if (RES) {
+#pragma unroll
+        for (int e = 0; e < COLS; ++e) part[cur][u][wave][lane + kScanCols * e] = acc[e];
+      }
     }
+    if (more) put(cur ^ 1, t + U);
+    __syncthreads();
     if (RES) {
 #pragma unroll
-      for (int e = 0; e < COLS; ++e) part[cur][wave][lane + kScanCols * e] = acc[e];
+      for (int p = 0; p < U * COLS; p += kScanWaves) {
+        const int u = (p + wave) / COLS, e = (p + wave) % COLS, at = lane + kScanCols * e, j = j0 + kScanCols * e;
+        if (p + wave < U * COLS && t + u < t1 && j < v_cols)
+          out[((size_t)(t + u) * H + h) * dv + j] =
+              (part[cur][u][0][at] + part[cur][u][1][at]) + (part[cur][u][2][at] + part[cur][u][3][at]);
+      }
+      if (ones && blockIdx.z == 0 && own < U && t + own < t1)
+        out[((size_t)(t + own) * H + h) * dv + v_cols] =
+            (npart[cur][own][0] + npart[cur][own][1]) + (npart[cur][own][2] + npart[cur][own][3]);
     }
-    if (t + 1 < t1) {
-      if (RES) qs[cur ^ 1][c] = fq;
-      ks[cur ^ 1][c] = fk;
-      if (!ONE) as[cur ^ 1][c] = fa;
-    }
-    __syncthreads();
-    if (RES && wave < COLS) {
-      const int at = lane + kScanCols * wave, j = j0 + kScanCols * wave;
-      if (j < v_cols)
-        out[((size_t)t * H + h) * dv + j] = (part[cur][0][at] + part[cur][1][at]) + (part[cur][2][at] + part[cur][3][at]);
-    }
-    if (RES && ones && blockIdx.z == 0 && threadIdx.x == 0)
-      out[((size_t)t * H + h) * dv + v_cols] = (npart[cur][0] + npart[cur][1]) + (npart[cur][2] + npart[cur][3]);
   }
   if (to >= 0) {
     float* D = state_out + (size_t)to * out_stride + (size_t)h * dk * dv;
@@ -201,9 +242,9 @@ __global__ __launch_bounds__(kScanWaves* kWave) void linear_scan_kernel(
         const int i = wave * RPT + r;
         if (col[e] && i < dk) D[(size_t)i * dv + j0 + kScanCols * e] = s[e][r];
       }
-    if (ones && blockIdx.z == 0 && c < dk) D[(size_t)c * dv + v_cols] = nc;
+    if (ones && blockIdx.z == 0 && own < dk) D[(size_t)own * dv + v_cols] = nc;
   }
-  if (decay_out && blockIdx.z == 0 && c < dk) decay_out[((size_t)b * H + h) * dk + c] = all_decays;
+  if (decay_out && blockIdx.z == 0 && own < dk) decay_out[((size_t)b * H + h) * dk + own] = all_decays;
 }
 
 // The states that the chunks of long portions start from.  Portion p has n[p] chunks, numbered from c0[p]:
@@ -330,14 +371,14 @@ extern "C" {
 // first[w] .. last[w] - 1 from the state state_in + in_idx[w] * in_stride ([H, dk, dv] float32; in_idx null or a
 // negative entry: from zeros) and leaves its last state at state_out + out_idx[w] * out_stride (null or negative:
 // nowhere); out float32 [T, H, dv] or null (no results); decay_out float32 [items, H, dk] or null: the product of
-// each channel's decays over the item.
+// each channel's decays over the item.  singles: the items are single tokens (the results do not depend on it).
 int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k_stride, const void* v, long long v_stride,
                    int dtype, const float* z, const float* z_bias, float tau, const float* head_decay, const void* step,
                    long long step_stride, const float* step_bias, const float* decay_log, const float* gates, int v_cols,
                    int group_heads, const float* state_in,
                    long long in_stride, const long long* in_idx, float* state_out, long long out_stride,
                    const long long* out_idx, const int* first, const int* last, float* out, float* decay_out, int n_items, int H,
-                   int dk, int dv, float q_scale, float k_scale, int act, int skip_from, hipStream_t stream) {
+                   int dk, int dv, float q_scale, float k_scale, int act, int skip_from, int singles, hipStream_t stream) {
   if (skip_from <= 0) skip_from = 0x7fffffff;
   XI_CHECK(n_items >= 0 && H > 0 && dk > 0 && dv > 0, "linear_scan: bad sizes items=%d H=%d dk=%d dv=%d", n_items, H, dk, dv);
   XI_CHECK(dk <= kScanWaves * 64, "linear_scan: key heads of up to %d channels, not %d", kScanWaves * 64, dk);
@@ -367,18 +408,19 @@ int xi_linear_scan(const void* q, long long q_stride, const void* k, long long k
       (const TT*)q, q_stride, (const TT*)k, k_stride, (const TT*)v, v_stride, z, z_bias, inv_tau, head_decay, (const TT*)step,    \
       step_stride, step_bias, decay_log, gates, v_cols, group_heads, state_in, in_stride,                                                    \
       in_idx, state_out, out_stride, out_idx, first, last, out, decay_out, H, dk, dv, q_scale, k_scale, skip_from
-#define XI_SCAN_F(TT, R, COLS, RES)                                                                                           \
+#define XI_SCAN_F(TT, R, COLS, RES, U)                                                                                        \
   do {                                                                                                                        \
-    if (z) linear_scan_kernel<TT, R, false, false, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));     \
-    else if (act) linear_scan_kernel<TT, R, true, true, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT)); \
-    else linear_scan_kernel<TT, R, true, false, COLS, RES><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));        \
+    if (z) linear_scan_kernel<TT, R, false, false, COLS, RES, U><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));  \
+    else if (act) linear_scan_kernel<TT, R, true, true, COLS, RES, U><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT)); \
+    else linear_scan_kernel<TT, R, true, false, COLS, RES, U><<<grid, kScanWaves * kWave, 0, stream>>>(XI_SCAN_ARGS(TT));     \
   } while (0)
 #define XI_SCAN(TT, R)                          \
   do {                                          \
-    if (two && out) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), true);  \
-    else if (two) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), false);   \
-    else if (out) XI_SCAN_F(TT, R, 1, true);    \
-    else XI_SCAN_F(TT, R, 1, false);            \
+    if (two && out) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), true, together(R));  \
+    else if (two) XI_SCAN_F(TT, R, (R <= 32 ? 2 : 1), false, together(R));   \
+    else if (out && singles) XI_SCAN_F(TT, R, 1, true, 1); \
+    else if (out) XI_SCAN_F(TT, R, 1, true, together(R));    \
+    else XI_SCAN_F(TT, R, 1, false, together(R));            \
   } while (0)
 #define XI_SCAN_T(TT)            \
   do {                           \

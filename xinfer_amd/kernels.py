@@ -411,14 +411,15 @@ def _step_chunks(common, state, slot_stride, state_slots, cu_q, q_lens, plan_cac
 
 def _scan_launch(q, k, v, qs, ks, vs, z, z_bias, tau, head_decay, step, ss, step_bias, decay_log, gates, v_cols, group_heads, act,
                  state_in, in_stride, in_idx, state_out, out_stride, out_idx,
-                 first, last, out, decay_out, items, H, dk, dv, q_scale, k_scale, skip_from=0):
+                 first, last, out, decay_out, items, H, dk, dv, q_scale, k_scale, skip_from=0, singles=False):
     _ok(lib().xi_linear_scan(_p(q), ctypes.c_longlong(qs), _p(k), ctypes.c_longlong(ks), _p(v), ctypes.c_longlong(vs),
                              _code(q, "linear_scan"), _p(z), _p(z_bias), ctypes.c_float(tau), _p(head_decay),
                              _p(step), ctypes.c_longlong(ss), _p(step_bias), _p(decay_log), _p(gates), int(v_cols),
                              int(group_heads), _p(state_in),
                              ctypes.c_longlong(in_stride), _p(in_idx), _p(state_out), ctypes.c_longlong(out_stride),
                              _p(out_idx), ctypes.c_void_p(first), ctypes.c_void_p(last), _p(out), _p(decay_out), int(items),
-                             H, dk, dv, ctypes.c_float(q_scale), ctypes.c_float(k_scale), int(act), int(skip_from), _stream()))
+                             H, dk, dv, ctypes.c_float(q_scale), ctypes.c_float(k_scale), int(act), int(skip_from), int(singles),
+                             _stream()))
 
 
 def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor,
@@ -515,7 +516,7 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     whole, long, chunks = scan_chunk_plan(q_lens) if q_lens is not None else (None, [], [])
     if not long:            # every request in one piece, straight from the step's own arrays
         _scan_launch(*common, state, slot_stride, state_slots, state, slot_stride, state_slots, cu_q.data_ptr(),
-                     cu_q.data_ptr() + 4, out, None, B, H, dk, dv, q_scale, k_scale)
+                     cu_q.data_ptr() + 4, out, None, B, H, dk, dv, q_scale, k_scale, singles=T <= B)
         return out
     key = ("linear_scan_plan", SCAN_CHUNK)
     plan = plan_cache.get(key) if plan_cache is not None else None
