@@ -59,7 +59,7 @@ def test_low_tiles_are_one_round(split):
             taken += 1
             rows, features = {7: (64, 64), 8: (64, 128), 9: (128, 128)}[plan[0]]
             assert -(-M // rows) * -(-N // features) * plan[1] <= kernels.COMPUTE_UNITS and kernels.linear_tile_takes(M, N, K, plan[1])
-            assert 17 <= M <= 2048 and (split or (plan[1] == 1 and M >= 65)) and (plan[1] == 1 or K // 64 // plan[1] >= 4)
+            assert 17 <= M <= 2048 and (split or plan[1] == 1) and (plan[1] == 1 or K // 64 // plan[1] >= 4)
             assert not split or M > 128 or (N >= 1024 and N * K < 1 << 23)
     assert taken > 50
     plan = kernels.small_tile_plan

@@ -64,13 +64,15 @@ def _p(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# (torch.cuda.current_device makes sure of an initialised runtime first, which operands on the GPU have: 0.6 us a launch)
+_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream() -> ctypes.c_void_p:
     """The current HIP stream of the current device (asked for at every launch: the runner
     records graphs on a side stream)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return ctypes.c_void_p(_raw_stream(_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -1814,9 +1816,9 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
       24.1, with half the partial sums and less; 768 rows, K=8192 40.2 for 32.4).  (Wider ones are 5 to 20% ahead alone up to 256 rows, 2% of a step
       at 8B sizes; tests pin the slices there.)
       129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
-      otherwise, from 65 rows on: the library, where the time is below what that takes at its better sizes (8 us; 6 us and 0.7, 0.85 or 1.25 PFLOP/s up
-      to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
-    if not 17 <= M <= SMALL_TILE_ROWS or N % 4 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)) or (M < 65 and not split):
+      otherwise: the library, where the time is below what that takes at its better sizes (5.6 us under 32 rows and up to 2,048 features, 8 us; from 65
+      rows on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
+    if not 17 <= M <= SMALL_TILE_ROWS or N % 4 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)):
         return None
     k_tiles, best = K // 64, None
     for shape, rows, features, start, alone, more, out, full in SMALL_TILES:
@@ -1837,7 +1839,10 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
         return best[1:] if N <= 1024 or (N <= 2048 and M <= 512) else None
     if split and M <= 256:
         return best[1:]
-    library = max(8.0, 6 + 2e-9 * M * N * K / (0.7 if M <= 512 else 0.85 if M <= 1024 else 1.25))
+    if M < 65:
+        library = 8.0 if M >= 32 or N > 2048 else 5.6
+    else:
+        library = max(8.0, 6 + 2e-9 * M * N * K / (0.7 if M <= 512 else 0.85 if M <= 1024 else 1.25))
     return best[1:] if best[0] < library else None
 
 
@@ -2206,9 +2211,14 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
             and linear_mid_slices(w.shape[0], w.shape[1]) == 1:
         return linear_mid(x, w)[0]           # a wide output in float32 (the head): one slice is the result
     if out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15:
-        small = small_tile_plan(x.shape[0], w.shape[0], x.shape[1], bool(allow_split))
+        M, K = x.shape
+        N = w.shape[0]
+        small = small_tile_plan(M, N, K, allow_split)
         if small is not None:
-            return linear_tile(x, w, small[1], shape=small[0])
+            shape, slices = small
+            y = torch.empty((slices, M, N), dtype=torch.float32, device=x.device) if slices > 1 else torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+            _ok(lib().xi_linear_tile(_p(x), _p(w), _p(y), M, N, K, slices, int(slices > 1), shape, _stream()))
+            return y
     if allow_split and MID_BLOCK < x.shape[0] <= TILE_SPLIT_ROWS:
         slices, shape = tile_split_plan(x.shape[0], w.shape[0], w.shape[1])
         if slices > 1:
