@@ -155,6 +155,11 @@ class CausalLM:
                 want_rows: torch.Tensor) -> torch.Tensor:
         """ids int32 [T]; caches: layer index -> the cache that layer owns; want_rows int32
         [R].  Returns float32 logits [R, vocab]."""
+        return self.head.forward(self.hidden(ids, ctx, caches, want_rows))
+
+    def hidden(self, ids: torch.Tensor, ctx: StepContext, caches: Dict[int, LayerCache],
+               want_rows: torch.Tensor) -> torch.Tensor:
+        """What `forward` gives the head: the wanted rows behind the last norm."""
         ctx.ids = ids
         if EMBEDDING_CACHE in self.state_needs:
             first = self.embedding.forward(ids, ctx, cache=caches[EMBEDDING_CACHE])
@@ -192,12 +197,9 @@ class CausalLM:
             for op in e.after:
                 stream = run_op(self.stream_ops[id(op)], stream)
         if stream.open and joins(self.final_norm):
-            h = join(stream, self.dtype, (self.final_norm,), rows=want_rows)[2][0]
-            return self.head.forward(h)
+            return join(stream, self.dtype, (self.final_norm,), rows=want_rows)[2][0]
         stream = closed(stream)
         if stream.pending is not None and stream.pending_scale != 1.0:
-            h = self.final_norm.forward(stream.resid, stream.pending, self.dtype, rows=want_rows,
-                                        add_scale=stream.pending_scale)
-        else:
-            h = self.final_norm.forward(stream.resid, stream.pending, self.dtype, rows=want_rows)
-        return self.head.forward(h)
+            return self.final_norm.forward(stream.resid, stream.pending, self.dtype, rows=want_rows,
+                                           add_scale=stream.pending_scale)
+        return self.final_norm.forward(stream.resid, stream.pending, self.dtype, rows=want_rows)

@@ -106,15 +106,15 @@ class _DecodeGraph:
     graph: Any
     dev32: torch.Tensor
     dev64: torch.Tensor
-    logits: torch.Tensor            # [B, vocab], rewritten by every replay
+    hidden: torch.Tensor            # [B, width], the head's rows, rewritten by every replay
     want: torch.Tensor              # int32 [B]: this step's wanted rows (first R valid)
     keep: Tuple[Any, ...] = ()      # everything else the recorded kernels read: it must stay
                                     # allocated for as long as the graph may be replayed
 
     @property
     def nbytes(self) -> int:
-        """What the graph holds for itself between replays: its logits and its index arrays."""
-        return sum(t.numel() * t.element_size() for t in (self.dev32, self.dev64, self.logits))
+        """What the graph holds for itself between replays: the head's rows and its index arrays."""
+        return sum(t.numel() * t.element_size() for t in (self.dev32, self.dev64, self.hidden))
 
 
 def context_bucket(longest: int) -> int:
@@ -150,7 +150,7 @@ class ModelRunner:
         the runner, the count is 3 for a model whose step is bound by the host and 12 otherwise,
         and `graph_max_batch` 256 for such a model (its launches cost more than its kernels at
         any batch size) and 64 otherwise.  At most `graphs_most` graphs holding `graph_bytes_most`
-        bytes (their logits, 39 MB at 64 rows of 151,936, and index arrays) are kept; beyond that
+        bytes (the head's rows and index arrays) are kept; beyond that
         the least recently replayed one is dropped and its key starts counting sightings again
         (the reference records batch sizes 1 to 32 once, /root/reference/src/utils/graph.rs:415-420)."""
         if not torch.cuda.is_available():
@@ -407,9 +407,16 @@ class ModelRunner:
         self.graph_replays += 1
         if not reserved:
             self.cache.commit_many(rid_arr, np.ones(B, np.int32))
+        return self._logits(g, rows)
+
+    def _logits(self, g: _DecodeGraph, rows: np.ndarray) -> torch.Tensor:
+        """The head behind a replay, into a tensor of the caller's own: recorded with the rest, its logits would be the next replay's too and have to be
+        copied (256 rows of 151,936: 53 us of a step's 3,509)."""
+        logits = self.model.head.forward(g.hidden)
+        B = logits.shape[0]
         if rows.size == B and np.array_equal(rows, np.arange(B)):
-            return g.logits.clone()
-        return g.logits.index_select(0, g.want[:rows.size])
+            return logits
+        return logits.index_select(0, g.want[:rows.size])
 
     # ---- index arrays on the device -------------------------------------------------
     def _context(self, a: BatchArrays, ids32: np.ndarray, rows32: np.ndarray, dst32=None, dst64=None,
@@ -469,8 +476,8 @@ class ModelRunner:
             self.graphs_dropped += 1
 
     def _replay_decode(self, a: BatchArrays, ids32: np.ndarray, rows32: np.ndarray) -> torch.Tensor:
-        """A step of single tokens.  The graph of (batch size, context bucket) computes the
-        logits of every row; the wanted rows are gathered afterwards.  Kernels whose grid
+        """A step of single tokens.  The graph of (batch size, context bucket) computes what the
+        head wants of every row; the wanted rows' logits are gathered afterwards.  Kernels whose grid
         depends on the longest context are recorded for the bucket's upper bound (work
         beyond a request's own length ends at once)."""
         B = a.num_seqs
@@ -501,7 +508,7 @@ class ModelRunner:
                 self._graph_pool = torch.cuda.graph_pool_handle()
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph, pool=self._graph_pool):
-                recorded = self.model.forward(ids, ctx, self.layer_caches, every_row)
+                recorded = self.model.hidden(ids, ctx, self.layer_caches, every_row)
             g = _DecodeGraph(graph, d32, d64, recorded, want, keep=(every_row, ctx, ids))
             self._graphs[key] = g
             self._drop_least_used(keep=key)
@@ -517,6 +524,4 @@ class ModelRunner:
             self._put_device_tokens(g.dev32[:B])
         g.graph.replay()
         self.graph_replays += 1
-        if rows32.size == B and np.array_equal(rows32, np.arange(B)):
-            return g.logits.clone()
-        return g.logits.index_select(0, g.want[:rows32.size])
+        return self._logits(g, rows32)
