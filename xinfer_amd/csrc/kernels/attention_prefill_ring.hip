@@ -18,6 +18,11 @@
 // attention_prefill.hip the keys of a 32-key step are permuted over the rows:
 // key k sits at row 16*((k>>2)&1) + 4*(k>>3) + (k&3).
 //
+// Bound by the issue of vector instructions beside the matrix ones, then by LDS reads.  A step's operands asked for together and the tiles'
+// addresses kept in scalar registers, without | with, us on MI355X, heads of 128 on 8 kv heads: 32 heads, 1,024 tokens 27.1 | 25.5, 2,048 55 | 51,
+// 4,096 147 | 135; 64 heads, 2,048 tokens 83 | 77, the last 2,048 of 8,192 448 | 409 (1.18 PFLOP/s); 32 heads of 256, 2,048 tokens 105 | 96, of 64
+// 39.0 | 34.4.  A higher priority for the matrix instructions, a barrier for two tiles, V^T asked for before the scores: level to 5% slower.
+//
 // Head sizes 32, 64, 128 and 256 (whole 32-wide steps of the matrix product and a power of two
 // of chunks a row); other sizes stay with attention_prefill.hip.
 //
@@ -94,7 +99,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
   int* bt_s = reinterpret_cast<int*>(smem + (size_t)S * STAGE);      // [max_pages]
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave_abs = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave_abs = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave = wave_abs % WPG, grp = wave_abs / WPG;     // the wave within its group, and the group
   const int r = lane & 15, j = lane >> 4;
   const int page = 1 << page_shift;
@@ -196,22 +201,20 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
   // from the last one's place (they are masked); tiles past the workgroup's last are asked for
   // all the same, so that the number of loads in flight does not depend on where the walk is.
   const int last_tile = k_last & ~(kKeys - 1);
+  int pid_next = 0;                   // BIGPAGE: the page of the tile that is asked for next (an LDS read away otherwise)
   auto fetch = [&](int kb, int st) {
     const unsigned base = lds0 + (unsigned)st * STAGE;
     if (BIGPAGE) {
       kb = kb > last_tile ? last_tile : kb;        // a tile past the end: the last one again (nobody reads it)
-      const int pid = __builtin_amdgcn_readfirstlane(bt_s[kb >> page_shift]);
+      const int pid = __builtin_amdgcn_readfirstlane(pid_next);
+      pid_next = bt_s[min(kb + kKeys, last_tile) >> page_shift];
       const size_t blk = ((size_t)pid * nkv + kvh) * kv_head_stride;
       const bf16* kbase = k_cache + blk + (size_t)(kb & (page - 1)) * D;
       const bf16* vbase = vt_cache + blk + (size_t)((kb & (page - 1)) >> 3) * D * 8;
 #pragma unroll
       for (int t = 0; t < LPW; ++t) {
         const int ii = wave_abs + NWV * t;
-        // (which of the two a wave's t-th load takes is the same in all its lanes: made a scalar by hand)
-        const unsigned long long a = (unsigned long long)(uintptr_t)(ii < KI ? kbase : vbase);
-        const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
-        load_lds16(reinterpret_cast<const void*>((uintptr_t)(((unsigned long long)hi << 32) | lo)), ld_lane[t],
-                   __builtin_amdgcn_readfirstlane(base + ld_dst[t]));
+        load_lds16(ii < KI ? kbase : vbase, ld_lane[t], base + ld_dst[t]);
       }
       return;
     }
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
         const int vp = bt_s[key0 >> page_shift];
         src = vt_cache + ((size_t)vp * nkv + kvh) * kv_head_stride + ((size_t)((key0 & (page - 1)) >> 3) * D + ld_off[t]) * 8;
       }
-      load_lds16(src, __builtin_amdgcn_readfirstlane(base + ld_dst[t]));
+      load_lds16(src, base + ld_dst[t]);
     }
   };
 
@@ -238,6 +241,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
   // the queries have landed before the first tile is asked for: from here on the tiles' loads are
   // the only ones in flight, and the counts they are waited for with mean what they say
   wait_loads<0>();
+  if (BIGPAGE) pid_next = bt_s[min(k_begin, last_tile) >> page_shift];
 #pragma unroll
   for (int p = 0; p < S - 1; ++p) fetch(k_begin + kKeys * p, p);
   int st = 0;
@@ -253,12 +257,15 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
     if ((KS == 1 || sub == grp) && active && kb >= wave_k_begin && kb <= last_pos) {
       // a step needs the mask unless every key is at or before every query and inside every window
       const bool masked = (kb + 31 > first_pos) || (kb < lo_last);
+      // All of a step's K is asked for before its first product, and its V^T ahead of the softmax: left to itself the compiler takes both
+      // through a few registers at a time, and a wave waits for LDS eight times a step.
       bf16x8 ka[2][KC];
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         ka[0][c] = ld8(reinterpret_cast<const bf16*>(Kt + k_rd[c] + 2 * D * (32 * sub)));
         ka[1][c] = ld8(reinterpret_cast<const bf16*>(Kt + k_rd[c] + 2 * D * (32 * sub + 16)));
       }
+      __builtin_amdgcn_sched_barrier(0);
       // ---- all scores of the step first
       f32x4 s0[NQT], s1[NQT];
 #pragma unroll
@@ -273,6 +280,11 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
           s0[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[0][c], qb[ct][c], s0[ct], 0, 0, 0);
           s1[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[1][c], qb[ct][c], s1[ct], 0, 0, 0);
         }
+      bf16x8 va[DT];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) va[dt] = ld8(reinterpret_cast<const bf16*>(Vt + v_rd[sub] + 2 * kKeys * (16 * dt)));
+      __builtin_amdgcn_sched_barrier(0);
       if (masked) {
         const int key0 = kb + 8 * j;
 #pragma unroll
@@ -328,13 +340,12 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_ring_kernel(
         }
         l_run[ct] += psum;
       }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const bf16x8 va = ld8(reinterpret_cast<const bf16*>(Vt + v_rd[sub] + 2 * kKeys * (16 * dt)));
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int ct = 0; ct < NQT; ++ct)
-          acc[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb_[ct], acc[dt][ct], 0, 0, 0);
-      }
+          acc[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb_[ct], acc[dt][ct], 0, 0, 0);
     }
     }
     st = st + 1 == S ? 0 : st + 1;
