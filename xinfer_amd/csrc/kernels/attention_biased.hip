@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_biased_lds_kernel(
   bf16* lds = reinterpret_cast<bf16*>(smem);
   int* bt_s = reinterpret_cast<int*>(smem + 2 * (size_t)stage * sizeof(bf16));  // [max_pages]
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, j = lane >> 4;
   const int g = nq / nkv, groups = g / GH;
   const int kvh = blockIdx.x / groups;
@@ -243,13 +243,18 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_biased_lds_kernel(
       const bf16* Vs = lds + buf * stage + kKeysB * krow + 32 * sub;
       // a step needs the mask unless every key is at or before every query and inside every window
       const bool masked = (kb + 31 > first_pos) || (kb < lo_last);
-      bf16x8 ka[2][KC];
+      // Four waves: all of a step's K is asked for before its first product, and its V^T ahead of the scores' options and the softmax; left to itself
+      // the compiler takes both through a few registers at a time (32 heads of 128, 2,048 tokens 81.2 us, 79.1 so, with a soft cap 92.3 | 90.0; with
+      // eight waves, where another wave of the SIMD fills the waits, 6,000 tokens 330 | 335).
+      constexpr bool kEarly = NWV == 4 && FULLD && DT <= 8;
+      bf16x8 ka[2][KC], va[kEarly ? DT : 1];
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         const int off = 32 * c + 8 * j;
         ka[0][c] = ld8(Ks + r * krow + off);
         ka[1][c] = ld8(Ks + (16 + r) * krow + off);
       }
+      if constexpr (kEarly) __builtin_amdgcn_sched_barrier(0);
       // ---- all scores of the step first: 2 * KC * NQT matrix instructions with nothing
       // between them that waits for their results
       f32x4 s0[NQT], s1[NQT];
@@ -265,6 +270,12 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_biased_lds_kernel(
           s0[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[0][c], qb[ct][c], s0[ct], 0, 0, 0);
           s1[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[1][c], qb[ct][c], s1[ct], 0, 0, 0);
         }
+      if constexpr (kEarly) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) va[dt] = ld8(Vs + (16 * dt + r) * vrow + 8 * j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // ---- the score itself, in the exponent's unit: scale, soft cap, distance bias; then the mask
       {
         const int key0 = kb + 8 * j;
@@ -345,10 +356,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_biased_lds_kernel(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         if (FULLD || 16 * dt < dv) {
-          const bf16x8 va = ld8(Vs + (16 * dt + r) * vrow + 8 * j);
+          if constexpr (!kEarly) va[0] = ld8(Vs + (16 * dt + r) * vrow + 8 * j);
 #pragma unroll
           for (int ct = 0; ct < NQT; ++ct)
-            acc[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb_[ct], acc[dt][ct], 0, 0, 0);
+            acc[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[kEarly ? dt : 0], pb_[ct], acc[dt][ct], 0, 0, 0);
         }
       }
     }
