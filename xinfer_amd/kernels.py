@@ -1309,7 +1309,7 @@ def prefill_tiles(q_lens, ctx_lens, d: int, nq: int, nkv: int, small=None, first
     with so few blocks that even those leave compute units with one workgroup (a prompt of 2,048
     tokens on 8 kv heads) 2, where the head size allows: eight waves in two groups that split a
     tile's keys, so that the longest block, which ends up alone on its unit, walks its keys with
-    twice the waves (2,048 tokens, 32 query heads: 60 -> 56 us; 1,024: 31 -> 28).  Shape 0 has one
+    twice the waves (2,048 tokens, 32 query heads: 54.7 -> 53.5 us; 1,024: 28.8 -> 26.4).  Shape 0 has one
     workgroup per unit at a time: longest first."""
     g = nq // nkv
     heads = nkv * (g // (4 if g % 4 == 0 else 2 if g % 2 == 0 else 1))     # workgroups per query block
