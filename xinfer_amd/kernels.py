@@ -1818,7 +1818,7 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
       129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
       otherwise: the library, where the time is below what that takes at its better sizes (5.6 us under 32 rows and up to 2,048 features, 8 us; from 65
       rows on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
-    if not 17 <= M <= SMALL_TILE_ROWS or N % 4 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)):
+    if not 17 <= M <= SMALL_TILE_ROWS or N < 4 or N % 4 or K < 64 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)):
         return None
     k_tiles, best = K // 64, None
     for shape, rows, features, start, alone, more, out, full in SMALL_TILES:
@@ -2210,7 +2210,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     if out_dtype == torch.float32 and MID_WIDE_FROM <= x.shape[0] <= MID_GATED_ROWS \
             and linear_mid_slices(w.shape[0], w.shape[1]) == 1:
         return linear_mid(x, w)[0]           # a wide output in float32 (the head): one slice is the result
-    if out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15:
+    if out_dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15:
         M, K = x.shape
         N = w.shape[0]
         small = small_tile_plan(M, N, K, allow_split)
