@@ -55,3 +55,12 @@ def test_operands_that_are_no_product_of_the_tiles(launches, M, x_shape, w_shape
     else:
         assert torch.equal(kernels.linear_bf16(x, w), want)
     assert not launches
+
+
+@pytest.mark.parametrize("M,asked,kernel", [(17, 64, "xi_linear_skinny"), (64, 64, "xi_linear_skinny"), (48, 48, "xi_linear_skinny"), (32, 17, "xi_linear_tile"),
+                                            (32, None, "xi_linear_tile"), (65, 100, "xi_linear_tile")])
+def test_rows_for_the_streaming_kernel(launches, M, asked, kernel):
+    """`skinny_rows` is a caller's choice, up to the 64 rows that the streaming kernel takes: what is whole goes there up to that many."""
+    x, w = _rows(M, 1024), _rows(4096, 1024)
+    kernels.linear_bf16(x, w, **({} if asked is None else {"skinny_rows": asked}))
+    assert [name for name, _ in launches] == [kernel]

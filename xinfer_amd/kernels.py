@@ -2213,7 +2213,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     if out_dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15:
         M, K = x.shape
         N = w.shape[0]
-        small = small_tile_plan(M, N, K, allow_split)
+        small = small_tile_plan(M, N, K, allow_split) if allow_split or M > min(skinny_rows, SKINNY_MAX_ROWS) else None
         if small is not None:
             shape, slices = small
             y = torch.empty((slices, M, N), dtype=torch.float32, device=x.device) if slices > 1 else torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
