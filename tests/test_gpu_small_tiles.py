@@ -66,3 +66,27 @@ def test_low_tiles_are_one_round(split):
     assert plan(256, 4096, 1024, True) == (7, 1) and plan(256, 1024, 2048, True) == (7, 4) and plan(61, 1024, 4096, True) == (7, 11) and plan(40, 4096, 2048, True) is None and plan(61, 4096, 4096, True) is None
     assert plan(256, 10240, 5120, True) is None and plan(256, 5120, 25600, True) is None and plan(2048, 4096, 4096, True) is None
     assert plan(512, 2048, 6144, True) == (9, 4) and plan(768, 2048, 8192, True) is None and plan(512, 4096, 8192, True) is None and plan(256, 1024, 3072, False) is None
+
+
+SPLIT_SIZES = [(N, K) for N in (1024, 1500, 1536, 2048, 3072, 4096, 6144, 8192, 16768, 32768) for K in (64, 192, 512, 1024, 1536, 2048, 3072, 4096, 5632, 8128)]
+
+
+def test_sums_of_decode_rows_do_not_follow_the_batch():
+    """17 to 128 rows with partial sums: whether a product goes to the low tiles, and in how many slices of K, follows from (N, K) alone."""
+    taken = 0
+    for N, K in SPLIT_SIZES:
+        plans = [kernels.small_tile_plan(M, N, K, True) for M in range(17, 129)]
+        assert len({None if p is None else p[1] for p in plans}) == 1, (N, K)
+        taken += plans[0] is not None
+    assert taken > 20
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(1024, 3072), (4096, 1024), (1536, 3584), (1536, 4096), (1028, 1024), (640, 2560)])
+def test_a_row_beside_others(N, K):
+    """... and so a row's partial sums are the same bits beside 16 others and beside 127."""
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn(128, K, generator=g).to(torch.bfloat16).to(DEV), torch.randn(N, K, generator=g).to(torch.bfloat16).to(DEV)
+    y = kernels.linear_bf16(x, w, allow_split=True)
+    for M in (17, 32, 37, 64, 65, 66, 100, 127):
+        assert torch.equal(kernels.linear_bf16(x[:M].contiguous(), w, allow_split=True), y[:, :M])

@@ -1795,35 +1795,20 @@ def tile_split_plan(M: int, N: int, K: int):
 
 SMALL_TILE_ROWS = 2048        # rows up to which the low tiles were measured
 SMALL_TILE_SLICES = 12
+SMALL_TILE_SUMS = 32          # the rows whose slices 17 to 128 rows with partial sums have
+SMALL_TILE_SPLIT = 6 << 20    # elements of a weight from which on linear_mid stays there
 SMALL_TILES = (               # shape of `linear_tile`, rows, features; us: a kernel's start, a tile of 64 k alone and what the others of a round add to
     (7, 64, 64, 2.72, 0.239, 0.073, 0.270, 0.0),           # it, a MB of results, a round of workgroups
     (8, 64, 128, 2.64, 0.376, 0.086, 0.130, 1.08),
     (9, 128, 128, 3.31, 0.448, 0.164, 0.254, 0.0))
 
 
-@functools.lru_cache(maxsize=4096)
-def small_tile_plan(M: int, N: int, K: int, split: bool):
-    """(shape of `linear_tile`, slices of K) of x [M, K] @ w [N, K]^T in one round of low tiles, None: not there.  `split`: the caller takes float32
-    partial sums.
-
-    The least of `SMALL_TILES`' times and the reader's of the partial sums (6 TB/s), by a fit to 4,100 measured times on MI355X with weights from memory
-    (1% of them more than 20 to 35% off).  What it stands against, with 38 weights of 256 to 10,240 features by 512 to 25,600 and 17 to 2,048 rows:
-      up to 128 rows, split, weights under 16 MB: `linear_mid`.  17 to 64 rows 12% ahead in the median, 2% behind at most, 65 to 128 35%, never
-      behind; a step of 20, 61 and 128 requests at Qwen3-0.6B sizes 1,333, 1,635 and 2,483 us with linear_mid, 1,303, 1,569 and 2,232 so.  (Larger
-      weights are 0 to 15% ahead alone and level to 3% behind in a step: 20 requests of 8 layers at 8B sizes 1,083 for 1,117.  Under 1,024 features
-      linear_mid stays: tests pin its bits there.)
-      where `tile_split_plan` cuts K, narrow ones: N up to 1,024, and up to 2,048 to 512 rows (256 rows, K=6144 15.1 for 18.5, 512 rows 21.5 for
-      24.1, with half the partial sums and less; 768 rows, K=8192 40.2 for 32.4).  (Wider ones are 5 to 20% ahead alone up to 256 rows, 2% of a step
-      at 8B sizes; tests pin the slices there.)
-      129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
-      otherwise: the library, where the time is below what that takes at its better sizes (5.6 us under 32 rows and up to 2,048 features, 8 us; from 65
-      rows on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
-    if not 17 <= M <= SMALL_TILE_ROWS or N < 4 or N % 4 or K < 64 or K % 64 or (M <= 128 and split and (N < 1024 or N * K >= 1 << 23)):
-        return None
+def _least_small_tiles(M: int, N: int, K: int, cuts):
+    """(us, shape of `linear_tile`, slices) of the low tiles that take least, of those in one round, `cuts`: the slices to look at in rising order."""
     k_tiles, best = K // 64, None
     for shape, rows, features, start, alone, more, out, full in SMALL_TILES:
         tiles = -(-M // rows) * -(-N // features)
-        for slices in range(1, SMALL_TILE_SLICES + 1 if split else 2):
+        for slices in cuts:
             share = tiles * slices / COMPUTE_UNITS
             if share > 1 or (slices > 1 and k_tiles // slices < 4):
                 break
@@ -1833,6 +1818,39 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
                 cost += M * N * (4 * slices - 2) / 6e6
             if best is None or cost < best[0]:
                 best = (cost, shape, slices)
+    return best
+
+
+@functools.lru_cache(maxsize=4096)
+def small_tile_plan(M: int, N: int, K: int, split: bool):
+    """(shape of `linear_tile`, slices of K) of x [M, K] @ w [N, K]^T in one round of low tiles, None: not there.  `split`: the caller takes float32
+    partial sums.
+
+    The least of `SMALL_TILES`' times and the reader's of the partial sums (6 TB/s), by a fit to 4,100 measured times on MI355X with weights from memory
+    (1% of them more than 20 to 35% off).  What it stands against, with 38 weights of 256 to 10,240 features by 512 to 25,600 and 17 to 2,048 rows:
+      up to 128 rows, split, 1,024 features and more, weights under 12 MB: `linear_mid`.  As there, a row's sums must not follow the rows beside it, so the
+      slices are those of 32 rows at any number of them, and the tile's shape, on which no sum depends, is what follows from it.  Of 19 weights, us,
+      linear_mid / so: N=1024 K=2048, 17 rows 4.5 / 4.0, 64 5.5 / 4.7, 128 8.2 / 5.4; N=1024 K=3072 4.8 / 4.4, 6.0 / 5.5, 9.1 / 7.3 (6.3 in the 8 slices that
+      128 rows alone would choose); N=4096 K=1024 5.1 / 4.8, 6.5 / 6.3, 9.8 / 8.9 (7.4 in 2); N=1024 K=4096 5.1 / 5.2, 6.6 / 6.3, 10.0 / 8.2; 17 to 64 rows
+      2% behind at most, 65 to 128 8% ahead at least; a step of 20, 61, 100 and 128 requests at Qwen3-0.6B sizes 1,319, 1,650, 2,101 and 2,428 us with
+      linear_mid, 1,291, 1,598, 1,957 and 2,270 so (1,293, 1,588, 1,913 and 2,209 if every number of rows chose its own slices).  Not from 12 MB on: N=6144 K=1024 5.5 / 5.9, 7.5 / 7.2, 11.5 / 9.2, N=1536 K=4096 5.6 / 6.0, 7.5 / 7.3,
+      11.7 / 9.7 (larger ones are level to 3% behind in a step: 20 requests of 8 layers at 8B sizes 1,083 for 1,117).  Nor under 1,024 features, where
+      linear_mid stays although it takes longer (N=640 K=2560 4.5 / 4.0, 5.5 / 4.9, 8.1 / 5.4): its sums there are what they have been.
+      where `tile_split_plan` cuts K, narrow ones: N up to 1,024, and up to 2,048 to 512 rows (256 rows, K=6144 15.1 for 18.5, 512 rows 21.5 for
+      24.1, with half the partial sums and less; 768 rows, K=8192 40.2 for 32.4).  (Wider ones are 5 to 20% ahead alone up to 256 rows, 2% of a step
+      at 8B sizes; they keep that plan's slices, and their sums with them.)
+      129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
+      otherwise: the library, where the time is below what that takes at its better sizes (5.6 us under 32 rows and up to 2,048 features, 8 us; from 65
+      rows on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
+    if not 17 <= M <= SMALL_TILE_ROWS or N < 4 or N % 4 or K < 64 or K % 64:
+        return None
+    cuts = range(1, SMALL_TILE_SLICES + 1 if split else 2)
+    if split and M <= MID_BLOCK:
+        if N < 1024 or N * K >= SMALL_TILE_SPLIT:
+            return None
+        sums = _least_small_tiles(SMALL_TILE_SUMS, N, K, cuts)
+        return _least_small_tiles(M, N, K, (sums[2],))[1:] if sums is not None else None
+    best = _least_small_tiles(M, N, K, cuts)
     if best is None:
         return None
     if split and tile_split_plan(M, N, K)[0] > 1:
