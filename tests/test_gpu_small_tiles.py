@@ -90,3 +90,15 @@ def test_a_row_beside_others(N, K):
     y = kernels.linear_bf16(x, w, allow_split=True)
     for M in (17, 32, 37, 64, 65, 66, 100, 127):
         assert torch.equal(kernels.linear_bf16(x[:M].contiguous(), w, allow_split=True), y[:, :M])
+
+
+def test_whole_products_where_they_are_ahead():
+    """No gaps between rows at which nothing was measured behind, and nothing where it was."""
+    plan = kernels.small_tile_plan
+    for N, M in ((1024, 1024), (2048, 1024), (4096, 512)):
+        assert all(plan(m, N, 1024, False) is not None for m in range(32, M + 1))
+    for M, N, K in ((493, 6144, 4096), (512, 6144, 4096), (512, 6144, 2560), (512, 7168, 5120), (384, 8192, 1280), (400, 8192, 1024)):
+        assert plan(M, N, K, False) is None and plan(M, N, K, M > 256) is None
+    for N in (512, 1024):
+        assert all(plan(m, N, K, False) is None for m in (32, 64, 128, 256) for K in (1152, 1280))
+    assert plan(960, 4096, 2048, False) == (9, 1) and plan(96, 3072, 1152, False) is not None and plan(300, 10240, 1024, False) == (9, 1)

@@ -1840,8 +1840,19 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
       24.1, with half the partial sums and less; 768 rows, K=8192 40.2 for 32.4).  (Wider ones are 5 to 20% ahead alone up to 256 rows, 2% of a step
       at 8B sizes; they keep that plan's slices, and their sums with them.)
       129 to 256 rows, split, what that leaves to the library: 27% ahead in the median, never behind.
-      otherwise: the library, where the time is below what that takes at its better sizes (5.6 us under 32 rows and up to 2,048 features, 8 us; from 65
-      rows on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above): 21% ahead in the median of 80 sizes, one more than 1% behind (512 rows of N=6144 K=4096 39.7 for 36.6)."""
+      otherwise: the library (3,300 pairs of times at 55 weights, from memory but for the smallest; us, the library / low tiles).
+        Where the low tiles' time is below what the library takes at its better sizes: 8 us (5.6 under 32 rows and up to 2,048 features), from 65 rows
+        on 6 us and 0.7, 0.85 or 1.25 PFLOP/s up to 512, up to 1,024 and above.  N=1024 K=1024: 32 rows 8.1 / 6.3, 128 8.1 / 6.6, 512 8.4 / 6.7, 1024 8.8 /
+        7.0; N=4096 K=1024: 17 11.2 / 6.8, 64 11.6 / 8.0, 256 11.9 / 8.2.
+        K up to 1,088 besides: up to 12 us and 1,024 rows; the library's times go up and down with the rows there and hardly below that.  N=4096 K=1024: 257 rows
+        12.6 / 9.2, 460 13.3 / 9.9, 512 13.2 / 10.7 (640 13.8 / 13.3, 768 level); N=2048: 700 9.5 / 8.3; N=3072: 400 11.3 / 9.1; N=6144: 129 12.6 / 9.6, 257 13.2
+        / 9.9.  30% ahead in the median with weights from memory, 15 to 20% with weights in a cache.
+        Larger K only from 3,072 features or 2^19 results on, not for 49 to 64 rows, and above 2,048 only from 513 rows on.  Left out so: N=512 K=1280: 64 rows
+        6.7 / 7.9, N=1024 K=1280: 48 7.2 / 7.8, 128 7.0 / 7.9, 192 7.2 / 7.9; N=3072 K=1280: 64 9.1 / 9.9; K=2560 N=6144: 512 27.0 / 30.4, K=4096 37.6 / 39.9.
+        Nor K above 512 with 6,145 to 8,192 features at 257 to 400 rows (N=8192 K=1024: 384 14.3 / 14.2, 400 15.4 / 16.5, K=1280: 384 17.0 / 18.3;
+        N=10240 K=1024: 300 15.7 / 13.8).
+        What is taken is 29% ahead in the median with weights from memory, 3 of 1,100 sizes more than 3% behind (N=8192 K=1024: 448 rows 15.2 / 15.9); with
+        all weights in a cache N=256 to 512 K=1024 at 65 to 192 rows are up to 1.4 us behind (5.2 / 6.6; from memory 9.5 / 7.0)."""
     if not 17 <= M <= SMALL_TILE_ROWS or N < 4 or N % 4 or K < 64 or K % 64:
         return None
     cuts = range(1, SMALL_TILE_SLICES + 1 if split else 2)
@@ -1861,6 +1872,12 @@ def small_tile_plan(M: int, N: int, K: int, split: bool):
         library = 8.0 if M >= 32 or N > 2048 else 5.6
     else:
         library = max(8.0, 6 + 2e-9 * M * N * K / (0.7 if M <= 512 else 0.85 if M <= 1024 else 1.25))
+    if K <= 1088 and M <= 1024 and (M >= 32 or N > 2048):
+        library = max(library, 12.0)
+    elif K > 1088 and ((N < 3072 and M * N < 1 << 19) or 48 < M < 65 or (K > 2048 and M <= 512)):
+        return None
+    if K > 512 and 6144 < N <= 8192 and 256 < M <= 400:
+        return None
     return best[1:] if best[0] < library else None
 
 
