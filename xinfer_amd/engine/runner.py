@@ -415,7 +415,7 @@ class ModelRunner:
         logits = self.model.head.forward(g.hidden)
         B = logits.shape[0]
         if rows.size == B and np.array_equal(rows, np.arange(B)):
-            return logits
+            return logits if self.model.head.fresh else logits.clone()
         return logits.index_select(0, g.want[:rows.size])
 
     # ---- index arrays on the device -------------------------------------------------

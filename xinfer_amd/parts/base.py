@@ -317,6 +317,9 @@ class StreamOp(Part):
 
 class Head(Part):
     tied = False
+    # `forward`'s result is a tensor of the caller's own: not its input or a view of it, and nothing that a later call writes.  Behind a recorded
+    # step the input is the recording's and is written again by the next one; what a head returns that does not say so is copied there.
+    fresh = False
 
     def load(self, store: WeightStore, prefix: str, device, shared: Optional[torch.Tensor] = None) -> None:
         raise NotImplementedError

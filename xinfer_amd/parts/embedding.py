@@ -102,6 +102,7 @@ class Embedding(TokenEmbedding):
 @register_head("lm_head")
 class LMHead(Head):
     graph_safe = True
+    fresh = True
 
     def __init__(self, spec: PartSpec, dtype: torch.dtype):
         super().__init__(spec, dtype)
