@@ -114,7 +114,8 @@ def test_tall_tile_rule(M, N, K, rows):
 @pytest.mark.gpu
 @pytest.mark.parametrize("k_tiles", [1, 2, 3, 4, 5, 6, 7])
 def test_rings_of_unequal_depth(k_tiles):
-    """Every walk at fewer tiles of k than its rings have stages, and at their first turns: whole numbers of which every partial sum is exact in float32."""
+    """Every walk but those of cut last tiles (below) at fewer tiles of k than its rings have stages, and at their first turns: whole numbers of which
+    every partial sum is exact in float32."""
     M, N, K = 260, 520, 64 * k_tiles
     g = torch.Generator().manual_seed(k_tiles)
     x, w = (torch.randint(-4, 5, (n, K), generator=g).to(torch.bfloat16).to(DEV) for n in (M, N))
@@ -129,6 +130,24 @@ def test_rings_of_unequal_depth(k_tiles):
     want = torch.nn.functional.silu(a) * b
     assert bool(((got[0].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * (1 + (a * b).abs())).all())
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k_tiles", [1, 3, 5, 7, 11])
+@pytest.mark.parametrize("M,N", [(2049, 3716), (2300, 3840), (2290, 5100), (1793, 5888)])
+def test_walks_of_cut_last_tiles(M, N, k_tiles):
+    """A whole round of tiles of 256 by 128 and up to 64 (in quarters) or 128 more (in halves), past fewer and more tiles of k than the rings of their three walks
+    have stages, rows and features past the last tile: bit for bit the sums of the other shapes, whole numbers that are exact."""
+    K = 64 * k_tiles
+    rest = -(-M // 256) * -(-N // 128) - 256
+    assert (0 < rest <= 64) == (N < 4000) and 0 < rest <= 128
+    g = torch.Generator().manual_seed(M + k_tiles)
+    x, w = (torch.randint(-4, 5, (n, K), generator=g).to(torch.bfloat16).to(DEV) for n in (M, 2 * N))
+    cut, low, one = (kernels.linear_gated_tile(x, w, "silu", shape) for shape in (2, 0, 1))
+    assert torch.equal(cut, low) and torch.equal(cut, one)
+    a, b = (x.double() @ w.double().t()).split(N, 1)
+    want = torch.nn.functional.silu(a) * b
+    assert bool(((cut.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * (1 + (a * b).abs())).all())
 
 
 @pytest.mark.parametrize("M,F,K,shape", [
