@@ -32,8 +32,8 @@ HIP_FLAGS = [
     # no packed-FP32 instructions in the generated code: some of their forms have given wrong results on gfx950
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # A kernel's arguments are in scalar registers when it starts, as many as fit, instead of behind a first trip to memory: a chain of short
-    # kernels waits for that once a kernel.  0.18 us each of the 175 of a step of one request at Qwen3-0.6B sizes (977 -> 946 us); 8B sizes, 8
-    # requests 4,323 -> 4,246.
+    # kernels waits for that once a kernel.  0.18 us each of the 175 of a step of one request at Qwen3-0.6B sizes (977 -> 946 us); at
+    # 8B sizes, 8 requests, about 1%, as much as its runs differ.
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument",
 ]

@@ -244,7 +244,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_biased_lds_kernel(
       // a step needs the mask unless every key is at or before every query and inside every window
       const bool masked = (kb + 31 > first_pos) || (kb < lo_last);
       // Four waves: all of a step's K is asked for before its first product, and its V^T ahead of the scores' options and the softmax; left to itself
-      // the compiler takes both through a few registers at a time (32 heads of 128, 2,048 tokens 81.2 us, 79.1 so, with a soft cap 92.3 | 90.0; with
+      // the compiler takes both through a few registers at a time (32 heads of 128, 2,048 tokens 86.2 us, 82.1 so, with a soft cap 97.2 | 92.8; with
       // eight waves, where another wave of the SIMD fills the waits, 6,000 tokens 330 | 335).
       constexpr bool kEarly = NWV == 4 && FULLD && DT <= 8;
       bf16x8 ka[2][KC], va[kEarly ? DT : 1];

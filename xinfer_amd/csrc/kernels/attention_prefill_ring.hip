@@ -21,7 +21,8 @@
 // Bound by the issue of vector instructions beside the matrix ones, then by LDS reads.  A step's operands asked for together and the tiles'
 // addresses kept in scalar registers, without | with, us on MI355X, heads of 128 on 8 kv heads: 32 heads, 1,024 tokens 27.1 | 25.5, 2,048 55 | 51,
 // 4,096 147 | 135; 64 heads, 2,048 tokens 83 | 77, the last 2,048 of 8,192 448 | 409 (1.18 PFLOP/s); 32 heads of 256, 2,048 tokens 105 | 96, of 64
-// 39.0 | 34.4.  A higher priority for the matrix instructions, a barrier for two tiles, V^T asked for before the scores: level to 5% slower.
+// 39.0 | 34.4.  (Another card gave 59.5 | 55.9 for 2,048 tokens of 32 heads, 159 | 143 for 4,096 and 453 | 422 for the last of 64 heads'; in a step the
+// launch takes 55 to 56.)  A higher priority for the matrix instructions, a barrier for two tiles, V^T asked for before the scores: level to 5% slower.
 //
 // Head sizes 32, 64, 128 and 256 (whole 32-wide steps of the matrix product and a power of two
 // of chunks a row); other sizes stay with attention_prefill.hip.

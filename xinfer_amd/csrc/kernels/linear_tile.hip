@@ -44,7 +44,7 @@
 // (0.80, and 7% behind with the reads between the products); the operands of one step only in registers (the second step's reads then wait: -8%).
 //
 // Products of a few MB at up to 1,024 rows (and any of one round of them: `kernels.small_tile_plan`) go in tiles of 64 x 64, 64 x 128 or 128 x 128 with
-// rings of four to eight stages: a workgroup has 96 to 128 KB on their way from its first clocks on, which for 512 k of 64 x 64 is all it
+// rings of four to eight stages: a workgroup has 128 to 144 KB on their way from its first clocks on, which for 512 k of 64 x 64 is all it
 // will need, and the time is a kernel's start, one way to memory and the results' way out.  With slices of K the reader adds partial sums.
 // Rows, N, K, us, weights from memory, the library | the tiles for 128 rows a block (linear_mid) | this: 256, 1024, 2048 8.4 | 15.6 | 5.8 (four
 // slices of 64 x 64), 256, 1024, 3072 9.7 | 16.6 | 7.3, 256, 4096, 1024 12.0 | 17.1 | 8.1 (whole), 512, 2048, 4096 21.7 | - | 15.8 (20.1 in six slices of

@@ -36,7 +36,8 @@ constexpr int kHeights = 5;
 // heights that an expert's rows may be cut into, highest first, and the height of the walk that a tile of `rows` takes
 __host__ __device__ constexpr int height(int i) { return i == 0 ? 256 : i == 1 ? 224 : i == 2 ? 192 : i == 3 ? 160 : 128; }
 __device__ __forceinline__ int lowest(int rows) { return rows <= 64 ? 64 : rows <= 128 ? 128 : (rows + 31) & ~31; }
-// a round's time, in rows: 1.95 us for 64 k of 256 rows, and what a tile costs beyond its products
+// a round's time, in rows: 1.95 us for 64 k of 256 rows, and what a tile costs beyond its products.  Measured with two stages of w in flight: since there are
+// three, tiles of 192 rows and more take up to a tenth less and lower ones do not, which these prices do not know.
 __device__ __forceinline__ int tile_time(int high) { return high + 16; }
 
 // ceil(n / d), n and d > 0, of up to 2^22: the float quotient is one off at most (the compiler's division is three times as many instructions).

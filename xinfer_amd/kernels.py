@@ -1763,8 +1763,10 @@ def tile_split_plan(M: int, N: int, K: int):
     tiles for the chip's 256 compute units (256 rows by 4,096 features: 32 tiles of 256 x 128), so K
     is cut into slices, each a workgroup's own, with float32 partial sums [slices, M, N] for the
     caller to add in order.  Slices (2 to 16, whole tiles of 64 k, a slice at least 512 long) and tile shape are
-    those with the least cost in a model of two terms that fits what was measured on MI355X within a
-    tenth: a workgroup brings (rows of x + rows of w of its tile) x its slice of K into LDS at 58 GB/s
+    those with the least cost in a model of two terms that orders what was measured on MI355X (with a
+    kernel's start and weights from memory products take 20 to 40% more than it says, and 60% more
+    for 192 rows of K = 4096; of 13 sizes the choice is the least of all shapes and slices, its reader
+    included, at 7 and 1 to 11% above it at the others): a workgroup brings (rows of x + rows of w of its tile) x its slice of K into LDS at 58 GB/s
     (that, not the matrix cores, bounds these shapes: x is fetched again by every workgroup, so
     tiles with as many rows of w as of x are ahead where x is a whole tile's rows), rounds of 256
     workgroups one after the other, never faster than the weight streams from memory; and the
@@ -1922,8 +1924,8 @@ def tall_tile_rows(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     """The rows of a tile in which x [M, K] @ w [N, K]^T goes to `linear_tall`, None: not there.  The lowest of `TALL_SHAPES` whose
     tiles of 256 features are one round of the compute units.  For K of 16,448 to 30,720 and 20 tiles of features (N of 4,865
     to 5,120), for which the library has kernels at half the matrix cores' rate beside its good ones.  Measured on MI355X, us,
-    library / this kernel: N=5120 K=17408, rows 1025 271/209, 1280 294/220, 1536 352/224, 1727 475/252 (160 rows a tile), 2400 544/364
-    (224), 2688 596/375; K=25600: 1025 412/311, 1536 509/332, 1727 682/395, 2400 774/575, 2688 830/594; N=4872 and 5000 within 6% of
+    library / this kernel: N=5120 K=17408, rows 1025 271/209, 1280 294/220, 1536 352/224, 1727 475/252 to 265 (160 rows a tile), 2400 544/340
+    (224), 2688 590/356; K=25600: 1025 412/311, 1536 509/332, 1727 682/390, 2400 768/501, 2688 830/594 (with two stages of w); N=4872 and 5000 within 6% of
     these, 20 K from 16,448 to 30,720 all ahead (1.04 to 1.9 times) but for up to 1,152 rows at K of 18,176 to 18,688 (1025 194/225).
     Not there: 1,761 to 2,304 rows (K=17408: 1790 251/266, 2048 276/365) and more than 2,688 (3072 359/414); K=13824 (1100 152/162,
     1600 200/210), K=16384 (1025 180/192, 1536 212/214, 1600 444/233); one tile of features less or more, where the library's good
@@ -1982,8 +1984,10 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
       M=65 12.1 / 9.1, M=1024 12.6 / 11.7, F=512 M=65 12.5 / 10.0, F=1024 M=128 13.2 / 12.5; 48: F=1536 M=65 13.2 / 13.1).
       2048 < K <= 4096: 128 rows where their workgroups are 3/4 of a round to one; otherwise 256 rows, of 257 to 3,584, where 0.74 of the rounds'
       room is rows and features (`_tile_room`).  F=12288 K=4096: M=200 62 / 68, 400 90 / 94, 700 129 / 163, 1024 175 / 180, 1400 225 / 259, 2048 296 /
-      302, 3000 436 / 597; F=6144: 400 52 / 60, 1400 127 / 153, 2048 153 / 180; K=2304 F=11008: 512 54 / 66, 1024 104 / 139; of 461 sizes, F of 1,536 to
-      14,336, 12% ahead in the median and up to 4% behind (F=14336: M=129 K=4096 66 / 63, 2049 398 / 388).  Left out: emptier rounds (F=12288 K=4096: 300 87 /
+      302, 3000 436 / 597; F=6144: 400 52 / 60, 1400 127 / 153, 2048 153 / 180; K=2304 F=11008: 512 54 / 66, 1024 104 / 139; of 2,100 sizes, F of 1,536 to
+      16,384, 12% ahead in the median, 27 more than 2% behind and 7 more than 4, next to sizes that gain more: F=12288 K=4096: 850 172 / 165, 1000 171 / 178;
+      F=16384: 384 102 / 97, 640 163 / 153, 1200 a third ahead; F=9728: 2049 287 / 273, 2048 a third ahead; level at 129 to 160 rows of F=13312 and 14336
+      (K=4096: 129 66 / 65).  Left out: emptier rounds (F=12288 K=4096: 300 87 /
       77, 800 161 / 152), and more rows, where the library has its best sizes (4096 600 / 589).
       4096 < K <= 6144, 512 rows and more, 8/9 of the rows of the tiles there: up to four rounds of 256 workgroups and a rest of up to
       64, which is cut (see the kernel) and for which the library has a whole round: K=4608 F=8192: 1230 155 / 163, F=10240: 1024 158
@@ -1996,7 +2000,8 @@ def gated_tile_shape(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
       less than these figures.)
       4096 < K <= 6144 besides: 128 rows where their workgroups are 7/8 of a round to one (F=8192 K=5120: 400 75 / 88, 512 83 / 92; K=6144 F=6144: 600
       106 / 118), and from 769 rows on also fewer rows than 8/9 of the tiles' where 0.74 of the rounds' room is filled (F=17408 K=5120: 900
-      267 / 410); 30 sizes, 13% ahead in the median, none behind.
+      267 / 410); 570 sizes of 4,608, 5,120 and 6,144 in all, 13% ahead in the median, 10 more than 2% behind, most of them 129 to 192 rows of F=14336 K=5120 (160
+      83 / 78; of F=16384 144 84 / 112).
       Left out: F=64 K=5120 M=512 87 / 17, F=1536 94 / 31, F=2048 K=7168 M=2048 162 / 107, F=12288 K=5120 M=1024 233 / 220, K=4608 M=1280 239 / 222,
       F=8192 K=8192 M=4096 855 / 731, F=17408 K=5120 M=384 182 / 173, 770 422 / 370."""
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] \
@@ -2236,7 +2241,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     """bfloat16 x @ w.T with float32 accumulation, rounded once to `out_dtype` (bfloat16 or
     float32).  Up to `skinny_rows` rows (decode): the hand-written streaming kernel, which with
     `allow_split` may answer with float32 partial sums [slices, M, N] for a narrow output.  More
-    rows: where K is long and the output narrow `linear_tall`, else the vendor library (hipBLASLt through torch), which the reference's engine also
+    rows: one round of low tiles where `small_tile_plan` says so (bfloat16 results, operands on 16 bytes), with
+    `allow_split` in slices of K; with `allow_split` the tiled kernels of `tile_split_plan` and `linear_mid`;
+    where K is long and the output narrow `linear_tall`, else the vendor library (hipBLASLt through torch), which the reference's engine also
     uses for its matrix products."""
     _dev(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
