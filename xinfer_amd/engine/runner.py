@@ -24,6 +24,7 @@ import numpy as np
 import torch
 
 from ..cache import DecodeStepError, BatchArrays, CacheGroup, PagedCacheManager
+from ..kernels import PINNED_BYTES, on_device
 from ..parts import LayerCache, StepContext, state_needs_of
 from .model import CausalLM
 
@@ -194,6 +195,8 @@ class ModelRunner:
                 c.states[st.name] = arena
         self._empty_f32 = torch.empty((1, 0), dtype=torch.float32, device=self.device)
         self._staging = _Staging(self.device)
+        # pinned blocks for the small arrays of a step or two, so that the first one does not make them (torch keeps them for `on_device`)
+        [torch.empty((PINNED_BYTES,), dtype=torch.uint8, pin_memory=True) for _ in range(8)]
         self.use_graphs = bool(use_graphs) and model.graph_safe
         # a step's kernels take about weights / 4 TB/s, its launches about 100 us a layer
         size = 2 if model.dtype == torch.bfloat16 else 4
@@ -232,7 +235,7 @@ class ModelRunner:
 
     def _clear_state(self, slots: Sequence[int]) -> None:
         """Zeroes the given state slots in every arena (a slot keeps what the request before left)."""
-        idx = torch.tensor([int(s) for s in slots], dtype=torch.int64, device=self.device)
+        idx = on_device([int(s) for s in slots], torch.int64, self.device)
         for arena in self._state_arenas:
             arena.index_fill_(0, idx, 0)
 

@@ -86,6 +86,21 @@ def _want(t: torch.Tensor, dtype: torch.dtype, what: str) -> None:
         raise KernelError(f"{what} must be {dtype}, got {t.dtype}")
 
 
+PINNED_BYTES = 4096
+
+
+def on_device(values, dtype: torch.dtype, device) -> torch.Tensor:
+    """A step's small array (a list, or rows of one) on the device, through pinned memory of its own: the host goes on launching.
+    From ordinary memory the copy waits for everything on the stream, and the GPU then for the host: 290 us of a 2,048-token prompt
+    of a design with states (5,485), 65 of any prompt.  (torch hands the pinned block out again when the copy has left it; blocks of
+    one size, PINNED_BYTES, serve almost all of them: a new one costs 100 us.)"""
+    host = torch.tensor(values, dtype=dtype)
+    if torch.device(device).type != "cuda":
+        return host.to(device)
+    pin = torch.empty((max(host.numel(), PINNED_BYTES // host.element_size()),), dtype=dtype, pin_memory=True)[:host.numel()].view(host.shape)
+    return pin.copy_(host).to(device, non_blocking=True)
+
+
 # ---------------------------------------------------------------------------------------
 def embed(table: torch.Tensor, ids: torch.Tensor, out: Optional[torch.Tensor] = None, scale: float = 1.0) -> torch.Tensor:
     """out[t] = float32(table[ids[t]]) * scale.  ids: int32 [T], values in [0, rows) (caller checks)."""
@@ -332,9 +347,9 @@ def _decay_chunks(common, state, slot_stride, state_slots, q_lens, plan_cache, o
         for b, c0, count in long:
             for c in range(c0, c0 + count):
                 first[c] = starts[b] + chunks[c][0]
-        i32 = torch.tensor(first + [f + n for f, (_, n) in zip(first, chunks)] + [c0 for _, c0, _ in long] + [n for _, _, n in long]
-                           + [starts[b] for b in whole] + [starts[b + 1] for b in whole], dtype=torch.int32).to(q.device)
-        i64 = torch.tensor([b for b, _, _ in long] + whole, dtype=torch.int64).to(q.device)
+        i32 = on_device(first + [f + n for f, (_, n) in zip(first, chunks)] + [c0 for _, c0, _ in long] + [n for _, _, n in long]
+                        + [starts[b] for b in whole] + [starts[b + 1] for b in whole], torch.int32, q.device)
+        i64 = on_device([b for b, _, _ in long] + whole, torch.int64, q.device)
         slots = state_slots.index_select(0, i64)
         plan = dict(C=C, L=L, W=W, first=i32[:C], last=i32[C:2 * C], c0=i32[2 * C:2 * C + L], n=i32[2 * C + L:2 * C + 2 * L],
                     wfirst=i32[2 * C + 2 * L:2 * C + 2 * L + W], wlast=i32[2 * C + 2 * L + W:], long_slots=slots[:L], whole_slots=slots[L:])
@@ -391,8 +406,8 @@ def _step_chunks(common, state, slot_stride, state_slots, cu_q, q_lens, plan_cac
     key = ("step_chunk_plan", STEP_FROM)
     plan = plan_cache.get(key) if plan_cache is not None else None
     if plan is None:
-        # from the first to the last row of either kind, straight from the step's own arrays (arrays of their own would be copied to
-        # a device that works, 65 us a step); rows of the other kind between them are passed over: 200 single tokens between two
+        # from the first to the last row of either kind, straight from the step's own arrays (arrays of their own would be copies of
+        # their own); rows of the other kind between them are passed over: 200 single tokens between two
         # portions of 40 tokens, 128 heads, 23 us beside a launch for each portion, 8 of them 4, and at 32 heads one launch is 6 ahead
         whole, long = step_chunk_plan(q_lens)
         plan = dict(long=(long[0], long[-1] - long[0] + 1), whole=(whole[0], whole[-1] - whole[0] + 1) if whole else None)
@@ -533,12 +548,12 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
                 first[c0 + c] = starts[b] + chunks[c0 + c][0]
                 last[c0 + c] = first[c0 + c] + chunks[c0 + c][1]
                 hands_on[c0 + c] = c + 1 < count          # a portion's last chunk hands no share on
-        i32 = torch.tensor(first + last
-                           + [f if h else 0 for f, h in zip(first, hands_on)] + [l if h else 0 for l, h in zip(last, hands_on)]
-                           + [c0 for _, c0, _ in long] + [n for _, _, n in long]
-                           + [starts[b] for b in whole] + [starts[b + 1] for b in whole], dtype=torch.int32).to(q.device)
-        i64 = torch.tensor([c if h else -1 for c, h in enumerate(hands_on)] + list(range(C)) + [-1] * C
-                           + [b for b, _, _ in long] + [c0 + n - 1 for _, c0, n in long] + whole, dtype=torch.int64).to(q.device)
+        i32 = on_device(first + last
+                        + [f if h else 0 for f, h in zip(first, hands_on)] + [l if h else 0 for l, h in zip(last, hands_on)]
+                        + [c0 for _, c0, _ in long] + [n for _, _, n in long]
+                        + [starts[b] for b in whole] + [starts[b + 1] for b in whole], torch.int32, q.device)
+        i64 = on_device([c if h else -1 for c, h in enumerate(hands_on)] + list(range(C)) + [-1] * C
+                        + [b for b, _, _ in long] + [c0 + n - 1 for _, c0, n in long] + whole, torch.int64, q.device)
         long_slots = state_slots.index_select(0, i64[3 * C:3 * C + L])
         keep = i64[2 * C:3 * C]         # where launch 3 leaves a chunk's last state: a portion's last chunk in the slot
         keep.index_copy_(0, i64[3 * C + L:3 * C + 2 * L], long_slots)
@@ -1604,7 +1619,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx
                     q_lens = [ctx.cu_q_host[b + 1] - ctx.cu_q_host[b] for b in range(ctx.num_seqs)]
                     rows, small = prefill_tiles(q_lens, ctx.ctx_lens_host, d, nq, nkv,
                                                 block_of=lambda shape: attention_biased_block(d, dv, nq // nkv, shape))
-                    cached = (torch.tensor(rows, dtype=torch.int32, device=q.device).reshape(-1, 2), small)
+                    cached = (on_device(rows, torch.int32, q.device).reshape(-1, 2), small)
                 ctx.scratch[key] = cached
             tiles, small = cached
             split, span = 0, 0
@@ -1642,7 +1657,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx
                     or not (lead * lead_ctx * reads >= MIXED_DECODE_WORK or lead_ctx >= MIXED_DECODE_CONTEXT)):
                 lead = 0
             rows, small = prefill_tiles(q_lens, ctx.ctx_lens_host, d, nq, nkv, first_seq=lead)
-            cached = (torch.tensor(rows, dtype=torch.int32, device=q.device).reshape(-1, 2), small, lead,
+            cached = (on_device(rows, torch.int32, q.device).reshape(-1, 2), small, lead,
                       lead_ctx if lead else 0)
             ctx.scratch[key] = cached
         tiles, small, lead, lead_ctx = cached
@@ -2850,7 +2865,7 @@ def channel_scan(gate: torch.Tensor, gate_act: str, state: torch.Tensor, state_s
         plan = plan_cache.get(key) if plan_cache is not None else None
         if plan is None:
             rows = channel_items(q_lens, channel_chunk(T))
-            plan = (torch.tensor(rows, dtype=torch.int32).to(gate.device) if len(rows) > B else None, len(rows))
+            plan = (on_device(rows, torch.int32, gate.device) if len(rows) > B else None, len(rows))
             if plan_cache is not None:
                 plan_cache[key] = plan
         items, n = plan
