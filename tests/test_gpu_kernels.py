@@ -1150,6 +1150,49 @@ def test_attention_decode_packed_gives_the_bits_of_the_two_kernels(nq, nkv, d, p
             assert (out[0].reshape(nq, d)[kvh * gsz].float().cpu() - new_v[kvh]).abs().max() < 0.05, kvh
 
 
+LEAN_CASES = [
+    # heads turned as a whole, pages of 32 keys and more: contexts at the edges of a step, a wave's turn, a chunk and a page; groups whose heads
+    # are one batch of a wave's or several; the most slices of the lean kernel and one more
+    (16, 8, 128, 64, 0, 128, False, True, False, 0, None, [513, 512, 511, 480, 449, 128, 129, 127, 97, 96, 33, 32, 31, 8, 7, 2, 1, 64]),
+    (8, 8, 128, 32, 0, 128, False, True, False, 1, 128, [1, 2, 32, 33, 128, 129, 160, 161, 640, 700]),
+    (14, 2, 128, 128, 0, 128, False, True, False, 8, 256, [300, 256, 257, 1000, 5, 100]),
+    (16, 1, 128, 64, 0, 128, False, True, False, 5, 384, [385, 384, 1200, 31, 50]),
+    (30, 2, 64, 32, 0, 64, False, False, False, 3, 128, [129, 128, 1, 70, 333]),
+    (6, 2, 64, 64, 0, 64, False, True, False, 0, None, [65, 64, 40, 200, 3]),
+    (4, 2, 128, 64, 0, 128, False, True, False, 9, 128, [130, 64, 3, 90]),
+    (8, 8, 128, 64, 0, 128, False, True, False, 0, 1152, list(range(70, 3, -2)) + [900]),       # 35 sequences: a run of 32 and the start of another
+    (4, 4, 64, 64, 0, 64, False, True, False, 2, 256, list(range(130, 0, -2))),                 # 65: a run of 64 and one more
+    (12, 3, 128, 64, 0, 128, False, True, False, 2, 512, [500, 400, 30, 20, 10]),               # no power of two of kv heads
+    (8, 8, 128, 64, 0, 128, False, False, False, 0, 2176, list(range(150, 10, -1))),            # more than are resident at once
+]
+
+
+@pytest.mark.parametrize("nq,nkv,d,page,window,rot,interleaved,norm,bias,slices,kpw,contexts", LEAN_CASES)
+def test_attention_decode_lean(nq, nkv, d, page, window, rot, interleaved, norm, bias, slices, kpw, contexts):
+    test_attention_decode_packed_gives_the_bits_of_the_two_kernels(nq, nkv, d, page, window, rot, interleaved, norm, bias, slices, kpw, contexts)
+
+
+def test_attention_decode_packed_slot_elsewhere():
+    """A slot that is not the position's place: the key and value go there, and the sequence reads what its own place holds."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(3)
+    nq, nkv, d, page, contexts = 4, 2, 128, 64, [70, 64]
+    case = _paged_case(g, torch.bfloat16, nq, nkv, d, page, [(c, 1) for c in contexts])
+    _, kc, vt, bt = _mfma_inputs(case)
+    _, ctx = _cu_ctx([(c, 1) for c in contexts])
+    used = {int(p) for b, c in enumerate(contexts) for p in case["bt"][b, :-(-c // page)]}
+    spare = next(p for p in range(kc.shape[0]) if p not in used)
+    slots = torch.tensor([spare * page + 3, spare * page + 9], device=DEV)
+    packed = _rand((2, (nq + 2 * nkv) * d), torch.bfloat16, g).to(DEV)
+    cos, sin = (t.to(DEV) for t in plain.rope_tables(10000.0, d, 80))
+    pos, k2, v2 = (ctx - 1).to(torch.int32).to(DEV), kc.clone(), vt.clone()
+    q = kernels.qk_norm_rope_kv(packed, None, None, 1e-5, cos, sin, d, False, pos, slots, kc, vt, nq, nkv, d, v_grouped=True,
+                                vector_min_tokens=1 << 30)
+    one = kernels.attention_decode_bf16(q, kc, vt, bt, ctx.to(DEV), 70, 0.1)
+    two = kernels.attention_decode_packed_bf16(packed, None, None, 1e-5, cos, sin, d, False, pos, slots, k2, v2, bt, ctx.to(DEV), 70, nq, 0.1)
+    assert torch.equal(one, two) and torch.equal(kc, k2) and torch.equal(vt, v2)
+
+
 def test_attention_decode_packed_refuses():
     from xinfer_amd import kernels
     nq, nkv, d, page = 4, 2, 32, 16

@@ -50,6 +50,14 @@ def test_decode_mixed_lengths_take_whole_sequences_where_there_are_many():
     assert kernels.decode_keys_per_workgroup(2048, 16384, False) == 2048
 
 
+def test_decode_keys_per_workgroup_of_even_lengths():
+    plan = lambda pairs, span: kernels.decode_keys_per_workgroup(pairs, span, kernels.EVEN_LENGTHS)
+    assert plan(488, 3072) == 3200 and plan(264, 2048) == 2176 and plan(240, 1024) == 1152 and plan(4096, 4096) == 4224
+    for pairs, span in ((217, 1024), (184, 2048), (256, 4096), (8, 1024), (600, 5000)):
+        assert plan(pairs, span) == kernels.decode_keys_per_workgroup(pairs, span, False)
+
+
+
 def test_float32_attention_sets_one_limit_a_kernel():
     """The dynamic LDS that the kernel of a class of head sizes is allowed: one number for the class, enough for all of it, so that
     two engines with different heads do not lower it between each other's setting and launch."""

@@ -29,6 +29,8 @@
 // (varlen prefill over cu_seqlens with a cached prefix; decode with split-K, workspace
 // /root/reference/src/utils/kvcache_allocator.rs:662-673); golden formula
 // /root/reference/tests/probes/compare_flashinfer_probe.py:51-73.
+#include <type_traits>
+
 #include "common.h"
 #include "qk_row.h"
 
@@ -86,13 +88,110 @@ struct PackedStep {
   const long long* slots;      // [sequences]; negative: the sequence's key and value are not stored
 };
 
+// The scores of a step's 32 keys (this lane: keys key0 .. key0 + 7 of its query's column) to weights, and the weighted values into
+// the sums; `edge`: some key of the step may be hidden.
+template <int DT>
+__device__ __forceinline__ void weigh_values(f32x4 s0, f32x4 s1, float scale_log2, bool edge, int key0, int pos, int lo, const bf16x8 (&va)[DT],
+                                             f32x4 (&acc)[DT], float& m_run, float& l_run) {
+  float sc[8];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    sc[v] = s0[v] * scale_log2;
+    sc[4 + v] = s1[v] * scale_log2;
+  }
+  if (edge) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int key = key0 + v;
+      if (key > pos || key < lo) sc[v] = -INFINITY;
+    }
+  }
+  float mx = sc[0];
+#pragma unroll
+  for (int v = 1; v < 8; ++v) mx = fmaxf(mx, sc[v]);
+  mx = fmaxf(mx, lane_xor<16>(mx));
+  mx = fmaxf(mx, lane_xor<32>(mx));
+  const float m_new = fmaxf(m_run, mx);
+  const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+  const float corr = __builtin_amdgcn_exp2f(m_run - m_safe);
+  float psum = 0.f;
+  bf16x8 pb;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) {
+    const float p = __builtin_amdgcn_exp2f(sc[v] - m_safe);
+    psum += p;
+    pb[v] = (__bf16)p;
+  }
+  l_run = l_run * corr + psum;
+  m_run = m_new;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    acc[dt][0] *= corr;
+    acc[dt][1] *= corr;
+    acc[dt][2] *= corr;
+    acc[dt][3] *= corr;
+    acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb, acc[dt], 0, 0, 0);
+  }
+}
+
+// The four waves' sums through LDS ([4][g][d] and [4][g][2]), added in wave order: the partial of (sequence, head, split), or with one
+// split for every sequence the result itself.  A thread takes four dims.
+template <int DT>
+__device__ __forceinline__ void merge_waves(float* lds_o, float* lds_ml, const f32x4 (&acc)[DT], float m_run, float l_run, int wave, int lane, int g,
+                                            int d, size_t head0, int split, int max_splits, float* __restrict__ part_o,
+                                            float* __restrict__ part_ml, bf16* __restrict__ out) {
+  const int r = lane & 15, j = lane >> 4;
+  // the column's sum over the four lane groups
+  float lt = l_run + lane_xor<16>(l_run);
+  lt += lane_xor<32>(lt);
+  if (r < g) {
+    if (j == 0) {
+      lds_ml[(wave * g + r) * 2] = m_run;
+      lds_ml[(wave * g + r) * 2 + 1] = lt;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      if (16 * dt >= d) break;
+      *reinterpret_cast<f32x4*>(lds_o + ((size_t)wave * g + r) * d + 16 * dt + 4 * j) = acc[dt];
+    }
+  }
+  lds_barrier();
+  for (int idx = threadIdx.x; idx < g * d / 4; idx += 256) {
+    const int h = idx / (d / 4), i = 4 * (idx - h * (d / 4));
+    float mm = -INFINITY;
+#pragma unroll
+    for (int wv = 0; wv < 4; ++wv) mm = fmaxf(mm, lds_ml[(wv * g + h) * 2]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float ll = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < 4; ++wv) {
+      const float mw = lds_ml[(wv * g + h) * 2];
+      const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - mm);
+      o += *reinterpret_cast<const f32x4*>(lds_o + ((size_t)wv * g + h) * d + i) * f;
+      ll += lds_ml[(wv * g + h) * 2 + 1] * f;
+    }
+    if (max_splits == 1) {   // the only split of every sequence: the result itself
+      const float inv = 1.f / ll;                                      // as the combine rounds
+      typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+      bf16x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = (__bf16)(o[e] * inv);
+      *reinterpret_cast<bf16x4*>(out + (head0 + h) * d + i) = y;
+      continue;
+    }
+    const size_t pidx = (head0 + h) * max_splits + split;
+    *reinterpret_cast<f32x4*>(part_o + pidx * d + i) = o;
+    if (i == 0) *reinterpret_cast<float2*>(part_ml + pidx * 2) = make_float2(mm, ll);
+  }
+}
+
 template <int KC, int DT, int PACKED>
 __global__ __launch_bounds__(256, DT > 8 ? 1 : 2) void attn_decode_split_kernel(
     const void* q_v, bf16* k_cache_w, bf16* vt_cache_w,
     const int* __restrict__ block_tables, int max_pages, const int* __restrict__ ctx_lens,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16* __restrict__ out, int max_splits, float scale_log2,
     int window, int page, int nq, int nkv, int d, int keys_per_wg, PackedStep ps) {
-  extern __shared__ float lds[];  // [4 waves][g][d] + [4][g][2] + page numbers of the chunk
+  extern __shared__ __align__(16) float lds[];  // [4 waves][g][d] + [4][g][2] + page numbers of the chunk
   const bf16* k_cache = k_cache_w;
   const bf16* vt_cache = vt_cache_w;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -246,92 +345,216 @@ __global__ __launch_bounds__(256, DT > 8 ? 1 : 2) void attn_decode_split_kernel(
       s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[1][c], qb[c], s1, 0, 0, 0);
     }
     if (more) load_k(kb + 128);
-    float sc[8];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      sc[v] = s0[v] * scale_log2;
-      sc[4 + v] = s1[v] * scale_log2;
-    }
-    if (kb + 31 > pos || kb < lo) {   // some key of the step is hidden from the query
-      const int key0 = kb + 8 * j;
-#pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int key = key0 + v;
-        if (key > pos || key < lo) sc[v] = -INFINITY;
-      }
-    }
-    float mx = sc[0];
-#pragma unroll
-    for (int v = 1; v < 8; ++v) mx = fmaxf(mx, sc[v]);
-    mx = fmaxf(mx, lane_xor<16>(mx));
-    mx = fmaxf(mx, lane_xor<32>(mx));
-    const float m_new = fmaxf(m_run, mx);
-    const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
-    const float corr = __builtin_amdgcn_exp2f(m_run - m_safe);
-    float psum = 0.f;
-    bf16x8 pb;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const float p = __builtin_amdgcn_exp2f(sc[v] - m_safe);
-      psum += p;
-      pb[v] = (__bf16)p;
-    }
-    l_run = l_run * corr + psum;
-    m_run = m_new;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      acc[dt][0] *= corr;
-      acc[dt][1] *= corr;
-      acc[dt][2] *= corr;
-      acc[dt][3] *= corr;
-      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb, acc[dt], 0, 0, 0);
-    }
+    weigh_values(s0, s1, scale_log2, kb + 31 > pos || kb < lo, kb + 8 * j, pos, lo, va, acc, m_run, l_run);
     if (more) load_v(kb + 128);
   }
-  // the column's sum over the four lane groups
-  float lt = l_run + lane_xor<16>(l_run);
-  lt += lane_xor<32>(lt);
-  if (col) {
-    if (j == 0) {
-      lds_ml[(wave * g + r) * 2] = m_run;
-      lds_ml[(wave * g + r) * 2 + 1] = lt;
-    }
+  merge_waves(lds_o, lds_ml, acc, m_run, l_run, wave, lane, g, d, (size_t)seq * nq + kvh * g, split, max_splits, part_o, part_ml, out);
+}
+
+// The same for what decoding usually is: heads of 64 or 128 dims (32 KC) that are turned as a whole in the half layout and have no bias, no
+// window, pages of 32 keys and more, projections of up to kTogether slices.  What bounds a launch over few keys is its start, a chain of trips
+// to memory and what is executed between them (every launch fetches its instructions anew), so there is little between a wave's first
+// instruction and its first keys:
+//   * the length, the position, the slot, the first step's page number, the chunk's row of page numbers and the heads' elements need nothing
+//     but the arguments and are asked for together, a head's slices and a wave's heads too (one after the other, the heads of 100
+//     sequences of 60 to 480 keys on 64 query heads took 14 us of 38);
+//   * the first keys and values go out as soon as the length is there, behind the heads' elements: loads return in order, so that the heads
+//     are normed and turned while the keys travel;
+//   * the new key and value go into the step that holds them from LDS: nobody waits for their stores;
+//   * a step's page number is one scalar.
+// Attention and combine, us, the kernel above | this, 8 kv heads of 128: 1 sequence of 513 keys 9.0 | 8.0, of 4,000 11.8 | 9.5, 8 of 4,013 31.9 | 29.3,
+// 48 of 100 to 768 27.0 | 20.3, 100 of 60 to 480 (64 query heads) 38.0 | 28.3, 200 of 30 to 240 34.5 | 27.7, 256 of 30 to 513 61 | 59.3, 64 of 4,096 187 |
+// 187 (5.7 TB/s).  A wave's registers leave room for four workgroups a compute unit where the heads stay in LDS.
+struct LeanStep {
+  const float* qw;             // per-head norm weights [d], or null (both)
+  const float* kw;
+  const float* cos_t;          // [positions, d / 2]
+  const float* sin_t;
+  size_t slice_stride;
+  float eps;
+  int slices, n_seq, run_shift;
+};
+
+template <int KC, bool PARTS>
+__global__ __launch_bounds__(256, 4) void attn_decode_lean_kernel(
+    const int* __restrict__ ctx_lens, const int* __restrict__ block_tables, const void* __restrict__ qkv, bf16* k_cache, bf16* v_cache,
+    const int* __restrict__ positions, const long long* __restrict__ slots, int max_pages, int keys_per_wg, int page_shift, int nq, int nkv,
+    int max_splits, float scale_log2, float* __restrict__ part_o, float* __restrict__ part_ml, bf16* __restrict__ out, LeanStep ps) {
+  constexpr int D = 32 * KC, DT = 2 * KC, kTogether = PARTS ? 8 : 1, kRows = 2;
+  extern __shared__ __align__(16) float lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, j = lane >> 4;
+  // Workgroups as above, and: a compute unit gets workgroups c, c + 256, .., and where all of them are resident at once none is left to
+  // hand out.  Sequences come longest first; every second run of 256 workgroups, the first among them, is taken from its end, so that the
+  // units that get another one have the short ones (61 sequences of 90 to 2,700 keys, 8 kv heads: units of 1,630 to 3,950 keys, of
+  // 2,620 to 2,790 so).
+  const int kvh = blockIdx.x, split = blockIdx.z, run = (int)blockIdx.y >> ps.run_shift;
+  const int seq = run & 1 ? (int)blockIdx.y : min((run + 1) << ps.run_shift, ps.n_seq) - 1 - ((int)blockIdx.y - (run << ps.run_shift));
+  const int g = nq / nkv, k_begin = split * keys_per_wg, kb0 = k_begin + 32 * wave;
+  float* lds_o = lds;                                        // [4][g][D]
+  float* lds_ml = lds + 4 * g * D;                           // [4][g][2]
+  bf16* qs = reinterpret_cast<bf16*>(lds_ml + 4 * g * 2);    // [g][D]
+  bf16* kv_new = qs + g * D;                                 // [2][D]
+  int* pages = reinterpret_cast<int*>(kv_new + 2 * D);       // [keys_per_wg / page + 2]
+
+  const int ctx = ctx_lens[seq], tok_pos = positions[seq];
+  const long long slot = slots[seq];
+  const int* bt = block_tables + (size_t)seq * max_pages;
+  const int first_page = k_begin >> page_shift;
+  const int page_begin = bt[min(first_page, max_pages - 1)], page_wave = bt[min(kb0 >> page_shift, max_pages - 1)];
+  const int n_row = min((keys_per_wg >> page_shift) + 2, max_pages - first_page);      // of the chunk's row of page numbers, the first 256
+  int my_page = 0;
+  if ((int)threadIdx.x < n_row) my_page = bt[first_page + threadIdx.x];
+  // head i of this workgroup (query heads, the new key, the new value), a lane's pair of dims `lane` and `lane` + D / 2
+  const int pair = lane < D / 2 ? lane : 0;
+  typedef std::conditional_t<PARTS, float, bf16> Raw;
+  auto row_of = [&](int i) {
+    return reinterpret_cast<const Raw*>(qkv) + ((size_t)seq * (nq + 2 * nkv) + (i < g ? kvh * g + i : nq + (i - g) * nkv + kvh)) * D;
+  };
+  Raw ra[kRows][kTogether], rb[kRows][kTogether];
+  auto ask = [&](int i0, int rows) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      if (16 * dt >= d) break;
-      float* o = lds_o + ((size_t)wave * g + r) * d + 16 * dt + 4 * j;
-      o[0] = acc[dt][0];
-      o[1] = acc[dt][1];
-      o[2] = acc[dt][2];
-      o[3] = acc[dt][3];
+    for (int u = 0; u < kRows; ++u)
+      if (i0 + 4 * u < rows) {
+        const Raw* p = row_of(i0 + 4 * u);
+#pragma unroll
+        for (int sl = 0; sl < kTogether; ++sl)
+          if (!PARTS || sl < ps.slices) {
+            ra[u][sl] = p[pair];
+            rb[u][sl] = p[pair + D / 2];
+            p += ps.slice_stride;
+          }
+      }
+  };
+  ask(wave, g + 2);
+  const bool normed = ps.qw != nullptr;
+  float qwa = 1.f, qwb = 1.f, kwa = 1.f, kwb = 1.f;
+  if (normed) {
+    qwa = ps.qw[pair];
+    qwb = ps.qw[pair + D / 2];
+    kwa = ps.kw[pair];
+    kwb = ps.kw[pair + D / 2];
+  }
+  if (k_begin >= ctx) return;  // no keys for this split (the combine kernel knows)
+  const float cs = ps.cos_t[(size_t)tok_pos * (D / 2) + pair], sn = ps.sin_t[(size_t)tok_pos * (D / 2) + pair];
+  const int pos = ctx - 1, k_end = min(ctx, k_begin + keys_per_wg);     // exclusive
+
+  // Operands of keys kb .. + 31 (kb <= pos), all of one page; keys past the sequence are read from its last group of 8 (and masked).
+  const int page = 1 << page_shift;
+  bf16x8 ka[2][KC], va[DT];
+  auto load_k = [&](int kb, int number) {
+    const bf16* from = k_cache + ((size_t)number * nkv + kvh) * page * D;
+    const unsigned at = (unsigned)((kb & (page - 1)) + min(8 * (r >> 2), (pos & ~7) - kb) + (r & 3)) * D + 8 * j;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      ka[0][c] = load8(from + at + 32 * c);
+      ka[1][c] = load8(from + at + 32 * c + 4 * D);
+    }
+  };
+  auto load_v = [&](int kb, int number) {
+    const bf16* from = v_cache + ((size_t)number * nkv + kvh) * page * D;
+    const unsigned at = (unsigned)(((kb & (page - 1)) + min(8 * j, (pos & ~7) - kb)) >> 3) * (8 * D) + 8 * r;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) va[dt] = load8(from + at + 128 * dt);
+  };
+  const bool mine = kb0 < k_end;             // (a wave without keys gets the chunk's first ones)
+  load_k(mine ? kb0 : k_begin, mine ? page_wave : page_begin);
+  load_v(mine ? kb0 : k_begin, mine ? page_wave : page_begin);
+  if ((int)threadIdx.x < n_row) pages[threadIdx.x] = my_page;
+  const int n_pages = ((k_end - 1) >> page_shift) - first_page + 1;
+  for (int i = threadIdx.x + 256; i < n_pages; i += 256) pages[i] = bt[first_page + i];
+
+  const bool owner = pos < k_begin + keys_per_wg && slot >= 0;
+  const int rows = owner ? g + 2 : g;
+  for (int i0 = wave; i0 < rows; i0 += 4 * kRows) {
+    if (i0 != wave) ask(i0, rows);
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int i = i0 + 4 * u;
+      if (i >= rows) break;
+      // (sums and products written out as in qk_row.h: the same bits)
+      float a, b;
+      if constexpr (PARTS) {
+        a = b = 0.f;
+#pragma unroll
+        for (int sl = 0; sl < kTogether; ++sl)
+          if (sl < ps.slices) {
+            a += ra[u][sl];
+            b += rb[u][sl];
+          }
+      } else {
+        a = to_float(ra[u][0]);
+        b = to_float(rb[u][0]);
+      }
+      if (lane >= D / 2) a = b = 0.f;
+      bf16* to = i < g ? qs + i * D : kv_new + (i - g) * D;
+      if (i <= g) {
+#pragma clang fp contract(off)
+        float inv = 1.f;
+        if (normed) inv = rsqrtf(wave_sum(__builtin_fmaf(b, b, __builtin_fmaf(a, a, 0.f))) / (float)D + ps.eps);
+        const float x = a * inv * (i < g ? qwa : kwa), y = b * inv * (i < g ? qwb : kwb);
+        a = __builtin_fmaf(x, cs, -(y * sn));
+        b = __builtin_fmaf(x, sn, y * cs);
+      }
+      if (lane < D / 2) {
+        to[lane] = from_float<bf16>(a);
+        to[lane + D / 2] = from_float<bf16>(b);
+        if (i >= g) {                          // into the cache too
+          const size_t base = ((size_t)(slot >> page_shift) * nkv + kvh) * page * D;
+          const int off = (int)(slot & (page - 1));
+          bf16* p = i == g ? k_cache + base + (size_t)off * D : v_cache + base + (size_t)(off >> 3) * 8 * D + (off & 7);
+          const int step = i == g ? 1 : 8;
+          p[lane * step] = from_float<bf16>(a);
+          p[(lane + D / 2) * step] = from_float<bf16>(b);
+        }
+      }
     }
   }
-  __syncthreads();
-  // merge the four waves, in wave order, and store the partial of (seq, head, split)
-  for (int idx = threadIdx.x; idx < g * d; idx += blockDim.x) {
-    const int h = idx / d, i = idx - h * d;
-    float mm = -INFINITY;
+  lds_barrier();     // heads and page numbers are in LDS
+  const bool col = r < g;        // this lane's query column: head kvh*g + r of the sequence, or none
+  const bf16* q_lane = qs + (col ? r : 0) * D + 8 * j;
+  const bool patched = owner && (long long)__builtin_amdgcn_readfirstlane(pages[(pos >> page_shift) - first_page]) * page + (pos & (page - 1)) == slot;
+
+  f32x4 acc[DT];
 #pragma unroll
-    for (int wv = 0; wv < 4; ++wv) mm = fmaxf(mm, lds_ml[(wv * g + h) * 2]);
-    float o = 0.f, ll = 0.f;
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;   // running max (log2 domain) and this lane's part of the sum
+  for (int kb = kb0; kb < k_end; kb += 128) {
+    const bool more = kb + 128 < k_end;
+    int number = 0;
+    if (more) number = __builtin_amdgcn_readfirstlane(pages[((kb + 128) >> page_shift) - first_page]);
+    if (patched && kb + 31 >= pos) {          // (kb <= pos)
+      const int o = pos - kb;                 // key o of the step: row r of tile t, element o & 7 of lane group o >> 3
 #pragma unroll
-    for (int wv = 0; wv < 4; ++wv) {
-      const float mw = lds_ml[(wv * g + h) * 2];
-      const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - mm);
-      o += lds_o[((size_t)wv * g + h) * d + i] * f;
-      ll += lds_ml[(wv * g + h) * 2 + 1] * f;
+      for (int c = 0; c < KC; ++c)
+        if (r >> 2 == o >> 3 && (r & 3) == (o & 3)) {
+          const bf16x8 k = load8(kv_new + 32 * c + 8 * j);
+          if (o & 4) ka[1][c] = k;
+          else ka[0][c] = k;
+        }
+      const __bf16* v = reinterpret_cast<const __bf16*>(kv_new + D);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        if (j == o >> 3) {
+          const __bf16 x = v[16 * dt + r];
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (e == (o & 7)) va[dt][e] = x;
+        }
     }
-    if (max_splits == 1) {   // the only split of every sequence: the result itself
-      out[((size_t)seq * nq + kvh * g + h) * d + i] = __float2bfloat16(o * (1.f / ll));   // as the combine rounds
-      continue;
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+    asm volatile("" ::: "memory");       // (the heads are read from LDS in every step: held in registers they cost a wave a SIMD)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const bf16x8 qb = load8(q_lane + 32 * c);
+      s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[0][c], qb, s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[1][c], qb, s1, 0, 0, 0);
     }
-    const size_t pidx = ((size_t)seq * nq + kvh * g + h) * max_splits + split;
-    part_o[pidx * d + i] = o;
-    if (i == 0) {
-      part_ml[pidx * 2] = mm;
-      part_ml[pidx * 2 + 1] = ll;
-    }
+    if (more) load_k(kb + 128, number);
+    weigh_values(s0, s1, scale_log2, kb + 31 > pos, kb + 8 * j, pos, 0, va, acc, m_run, l_run);
+    if (more) load_v(kb + 128, number);
   }
+  merge_waves(lds_o, lds_ml, acc, m_run, l_run, wave, lane, g, D, (size_t)seq * nq + kvh * g, split, max_splits, part_o, part_ml, out);
 }
 
 // One wave per (head, sequence).  Lanes first share out the splits to find the common
@@ -496,6 +719,27 @@ static int launch_decode(int packed, const void* q, const PackedStep& ps, void* 
   if (n_seq == 0) return 0;
   dim3 grid(nkv, n_seq, max_splits);
   const float sl = scale * kLog2e;
+  const int slices = packed == 2 ? ps.slices : 0;
+  const size_t lean_lds = lds + (size_t)(g + 2) * d * sizeof(bf16);
+  if (packed && (d == 64 || d == 128) && ps.rot == d && !ps.interleaved && !ps.bias && window <= 0 && page >= 32 && slices <= 8 && lean_lds <= 64 * 1024) {
+    // (run_shift 0: the sequences' own order, where the units take further workgroups in turn, a sequence's splits are workgroups of their own or
+    // 256 workgroups are no run of sequences)
+    LeanStep step{ps.qw, ps.kw, ps.cos_t, ps.sin_t, ps.slice_stride, ps.eps, slices, n_seq, 0};
+    for (int s = 1; s <= 8; ++s)
+      if (nkv << s == 256 && max_splits == 1 && (long long)nkv * n_seq <= 1024) step.run_shift = s;
+#define XI_LEAN(KC, PARTS)                                                                                                       \
+  attn_decode_lean_kernel<KC, PARTS><<<grid, 256, lean_lds, stream>>>(ctx_lens, block_tables, q, (bf16*)k_cache, (bf16*)vt_cache, ps.positions, \
+                                                                      ps.slots, max_pages, keys_per_wg, __builtin_ctz(page), nq, nkv,  \
+                                                                      max_splits, sl, part_o, part_ml, (bf16*)out, step)
+    if (d == 64) {
+      if (slices) XI_LEAN(2, true);
+      else XI_LEAN(2, false);
+    } else {
+      if (slices) XI_LEAN(4, true);
+      else XI_LEAN(4, false);
+    }
+#undef XI_LEAN
+  } else {
 #define XI_DC(KC, DT, PACKED)                                                                      \
   attn_decode_split_kernel<KC, DT, PACKED><<<grid, 256, lds, stream>>>(                            \
       q, (bf16*)k_cache, (bf16*)vt_cache, block_tables, max_pages, ctx_lens,                       \
@@ -511,6 +755,7 @@ static int launch_decode(int packed, const void* q, const PackedStep& ps, void* 
   else XI_DCP(8, 16);
 #undef XI_DCP
 #undef XI_DC
+  }
   XI_LAUNCH_CHECK("attention_decode_split");
   if (max_splits == 1) return 0;   // the split kernel has written the result
   if (max_splits > kCombineWideFrom) {

@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from ..cache import DecodeStepError, BatchArrays, CacheGroup, PagedCacheManager
-from ..kernels import PINNED_BYTES, on_device
+from ..kernels import EVEN_LENGTHS, PINNED_BYTES, on_device
 from ..parts import LayerCache, StepContext, state_needs_of
 from .model import CausalLM
 
@@ -40,10 +40,14 @@ class StepError(ValueError):
     pass
 
 
-def _similar(ctx_lens: np.ndarray) -> bool:
-    """The sequences of a step are about equally long (kernels may then give each a workgroup of
-    its own instead of cutting all into equal pieces)."""
-    return bool(ctx_lens.size) and float(ctx_lens.mean()) >= 0.9 * float(ctx_lens.max())
+def _similar(ctx_lens: np.ndarray) -> int:
+    """How even the sequences of a step are: True, about equally long (kernels may then give each a
+    workgroup of its own instead of cutting all into equal pieces), EVEN_LENGTHS, not a few long ones among many short (of sixteen
+    sequences and more), or False."""
+    if not ctx_lens.size:
+        return False
+    mean, longest = float(ctx_lens.mean()), float(ctx_lens.max())
+    return True if mean >= 0.9 * longest else EVEN_LENGTHS if mean >= 0.4 * longest and ctx_lens.size >= 16 else False
 
 
 class _Staging:
@@ -208,11 +212,11 @@ class ModelRunner:
             graph_max_batch = 256 if host_bound else 64
         self.graph_after = max(1, int(graph_after))
         self.graph_max_batch = int(graph_max_batch)
-        self._graphs: Dict[Tuple[int, int, bool], _DecodeGraph] = {}     # in order of last use, oldest first
+        self._graphs: Dict[Tuple[int, int, int], _DecodeGraph] = {}     # in order of last use, oldest first
         self.graphs_most = max(1, int(graphs_most))
         self.graph_bytes_most = int(graph_bytes_most)
         self.graphs_dropped = 0
-        self._seen: Dict[Tuple[int, int, bool], int] = {}
+        self._seen: Dict[Tuple[int, int, int], int] = {}
         self._graph_pool = None
         self._device_tokens = None          # the step's tokens that live on the device (see `step`)
         self._tok_pin: Optional[torch.Tensor] = None
@@ -397,6 +401,8 @@ class ModelRunner:
                              -3: f"request {rid}: its tokens exceed the model's {spec.max_positions} positions",
                              -4: f"a token id is outside the vocabulary of {spec.vocab_size}"}.get(
                                  ex.kind, f"the step could not be prepared ({ex.kind})")) from None
+        if not similar and B >= 16:
+            similar = _similar(host32[4 * B + 1:5 * B + 1])       # (the lengths just written)
         bucket = context_bucket(longest)
         g = self._graphs.get((B, bucket, similar))
         if g is None:

@@ -1193,12 +1193,16 @@ DECODE_SPLITS_MOST = 1024           # splits of a sequence that the search below
 DECODE_WHOLE_KEYS = 2048            # mixed lengths, one and a half pairs a compute unit and more: a workgroup's keys at most
 
 
-def decode_keys_per_workgroup(pairs: int, span: int, similar: bool = False) -> int:
-    return _decode_keys_per_workgroup(int(pairs), int(span), bool(similar))
+EVEN_LENGTHS = 2                    # a third value for `similar`: the mean length is at least 0.4 of the longest (True: 0.9)
+DECODE_EVEN_KEYS = 4096             # such lengths: a workgroup's keys at most
+
+
+def decode_keys_per_workgroup(pairs: int, span: int, similar: int = False) -> int:
+    return _decode_keys_per_workgroup(int(pairs), int(span), int(similar) if similar == EVEN_LENGTHS else int(bool(similar)))
 
 
 @functools.lru_cache(maxsize=4096)
-def _decode_keys_per_workgroup(pairs: int, span: int, similar: bool) -> int:
+def _decode_keys_per_workgroup(pairs: int, span: int, similar: int) -> int:
     """Keys per workgroup of the split-K decode kernel for `pairs` (sequence, kv head) pairs of
     up to `span` keys (a multiple of 128; more than `span`: a workgroup takes a whole sequence and
     there is no second kernel).
@@ -1221,7 +1225,19 @@ def _decode_keys_per_workgroup(pairs: int, span: int, similar: bool) -> int:
     sequences of 100 to 768 keys, longest first: 64 us against 72 in chunks of 512, and 80 in chunks
     of 512 in random order; 64 of 256 to 2,304: 64 against 68; 48 of 100 to 768: 20.5 against 21.9);
     from one pair a compute unit on chunks of 1,024 (32 sequences of 500 to 4,000: 60 us against 65
-    at 512 and 63 whole)."""
+    at 512 and 63 whole).
+
+    EVEN_LENGTHS: spread out, but not a few long ones among many short.  Whole sequences where the longest outlasts a unit's share of
+    all keys (0.55 pairs span / 256) by less than what the second kernel and the splits' uneven share-out cost, about 800 keys and a fifth
+    of the share, from 7 pairs for 8 units on.  Us, the rules above | whole, both in the kernel for such steps: 61 sequences of 90 to 2,700
+    keys 71 | 66, 64 of 256 to 2,304 67 | 63, 40 of 300 to 3,000 62 | 58, 33 of 700 to 1,400 39 | 32, 45 of 130 to 1,060 (64 query heads) 33 |
+    26, 30 of 40 to 300 14 | 10, 31 of 200 to 1,900 36 | 33; beyond the rule 25 of 200 to 1,500 26 | 26, 23 of 130 to 1,900 28 | 29, 16 of 500
+    to 2,500 30 | 34; a few long ones, 61 of 600 in the middle and one of 4,000, 54 | 63."""
+    if similar == EVEN_LENGTHS:
+        p = pairs / COMPUTE_UNITS
+        if p >= 0.85 and span <= DECODE_EVEN_KEYS and span * (1 - 0.76 * p) <= 800:
+            return (span + 128) // 128 * 128          # more than span: one split
+        similar = 0
     if similar:
         chunks = max(1, -(-int(span) // 128))
         plans = []
