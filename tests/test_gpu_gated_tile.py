@@ -163,3 +163,18 @@ def test_gated_tile_rule_by_rounds(M, F, K, shape):
     assert kernels.gated_tile_shape(x, w) == shape
     for other in (_Rows(M, K, start=8), _Rows(M, K, contiguous=False), _Rows(M, K, dtype=torch.float32), _Rows(M, K + 64)):
         assert kernels.gated_tile_shape(other, w) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1793, 4092, 5120), (2048, 4096, 6144), (1025, 5764, 5184)])
+def test_round_tiles(M, N, K):
+    """One full round of tiles of 256 by 128: remainders of rows and features, an odd number of tiles of K."""
+    from xinfer_amd import kernels
+    assert kernels.round_tiles_ahead(M, N, K)
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    x, w = (torch.randn(s, generator=g, device="cuda:0").to(torch.bfloat16) for s in ((M, K), (N, K)))
+    y = kernels.linear_bf16(x, w)
+    assert torch.equal(y, kernels.linear_tile(x, w, shape=1))
+    # float32 sums of K products of about one, 2^-24 of sqrt(K) each step at worst, and one rounding to 8 bits
+    ref = x.float() @ w.float().T
+    assert float(((y.float() - ref).abs() - ref.abs() * 2.0 ** -8).max()) < K * 2.0 ** -24 * K ** 0.5

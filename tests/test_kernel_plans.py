@@ -177,3 +177,12 @@ def test_three_parts_of_a_float32():
     perm = torch.cat([torch.arange(len(worst)), len(worst) + torch.randperm(len(x) - len(worst), generator=g)])
     out = mid * lo[perm] + lo * mid[perm] + lo * lo[perm]
     assert bool((out.abs() <= (2.0 ** -24 + 2.0 ** -34) * (x.double() * x.double()[perm]).abs() * 2.0 ** 48).all())
+
+
+def test_round_tiles_ahead():
+    """One full round of tiles of 256 by 128, long K."""
+    ahead = kernels.round_tiles_ahead
+    assert ahead(2048, 4096, 12288) and ahead(1793, 4096, 6144) and ahead(1537 - 256, 5120, 5120) and ahead(1025, 6144, 20480)
+    assert ahead(1792, 4096, 8192) and not ahead(1791 - 255, 4096, 8192)       # 7 x 32 tiles, 6 x 32
+    for M, N, K in ((2048, 4096, 4096), (2049, 4096, 12288), (1536, 4096, 12288), (2048, 2048, 8192), (4096, 2048, 16384), (8, 4096, 12288)):
+        assert not ahead(M, N, K), (M, N, K)

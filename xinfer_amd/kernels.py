@@ -1981,6 +1981,19 @@ def tall_tile_rows(x: torch.Tensor, w: torch.Tensor) -> Optional[int]:
     return rows
 
 
+ROUND_TILES = (224, 256)            # tiles of 256 rows by 128 features that are one full round of the compute units
+
+
+def round_tiles_ahead(M: int, N: int, K: int) -> bool:
+    """Whether x [M, K] @ w [N, K]^T goes in tiles of 256 rows by 128 features (shape 1 of `linear_tile`) because they are one full round of
+    the compute units (224 to 256 of them) and K is long, from 5,120 on.  Weights from memory, library / this, over N of 2,048 to 8,192 and the
+    rows that make 224 tiles and more: K = 5,120 1.00 to 1.18, 6,144 1.03 to 1.11, 8,192 0.99 to 1.12, 12,288 1.03 to 1.15, 16,384 1.01 to 1.15,
+    20,480 (the library at half its rate) 1.5 to 1.6.  2,048 rows, us: N=4096 K=6144 91 / 87, K=12288 178 / 167, K=17408 377 / 231.  Not there: K = 4,096 (0.93
+    to 1.14 alone, inside a prompt of 2,048 tokens 59 / 61 us), 200 tiles (0.97 to 1.15) and fewer, N up to 2,048 around K = 16,384 (0.74), two
+    rounds (the library ahead by 5 to 12%)."""
+    return ROUND_TILES[0] <= -(-M // 256) * -(-N // 128) <= ROUND_TILES[1] and 5120 <= K < 1 << 22 and not (N <= 2048 and 14336 < K < 18432)
+
+
 def linear_tall(x: torch.Tensor, w: torch.Tensor, rows: int) -> torch.Tensor:
     """bfloat16 x [M, K] @ w [N, K]^T, [M, N] bfloat16, in the many-row tiled kernel's tiles of `rows` (`TALL_SHAPES`) by 256; the
     value of an element does not depend on `rows`."""
@@ -2274,7 +2287,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     `allow_split` may answer with float32 partial sums [slices, M, N] for a narrow output.  More
     rows: one round of low tiles where `small_tile_plan` says so (bfloat16 results, operands on 16 bytes), with
     `allow_split` in slices of K; with `allow_split` the tiled kernels of `tile_split_plan` and `linear_mid`;
-    where K is long and the output narrow `linear_tall`, else the vendor library (hipBLASLt through torch), which the reference's engine also
+    where K is long and the output narrow `linear_tall`, one full round of larger tiles `round_tiles_ahead`, else the vendor library (hipBLASLt through torch), which the reference's engine also
     uses for its matrix products."""
     _dev(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
@@ -2313,6 +2326,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtyp
     rows = tall_tile_rows(x, w)
     if rows is not None:
         return linear_tall(x, w, rows)
+    if (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and not (x.data_ptr() | w.data_ptr()) & 15
+            and round_tiles_ahead(x.shape[0], w.shape[0], x.shape[1]) and linear_tile_takes(x.shape[0], w.shape[0], x.shape[1])):
+        return linear_tile(x, w, shape=1)
     return torch.nn.functional.linear(x, w)
 
 
