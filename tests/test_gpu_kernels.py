@@ -294,6 +294,15 @@ def test_linear_thin_and_its_folded_norm(M, N, K, N2):
         assert (y3.cpu().double() - ref2).abs().max() / ref2.abs().max() < 2.0 ** -6
 
 
+# K: every number of tiles that is asked for together, and one more; N: one to four features a workgroup (held alone), five, and more; rows: a group of
+# the copying and one more; N2 behind N = 8,192: 512 parts of a row's squares
+@pytest.mark.parametrize("M,N,K,N2", [(1, 1024, 512, 256), (4, 1000, 1024, 300), (5, 256, 1536, 4096), (8, 768, 2048, 1024), (9, 1021, 2560, 64),
+                                      (16, 1024, 3072, 512), (3, 700, 3584, 80), (16, 1280, 2048, 96), (7, 5, 3072, 512), (1, 4096, 1024, 6144),
+                                      (16, 8192, 512, 48), (2, 8192, 256, 1000)])
+def test_linear_thin_asked_for_together(M, N, K, N2):
+    test_linear_thin_and_its_folded_norm(M, N, K, N2)
+
+
 def test_linear_thin_refuses():
     from xinfer_amd import kernels
     x = torch.zeros((17, 256), dtype=torch.bfloat16, device=DEV)

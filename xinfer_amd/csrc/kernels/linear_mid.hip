@@ -37,6 +37,7 @@
 // Reference call site: candle matmul in /root/reference/src/models/layers/linear.rs:76-124
 // (vendor BLAS).
 #include "common.h"
+#include "fold_parts.h"
 
 namespace xi {
 
@@ -51,7 +52,7 @@ constexpr int kMidDepth = 2;           // tiles whose loads are in flight (the d
 constexpr int kMidTile = 128 * kMidLdsRow;   // elements of one operand's tile in LDS
 constexpr size_t kMidLdsBytes = 2 * 2 * (size_t)kMidTile * sizeof(bf16) + 16 * sizeof(float);
 constexpr size_t kMidWideLdsBytes = 2 * 3 * (size_t)kMidTile * sizeof(bf16) + 16 * sizeof(float);   // WR = 8
-constexpr int kMidSsLoads = 32;        // 16 threads x 32 loads: up to 512 parts of a row's sum of squares
+constexpr int kMidParts = 512;         // most parts of a row's sum of squares
 
 struct MidFold {
   const float* ss_in;   // [M, parts] parts of each row's sum of squares
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
   extern __shared__ __align__(16) unsigned char mid_smem[];
   bf16* lds = reinterpret_cast<bf16*>(mid_smem);   // [buffer][w tile [WROWS] | x tile [128]][kMidLdsRow]
   float* inv_s = reinterpret_cast<float*>(mid_smem + 2 * (size_t)(WT + kMidTile) * sizeof(bf16));   // [16]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, j = lane >> 4;
   constexpr int TI = FULL ? 4 : WR / 2;               // 16-row tiles of w a wave multiplies
   constexpr int TG = GATED ? TI / 2 : TI;             // of them gate tiles (the others: their up tiles)
@@ -96,18 +97,10 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
   // Workgroups start at different tiles of their slice and wrap around, so that they do not all
   // ask for the same offset of their rows of w at the same time; where a workgroup starts
   // depends on its features alone, so an output element's sum has one order whatever M is.
-  const int start = (int)(((long long)tile * rotate) % nkt);
+  const int start = rotate == 1 ? (int)((unsigned)tile % (unsigned)nkt) : rotate ? (int)(((long long)tile * rotate) % nkt) : 0;
 
-  // FOLD: 16 threads per row add up the parts of its sum of squares; the loads start now
-  float ss_mine[FOLD ? kMidSsLoads : 1];
-  if constexpr (FOLD) {
-    const int token = tid >> 4, sub = tid & 15;
-#pragma unroll
-    for (int i = 0; i < kMidSsLoads; ++i) {
-      const int p = sub + 16 * i;
-      ss_mine[i] = (token < M && p < fold.parts) ? fold.ss_in[(size_t)token * fold.parts + p] : 0.f;
-    }
-  }
+  float* parts_s = inv_s + 16;                        // FOLD: [M][parts]
+  if constexpr (FOLD) fetch_fold_parts<4>(fold.ss_in, M * fold.parts, parts_s, wave, lane);
 
   // ---- copying: a tile is 128 rows (of w: WROWS) of 8 16-byte chunks; thread t moves chunk t % 8 of rows
   // t / 8 + 32 i.  Row q of the w tile is feature n0 + q (GATED: the gate row of feature
@@ -159,6 +152,7 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
   const int last = nkt - 1;
 #pragma unroll
   for (int s = 0; s < D; ++s) XI_MID_ISSUE(s, s < last ? s : last);
+  if constexpr (FOLD) wait_all_but<D * (WR + XI)>();            // this wave's parts are in LDS (the first tile is waited for anyway)
 
   // One tile: registers of slot s to LDS, the slot loaded again D tiles ahead, barrier,
   // products.  One barrier a tile is enough: whoever writes this buffer again, two tiles on, has
@@ -205,14 +199,11 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
 #undef XI_MID_ISSUE
 
   if constexpr (FOLD) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < kMidSsLoads; ++i) t += ss_mine[i];
-    t += lane_xor<8>(t);
-    t += lane_xor<4>(t);
-    t += lane_xor<2>(t);
-    t += lane_xor<1>(t);
-    if ((tid & 15) == 0) inv_s[tid >> 4] = rsqrtf(t * fold.inv_h + fold.eps);
+    const int token = tid >> 4;
+    if (token < M) {
+      const float inv = fold_inverse<16>(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
+      if ((tid & 15) == 0) inv_s[token] = inv;
+    }
     __syncthreads();
   }
   if (!active) return;
@@ -374,8 +365,8 @@ int xi_linear_mid_gated(const void* x, const void* w, void* y, int M, int N, int
            K, kMidK);
   XI_CHECK(((uintptr_t)x | (uintptr_t)w) % 16 == 0, "linear_mid_gated: operands must be 16-byte aligned");
   XI_CHECK(rotate >= 0, "linear_mid_gated: rotate=%d", rotate);
-  XI_CHECK(ss == nullptr || (M <= 16 && parts >= 1 && parts <= 16 * kMidSsLoads),
-           "linear_mid_gated: a folded norm takes up to 16 rows and %d parts (M=%d, parts=%d)", 16 * kMidSsLoads, M, parts);
+  XI_CHECK(ss == nullptr || (M <= 16 && parts >= 1 && parts <= kMidParts),
+           "linear_mid_gated: a folded norm takes up to 16 rows and %d parts (M=%d, parts=%d)", kMidParts, M, parts);
   const int R = features > 0 ? features : xi_linear_mid_gated_features(N, M);     // features: an override, for measurements
   const long long wgs = (N + R - 1) / R;
   XI_CHECK(R >= 1 && R <= 128 && wgs < (1ll << 31), "linear_mid_gated: %d features per workgroup", R);
@@ -399,8 +390,10 @@ int xi_linear_mid_gated(const void* x, const void* w, void* y, int M, int N, int
 #define XI_MIDG(TJ, FULL, FOLD)                                                                               \
   do {                                                                                                        \
     static bool lds_set = false;                                                                              \
-    if (mid_lds(linear_mid_kernel<kMidDepth, TJ, FULL, true, FOLD>, &lds_set)) return 1;                      \
-    linear_mid_kernel<kMidDepth, TJ, FULL, true, FOLD><<<(unsigned)wgs, 256, kMidLdsBytes, stream>>>(         \
+    constexpr size_t most = kMidLdsBytes + (FOLD ? 16 * kMidParts * sizeof(float) : 0);                       \
+    const size_t lds = kMidLdsBytes + (FOLD ? fold_parts_room(M * parts) * sizeof(float) : 0);                \
+    if (mid_lds(linear_mid_kernel<kMidDepth, TJ, FULL, true, FOLD>, &lds_set, most)) return 1;                \
+    linear_mid_kernel<kMidDepth, TJ, FULL, true, FOLD><<<(unsigned)wgs, 256, lds, stream>>>(                  \
         (const bf16*)x, (const bf16*)w, y, M, N, K, 1, 0, R, rotate, fold);                                   \
   } while (0)
   if (ss != nullptr) XI_MIDG(1, false, true);

@@ -83,11 +83,13 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16* __re
   constexpr int kSsLoads = 16;   // 32 threads x 16 loads: up to 512 parts of a row's sum
   float ss_mine[kSsLoads];
   if constexpr (MODE == kFoldIn) {
+    // (waves without a row and steps past the parts are passed over as a whole: the first weights wait for what is issued here)
     const int token = threadIdx.x >> 5, sub = threadIdx.x & 31;
+    const float* row = fold.ss_in + (size_t)(token < M ? token : M - 1) * fold.parts;
+    if (2 * __builtin_amdgcn_readfirstlane(wave) < M) {
 #pragma unroll
-    for (int i = 0; i < kSsLoads; ++i) {
-      const int p = sub + 32 * i;
-      ss_mine[i] = (token < M && p < fold.parts) ? fold.ss_in[(size_t)token * fold.parts + p] : 0.f;
+      for (int i = 0; i < kSsLoads; ++i)
+        if (32 * i < fold.parts) ss_mine[i] = row[min(sub + 32 * i, fold.parts - 1)];
     }
   }
   // The workgroup owns output features n0 .. n0 + R - 1 (R <= 16 * PAIRS, any number: the grid
@@ -213,7 +215,8 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16* __re
   if constexpr (MODE == kFoldIn) {   // read after the barriers of the merge below
     float t = 0.f;
 #pragma unroll
-    for (int i = 0; i < kSsLoads; ++i) t += ss_mine[i];
+    for (int i = 0; i < kSsLoads; ++i)
+      if (32 * i < fold.parts) t += (int)(threadIdx.x & 31) + 32 * i < fold.parts ? ss_mine[i] : 0.f;
     t += lane_xor<16>(t);
     t += lane_xor<8>(t);
     t += lane_xor<4>(t);

@@ -22,6 +22,7 @@
 //
 // Reference call site: candle matmul in /root/reference/src/models/layers/linear.rs:76-124.
 #include "common.h"
+#include "fold_parts.h"
 
 namespace xi {
 
@@ -32,10 +33,11 @@ constexpr int kThinRows = 16;            // rows of x
 constexpr int kThinFeatures = 32;        // most rows of w in a workgroup's tile
 constexpr int kThinK = 256;              // k per tile of 32 rows of w (a tile of 16 rows takes 512: the same bytes)
 constexpr int kThinDepth = 2;            // tiles whose loads are in flight
-constexpr int kThinSsLoads = 32;         // 16 threads x 32 loads: up to 512 parts of a row's sum of squares
+constexpr int kThinParts = 512;          // most parts of a row's sum of squares
 constexpr size_t thin_lds_bytes(int tr) {     // two buffers of a w tile and an x tile, rows padded by 8 elements
   return 2 * (size_t)(tr + kThinRows) * (8192 / tr + 8) * sizeof(bf16);
 }
+constexpr size_t kThinLdsMost = thin_lds_bytes(16) + kThinRows * kThinParts * sizeof(float);     // and MODE 2's parts
 
 struct ThinFold {
   float* resid;         // MODE 1: [M, N] float32, updated in place
@@ -53,39 +55,45 @@ struct ThinFold {
 // two from M up that the copying takes (a workgroup reads all of x, as many bytes per row as of
 // a row of w, so rows that are not there cost as much as features); the product's rows past XR
 // repeat earlier ones and are dropped.
-template <int MODE, typename TO, int TR, int XR>
+// D: tiles whose loads are in flight; WHOLE: K has no more of them than that, and all are asked for at the start.  WR: rows of w that are
+// copied and held, 4 for workgroups of up to 4 features (the other rows of the products repeat them and are dropped): the load unit takes 64
+// bytes a clock, and 16 rows for 4 were 0.9 us of a product of 4 (N = 1024, K = 3072).
+template <int MODE, typename TO, int TR, int XR, int D = kThinDepth, bool WHOLE = false, int WR = TR>
 __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                           TO* __restrict__ y, int M, int N, int K, int R, int rotate,
                                                           ThinFold fold) {
-  constexpr int D = kThinDepth;
   constexpr int BK = 8192 / TR;              // k per tile
   constexpr int LROW = BK + 8;               // elements of a row in LDS
   constexpr int CPR = BK / 8;                // 16-byte chunks of a row
   constexpr int RPP = 256 / CPR;             // rows the 256 threads copy at once
-  constexpr int WP = TR / RPP, XP = XR / RPP;
-  static_assert(XR % RPP == 0 && XP >= 1, "rows of x in a tile");     // copies of a thread per tile of w, of x
+  constexpr int WP = WR / RPP, XP = XR / RPP;
+  static_assert(XR % RPP == 0 && XP >= 1 && WR % RPP == 0 && WP >= 1, "rows of x and w in a tile");     // copies of a thread per tile of w, of x
   constexpr int RT = TR / 16;                // 16-feature tiles
   constexpr int SPW = BK / 32 / 4;           // 32-wide k steps of a tile that a wave multiplies
-  constexpr int STAGE = (TR + XR) * LROW;         // elements of one buffer
+  constexpr int STAGE = (WR + XR) * LROW;         // elements of one buffer
   extern __shared__ __align__(16) unsigned char thin_smem[];
-  bf16* lds = reinterpret_cast<bf16*>(thin_smem);        // [buffer][w tile TR rows | x tile 16 rows][LROW]
+  bf16* lds = reinterpret_cast<bf16*>(thin_smem);        // [buffer][w tile WR rows | x tile XR rows][LROW], then MODE 2's parts [M][parts]
+  float* parts_s = reinterpret_cast<float*>(thin_smem + 2 * (size_t)STAGE * sizeof(bf16));
   __shared__ __align__(16) float red[4 * RT * 256];      // [wave][feature tile][lane * 4 + i]
   __shared__ float side[MODE == 1 ? kThinRows * TR : kThinRows];   // squares [row][feature], or 1/rms [row]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, j = lane >> 4;
   const int n0 = blockIdx.x * R;
   const int n_last = (n0 + R < N ? n0 + R : N) - 1;
   const int nkt = K / BK;
-  const int start = (int)(((long long)blockIdx.x * rotate) % nkt);
+  const int start = rotate ? (int)(((long long)blockIdx.x * rotate) % nkt) : 0;
 
-  // MODE 2: 16 threads per row add up the parts of its sum of squares; the loads start now
-  float ss_mine[MODE == 2 ? kThinSsLoads : 1];
-  if constexpr (MODE == 2) {
-    const int token = tid >> 4, sub = tid & 15;
+  if constexpr (MODE == 2) fetch_fold_parts<4>(fold.ss_in, M * fold.parts, parts_s, wave, lane);
+  // element `tid` of a tile of 16 features of the result: feature and row
+  const int e_token = (tid >> 2) & 15, e_f = 4 * (tid >> 6) + (tid & 3);
+  // MODE 1: what the result is added to and the norm's weight, asked for now (at the end they were 0.6 us)
+  float old[MODE == 1 ? RT : 1], norm_w[MODE == 1 ? RT : 1];
+  if constexpr (MODE == 1) {
 #pragma unroll
-    for (int i = 0; i < kThinSsLoads; ++i) {
-      const int p = sub + 16 * i;
-      ss_mine[i] = (token < M && p < fold.parts) ? fold.ss_in[(size_t)token * fold.parts + p] : 0.f;
+    for (int h = 0; h < RT; ++h) {
+      const int n = n0 + 16 * h + e_f < n_last ? n0 + 16 * h + e_f : n_last;
+      old[h] = fold.resid[(size_t)(e_token < M ? e_token : M - 1) * N + n];
+      norm_w[h] = fold.g[n];
     }
   }
 
@@ -127,23 +135,24 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
   const int last = nkt - 1;
 #pragma unroll
   for (int s = 0; s < D; ++s) XI_THIN_ISSUE(s, s < last ? s : last);
+  if constexpr (MODE == 2) wait_all_but<D * (WP + XP)>();       // this wave's parts are in LDS (the first tile is waited for anyway)
 
   int buf = 0;
 #define XI_THIN_TILE(s, t)                                                                                \
   do {                                                                                                    \
     bf16* Ws = lds + buf * STAGE;                                                                         \
-    bf16* Xs = Ws + TR * LROW;                                                                            \
+    bf16* Xs = Ws + WR * LROW;                                                                            \
     _Pragma("unroll") for (int i = 0; i < WP; ++i)                                                        \
       *reinterpret_cast<bf16x8*>(Ws + sdst + RPP * i * LROW) = wr[s][i];                                  \
     _Pragma("unroll") for (int i = 0; i < XP; ++i)                                                        \
       *reinterpret_cast<bf16x8*>(Xs + sdst + RPP * i * LROW) = xr[s][i];                                  \
-    XI_THIN_ISSUE(s, (t) + D < last ? (t) + D : last);                                                    \
+    if constexpr (!WHOLE) XI_THIN_ISSUE(s, (t) + D < last ? (t) + D : last);                              \
     __syncthreads();                                                                                      \
     _Pragma("unroll") for (int kk = 0; kk < SPW; ++kk) {                                                  \
       const int col = 32 * (SPW * wave + kk) + 8 * j;                                                     \
       const bf16x8 b = *reinterpret_cast<const bf16x8*>(Xs + (r & (XR - 1)) * LROW + col);                             \
       _Pragma("unroll") for (int t_ = 0; t_ < RT; ++t_) {                                                 \
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(Ws + (16 * t_ + r) * LROW + col);               \
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(Ws + ((16 * t_ + r) & (WR - 1)) * LROW + col);  \
         acc[t_] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t_], 0, 0, 0);                        \
       }                                                                                                   \
     }                                                                                                     \
@@ -168,21 +177,17 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
 #pragma unroll
   for (int t = 0; t < RT; ++t) *reinterpret_cast<f32x4*>(&red[(wave * RT + t) * 256 + lane * 4]) = acc[t];
   if constexpr (MODE == 2) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < kThinSsLoads; ++i) t += ss_mine[i];
-    t += lane_xor<8>(t);
-    t += lane_xor<4>(t);
-    t += lane_xor<2>(t);
-    t += lane_xor<1>(t);
-    if ((tid & 15) == 0) side[tid >> 4] = rsqrtf(t * fold.inv_h + fold.eps);
+    const int token = tid >> 4;
+    if (token < M) {
+      const float inv = fold_inverse<16>(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
+      if ((tid & 15) == 0) side[token] = inv;
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int h = 0; h < RT; ++h) {
     const int e = tid;                       // element of feature tile h
-    const int ln = e >> 2, v = e & 3;
-    const int token = ln & 15, f = 16 * h + 4 * (ln >> 4) + v;      // feature within the workgroup's tile
+    const int token = e_token, f = 16 * h + e_f;                    // feature within the workgroup's tile
     const int n = n0 + f;
     float a = 0.f;
 #pragma unroll
@@ -191,9 +196,9 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
     if constexpr (MODE == 1) {
       float sq = 0.f;
       if (mine) {
-        const float rr = fold.resid[(size_t)token * N + n] + a;
+        const float rr = old[h] + a;
         fold.resid[(size_t)token * N + n] = rr;
-        fold.xg[(size_t)token * N + n] = from_float<bf16>(rr * fold.g[n]);
+        fold.xg[(size_t)token * N + n] = from_float<bf16>(rr * norm_w[h]);
         sq = rr * rr;
       }
       side[token * TR + f] = sq;
@@ -251,30 +256,42 @@ static int thin_check(const char* what, const void* x, const void* w, int M, int
 // A tile of 16 rows of w where the workgroups own at most 16 features and K is a multiple of 512.
 static int thin_tile_rows(int R, int K) { return (R <= 16 && K % 512 == 0) ? 16 : 32; }
 
-#define XI_THIN_LAUNCH_(MODE, TO, TR, XR, yptr)                                                                      \
+#define XI_THIN_LAUNCH_(MODE, TO, TR, yptr, ...)                                                                     \
   do {                                                                                                          \
+    auto kern = linear_thin_kernel<MODE, TO, TR, __VA_ARGS__>;                                                  \
     static bool lds_set = false;                                                                                \
     if (!lds_set) {                                                                                             \
-      hipError_t e = hipFuncSetAttribute((const void*)linear_thin_kernel<MODE, TO, TR, XR>,                         \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)thin_lds_bytes(TR));  \
-      XI_CHECK(e == hipSuccess, "linear_thin: cannot get %zu bytes of LDS: %s", thin_lds_bytes(TR),             \
+      hipError_t e = hipFuncSetAttribute((const void*)kern,                                                     \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kThinLdsMost);        \
+      XI_CHECK(e == hipSuccess, "linear_thin: cannot get %zu bytes of LDS: %s", kThinLdsMost,                   \
                hipGetErrorString(e));                                                                           \
       lds_set = true;                                                                                           \
     }                                                                                                           \
-    linear_thin_kernel<MODE, TO, TR, XR><<<wgs, 256, thin_lds_bytes(TR), stream>>>(                             \
-        (const bf16*)x, (const bf16*)w, (TO*)(yptr), M, N, K, R, rotate, fold);                                 \
+    const size_t parts_lds = MODE == 2 ? fold_parts_room(M * fold.parts) * sizeof(float) : 0;                  \
+    kern<<<wgs, 256, thin_lds_bytes(TR) + parts_lds, stream>>>((const bf16*)x, (const bf16*)w, (TO*)(yptr), M, N, K, R, rotate, fold); \
+  } while (0)
+// tiles of 16 rows of w (512 k): up to six of them are asked for together
+#define XI_THIN_DEPTH(MODE, TO, yptr, XR)                                          \
+  do {                                                                             \
+    constexpr int kLow = MODE == 1 ? 4 : 16;                                       \
+    if (MODE == 1 && R <= 4) {                                                     \
+      if (K <= 2048) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true, kLow);       \
+      else if (K <= 3072) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 6, true, kLow);  \
+      else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, false, kLow);                \
+    } else if (K <= 1024) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, true);               \
+    else if (K <= 2048) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true);          \
+    else if (K <= 3072) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 6, true);          \
+    else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR);                                  \
   } while (0)
 // rows of x in a tile: 4 (tiles of 16 rows of w only: their copying takes 4 rows at once), 8 or 16
-#define XI_THIN_LAUNCH(MODE, TO, TR, yptr)                                    \
-  do {                                                                        \
-    if (M <= 4 && TR == 16) XI_THIN_LAUNCH_(MODE, TO, 16, 4, yptr);           \
-    else if (M <= 8) XI_THIN_LAUNCH_(MODE, TO, TR, 8, yptr);                  \
-    else XI_THIN_LAUNCH_(MODE, TO, TR, 16, yptr);                             \
-  } while (0)
-#define XI_THIN_TILE_ROWS(MODE, TO, yptr)                   \
-  do {                                                      \
-    if (thin_tile_rows(R, K) == 16) XI_THIN_LAUNCH(MODE, TO, 16, yptr); \
-    else XI_THIN_LAUNCH(MODE, TO, 32, yptr);                \
+#define XI_THIN_TILE_ROWS(MODE, TO, yptr)                                  \
+  do {                                                                     \
+    if (thin_tile_rows(R, K) == 16) {                                      \
+      if (M <= 4) XI_THIN_DEPTH(MODE, TO, yptr, 4);                        \
+      else if (M <= 8) XI_THIN_DEPTH(MODE, TO, yptr, 8);                   \
+      else XI_THIN_DEPTH(MODE, TO, yptr, 16);                              \
+    } else if (M <= 8) XI_THIN_LAUNCH_(MODE, TO, 32, yptr, 8);             \
+    else XI_THIN_LAUNCH_(MODE, TO, 32, yptr, 16);                          \
   } while (0)
 
 // y [M, N] bfloat16 (out_dtype 1) or float32 (0).
@@ -309,8 +326,8 @@ int xi_linear_thin_fold_out(const void* x, const void* w, int M, int N, int K, f
 int xi_linear_thin_fold_in(const void* x, const void* w, void* y, int M, int N, int K, int out_dtype, const float* ss,
                            int parts, float eps, int rotate, hipStream_t stream) {
   if (thin_check("linear_thin_fold_in", x, w, M, N, K)) return 1;
-  XI_CHECK(ss && parts >= 1 && parts <= 16 * kThinSsLoads && rotate >= 0, "linear_thin_fold_in: %d parts (1..%d)", parts,
-           16 * kThinSsLoads);
+  XI_CHECK(ss && parts >= 1 && parts <= kThinParts && rotate >= 0, "linear_thin_fold_in: %d parts (1..%d)", parts,
+           kThinParts);
   const int R = thin_features(N);
   const unsigned wgs = (unsigned)((N + R - 1) / R);
   const ThinFold fold{nullptr, nullptr, nullptr, nullptr, ss, parts, eps, 1.f / (float)K};
@@ -321,7 +338,7 @@ int xi_linear_thin_fold_in(const void* x, const void* w, void* y, int M, int N, 
   return 0;
 }
 #undef XI_THIN_TILE_ROWS
-#undef XI_THIN_LAUNCH
+#undef XI_THIN_DEPTH
 #undef XI_THIN_LAUNCH_
 
 }  // extern "C"
