@@ -308,3 +308,23 @@ def test_attention_tiles_are_one(nq, nkv, d):
         run(tile=most + 1)
     with pytest.raises(kernels.KernelError):
         run(lead=q.shape[0] + 1)
+
+
+@pytest.mark.parametrize("page,window,d,news", [(16, 0, 64, 5), (24, 0, 128, 3), (64, 9000, 128, 4), (40, 130, 32, 4), (16, 0, 144, 2)])
+def test_attention_past_a_waves_pages(page, window, d, news):
+    """Contexts around the 8,192 keys whose pages a wave asks for at once, with pages of whole blocks of 16 keys and others: tokens by
+    themselves and in tiles give the same bits, and those of the kernel for every size but for the sums' order."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(page + d)
+    lens, nq, nkv = [8192, 8207, 16500, 129], 4, 2
+    mp = -(-max(lens) // page)
+    kc, vc = (torch.randn(4 * mp, nkv, page, d, generator=g).to(DEV) for _ in range(2))
+    bt = torch.randperm(4 * mp, generator=g).to(torch.int32).view(4, mp).to(DEV)
+    q = torch.randn(4 * news, nq, d, generator=g).to(DEV)
+    seq = torch.arange(4, dtype=torch.int32).repeat_interleave(news).to(DEV)
+    pos = torch.tensor([n - news + i for n in lens for i in range(news)], dtype=torch.int32, device=DEV)
+    run = lambda **kw: kernels.attention_generic(q, kc, vc, bt, seq, pos, d ** -0.5, window, **kw).cpu()
+    one = run(tile=1)
+    assert float((one - run(matrix=False)).abs().max()) < 2e-5           # as in `test_attention`
+    assert torch.equal(run(tile=min(8, news + 1)), one)
+    assert torch.equal(run(tile=8, lead=1), one)

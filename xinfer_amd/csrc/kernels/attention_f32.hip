@@ -17,13 +17,15 @@
 //                    block), A = V: a lane brings dims 4 r .. 4 r + 3 of a key, element e belongs to
 //                    tile e, whose 16 rows are the dims 4 i + e of 64.
 //
-// A block's K is asked for a block ahead, its V before its scores are made: a wave would wait for the
-// page number, K and V one after the other.
+// A block's K is asked for a block ahead, its V before its scores are made: a wave would wait for the page number, K and V one after the
+// other.  The page numbers of a wave's next 64 blocks are one load, a lane a block (pages in whole blocks; others are looked up key by key);
+// heads of whole tiles (WHOLE) are a kernel without tests around their loads, behind which the compiler waits for more than it needs.
 //
-// Measured on MI355X, 32 heads of 128 on 8 kv heads, against one lane a key (us): prompts of 200, 127, 54,
-// 172 and 9 tokens 81 (396), a prompt of 1,024 245 (1,990; 32 kv heads 424, 2,220), 8 single tokens at up
-// to 330 keys 18 (54), one at 4,096 keys 125 (738).  Bound by the chain of a block (page, K, scores, sum,
-// V) in the few waves that a long head leaves room for; the matrix instructions are a third of it.
+// Measured on MI355X, 32 heads of 128 on 8 kv heads, against a page's number looked up for every block and tests around every load (us):
+// prompts of 200, 127, 54, 172 and 9 tokens 67.6 (79.4), a prompt of 1,024 208 (248), 8 single tokens at up to 330 keys 15.9 (17.3), one at
+// 4,096 keys 99 (125); 16 heads on 8, a prompt of 1,024, heads of 64 71 (113), a prompt of 512, heads of 256 118 (182).  One lane a key took 396,
+// 1,990, 54 and 738 for the first four.  Bound by the issue of the matrix and vector instructions of two waves a SIMD, of whose 16 columns a
+// decode step uses the heads of a kv head.
 //
 // A value that a token does not see never reaches it, not even with a weight of 0 (an infinite or
 // undefined one would): in a block that some token of the tile does not see in full, each token's
@@ -42,20 +44,22 @@ constexpr int kWaves = 8, kBlock = 16;
 // Bytes of LDS for `rows` (token, head) rows of heads of d and dv.
 constexpr size_t lds_bytes(int rows, int d, int dv) { return ((size_t)kWaves * (rows * dv + 2 * 16) + 16 * (d + 4)) * sizeof(float); }
 
-// DT: 16-dim tiles that the registers have room for (head sizes up to 16 DT)
-template <int DT>
+// DT: 16-dim tiles that the registers have room for (head sizes up to 16 DT); SINGLE: every workgroup has one token;
+// WHOLE: both head sizes are 16 DT
+template <int DT, bool SINGLE, bool WHOLE>
 __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_pages, const int* __restrict__ tok_seq, const int* __restrict__ positions,
-    float* __restrict__ out, float scale, int window, int page_size, int n_tok, int lead, int tile_tokens, int nq, int nkv, int d, int dv,
+    float* __restrict__ out, float scale, int window, int page_size, int n_tok, int lead, int tile_tokens, int nq, int nkv, int d_, int dv_,
     float softcap, const float* __restrict__ slopes, const float* __restrict__ sinks, int values_in_keys, int chunk) {
   constexpr int DG = (DT + 3) / 4;                  // groups of 64 value dims
+  const int d = WHOLE ? 16 * DT : d_, dv = WHOLE ? 16 * DT : dv_;
   extern __shared__ float lds[];                    // m and l [kWaves][16] each, then q [16][d + 4], then [kWaves][rows][dv]
   float *m_s = lds, *l_s = lds + kWaves * 16, *q_s = lds + 2 * kWaves * 16, *acc_s = q_s + 16 * (d + 4);
   const int group = nq / nkv, kvh = blockIdx.y, hb = blockIdx.z * 16;
   const int heads = group - hb < 16 ? group - hb : 16;
   const int bx = blockIdx.x, t0 = bx < lead ? bx : lead + (bx - lead) * tile_tokens;
-  const int t1 = bx < lead ? t0 + 1 : t0 + tile_tokens < n_tok ? t0 + tile_tokens : n_tok;
+  const int t1 = SINGLE || bx < lead ? t0 + 1 : t0 + tile_tokens < n_tok ? t0 + tile_tokens : n_tok;
   const int rows = (t1 - t0) * heads;               // row: token by token, its heads side by side
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, j = lane >> 4;
@@ -74,7 +78,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
   // the rows' queries; a row's 16-byte pieces lie in other banks than the next row's
   const float* qp = q + ((size_t)t * nq + h) * d + 4 * j;
   float* qr = q_s + r * (d + 4) + 4 * j;
-  for (int i = wave; i < nd; i += kWaves) *reinterpret_cast<f4*>(qr + 16 * i) = *reinterpret_cast<const f4*>(qp + 16 * i);
+  constexpr int kQ = (DT + kWaves - 1) / kWaves;
+  constexpr bool kHold = DT == 8;                   // (in registers from then on)
+  f4 qx[kQ], qh[kHold ? DT : 1];
+#pragma unroll
+  for (int i = 0; i < kQ; ++i)
+    if (wave + i * kWaves < nd) qx[i] = *reinterpret_cast<const f4*>(qp + 16 * (wave + i * kWaves));
   f4 o[DG][4];
 #pragma unroll
   for (int g = 0; g < DG; ++g)
@@ -83,13 +92,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
   const float slope = slopes ? slopes[h] : 0.f;
   const float inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
   float m = -INFINITY, l = 0.f;
-  __syncthreads();
+  const bool in_page = page_size % kBlock == 0;
 
   // a tile's tokens are of one request, but where two meet: then each request's are walked by themselves
   for (int ta = t0; ta < t1;) {
     const int seq = tok_seq[ta];
     int tb = ta, low = 0x7fffffff, lo_most = 0, pos_least = 0x7fffffff, high = 0;      // the first key that any, that every
-    for (; tb < t1 && tok_seq[tb] == seq; ++tb) {                                      // token sees, and the last ones
+    for (; tb < t1 && (SINGLE || tok_seq[tb] == seq); ++tb) {                          // token sees, and the last ones
       const int p = positions[tb], f = first_seen(p);
       low = min(low, f);
       lo_most = max(lo_most, f);
@@ -99,20 +108,30 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
     const bool one = ta == t0 && tb == t1, own = t >= ta && t < tb;
     const int* bt = block_tables + (size_t)seq * max_pages;
     const int last = high / kBlock;
-    int b = low / kBlock + ((wave - low / kBlock) & (kWaves - 1));
-    // the row of the lane's key of block bb in either pool
-    auto row_of = [&](int bb) {
-      const int key = bb * kBlock + (lane & (kBlock - 1));
-      const int seen = key < low ? low : key > high ? high : key;
+    const int b0 = low / kBlock + ((wave - low / kBlock) & (kWaves - 1));
+    // Pages in whole blocks: lane i keeps what is added to a key of the wave's block b0 + kWaves (64 n + i) to give its row, so that 64
+    // blocks' pages are one trip to memory.
+    int place = 0;
+    auto ask_pages = [&](int from) {
+      const int bb = from + kWaves * lane < last ? from + kWaves * lane : last, page = bb * kBlock / page_size;
+      place = (bt[page] * nkv + kvh - page) * page_size;
+    };
+    // the row in either pool of the lane's key of block b, or of the nearest one from `from` to `to`
+    auto row_of = [&](int b, int at, int from, int to) {           // (at: what belongs to block b's page)
+      const int key = b * kBlock + (lane & (kBlock - 1));
+      const int seen = key < from ? from : key > to ? to : key;
+      if (in_page) return at + seen;
       return (bt[seen / page_size] * nkv + kvh) * page_size + seen % page_size;
     };
     constexpr bool kEarly = DT <= 8;                // (larger heads: no registers for V ahead of its use)
-    f4 ka[DT], va[kEarly ? 4 : 1][DG];
-    auto ask_k = [&](int row) {
+    constexpr int kSlots = SINGLE && kEarly ? 2 : 1;               // blocks whose operands have registers
+    f4 ka[kSlots][DT], va[kSlots][kEarly ? 4 : 1][DG];
+    int row[kSlots], at[kSlots], row_next = 0, at_next = 0;
+    auto ask_k = [&](int row, f4 (&to)[DT]) {
       const float* kp = k_cache + (size_t)__shfl(row, r, kWave) * d + 4 * j;
 #pragma unroll
       for (int i = 0; i < DT; ++i)
-        if (i < nd) ka[i] = *reinterpret_cast<const f4*>(kp + 16 * i);
+        if (i < nd) to[i] = *reinterpret_cast<const f4*>(kp + 16 * i);
     };
     auto ask_v = [&](int row, int v, f4 (&to)[DG]) {
       const float* vp = vbase + (size_t)__shfl(row, 4 * j + v, kWave) * vd + 4 * r;
@@ -120,27 +139,42 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
       for (int g = 0; g < DG; ++g)
         if (64 * g < dv) to[g] = 64 * g + 4 * r < dv ? *reinterpret_cast<const f4*>(vp + 64 * g) : f4{0.f, 0.f, 0.f, 0.f};
     };
-    int row = b <= last ? row_of(b) : 0, row_next = 0;
-    if (b <= last) ask_k(row);
-    for (; b <= last; b += kWaves) {
-      const bool full = b * kBlock >= lo_most && b * kBlock + kBlock - 1 <= pos_least, whole = one && full;
-      const bool more = b + kWaves <= last;
-      if (more) row_next = row_of(b + kWaves);
-      if (kEarly && whole) {
+    auto full = [&](int b) { return b * kBlock >= lo_most && b * kBlock + kBlock - 1 <= pos_least; };
+    // (a token by itself: what it does not see of a block reads its nearest key already)
+    auto whole = [&](int b) { return SINGLE || (one && full(b)); };
+    auto ask_vs = [&](int b, int slot) {
+      if (kEarly && whole(b)) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) ask_v(row, v, va[kEarly ? v : 0]);
+        for (int v = 0; v < 4; ++v) ask_v(row[slot], v, va[slot][kEarly ? v : 0]);
+      }
+    };
+    // Block b, the wave's n-th: its K (two slots: and V) is in the slot or on its way there; the slot's next block is asked for.
+    auto next_row = [&](int b, int n) {
+      if (in_page && ((n + kSlots) & 63) == 0) ask_pages(b + kSlots * kWaves);
+      at_next = __builtin_amdgcn_readlane(place, (n + kSlots) & 63);
+      return row_of(b + kSlots * kWaves, at_next, low, high);
+    };
+    auto block = [&](int b, int n, auto slot_c) {
+      constexpr int slot = decltype(slot_c)::value;
+      const bool more = b + kSlots * kWaves <= last;
+      if (kSlots == 1) {
+        if (more) row_next = next_row(b, n);
+        ask_vs(b, slot);
       }
       __builtin_amdgcn_sched_barrier(0);
       f4 s = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < DT; ++i)
         if (i < nd) {
-          const f4 qv = *reinterpret_cast<const f4*>(qr + 16 * i);
+          const f4 qv = kHold ? qh[kHold ? i : 0] : *reinterpret_cast<const f4*>(qr + 16 * i);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i][e], qv[e], s, 0, 0, 0);
+          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[slot][i][e], qv[e], s, 0, 0, 0);
         }
       __builtin_amdgcn_sched_barrier(0);
-      if (more) ask_k(row_next);
+      if (more) {
+        if (kSlots > 1) row_next = next_row(b, n);
+        ask_k(row_next, ka[slot]);
+      }
       __builtin_amdgcn_sched_barrier(0);
       float most = -INFINITY;
       bool sees[4];
@@ -174,25 +208,23 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
       for (int g = 0; g < DG; ++g)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[g][e] *= corr;
-      if (whole) {
+      if (whole(b)) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          if (!kEarly) ask_v(row, v, va[0]);
+          if (!kEarly) ask_v(row[slot], v, va[slot][0]);
 #pragma unroll
           for (int g = 0; g < DG; ++g)
             if (64 * g < dv) {
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[kEarly ? v : 0][g][e], s[v], o[g][e], 0, 0, 0);
+              for (int e = 0; e < 4; ++e) o[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[slot][kEarly ? v : 0][g][e], s[v], o[g][e], 0, 0, 0);
             }
         }
       } else {
-        const int per = full ? tb - ta : 1;
+        const int per = full(b) ? tb - ta : 1;
         for (int x = ta; x < tb; x += per) {     // (beside another request's tokens: one product for all of this one's)
           const int px = positions[x], lx = first_seen(px);
           if ((b + 1) * kBlock <= lx || b * kBlock > px) continue;
-          const int key = b * kBlock + (lane & (kBlock - 1));
-          const int seen = key < lx ? lx : key > px ? px : key;
-          const int rx = (bt[seen / page_size] * nkv + kvh) * page_size + seen % page_size;
+          const int rx = row_of(b, at[slot], lx, px);
           f4 ox[DG][4];
 #pragma unroll
           for (int g = 0; g < DG; ++g)
@@ -200,12 +232,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
             for (int e = 0; e < 4; ++e) ox[g][e] = o[g][e];
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            ask_v(rx, v, va[kEarly ? v : 0]);
+            ask_v(rx, v, va[slot][kEarly ? v : 0]);
 #pragma unroll
             for (int g = 0; g < DG; ++g)
               if (64 * g < dv) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ox[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[kEarly ? v : 0][g][e], s[v], ox[g][e], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) ox[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[slot][kEarly ? v : 0][g][e], s[v], ox[g][e], 0, 0, 0);
               }
           }
 #pragma unroll
@@ -214,7 +246,33 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
             for (int e = 0; e < 4; ++e) o[g][e] = (unsigned)(t - x) < (unsigned)per ? ox[g][e] : o[g][e];
         }
       }
-      row = row_next;
+      row[slot] = row_next;
+      at[slot] = at_next;
+      if (kSlots > 1 && more) ask_vs(b + kSlots * kWaves, slot);
+    };
+    if (in_page) ask_pages(b0);
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+      if (b0 + s * kWaves <= last) {
+        at[s] = __builtin_amdgcn_readlane(place, s);
+        row[s] = row_of(b0 + s * kWaves, at[s], low, high);
+        ask_k(row[s], ka[s]);
+        if (kSlots > 1) ask_vs(b0 + s * kWaves, s);
+      }
+    if (ta == t0) {                // (asked for above, wanted now)
+#pragma unroll
+      for (int i = 0; i < kQ; ++i)
+        if (wave + i * kWaves < nd) *reinterpret_cast<f4*>(qr + 16 * (wave + i * kWaves)) = qx[i];
+      __syncthreads();
+      if constexpr (kHold)
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+          if (i < nd) qh[i] = *reinterpret_cast<const f4*>(qr + 16 * i);
+    }
+    for (int n = 0, b = b0; b <= last; n += kSlots, b += kSlots * kWaves) {
+      block(b, n, std::integral_constant<int, 0>{});
+      if constexpr (kSlots > 1)
+        if (b + kWaves <= last) block(b + kWaves, n + 1, std::integral_constant<int, kSlots - 1>{});
     }
     ta = tb;
   }
@@ -306,16 +364,27 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
   if (tile == 0) tile = xi_attention_f32_tile((int)rest, n_seqs - lead, nq, nkv);
   dim3 grid((unsigned)(lead + (rest + tile - 1) / tile), (unsigned)nkv, (unsigned)((nq / nkv + 15) / 16));
   XI_CHECK(grid.z <= 65535u, "attention_f32: too many heads (%d)", nq);
+  // Single tokens with their operands two blocks ahead where half of the compute units are idle: 64 and 128 workgroups of up to 400 keys 15.9 | 18.5
+  // us, 17.3 | 19.4 one block ahead; at 256 memory is what they wait for (23.3 | 22.7) and at 512 the kernel of the tiles is ahead, 40.3 | 44.4.
+  const bool single = (rest == 0 || tile == 1) && (long long)grid.x * grid.y * grid.z <= 128;
   const size_t lds = attn_f32::lds_bytes(tile * heads, d, dv);
   const int most = d > dv ? d : dv;
 #define XI_AF(DT)                                                                                                             \
   do {                                                                                                                        \
+    const bool whole = d == 16 * DT && dv == d;                                                                               \
+    if (single && whole) XI_AF1(DT, true, true);                                                                              \
+    else if (single) XI_AF1(DT, true, false);                                                                                 \
+    else if (whole) XI_AF1(DT, false, true);                                                                                  \
+    else XI_AF1(DT, false, false);                                                                                            \
+  } while (0)
+#define XI_AF1(DT, SINGLE, WHOLE)                                                                                                    \
+  do {                                                                                                                        \
     if (lds > 65536) {     /* always the most this kernel may want: another thread's launch may lie between */                \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32::attention_f32_kernel<DT>),              \
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32::attention_f32_kernel<DT, SINGLE, WHOLE>),              \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, xi_attention_f32_lds(d, dv));      \
       XI_CHECK(e == hipSuccess, "attention_f32: %s", hipGetErrorString(e));                                                   \
     }                                                                                                                         \
-    attn_f32::attention_f32_kernel<DT><<<grid, 64 * attn_f32::kWaves, lds, stream>>>(                                         \
+    attn_f32::attention_f32_kernel<DT, SINGLE, WHOLE><<<grid, 64 * attn_f32::kWaves, lds, stream>>>(                                         \
         q, k_cache, v_cache, block_tables, max_pages, tok_seq, positions, out, scale, window, page_size, n_tok, lead, tile, nq, nkv, d, dv, softcap, \
         slopes, sinks, values_in_keys, chunk);                                                                                \
   } while (0)
@@ -323,6 +392,7 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
   else if (most <= 128) XI_AF(8);
   else XI_AF(16);
 #undef XI_AF
+#undef XI_AF1
   XI_LAUNCH_CHECK("attention_f32");
   return 0;
 }
