@@ -168,6 +168,35 @@ def test_many_rows_of_few_features(M, N, K):
     assert torch.equal(kernels.gemm_tn(x[-50:], w), y[-50:])
 
 
+# I: one tile, one feature past four, walks of one to three tiles with short last ones; K: no multiple of 4, chunks that end inside a step
+@pytest.mark.parametrize("I,K", [(40, 4100), (17, 130), (1000, 96), (3072, 1024), (4090, 257), (8190, 64), (12288, 72)])
+@pytest.mark.parametrize("M", [1, 7, 16])
+def test_gated_product_is_the_two_kernels(M, I, K):
+    """Gate, up and silu(gate) * up in one pass: the bits of the product and the activation behind it, operands without a bound among them."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(M + I + K)
+    x, w = torch.randn(M, K, generator=g).to(DEV), (torch.randn(2 * I, K, generator=g) * 2 * K ** -0.5).to(DEV)
+    assert kernels.gemm_gated_rows(I, K) >= M
+    assert torch.equal(kernels.gemm_gated(x, w), kernels.silu_mul(kernels.gemm_tn(x, w)))
+    flat = torch.zeros(M * K + 1, device=DEV)          # x not on 16 bytes
+    flat[1:] = x.reshape(-1)
+    assert torch.equal(kernels.gemm_gated(flat[1:].view(M, K), w), kernels.silu_mul(kernels.gemm_tn(x, w)))
+    w[I - 1, 0], w[2 * I - 1, 1], w[I, K - 1] = float("inf"), float("nan"), 3.4e38
+    x[M - 1, 2] = float("-inf")
+    got, want = kernels.gemm_gated(x, w), kernels.silu_mul(kernels.gemm_tn(x, w))
+    assert torch.equal(got.nan_to_num(1.5, 2.5, 3.5), want.nan_to_num(1.5, 2.5, 3.5)) and torch.equal(got.isnan(), want.isnan())
+
+
+def test_gated_product_refused():
+    """More rows than go in the kernel for few rows, and outputs with an empty last round of workgroups: the two kernels."""
+    from xinfer_amd import kernels
+    assert kernels.gemm_gated_rows(17408, 5120) == 0 and kernels.gemm_gated_rows(0, 64) == 0
+    with pytest.raises(kernels.KernelError):
+        kernels.gemm_gated(torch.zeros(17, 64, device=DEV), torch.zeros(64, 64, device=DEV))
+    with pytest.raises(kernels.KernelError):
+        kernels.gemm_gated(torch.zeros(4, 64, device=DEV), torch.zeros(65, 64, device=DEV))
+
+
 def test_product_form_refused():
     from xinfer_amd import kernels
     x, w = torch.zeros(65, 32, device=DEV), torch.zeros(8, 32, device=DEV)

@@ -1185,6 +1185,27 @@ def gemm_tn(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def gemm_gated_rows(I: int, K: int) -> int:
+    """Most rows that `gemm_gated` takes for I features (w is [2 I, K]); 0: none."""
+    return int(lib().xi_gemm_gated_f32_rows(int(I), int(K)))
+
+
+def gemm_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate.T) * (x @ up.T) in float32 in one pass over w = [gate; up] [2 I, K], for up to `gemm_gated_rows` rows: the bits of
+    `silu_mul(gemm_tn(x, w))`."""
+    _dev(x, w)
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or w.shape[0] % 2:
+        raise KernelError(f"gemm_gated: x {tuple(x.shape)} and w {tuple(w.shape)} do not match")
+    if x.dtype != torch.float32 or w.dtype != torch.float32:
+        raise KernelError(f"gemm_gated: x is {x.dtype} and w {w.dtype}, not float32")
+    M, K = x.shape
+    I = w.shape[0] // 2
+    out = torch.empty((M, I), dtype=torch.float32, device=x.device)
+    _ok(lib().xi_gemm_gated_f32(_p(x), _p(w), _p(out), M, I, K, _stream()))
+    return out
+
+
 DECODE_WORKGROUPS = 512             # workgroups of the split-K decode kernel a launch of mixed lengths aims at: two a compute unit
 DECODE_KEYS_LEAST = 128             # keys of a workgroup: from one 32-key step a wave
 DECODE_KEYS_MOST = 512              # to four, in batches of mixed lengths

@@ -68,6 +68,9 @@ class Linear:
             if (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                     and 0 < x.shape[0] <= kernels.SKINNY_GATED_ROWS and x.shape[1] % 8 == 0):
                 return kernels.linear_skinny(x, w, gated=True)        # the same with the streaming kernel
+            if (x.dtype == torch.float32 and w.dtype == torch.float32 and out_dtype in (None, torch.float32) and x.dim() == 2
+                    and 0 < x.shape[0] <= kernels.gemm_gated_rows(w.shape[0] // 2, w.shape[1])):
+                return kernels.gemm_gated(x, w)                       # the same in float32
             return None
         if (sink is not None and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
                 and 0 < x.shape[0] <= kernels.FOLD_ROWS and x.shape[1] % 8 == 0 and w.shape[0] % 8 == 0
