@@ -712,6 +712,36 @@ def test_qk_norm_rope_kv_many_tokens(nq, nkv, d, rot, interleaved):
     assert torch.equal(got_v, want_v)
 
 
+@pytest.mark.parametrize("d", [16, 24, 96, 128, 160, 256])
+@pytest.mark.parametrize("first", [0, 3])
+@pytest.mark.parametrize("normed", [True, False])
+def test_qk_norm_rope_kv_whole_heads(d, first, normed):
+    """Whole-rotated heads in halves, with blocks of 8 to 64 tokens and groups of eight keys that are full and that are not: as the
+    form of one wave per head, q and k but for the order of a head's sum of squares, v as it is."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d + first)
+    T, page, nq, nkv = 203, 16, 3, 2
+    cos, sin = plain.rope_tables(1e6, d, 256)
+    qkv = _rand((T, (nq + 2 * nkv) * d), torch.bfloat16, g)
+    qw, kw = (1 + 0.2 * torch.randn(d, generator=g) if normed else None for _ in range(2))
+    slots = (torch.arange(T) + first).to(torch.int64)
+    slots[torch.tensor([17, 90])] = -1
+    dev = lambda t: None if t is None else t.to(DEV)
+    both = []
+    for least in (1, 1000):
+        kc = torch.zeros((14, nkv, page, d), dtype=torch.bfloat16, device=DEV)
+        vt = torch.zeros((14, nkv, page // 8, d, 8), dtype=torch.bfloat16, device=DEV)
+        q = kernels.qk_norm_rope_kv(dev(qkv), dev(qw), dev(kw), 1e-6, dev(cos), dev(sin), d, False, torch.arange(T, dtype=torch.int32, device=DEV),
+                                    dev(slots), kc, vt, nq, nkv, d, v_grouped=True, vector_min_tokens=least)
+        both.append((q.cpu().float(), kc.cpu().float(), vt.cpu()))
+    (q1, k1, v1), (q0, k0, v0) = both
+    assert torch.equal(v1, v0)
+    # float32 up to the one rounding to bfloat16: apart by a last place of it where the float32 values fall on two sides of a tie
+    for a, b in ((q1, q0), (k1, k0)):
+        assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-6).all())
+        assert float((a != b).float().mean()) < 0.01
+
+
 @pytest.mark.parametrize("dtype,T,nq,nkv,d,rot,interleaved", [
     (torch.float32, 11, 3, 1, 48, 48, False), (torch.bfloat16, 11, 4, 2, 32, 16, True),
     (torch.bfloat16, 150, 5, 5, 48, 48, False), (torch.bfloat16, 150, 2, 1, 128, 64, True)])

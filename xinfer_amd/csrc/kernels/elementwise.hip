@@ -304,17 +304,22 @@ __global__ void qk_norm_rope_kv_kernel(const void* __restrict__ qkv_v, int slice
 // workgroup owns one head of the packed row for a block of consecutive tokens.  A head of a
 // token is d/8 lanes of 8 elements (sums and the rotary partner are exchanged inside that
 // group of lanes), a wave holds 64/(d/8) tokens, the workgroup's waves hold the block.  The
-// workgroup of a V head turns its [tokens, d] tile through LDS so that a wave's store takes eight
-// tokens by eight dims: where the eight tokens follow each other in a group of the pool, one line
-// of 128 bytes.  Value heads may have a size of their own, dv.
+// workgroup of a V head turns its [tokens, d] tile through LDS so that where eight tokens follow each other
+// in a group of the pool a lane stores their 16 bytes of a dim.  Value heads may have a size of their own, dv.
+// Measured, us (bytes moved at): 2,048 tokens of 32 + 16 heads of 128 under 13.4 (3.7 TB/s and more), 16.2 where a lane held eight elements side by
+// side, whose partners' came from other lanes, V went two bytes at a time and workgroups had 64 tokens; 64 + 16 heads 22.1 (28.0).  Bound by
+// vector instructions (conversions, norm, rotation) and the pass's few trips to memory; asking for all of a head at once without the pairs was
+// slower (18.1: the tables' rows are read twice).
 // Rows may be longer than their heads (`width`), the values' first column is `v_col` (behind the keys, or the keys' own: the
 // values are then the keys as projected), and with `vcos` / `vsin` (float32 [positions, dv / 2]; dv % 16 == 0) value heads turn
 // by their position in pairs (i, i + dv / 2).
 // Needs d % 8 == 0, dv % 8 == 0 and, for the half layout, rotary_dim % 16 == 0 (the partner of a lane's
 // 8 elements is then another lane's 8 elements).
 struct alignas(16) bf16x8v { bf16 v[8]; };
+struct alignas(8) bf16x4v { bf16 v[4]; };
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f4_any;       // (from any float on)
 
-__global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
+__global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
     const bf16* __restrict__ qkv, const float* __restrict__ bias, const float* __restrict__ qw, const float* __restrict__ kw, float eps,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, int rot, int interleaved,
     const int* __restrict__ positions, const long long* __restrict__ slots, bf16* __restrict__ q_out,
@@ -326,7 +331,7 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
   const int hpw = 64 / lph;        // tokens a wave holds
   const int tpw = (blockDim.x >> 6) * hpw;   // tokens of the workgroup (at most 64)
   const int sub = lane / lph, c = lane - sub * lph;
-  const int h = blockIdx.y;
+  const int h = gridDim.y - 1 - blockIdx.y;           // (the values, which take longest, first)
   const int t0 = blockIdx.x * tpw;
   const int tl = wave * hpw + sub;  // this lane's token within the block
   const int t = t0 + tl;
@@ -337,16 +342,10 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
     const int kvh = h - nq - nkv;
     bf16* vs = reinterpret_cast<bf16*>(smem_raw);  // [tpw][dv + 2]
     const int vstride = dv + 2;                      // an odd number of 32-bit words per row
-    // Every lane looks up where its own token of the block goes (lane = token); a store then takes eight
-    // tokens by eight dims: lane -> token 8 tg + (lane & 7), dim i0 + (lane >> 3), the place handed over
-    // from the token's lane.
+    // Every lane looks up where its own token of the block goes (lane = token).  Eight tokens that fill a group of the pool go as 16 bytes a
+    // dim, others two bytes at a time.
+    unsigned long long* place_s = reinterpret_cast<unsigned long long*>(vs + (((size_t)tpw * vstride + 3) & ~(size_t)3));
     const long long slot = (lane < tpw && t0 + lane < n_tok) ? slots[t0 + lane] : -1;
-    unsigned long long place = ~0ull;          // of the token's dim 0 in the pool, in elements
-    if (slot >= 0) {
-      const long long page = slot / page_size;
-      const int off = (int)(slot - page * page_size);
-      place = ((unsigned long long)page * nkv + kvh) * dv * page_size + (unsigned long long)(off >> 3) * dv * 8 + (off & 7);
-    }
     const size_t col0 = (size_t)v_col + (size_t)kvh * dv;
     const int vhalf = dv >> 1;
     for (int u = tid; u < tpw * (dv >> 3); u += (int)blockDim.x) {
@@ -386,24 +385,138 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
       dst[2] = raw.z;
       dst[3] = raw.w;
     }
+    unsigned long long place = ~0ull;          // of the token's dim 0 in the pool, in elements
+    if (slot >= 0) {
+      const long long page = slot / page_size;
+      const int off = (int)(slot - page * page_size);
+      place = ((unsigned long long)page * nkv + kvh) * dv * page_size + (unsigned long long)(off >> 3) * dv * 8 + (off & 7);
+    }
+    const unsigned lo = __shfl((unsigned)place, lane & ~7, kWave), hi = __shfl((unsigned)(place >> 32), lane & ~7, kWave);
+    const unsigned long long first = ((unsigned long long)hi << 32) | lo;
+    const unsigned long long follows = __ballot(slot >= 0 && (first & 7) == 0 && place == first + (lane & 7) && ((uintptr_t)vt_cache & 15) == 0);
+    if (wave == 0 && lane < tpw) place_s[lane] = place;
     __syncthreads();
-    const int units = ((tpw + 7) >> 3) * (dv >> 3);
-    for (int u = wave; u < units; u += (int)(blockDim.x >> 6)) {
-      const int tg = u / (dv >> 3), i = 8 * (u - tg * (dv >> 3)) + (lane >> 3);
-      const int tok = 8 * tg + (lane & 7);
-      const unsigned lo = __shfl((unsigned)place, tok, kWave), hi = __shfl((unsigned)(place >> 32), tok, kWave);
-      const unsigned long long at = ((unsigned long long)hi << 32) | lo;
-      if (at != ~0ull) vt_cache[at + (size_t)i * 8] = vs[tok * vstride + i];
+    const int units = ((tpw + 7) >> 3) * dv;
+    for (int u = tid; u < units; u += (int)blockDim.x) {
+      const int tg = u / dv, i = u - tg * dv;
+      const bf16* from = vs + 8 * tg * vstride + i;
+      if (((follows >> (8 * tg)) & 0xff) == 0xff) {
+        bf16x8v y;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y.v[e] = from[e * vstride];
+        *reinterpret_cast<bf16x8v*>(vt_cache + place_s[8 * tg] + (size_t)i * 8) = y;
+      } else {
+        for (int e = 0; e < 8 && 8 * tg + e < tpw; ++e) {
+          const unsigned long long at = place_s[8 * tg + e];
+          if (at != ~0ull) vt_cache[at + (size_t)i * 8] = from[e * vstride];
+        }
+      }
     }
     return;
   }
 
   // ---- a query head or a k head
+  // ---- a whole-rotated head in halves: a lane holds four elements of either half, pairs that turn together, so that nothing is handed over
+  // between lanes and a pair's angle is read once
+  if (!interleaved && rot == d) {
+    const bool is_k = h >= nq;
+    const float* w = is_k ? kw : qw;
+    const int half = d >> 1, tc = t < n_tok ? t : n_tok - 1, cl = sub < hpw ? c : 0;
+    const bf16* from = qkv + (size_t)tc * width + (size_t)h * d + 4 * cl;
+    const bf16x4v xa = *reinterpret_cast<const bf16x4v*>(from), xb = *reinterpret_cast<const bf16x4v*>(from + half);
+    const int pos = positions[tc];
+    const long long slot = is_k ? slots[tc] : 0;
+    f4_any wa = {1.f, 1.f, 1.f, 1.f}, wb = wa;
+    if (w) {
+      wa = *reinterpret_cast<const f4_any*>(w + 4 * cl);
+      wb = *reinterpret_cast<const f4_any*>(w + half + 4 * cl);
+    }
+    const f4_any cs = *reinterpret_cast<const f4_any*>(cos_t + (size_t)pos * half + 4 * cl);
+    const f4_any sn = *reinterpret_cast<const f4_any*>(sin_t + (size_t)pos * half + 4 * cl);
+    float va[4], vb[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      va[e] = to_float(xa.v[e]);
+      vb[e] = to_float(xb.v[e]);
+      if (bias) {
+        va[e] += bias[(size_t)h * d + 4 * cl + e];
+        vb[e] += bias[(size_t)h * d + half + 4 * cl + e];
+      }
+    }
+    if (w) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += va[e] * va[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += vb[e] * vb[e];
+      float total;
+      if ((lph & (lph - 1)) == 0) {
+        total = ss;
+        if (lph > 1) total += lane_xor<1>(total);
+        if (lph > 2) total += lane_xor<2>(total);
+        if (lph > 4) total += lane_xor<4>(total);
+        if (lph > 8) total += lane_xor<8>(total);
+        if (lph > 16) total += lane_xor<16>(total);
+        if (lph > 32) total += lane_xor<32>(total);
+      } else {
+        total = 0.f;
+        const int begin = lane - c;
+        for (int o = 0; o < lph; ++o) total += __shfl(ss, begin + o, kWave);
+      }
+      const float inv = rsqrtf(total / (float)d + eps);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        va[e] = va[e] * inv * wa[e];
+        vb[e] = vb[e] * inv * wb[e];
+      }
+    }
+    if (!on) return;
+    bf16x4v ya, yb;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      ya.v[e] = from_float<bf16>(va[e] * cs[e] - vb[e] * sn[e]);
+      yb.v[e] = from_float<bf16>(va[e] * sn[e] + vb[e] * cs[e]);
+    }
+    bf16* to = q_out + ((size_t)t * nq + h) * d;
+    if (is_k) {
+      if (slot < 0) return;
+      const long long page = slot / page_size;
+      const int off = (int)(slot - page * page_size);
+      to = k_cache + (((size_t)page * nkv + (h - nq)) * page_size + off) * d;
+    }
+    *reinterpret_cast<bf16x4v*>(to + 4 * c) = ya;
+    *reinterpret_cast<bf16x4v*>(to + half + 4 * c) = yb;
+    return;
+  }
   const bool is_k = h >= nq;
+  const int half = rot >> 1;
+  const int pos = positions[t < n_tok ? t : n_tok - 1];
+  const long long slot = is_k ? slots[t < n_tok ? t : n_tok - 1] : 0;
+  const float* w = is_k ? kw : qw;
+  bf16x8v x;
+  if (on) x = *reinterpret_cast<const bf16x8v*>(qkv + (size_t)t * width + (size_t)h * d + 8 * c);
+  const int cl = sub < hpw ? c : 0;             // (lanes behind the last head read its numbers and keep none)
+  f4_any w0 = {1.f, 1.f, 1.f, 1.f}, w1 = w0;
+  if (w) {
+    w0 = *reinterpret_cast<const f4_any*>(w + 8 * cl);
+    w1 = *reinterpret_cast<const f4_any*>(w + 8 * cl + 4);
+  }
+  const bool in_rot = 8 * cl < rot;
+  const bool first = 8 * cl < half;
+  float4 c0 = float4{1.f, 1.f, 1.f, 1.f}, c1 = c0, s0 = float4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+  if (in_rot && (!interleaved || rot % 8 == 0)) {
+    const int p0 = interleaved ? 4 * cl : first ? 8 * cl : 8 * cl - half;   // pair index of this lane's first element
+    const float4* cp = reinterpret_cast<const float4*>(cos_t + (size_t)pos * half + p0);
+    const float4* sp = reinterpret_cast<const float4*>(sin_t + (size_t)pos * half + p0);
+    c0 = cp[0];
+    s0 = sp[0];
+    if (!interleaved) {
+      c1 = cp[1];
+      s1 = sp[1];
+    }
+  }
   float v[8];
   {
-    bf16x8v x;
-    if (on) x = *reinterpret_cast<const bf16x8v*>(qkv + (size_t)t * width + (size_t)h * d + 8 * c);
     float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (bias) {
       const float4* bp = reinterpret_cast<const float4*>(bias + (size_t)h * d + 8 * c);
@@ -413,7 +526,6 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = on ? to_float(x.v[e]) + bv[e] : 0.f;
   }
-  const float* w = is_k ? kw : qw;
   if (w) {
     float ss = 0.f;
 #pragma unroll
@@ -431,20 +543,12 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       v[e] *= inv;
-      v[e] *= w[8 * c + e];
+      v[e] *= e < 4 ? w0[e & 3] : w1[e & 3];
     }
   }
-  const int half = rot >> 1;
-  const int pos = positions[t < n_tok ? t : n_tok - 1];
   float o[8];
   if (interleaved && rot % 8 == 0) {       // a lane's 8 elements turn together or not at all: its 4 pairs' angles in two loads
-    const bool in_rot = 8 * c < rot;
-    float4 cs = float4{1.f, 1.f, 1.f, 1.f}, sn = float4{0.f, 0.f, 0.f, 0.f};
-    if (in_rot) {
-      cs = *reinterpret_cast<const float4*>(cos_t + (size_t)pos * half + 4 * c);
-      sn = *reinterpret_cast<const float4*>(sin_t + (size_t)pos * half + 4 * c);
-    }
-    const float c4[4] = {cs.x, cs.y, cs.z, cs.w}, s4[4] = {sn.x, sn.y, sn.z, sn.w};
+    const float c4[4] = {c0.x, c0.y, c0.z, c0.w}, s4[4] = {s0.x, s0.y, s0.z, s0.w};
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
       o[e] = in_rot ? v[e] * c4[e / 2] - v[e + 1] * s4[e / 2] : v[e];
@@ -465,19 +569,9 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
     }
   } else {
     const int hop = rot >> 4;        // lanes between rotary partners
-    const bool in_rot = 8 * c < rot;
-    const bool first = 8 * c < half;
     int partner = first ? lane + hop : lane - hop;
     if (!in_rot) partner = lane;
-    const int p0 = first ? 8 * c : 8 * c - half;   // pair index of this lane's first element
-    float cs[8], sn[8];
-    if (in_rot) {
-      const float4* cp = reinterpret_cast<const float4*>(cos_t + (size_t)pos * half + p0);
-      const float4* sp = reinterpret_cast<const float4*>(sin_t + (size_t)pos * half + p0);
-      const float4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
-      cs[0] = c0.x; cs[1] = c0.y; cs[2] = c0.z; cs[3] = c0.w; cs[4] = c1.x; cs[5] = c1.y; cs[6] = c1.z; cs[7] = c1.w;
-      sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
-    }
+    const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float pv = __shfl(v[e], partner, kWave);
@@ -491,7 +585,6 @@ __global__ __launch_bounds__(1024) void qk_norm_rope_kvt_bf16_kernel(
   if (!is_k) {
     *reinterpret_cast<bf16x8v*>(q_out + ((size_t)t * nq + h) * d + 8 * c) = y;
   } else {
-    const long long slot = slots[t];
     if (slot >= 0) {
       const long long page = slot / page_size;
       const int off = (int)(slot - page * page_size);
@@ -1126,12 +1219,13 @@ int xi_qk_norm_rope_kv(const void* qkv, int dtype, int slices, const float* bias
       (vcos == nullptr || (!interleaved && dv % 16 == 0 && ((uintptr_t)vcos | (uintptr_t)vsin) % 16 == 0)) &&
       ((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16 == 0) {
     const int lph = d / 8, hpw = 64 / lph;
-    int n_waves = 64 / hpw;                       // waves of a workgroup: at most 64 tokens, at most 16 waves
-    if (n_waves > 16) n_waves = 16;
+    // Small workgroups, which start as soon as four waves have ended (2,048 tokens of 64 + 16 heads of 128 in workgroups of 4 | 8 | 16 waves 22.1 |
+    // 24.0 | 27.6 us), of whole groups of eight tokens (40 tokens of heads of 96: 32.0 | 34.1 in workgroups of 20); at most 64 tokens.
+    const int fit = 64 / hpw, n_waves = fit < (hpw % 2 ? 8 : 4) ? fit : hpw % 2 ? 8 : 4;
     const int tpw = n_waves * hpw;
     const unsigned blocks_x = (unsigned)((n_tok + tpw - 1) / tpw);
     XI_CHECK(nq + 2 * nkv <= 65535, "qk_norm_rope_kv: too many heads");
-    const size_t lds = (size_t)tpw * (dv + 2) * sizeof(bf16);
+    const size_t lds = (((size_t)tpw * (dv + 2) + 3) & ~(size_t)3) * sizeof(bf16) + (size_t)tpw * sizeof(long long);
     qk_norm_rope_kvt_bf16_kernel<<<dim3(blocks_x, nq + 2 * nkv), n_waves * 64, lds, stream>>>(
         (const bf16*)qkv, bias, qw, kw, eps, cos_t, sin_t, rot, interleaved, positions, slots, (bf16*)q_out,
         (bf16*)k_cache, (bf16*)v_cache, page_size, n_tok, nq, nkv, d, dv, row_stride, v_col, vcos, vsin);
