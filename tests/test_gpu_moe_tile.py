@@ -60,6 +60,27 @@ def test_experts_in_tiles(H, F, act, gated, weigh, identity, shared, monkeypatch
         assert torch.equal(kernels.moe_experts_tiled(*dev, act, **kw), few), pair
 
 
+@pytest.mark.parametrize("H,F,act,gated,weigh,identity", [
+    (64, 64, "silu", True, False, 2), (192, 320, "gelu_tanh", True, True, 0), (320, 192, "relu2", False, False, 1), (1088, 576, "silu", True, False, 0),
+    (512, 2112, "silu", False, False, 0)])
+def test_tiles_of_few_rows(H, F, act, gated, weigh, identity):
+    """Tiles of up to 16 rows: the bits of the higher ones, for rows at the edges of a tile and more tiles an expert than there should be."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(H + F)
+    rb = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    for rows in ([0, 1, 15, 16, 17, 33], [0, 0, 2, 0, 0, 0], [3] * 6):
+        E = len(rows)
+        gate_up, down = rb(E, (2 if gated else 1) * F, H) * H ** -0.5, rb(E, H, F) * F ** -0.5
+        pairs = [e for e, n in enumerate(rows) for _ in range(n)] + [E + i % max(1, identity) for i in range(6) if identity]
+        idx = torch.tensor(pairs)[torch.randperm(len(pairs), generator=g)].view(-1, 2).to(torch.int32)
+        T = idx.shape[0]
+        dev = [t.to(DEV) for t in (rb(T, H), gate_up, down, idx, torch.rand(T, 2, generator=g) + 0.1)]
+        kw = dict(gated=gated, weigh_input=weigh, identity=identity, add=rb(T, H).to(DEV))
+        want = kernels.moe_experts_tiled(*dev, act, tile_rows=64, **kw)
+        assert torch.equal(kernels.moe_experts_tiled(*dev, act, tile_rows=16, **kw), want), rows
+    assert kernels.moe_tile_rows(8 * E, E, F, H, gated) == (16, 16) and kernels.moe_tile_rows(8 * E + 1, E, F, H, gated) == (64, 64)
+
+
 @pytest.mark.parametrize("H,F,act,gated", [(2112, 1088, "silu", True), (192, 2112, "relu2", False)])
 def test_heights_from_the_counts(H, F, act, gated, monkeypatch):
     """Tiles whose heights are chosen on the device, at the edges of every walk, with columns that do and do not share out over the dies."""

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kSortThreads) void moe_plan_kernel(const int* __res
   const int n1 = routed ? share(routed, high[0]) : 0, n2 = routed ? share(routed, high[1]) : 0;
   int before[3] = {pairs, n1, n2};
   int busy = 0;
-  if (high[0] == 64 && high[1] == 64) {        // the same list twice, and one order for all (8 pairs on 1,000 experts, a layer: 17.4 -> 16.6 us)
+  if (high[0] == high[1] && high[0] <= 64) {        // the same list twice, and one order for all (8 pairs on 1,000 experts, a layer: 17.4 -> 16.6 us)
     int both[2] = {pairs, n1};
     moe_sums_before(both, A, across);
     before[0] = both[0], before[1] = before[2] = both[1];
@@ -134,16 +134,15 @@ __global__ __launch_bounds__(kSortThreads) void moe_plan_kernel(const int* __res
 }
 
 // One tile: BM rows of x by BN rows of w (gated: BN / 2 features), rings of S and SW stages.
-template <int BM, int BN, int S, int SW, int FORM, int ACT>
+template <int BM, int BN, int S, int SW, int FORM, int ACT, int WGM = 2, int WGN = 4>
 __device__ __forceinline__ void moe_one_tile(const bf16* __restrict__ x, const int* __restrict__ order, int top,
                                              const bf16* __restrict__ w, int e, int row0, int rows, int tn_i, void* __restrict__ out,
                                              int N, int K, const float* __restrict__ in_wt, unsigned char* smem) {
   constexpr bool GATED = FORM == 1, GATHER = FORM != 0;
-  constexpr int WGM = 2, WGN = 4;
   using W = Walk<BM, BN, WGM, WGN, S, SW>;
   constexpr int TM = W::TM, TN = W::TN;
   constexpr int TF = GATED ? TN / 2 : TN, WF = 16 * TF;            // 16-feature tiles of a wave, and its features
-  static_assert(TN % 2 == 0, "half of a wave's rows of w are gate rows");
+  static_assert(!GATED || TN % 2 == 0, "half of a wave's rows of w are gate rows");
   // (opaque, so that nothing made from them is made in front of the choice between the walks and held in registers through all)
   asm volatile("" : "+s"(row0), "+s"(rows), "+s"(tn_i));
   int tid = threadIdx.x;
@@ -194,9 +193,17 @@ __device__ __forceinline__ void moe_one_tile(const bf16* __restrict__ x, const i
   }
 }
 
-// LOW: tiles of up to 64 rows by 128 rows of w; otherwise of up to 256 by 256, each in the lowest walk that holds it.
-template <bool LOW, int FORM, int ACT>
-__global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict__ x, const int* __restrict__ order, int top,
+// Rows of w and stages of the tiles of up to 16 rows: two workgroups of four waves a compute unit, 70 KB on their way each.  Decode steps are
+// bound by the stream of the touched experts' weights: with tiles of 64 rows a third of what came into LDS was copies of the few rows of x, one
+// workgroup a compute unit left a gap at every round's start, and columns of 128 features of the down product were fewer than the compute
+// units.  16 pairs on 8 gated experts of 6144 at width 4096 219 -> 206 us, without a gate 167 -> 148; 8 on 16 of 4096 at 2048 68 -> 57.
+constexpr int few_wide(int form) { return form == 1 ? 128 : 64; }
+constexpr int few_stages(int form) { return form == 1 ? 4 : 7; }
+
+// HIGH 64: tiles of up to 64 rows by 128 rows of w; 16: of up to 16 rows by 64 features; 0: of up to 256 by 256, each in the lowest walk that
+// holds it.
+template <int HIGH, int FORM, int ACT>
+__global__ __launch_bounds__(HIGH == 16 ? 256 : 512, HIGH == 16 ? 2 : 1) void moe_tile_kernel(const bf16* __restrict__ x, const int* __restrict__ order, int top,
                                                           const bf16* __restrict__ w, const int* __restrict__ tiles, int most,
                                                           void* __restrict__ out, int N, int K, int columns,
                                                           const float* __restrict__ in_wt) {
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
     column = q / count;
     tile = first + (q - column * count);
   };
-  const int order_of = LOW ? 2 : tiles[5 * most + 1];
+  const int order_of = HIGH ? 2 : tiles[5 * most + 1];
   if (order_of == 2) {
     // Consecutive places a die, an expert after the other: a die's L2 holds an expert's rows and the rows of w that its tiles share.  For
     // tiles that take about as long as each other (within 3%, the list says): 16 experts of 4096 at width 2048, 1,024 rows each 577 us the other way,
@@ -235,7 +242,9 @@ __global__ __launch_bounds__(512, 1) void moe_tile_kernel(const bf16* __restrict
   }
   const int e = tiles[tile], row0 = tiles[most + tile], rows = tiles[2 * most + tile];
 #define XI_ONE(BM, BN, S, SW) moe_one_tile<BM, BN, S, SW, FORM, ACT>(x, order, top, w, e, row0, rows, column, out, N, K, in_wt, smem)
-  if constexpr (LOW) {
+  if constexpr (HIGH == 16) {
+    moe_one_tile<16, few_wide(FORM), few_stages(FORM), few_stages(FORM), FORM, ACT, 1, 4>(x, order, top, w, e, row0, rows, column, out, N, K, in_wt, smem);
+  } else if constexpr (HIGH == 64) {
     XI_ONE(64, 128, 6, 6);
   } else {
     if (rows > 224) XI_ONE(256, 256, 2, 3);
@@ -271,7 +280,7 @@ int xi_moe_tile_takes(long long rows_x, int N, int K, int gated) {
 // device, of 128 to 256, for that many columns of workgroups; most: xi_moe_tiles_most for high or for 128.
 int xi_moe_plan(const int* idx, int P, int E, int I, int high1, int high2, int columns1, int columns2, int* order, int* slot_of, int* tiles1,
                 int* tiles2, int most1, int most2, hipStream_t stream) {
-  auto fits = [](int h) { return h == 0 || h == 64 || h == 128 || h == 256; };
+  auto fits = [](int h) { return h == 0 || h == 16 || h == 64 || h == 128 || h == 256; };
   XI_CHECK(P > 0 && E > 0 && I >= 0 && E + I <= kSortExperts && fits(high1) && fits(high2) && columns1 > 0 && columns2 > 0,
            "moe_plan: bad sizes pairs=%d experts=%d rows=%d, %d", P, E, high1, high2);
   XI_CHECK(most1 >= xi_moe_tiles_most(P, E, high1 ? high1 : 128) && most2 >= xi_moe_tiles_most(P, E, high2 ? high2 : 128),
@@ -284,14 +293,14 @@ int xi_moe_plan(const int* idx, int P, int E, int I, int high1, int high2, int c
 
 // Columns of workgroups of a product of N features in tiles of up to `high` rows (0: chosen on the device).
 int xi_moe_tile_columns(int N, int high, int gated) {
-  const int features = (high == 64 ? 128 : 256) / (gated ? 2 : 1);
+  const int features = high == 16 ? 64 : (high == 64 ? 128 : 256) / (gated ? 2 : 1);
   return (N + features - 1) / features;
 }
 
 // The operands of `xi_moe_group` (moe_mfma.hip) for the tiles of `xi_moe_plan` with this `high`; rows_x: rows of A.
 int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, const void* W, const int* tiles, int most, void* out,
                 int N, int K, int high, int form, int act, const float* in_wt, hipStream_t stream) {
-  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && most > 0 && (high == 0 || high == 64 || high == 128 || high == 256),
+  XI_CHECK(xi_moe_tile_takes(rows_x, N, K, form == 1) && top > 0 && most > 0 && (high == 0 || high == 16 || high == 64 || high == 128 || high == 256),
            "moe_tile: bad sizes N=%d K=%d top=%d tiles=%d rows=%d", N, K, top, most, high);
   XI_CHECK(act >= 0 && act <= 2 && form >= 0 && form <= 2, "moe_tile: unknown activation %d or form %d", act, form);
   XI_CHECK(tiles && order, "moe_tile: an operand is missing");
@@ -300,27 +309,29 @@ int xi_moe_tile(const void* A, long long rows_x, const int* order, int top, cons
   const int columns = xi_moe_tile_columns(N, high, form == 1);
   XI_CHECK((long long)most * columns <= 0x3fffffffLL, "moe_tile: too many tiles");
   const long long places = 8 * ((long long)most * (columns / 8) + ((long long)most * (columns % 8) + 7) / 8);
-  const unsigned wgs = (unsigned)(high == 64 ? ((long long)most * columns + 7) / 8 * 8 : places);
-#define XI_MT(LOW, FORM, ACT)                                                                                               \
+  const unsigned wgs = (unsigned)(high == 64 || high == 16 ? ((long long)most * columns + 7) / 8 * 8 : places);
+#define XI_MT(HIGH, FORM, ACT)                                                                                              \
   do {                                                                                                                      \
-    auto kern = tile::moe_tile_kernel<LOW, FORM, ACT>;                                                                      \
-    const size_t lds = LOW ? tile::Walk<64, 128, 2, 4, 6>::LDS : tile::Walk<256, 256, 2, 4, 2, 3>::LDS;                        \
+    auto kern = tile::moe_tile_kernel<HIGH, FORM, ACT>;                                                                      \
+    const size_t lds = HIGH == 16 ? tile::Walk<16, tile::few_wide(FORM), 1, 4, tile::few_stages(FORM)>::LDS                  \
+                       : HIGH ? tile::Walk<64, 128, 2, 4, 6>::LDS : tile::Walk<256, 256, 2, 4, 2, 3>::LDS;                     \
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);      \
     XI_CHECK(e == hipSuccess, "moe_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));                      \
-    kern<<<wgs, 512, lds, stream>>>((const bf16*)A, order, top, (const bf16*)W, tiles, most, out, N, K, columns, in_wt); \
+    kern<<<wgs, HIGH == 16 ? 256 : 512, lds, stream>>>((const bf16*)A, order, top, (const bf16*)W, tiles, most, out, N, K, columns, in_wt); \
   } while (0)
-#define XI_MT_FORM(LOW)                                 \
+#define XI_MT_FORM(HIGH)                                \
   do {                                                  \
-    if (form == 0) XI_MT(LOW, 0, 0);                    \
-    else if (form == 1 && act == 0) XI_MT(LOW, 1, 0);   \
-    else if (form == 1 && act == 1) XI_MT(LOW, 1, 1);   \
-    else if (form == 1) XI_MT(LOW, 1, 2);               \
-    else if (act == 0) XI_MT(LOW, 2, 0);                \
-    else if (act == 1) XI_MT(LOW, 2, 1);                \
-    else XI_MT(LOW, 2, 2);                              \
+    if (form == 0) XI_MT(HIGH, 0, 0);                    \
+    else if (form == 1 && act == 0) XI_MT(HIGH, 1, 0);   \
+    else if (form == 1 && act == 1) XI_MT(HIGH, 1, 1);   \
+    else if (form == 1) XI_MT(HIGH, 1, 2);               \
+    else if (act == 0) XI_MT(HIGH, 2, 0);                \
+    else if (act == 1) XI_MT(HIGH, 2, 1);                \
+    else XI_MT(HIGH, 2, 2);                              \
   } while (0)
-  if (high == 64) XI_MT_FORM(true);
-  else XI_MT_FORM(false);
+  if (high == 16) XI_MT_FORM(16);
+  else if (high == 64) XI_MT_FORM(64);
+  else XI_MT_FORM(0);
 #undef XI_MT_FORM
 #undef XI_MT
   XI_LAUNCH_CHECK("moe_tile");
