@@ -742,6 +742,33 @@ def test_qk_norm_rope_kv_whole_heads(d, first, normed):
         assert float((a != b).float().mean()) < 0.01
 
 
+@pytest.mark.parametrize("d", [16, 32, 48, 96, 128, 160, 256])
+@pytest.mark.parametrize("biased", [False, True])
+def test_qk_norm_rope_kv_orders_are_one(d, biased):
+    """A head's sum of squares has one order in both layouts of the pairs: turned by nothing (cos 1, sin 0) the heads have the same bits.
+    Without a norm, turned, they are those of the form of one wave per head."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d)
+    T, page, nq, nkv = 515, 16, 3, 2
+    qkv = (_rand((T, (nq + 2 * nkv) * d), torch.float32, g) * torch.exp(torch.randn(T, 1, generator=g))).to(torch.bfloat16).to(DEV)
+    bias = (0.1 * torch.randn((nq + 2 * nkv) * d, generator=g)).to(DEV) if biased else None
+    qw, kw = ((1 + 0.2 * torch.randn(d, generator=g)).to(DEV) for _ in range(2))
+    still = torch.ones(T, d // 2, device=DEV), torch.zeros(T, d // 2, device=DEV)
+    turned = tuple(t.to(DEV) for t in plain.rope_tables(1e6, d, T))
+
+    def run(tables, interleaved, least, *weights):
+        kc = torch.zeros((34, nkv, page, d), dtype=torch.bfloat16, device=DEV)
+        vt = torch.zeros((34, nkv, page // 8, d, 8), dtype=torch.bfloat16, device=DEV)
+        at = torch.arange(T, device=DEV)
+        q = kernels.qk_norm_rope_kv(qkv, *weights, 1e-6, *tables, d, interleaved, at.to(torch.int32), at, kc, vt, nq, nkv, d, v_grouped=True,
+                                    vector_min_tokens=least, bias=bias)
+        return q, kc
+    for a, b in zip(run(still, False, 1, qw, kw), run(still, True, 1, qw, kw)):
+        assert torch.equal(a, b)
+    for a, b in zip(run(turned, False, 1, None, None), run(turned, False, 10 ** 6, None, None)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,T,nq,nkv,d,rot,interleaved", [
     (torch.float32, 11, 3, 1, 48, 48, False), (torch.bfloat16, 11, 4, 2, 32, 16, True),
     (torch.bfloat16, 150, 5, 5, 48, 48, False), (torch.bfloat16, 150, 2, 1, 128, 64, True)])

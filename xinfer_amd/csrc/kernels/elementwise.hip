@@ -444,24 +444,29 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
       }
     }
     if (w) {
-      float ss = 0.f;
+      // The squares in the order of the lanes of eight elements below, so that a head's norm has one value whatever its rotation: an even lane's four
+      // and behind them the odd lane's of either half; then an even lane keeps the first half's sum of eight, the odd one the second's.
+      auto four = [](const float (&v)[4], float from) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ss += va[e] * va[e];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ss += vb[e] * vb[e];
+        for (int e = 0; e < 4; ++e) from = __builtin_fmaf(v[e], v[e], from);
+        return from;
+      };
+      const float sa = four(va, lane_xor<1>(four(va, 0.f))), sb = four(vb, lane_xor<1>(four(vb, 0.f)));
+      const float sa_odd = lane_xor<1>(sa), ss = lane & 1 ? sb : sa_odd;
       float total;
       if ((lph & (lph - 1)) == 0) {
         total = ss;
-        if (lph > 1) total += lane_xor<1>(total);
         if (lph > 2) total += lane_xor<2>(total);
         if (lph > 4) total += lane_xor<4>(total);
         if (lph > 8) total += lane_xor<8>(total);
         if (lph > 16) total += lane_xor<16>(total);
         if (lph > 32) total += lane_xor<32>(total);
+        total += lane_xor<1>(total);
       } else {
         total = 0.f;
         const int begin = lane - c;
-        for (int o = 0; o < lph; ++o) total += __shfl(ss, begin + o, kWave);
+        for (int o = 0; o < lph; o += 2) total += __shfl(ss, begin + o, kWave);
+        for (int o = 1; o < lph; o += 2) total += __shfl(ss, begin + o, kWave);
       }
       const float inv = rsqrtf(total / (float)d + eps);
 #pragma unroll
@@ -474,8 +479,8 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
     bf16x4v ya, yb;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      ya.v[e] = from_float<bf16>(va[e] * cs[e] - vb[e] * sn[e]);
-      yb.v[e] = from_float<bf16>(va[e] * sn[e] + vb[e] * cs[e]);
+      ya.v[e] = from_float<bf16>(__builtin_fmaf(va[e], cs[e], -(vb[e] * sn[e])));       // (as in qk_row.h)
+      yb.v[e] = from_float<bf16>(__builtin_fmaf(va[e], sn[e], vb[e] * cs[e]));
     }
     bf16* to = q_out + ((size_t)t * nq + h) * d;
     if (is_k) {
