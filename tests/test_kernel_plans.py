@@ -1,5 +1,8 @@
 """What the host decides before a kernel is launched (no GPU): how a narrow product is cut
 along K for the many-row tiled kernel, and how a decode step's keys are shared out among workgroups."""
+import os
+import re
+
 import pytest
 
 from xinfer_amd import kernels
@@ -186,3 +189,18 @@ def test_round_tiles_ahead():
     assert ahead(1792, 4096, 8192) and not ahead(1791 - 255, 4096, 8192)       # 7 x 32 tiles, 6 x 32
     for M, N, K in ((2048, 4096, 4096), (2049, 4096, 12288), (1536, 4096, 12288), (2048, 2048, 8192), (4096, 2048, 16384), (8, 4096, 12288)):
         assert not ahead(M, N, K), (M, N, K)
+
+
+def test_loads_into_lds_wait_for_m0():
+    """An asm that writes m0 and loads into LDS behind it has the wait state that the pair wants: the compiler puts none inside an asm."""
+    folder = os.path.join(os.path.dirname(kernels.__file__), "csrc", "kernels")
+    found = 0
+    for name in sorted(os.listdir(folder)):
+        with open(os.path.join(folder, name)) as f:
+            for text in re.findall(r'asm volatile\("((?:[^"\\]|\\.)*)"', f.read()):
+                lines = [line.strip() for line in text.replace("\\t", "").split("\\n")]
+                for before, line in zip(lines, lines[1:] + [""]):
+                    if re.match(r"s_\w+ m0,", before):
+                        found += 1
+                        assert line.startswith("s_nop"), (name, text)
+    assert found >= 4

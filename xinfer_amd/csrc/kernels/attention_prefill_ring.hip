@@ -53,14 +53,15 @@ __device__ __forceinline__ bf16x8 zero8() {
 
 // One 16-byte chunk per lane from global memory to LDS at `lds_addr` (the same in all lanes) +
 // 16 * lane.  The compiler does not see that LDS is written: whoever reads it waits for the load
-// with an explicit vmcnt and a barrier first.
+// with an explicit vmcnt and a barrier first.  (Behind a scalar write of m0 such a load wants one wait state, which the compiler gives its own
+// loads and cannot give inside an asm.)
 __device__ __forceinline__ void load_lds16(const void* g, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr) : "memory", "m0");
 }
 
 // The same with the address as a base that is the same in all lanes plus a byte offset per lane.
 __device__ __forceinline__ void load_lds16(const void* base, unsigned lane_off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
                : "memory", "m0");
 }
 

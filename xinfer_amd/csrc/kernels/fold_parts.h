@@ -11,13 +11,13 @@ namespace xi {
 constexpr int fold_parts_room(int n) { return (n + kWave - 1) / kWave * kWave; }
 
 // n numbers from `from` on into `to` (LDS, room for fold_parts_room(n)), by WAVES waves.  The caller waits for them (they are the oldest of its
-// loads) and for the other waves.
+// loads) and for the other waves.  (s_nop: the wait state that such a load wants behind a scalar write of m0.)
 template <int WAVES>
 __device__ __forceinline__ void fetch_fold_parts(const float* __restrict__ from, int n, float* to, int wave, int lane) {
   const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)to);
   for (int i = wave * kWave; i < n; i += WAVES * kWave) {
     const int at = i + lane < n ? i + lane : n - 1;
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(at * 4u), "s"(from), "s"(lds + 4u * i) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(at * 4u), "s"(from), "s"(lds + 4u * i) : "memory", "m0");
   }
 }
 

@@ -14,8 +14,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 namespace tile {
 
+// (A load that writes LDS wants one wait state behind a scalar write of m0, which the compiler gives its own loads and cannot give inside an asm.)
 __device__ __forceinline__ void load_lds16(const void* base, unsigned lane_off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_addr)
                : "memory", "m0");
 }
 
