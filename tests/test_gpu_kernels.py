@@ -1259,6 +1259,34 @@ def test_attention_decode_packed_slot_elsewhere():
     assert torch.equal(one, two) and torch.equal(kc, k2) and torch.equal(vt, v2)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("left", [float("inf"), float("nan")])
+def test_attention_decode_lean_overwrites_what_was_left(d, left):
+    """A place that its key and value are written to in this step held an infinity or no number: nothing of it is seen, also where the step's
+    other lanes read the place's group again for keys that are not there."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d)
+    nq, nkv, page, contexts = 4, 2, 64, [8, 16, 24, 32, 40, 72, 136, 200, 264, 5, 1]
+    case = _paged_case(g, torch.bfloat16, nq, nkv, d, page, [(c, 1) for c in contexts])
+    _, kc, vt, bt = _mfma_inputs(case)
+    _, ctx = _cu_ctx([(c, 1) for c in contexts])
+    slots = torch.tensor([int(case["bt"][b, (c - 1) // page]) * page + (c - 1) % page for b, c in enumerate(contexts)], device=DEV)
+    packed = _rand((len(contexts), (nq + 2 * nkv) * d), torch.bfloat16, g).to(DEV)
+    cos, sin = (t.to(DEV) for t in plain.rope_tables(10000.0, d, 300))
+    pos = (ctx - 1).to(torch.int32).to(DEV)
+    outs = []
+    for fill in (0.0, left):
+        k2, v2 = kc.clone(), vt.clone()
+        at, off = slots // page, slots % page
+        k2[at, :, off] = fill
+        v2[at, :, off // 8, :, off % 8] = fill
+        out = kernels.attention_decode_packed_bf16(packed, None, None, 1e-5, cos, sin, d, False, pos, slots, k2, v2, bt, ctx.to(DEV), 300, nq, 0.1)
+        outs.append((out, k2, v2))
+    assert bool(outs[1][0].float().isfinite().all())
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def test_attention_decode_packed_refuses():
     from xinfer_amd import kernels
     nq, nkv, d, page = 4, 2, 32, 16

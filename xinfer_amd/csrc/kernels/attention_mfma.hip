@@ -535,7 +535,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_lean_kernel(
       const __bf16* v = reinterpret_cast<const __bf16*>(kv_new + D);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        if (j == o >> 3) {
+        if (j >= o >> 3) {                    // (the groups behind it hold the same one: an infinity left in the place would get through a weight of 0)
           const __bf16 x = v[16 * dt + r];
 #pragma unroll
           for (int e = 0; e < 8; ++e)
