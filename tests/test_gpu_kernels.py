@@ -1287,6 +1287,21 @@ def test_attention_decode_lean_overwrites_what_was_left(d, left):
         assert torch.equal(a, b)
 
 
+def test_attention_decode_packed_without_pages():
+    """Sequences without a key and a table without columns: nothing is read or stored."""
+    from xinfer_amd import kernels
+    nq, nkv, d, B = 4, 2, 128, 3
+    kc, vt = torch.ones(2, nkv, 64, d, dtype=torch.bfloat16, device=DEV), torch.ones(2, nkv, 8, d, 8, dtype=torch.bfloat16, device=DEV)
+    none = torch.zeros(B, dtype=torch.int32, device=DEV)
+    out = torch.zeros(B, nq * d, dtype=torch.bfloat16, device=DEV)
+    kernels.attention_decode_packed_bf16(torch.ones(B, (nq + 2 * nkv) * d, dtype=torch.bfloat16, device=DEV), None, None, 1e-5,
+                                         torch.ones(4, d // 2, device=DEV), torch.zeros(4, d // 2, device=DEV), d, False, none,
+                                         torch.full((B,), -1, dtype=torch.int64, device=DEV), kc, vt,
+                                         torch.empty((B, 0), dtype=torch.int32, device=DEV), none, 0, nq, 0.1, out=out)
+    torch.cuda.synchronize()
+    assert bool((kc == 1).all()) and bool((vt == 1).all()) and bool((out == 0).all())
+
+
 def test_attention_decode_packed_refuses():
     from xinfer_amd import kernels
     nq, nkv, d, page = 4, 2, 32, 16

@@ -721,7 +721,9 @@ static int launch_decode(int packed, const void* q, const PackedStep& ps, void* 
   const float sl = scale * kLog2e;
   const int slices = packed == 2 ? ps.slices : 0;
   const size_t lean_lds = lds + (size_t)(g + 2) * d * sizeof(bf16);
-  if (packed && (d == 64 || d == 128) && ps.rot == d && !ps.interleaved && !ps.bias && window <= 0 && page >= 32 && slices <= 8 && lean_lds <= 64 * 1024) {
+  // (that kernel asks for a page number before it knows the length: not from a table without columns)
+  if (packed && (d == 64 || d == 128) && ps.rot == d && !ps.interleaved && !ps.bias && window <= 0 && page >= 32 && slices <= 8 && lean_lds <= 64 * 1024 &&
+      max_pages > 0) {
     // (run_shift 0: the sequences' own order, where the units take further workgroups in turn, a sequence's splits are workgroups of their own or
     // 256 workgroups are no run of sequences)
     LeanStep step{ps.qw, ps.kw, ps.cos_t, ps.sin_t, ps.slice_stride, ps.eps, slices, n_seq, 0};
