@@ -4,6 +4,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from xinfer_amd import kernels
 
@@ -204,3 +205,15 @@ def test_loads_into_lds_wait_for_m0():
                         found += 1
                         assert line.startswith("s_nop"), (name, text)
     assert found >= 4
+
+
+def test_a_steps_small_array_is_not_recorded(monkeypatch):
+    """While a graph is recorded the copy from a pinned block, which is another array's by the next replay, is refused as one from ordinary
+    memory is; on the CPU it is a plain tensor."""
+    assert kernels.on_device([[1, 2], [3, 4]], torch.int32, "cpu").tolist() == [[1, 2], [3, 4]]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    made = []
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: made.append(kw))
+    with pytest.raises(kernels.KernelError, match="recorded"):
+        kernels.on_device([1, 2], torch.int64, "cuda:0")
+    assert not made

@@ -93,10 +93,13 @@ def on_device(values, dtype: torch.dtype, device) -> torch.Tensor:
     """A step's small array (a list, or rows of one) on the device, through pinned memory of its own: the host goes on launching.
     From ordinary memory the copy waits for everything on the stream, and the GPU then for the host: 290 us of a 2,048-token prompt
     of a design with states (5,485), 65 of any prompt.  (torch hands the pinned block out again when the copy has left it; blocks of
-    one size, PINNED_BYTES, serve almost all of them: a new one costs 100 us.)"""
+    one size, PINNED_BYTES, serve almost all of them: a new one costs 100 us.)  For the same reason it is refused while a graph is recorded, as
+    the copy from ordinary memory is: a replay would read what the block holds by then."""
     host = torch.tensor(values, dtype=dtype)
     if torch.device(device).type != "cuda":
         return host.to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise KernelError("an array made on the host for one step cannot be recorded into a graph")
     pin = torch.empty((max(host.numel(), PINNED_BYTES // host.element_size()),), dtype=dtype, pin_memory=True)[:host.numel()].view(host.shape)
     return pin.copy_(host).to(device, non_blocking=True)
 
