@@ -217,3 +217,39 @@ def test_a_steps_small_array_is_not_recorded(monkeypatch):
     with pytest.raises(kernels.KernelError, match="recorded"):
         kernels.on_device([1, 2], torch.int64, "cuda:0")
     assert not made
+
+
+def test_even_lengths_are_read_by_the_kernel_they_were_measured_in(monkeypatch):
+    """A step of even lengths goes as whole sequences in the kernel for whole-rotated heads without bias or window on pages of 32 keys and
+    more; with q given, a bias, a window, small pages, half of a head turned or pairs (2i, 2i + 1) it is cut up as lengths of any kind are."""
+    real, cut = kernels.lib(), []
+
+    class Noted:
+        def __getattr__(self, name):
+            if not name.startswith("xi_attention_decode_") or name == "xi_attention_decode_lean":
+                return getattr(real, name)
+            return lambda *args: cut.append(int(args[-9])) or 0
+    monkeypatch.setattr(kernels, "lib", Noted)
+    monkeypatch.setattr(kernels, "_dev", lambda *a: None)
+    monkeypatch.setattr(kernels, "_stream", lambda: None)
+    bf = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32)
+    B, nq, nkv, d, span = 264, 2, 1, 64, 2048
+
+    def packed(page=64, rot=d, interleaved=False, bias=None, window=0, slices=0, similar=kernels.EVEN_LENGTHS):
+        cut.clear()
+        qkv = torch.zeros(slices, B, (nq + 2 * nkv) * d) if slices else bf(B, (nq + 2 * nkv) * d)
+        kernels.attention_decode_packed_bf16(qkv, None, None, 1e-6, torch.zeros(4, rot // 2), torch.zeros(4, rot // 2), rot, interleaved, i32(B),
+                                             torch.zeros(B, dtype=torch.int64), bf(1, nkv, page, d), bf(1, nkv, page // 8, d, 8), i32(B, 1), i32(B), span, nq,
+                                             0.1, window, bias=bias, similar=similar)
+        return cut[0]
+    whole, mixed = 2176, kernels.decode_keys_per_workgroup(B * nkv, span, False)
+    assert whole != mixed
+    assert packed() == packed(slices=8) == whole and packed(similar=False) == mixed
+    for other in (dict(page=16), dict(rot=32), dict(interleaved=True), dict(bias=torch.zeros((nq + 2 * nkv) * d)), dict(slices=9)):
+        assert packed(**other) == mixed, other
+    assert packed(window=span) == packed(window=span, similar=False)
+    for similar in (kernels.EVEN_LENGTHS, False):
+        cut.clear()
+        kernels.attention_decode_bf16(bf(B, nq, d), bf(1, nkv, 64, d), bf(1, nkv, 8, d, 8), i32(B, 1), i32(B), span, 0.1, similar=similar)
+        assert cut == [mixed]

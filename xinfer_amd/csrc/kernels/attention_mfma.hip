@@ -702,6 +702,14 @@ int xi_attention_mfma_supported(int nq, int nkv, int d, int page) {
   return (d % 16 == 0 && d >= 16 && d <= 256 && page >= 8 && (page & (page - 1)) == 0 && nq % nkv == 0) ? 1 : 0;
 }
 
+// Whether the packed projection's decode step goes in `attn_decode_lean_kernel` (its page numbers must fit LDS too).
+int xi_attention_decode_lean(int nq, int nkv, int d, int page, int rot, int interleaved, int biased, int window, int slices) {
+  return ((d == 64 || d == 128) && rot == d && !interleaved && !biased && window <= 0 && page >= 32 && slices <= 8 &&
+          xi_attention_mfma_supported(nq, nkv, d, page) && nq / nkv <= 16)
+             ? 1
+             : 0;
+}
+
 // The decode launch: `packed` 0 takes q [sequences, nq, d]; 1 and 2 the packed projection, see PackedStep.
 static int launch_decode(int packed, const void* q, const PackedStep& ps, void* k_cache, void* vt_cache,
                          const int* block_tables, int max_pages, const int* ctx_lens, void* out, float* part_o,
@@ -722,8 +730,7 @@ static int launch_decode(int packed, const void* q, const PackedStep& ps, void* 
   const int slices = packed == 2 ? ps.slices : 0;
   const size_t lean_lds = lds + (size_t)(g + 2) * d * sizeof(bf16);
   // (that kernel asks for a page number before it knows the length: not from a table without columns)
-  if (packed && (d == 64 || d == 128) && ps.rot == d && !ps.interleaved && !ps.bias && window <= 0 && page >= 32 && slices <= 8 && lean_lds <= 64 * 1024 &&
-      max_pages > 0) {
+  if (packed && xi_attention_decode_lean(nq, nkv, d, page, ps.rot, ps.interleaved, ps.bias != nullptr, window, slices) && lean_lds <= 64 * 1024 && max_pages > 0) {
     // (run_shift 0: the sequences' own order, where the units take further workgroups in turn, a sequence's splits are workgroups of their own or
     // 256 workgroups are no run of sequences)
     LeanStep step{ps.qw, ps.kw, ps.cos_t, ps.sin_t, ps.slice_stride, ps.eps, slices, n_seq, 0};

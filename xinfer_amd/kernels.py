@@ -1229,6 +1229,15 @@ EVEN_LENGTHS = 2                    # a third value for `similar`: the mean leng
 DECODE_EVEN_KEYS = 4096             # such lengths: a workgroup's keys at most
 
 
+@functools.lru_cache(maxsize=256)
+def decode_lean(nq: int, nkv: int, d: int, page: int, rot: int, interleaved: bool, biased: bool, window: int, slices: int = 0) -> bool:
+    """Whether `attention_decode_packed_bf16` takes such a step to the kernel with little between its start and its first keys.
+    Only there EVEN_LENGTHS is read: in the other kernels, two workgroups a compute unit, whole sequences of such lengths lose from one to one
+    and a half pairs a unit on (us, the mixed lengths' chunks | whole, 8 kv heads of 128 with a bias: 40 sequences of 300 to 3,000 keys 62 | 66, 28
+    of 100 to 900 19 | 20, 48 of 1,000 to 4,000 104 | 109; heads of 64 35 | 39; pages of 16 keys 62 | 67)."""
+    return bool(lib().xi_attention_decode_lean(nq, nkv, d, page, rot, int(interleaved), int(biased), window, slices))
+
+
 def decode_keys_per_workgroup(pairs: int, span: int, similar: int = False) -> int:
     return _decode_keys_per_workgroup(int(pairs), int(span), int(similar) if similar == EVEN_LENGTHS else int(bool(similar)))
 
@@ -1507,7 +1516,7 @@ def attention_decode_bf16(q, k_cache, vt_cache, block_tables, ctx_lens, max_ctx_
     if block_tables.shape[0] != B or ctx_lens.shape != (B,):
         raise KernelError("attention_decode: one block table row and one context length per sequence")
     span = min(int(max_ctx_len), int(window) + 31) if window > 0 else int(max_ctx_len)
-    kpw = int(keys_per_workgroup or decode_keys_per_workgroup(B * nkv, span, similar))
+    kpw = int(keys_per_workgroup or decode_keys_per_workgroup(B * nkv, span, similar != EVEN_LENGTHS and similar))
     max_splits = span // kpw + 1
     part_o = torch.empty((B, nq, max_splits, d), dtype=torch.float32, device=q.device)
     part_ml = torch.empty((B, nq, max_splits, 2), dtype=torch.float32, device=q.device)
@@ -1561,6 +1570,8 @@ def attention_decode_packed_bf16(qkv, q_weight, k_weight, eps, cos, sin, rotary_
         if bias.shape != (qkv.shape[-1],):
             raise KernelError(f"attention_decode_packed: bias {tuple(bias.shape)} is not [{qkv.shape[-1]}]")
     span = min(int(max_ctx_len), int(window) + 31) if window > 0 else int(max_ctx_len)
+    if similar == EVEN_LENGTHS and not decode_lean(nq, nkv, d, page, int(rotary_dim), bool(interleaved), bias is not None, int(window), slices):
+        similar = False
     kpw = int(keys_per_workgroup or decode_keys_per_workgroup(B * nkv, span, similar))
     max_splits = span // kpw + 1
     part_o = torch.empty((B, nq, max_splits, d), dtype=torch.float32, device=qkv.device)
