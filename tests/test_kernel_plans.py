@@ -1,12 +1,16 @@
 """What the host decides before a kernel is launched (no GPU): how a narrow product is cut
 along K for the many-row tiled kernel, and how a decode step's keys are shared out among workgroups."""
 import os
+import random
 import re
 
+import numpy as np
 import pytest
 import torch
 
 from xinfer_amd import kernels
+from xinfer_amd.cache import busiest_over_share
+from xinfer_amd.engine.runner import lengths_class
 
 SHAPES = [(6144, 4096), (4096, 4096), (4096, 12288), (7168, 5120), (5120, 5120), (5120, 17408), (10240, 5120),
           (5120, 8192), (5120, 25600), (4096, 1024), (1024, 2048), (1024, 3072), (24576, 4096), (1000, 2056), (48, 96)]
@@ -253,3 +257,36 @@ def test_even_lengths_are_read_by_the_kernel_they_were_measured_in(monkeypatch):
         cut.clear()
         kernels.attention_decode_bf16(bf(B, nq, d), bf(1, nkv, 64, d), bf(1, nkv, 8, d, 8), i32(B, 1), i32(B), span, 0.1, similar=similar)
         assert cut == [mixed]
+
+
+def _dealt_out(lengths, columns):
+    """Longest first, each to the column with the fewest keys: the busiest one's keys beyond the share, rounded down."""
+    keys = [0] * columns
+    for n in sorted(lengths, reverse=True):
+        keys[keys.index(min(keys))] += n
+    return max(keys) - sum(keys) // columns
+
+
+def test_busiest_over_share():
+    rng = random.Random(5)
+    for n, columns in ((1, 1), (3, 32), (16, 32), (33, 32), (61, 32), (200, 85), (256, 8), (17, 1)):
+        lengths = [rng.randint(1, 1 << rng.randint(0, 20)) for _ in range(n)]
+        assert busiest_over_share(np.asarray(lengths, np.int32), columns) == _dealt_out(lengths, columns), (n, columns)
+    assert busiest_over_share(np.empty(0, np.int32), 32) == 0
+    most = [2 ** 31 - 1] * 40                       # (sums beyond an int; the excess itself is never more than the longest)
+    assert busiest_over_share(np.asarray(most, np.int32), 39) == _dealt_out(most, 39)
+
+
+def test_lengths_class_looks_at_how_the_sequences_deal_out():
+    """Not the mean alone: one full round of long sequences and a few more leave most of the chip idle, whatever the short ones beside them."""
+    of = lambda lengths, heads=(8,), **kw: lengths_class(np.asarray(lengths, np.int32), heads, **kw)
+    rng = random.Random(6)
+    ragged = [rng.randint(90, 2700) for _ in range(61)]
+    assert of(ragged) == kernels.EVEN_LENGTHS and of(sorted(ragged)) == kernels.EVEN_LENGTHS
+    for n, longest, short in ((33, 4000, 15), (38, 4000, 10), (39, 3300, 61), (36, 4000, 54), (35, 2700, 37), (16, 4000, 24), (11, 2700, 17)):
+        assert of([longest] * n + [100] * short) is False, (n, longest, short)
+    assert of([4000] * 8) is True and of([3900] * 30 + [4000] * 30) is True and of([900] * 30, similar=False) == kernels.EVEN_LENGTHS
+    assert of(ragged[:15]) is False and of(ragged, ()) is False and of([]) is False
+    # several numbers of kv heads: every one has to deal out
+    uneven = [1800] * 33 + [100] * 12
+    assert of(uneven, (8,)) is False and of(uneven, (16,)) is False and of(uneven, (6,)) == kernels.EVEN_LENGTHS and of(uneven, (6, 8)) is False

@@ -2,7 +2,12 @@
 // kernels read.  The reference builds the same set in prepare_prefill / prepare_decode
 // (/root/reference/src/core/runner.rs:1303-1563, 1565-1750); here one builder serves both,
 // a decode token being a portion of one token.
+#include <algorithm>
+#include <climits>
 #include <cstring>
+#include <functional>
+#include <new>
+#include <queue>
 #include <vector>
 
 #include "cache.h"
@@ -64,6 +69,28 @@ int xi_cm_build_batch(CacheManager* cm, int B, const int64_t* ids, const int32_t
     cu_q[b + 1] = t;
   }
   return t == T ? 0 : -6;
+}
+
+// n sequences dealt out whole over `columns`, the longest first, each to the column with the fewest keys so far: what the busiest one has beyond
+// its share of all keys (rounded down; never more than the longest).
+int xi_busiest_over_share(int n, const int32_t* lengths, int columns) {
+  if (n <= 0 || columns <= 0) return 0;
+  try {
+    std::vector<int32_t> by(lengths, lengths + n);
+    std::sort(by.begin(), by.end(), std::greater<int32_t>());
+    std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> keys(std::greater<int64_t>(), std::vector<int64_t>((size_t)columns, 0));
+    int64_t busiest = 0, total = 0;
+    for (const int32_t length : by) {
+      const int64_t t = keys.top() + length;
+      keys.pop();
+      keys.push(t);
+      busiest = t > busiest ? t : busiest;
+      total += length;
+    }
+    return (int)(busiest - total / columns);
+  } catch (const std::bad_alloc&) {
+    return INT_MAX;
+  }
 }
 
 // A step in which every one of B requests brings one token, prepared in one call for the

@@ -23,8 +23,8 @@ from typing import Any, Dict, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
-from ..cache import DecodeStepError, BatchArrays, CacheGroup, PagedCacheManager
-from ..kernels import EVEN_LENGTHS, PINNED_BYTES, on_device
+from ..cache import DecodeStepError, BatchArrays, CacheGroup, PagedCacheManager, busiest_over_share
+from ..kernels import COMPUTE_UNITS, EVEN_LENGTHS, EVEN_SLACK, PINNED_BYTES, decode_lean, on_device
 from ..parts import LayerCache, StepContext, state_needs_of
 from .model import CausalLM
 
@@ -40,14 +40,17 @@ class StepError(ValueError):
     pass
 
 
-def _similar(ctx_lens: np.ndarray) -> int:
-    """How even the sequences of a step are: True, about equally long (kernels may then give each a
-    workgroup of its own instead of cutting all into equal pieces), EVEN_LENGTHS, not a few long ones among many short (of sixteen
-    sequences and more), or False."""
+def lengths_class(ctx_lens: np.ndarray, kv_heads: Sequence[int], similar: Optional[bool] = None) -> int:
+    """How even the cached lengths of a step of single tokens are (int32), for the plans of its attention: True, about equally long (kernels may
+    then give each a workgroup of its own instead of cutting all into equal pieces; `similar` if the caller knows), EVEN_LENGTHS for
+    every one of the numbers of kv heads of the layers whose kernel reads that, or False."""
     if not ctx_lens.size:
         return False
-    mean, longest = float(ctx_lens.mean()), float(ctx_lens.max())
-    return True if mean >= 0.9 * longest else EVEN_LENGTHS if mean >= 0.4 * longest and ctx_lens.size >= 16 else False
+    if similar is None:
+        similar = float(ctx_lens.mean()) >= 0.9 * float(ctx_lens.max())
+    if similar or ctx_lens.size < 16 or not kv_heads:
+        return bool(similar)
+    return EVEN_LENGTHS if all(busiest_over_share(ctx_lens, max(1, COMPUTE_UNITS // n)) <= EVEN_SLACK for n in kv_heads) else False
 
 
 class _Staging:
@@ -197,6 +200,9 @@ class ModelRunner:
                 if c.state is None:
                     c.state = arena
                 c.states[st.name] = arena
+        # numbers of kv heads of the layers whose decode kernel reads more than whether a step's lengths are about equal
+        forms = [kv.decode_form for kv in model.kv_needs.values() if kv.decode_form is not None]
+        self._even_heads = tuple(sorted({f["nkv"] for f in forms if decode_lean(page=self.page_size, **f)}))
         self._empty_f32 = torch.empty((1, 0), dtype=torch.float32, device=self.device)
         self._staging = _Staging(self.device)
         # pinned blocks for the small arrays of a step or two, so that the first one does not make them (torch keeps them for `on_device`)
@@ -401,8 +407,7 @@ class ModelRunner:
                              -3: f"request {rid}: its tokens exceed the model's {spec.max_positions} positions",
                              -4: f"a token id is outside the vocabulary of {spec.vocab_size}"}.get(
                                  ex.kind, f"the step could not be prepared ({ex.kind})")) from None
-        if not similar and B >= 16:
-            similar = _similar(host32[4 * B + 1:5 * B + 1])       # (the lengths just written)
+        similar = lengths_class(host32[4 * B + 1:5 * B + 1], self._even_heads, similar)      # (the lengths just written)
         bucket = context_bucket(longest)
         g = self._graphs.get((B, bucket, similar))
         if g is None:
@@ -450,7 +455,7 @@ class ModelRunner:
             ctx_lens_host=a.ctx_lens.tolist() if host_lengths else (),
             max_q_len=int(q_lens.max()),
             max_ctx_len=int(a.ctx_lens.max()) if max_ctx_len is None else int(max_ctx_len),
-            similar_lengths=_similar(a.ctx_lens),
+            similar_lengths=lengths_class(a.ctx_lens, self._even_heads if T == B else ()),
             no_slots=d64[o64[2]:o64[2] + T], empty_f32=self._empty_f32)
         return ctx, v32(0, T), v32(5, rows32.size), d32, d64
 
@@ -492,7 +497,7 @@ class ModelRunner:
         B = a.num_seqs
         longest = int(a.ctx_lens.max())
         bucket = context_bucket(longest)
-        key = (B, bucket, _similar(a.ctx_lens))     # what kernels choose their shapes from
+        key = (B, bucket, lengths_class(a.ctx_lens, self._even_heads))     # what kernels choose their shapes from
         all_rows = np.zeros(B, dtype=np.int32)
         all_rows[:rows32.size] = rows32
         g = self._graphs.get(key)

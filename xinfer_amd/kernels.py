@@ -1225,7 +1225,8 @@ DECODE_SPLITS_MOST = 1024           # splits of a sequence that the search below
 DECODE_WHOLE_KEYS = 2048            # mixed lengths, one and a half pairs a compute unit and more: a workgroup's keys at most
 
 
-EVEN_LENGTHS = 2                    # a third value for `similar`: the mean length is at least 0.4 of the longest (True: 0.9)
+EVEN_LENGTHS = 2                    # a third value for `similar`: not about equally long, but dealt out whole they leave no compute unit far behind
+EVEN_SLACK = 1150                   # that is: the busiest unit's keys beyond its share of all (`_decode_keys_per_workgroup`)
 DECODE_EVEN_KEYS = 4096             # such lengths: a workgroup's keys at most
 
 
@@ -1268,12 +1269,15 @@ def _decode_keys_per_workgroup(pairs: int, span: int, similar: int) -> int:
     from one pair a compute unit on chunks of 1,024 (32 sequences of 500 to 4,000: 60 us against 65
     at 512 and 63 whole).
 
-    EVEN_LENGTHS: spread out, but not a few long ones among many short.  Whole sequences where the longest outlasts a unit's share of
-    all keys (0.55 pairs span / 256) by less than what the second kernel and the splits' uneven share-out cost, about 800 keys and a fifth
-    of the share, from 7 pairs for 8 units on.  Us, the rules above | whole, both in the kernel for such steps: 61 sequences of 90 to 2,700
-    keys 71 | 66, 64 of 256 to 2,304 67 | 63, 40 of 300 to 3,000 62 | 58, 33 of 700 to 1,400 39 | 32, 45 of 130 to 1,060 (64 query heads) 33 |
-    26, 30 of 40 to 300 14 | 10, 31 of 200 to 1,900 36 | 33; beyond the rule 25 of 200 to 1,500 26 | 26, 23 of 130 to 1,900 28 | 29, 16 of 500
-    to 2,500 30 | 34; a few long ones, 61 of 600 in the middle and one of 4,000, 54 | 63."""
+    EVEN_LENGTHS: from 16 sequences on, whose pairs, dealt out whole over the units, the longest first, each to the one with the fewest keys,
+    give the busiest no more than EVEN_SLACK keys beyond its share of all (`cache.busiest_over_share`): about what the second kernel and a
+    workgroup's start for every chunk cost.  Whole sequences then, from 7 pairs for 8 units on; beyond span (1 - 0.76 pairs / 256) = 800 no lengths
+    spread evenly from a tenth of the longest on pass that test.  Us, the rules above | whole, 8 kv heads of 128, both in the kernel
+    for such steps (`decode_lean`): 61 sequences of 90 to 2,700 keys 77 | 65, 64 of 256 to 2,304 76 | 67, 40 of 300 to 3,000 60 | 56, 33 of 700 to 1,400
+    39 | 33, 30 of 40 to 300 13 | 9, 31 of 200 to 1,900 36 | 32, 28 of 100 to 900 18 | 16, 128 of 500 to 4,000 225 | 209, 45 of 130 to 1,060 (64 query
+    heads) 36 | 28.  Of 258 batches, most of n sequences of one length beside short ones, the 147 within the slack took 0.68 to 0.998 of the
+    time; beyond it (keys of excess in brackets) 11 of 1,900 and 17 of 100 (1,190) 1.01, 16 of 4,000 and 24 of 100 (1,925) 0.985, 39 of 2,700 and 61 of 100 (1,920) 1.02, 36 of
+    4,000 and 54 of 100 (3,330) 1.14."""
     if similar == EVEN_LENGTHS:
         p = pairs / COMPUTE_UNITS
         if p >= 0.85 and span <= DECODE_EVEN_KEYS and span * (1 - 0.76 * p) <= 800:

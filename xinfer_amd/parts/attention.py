@@ -50,6 +50,7 @@ own kv head.
 """
 from __future__ import annotations
 
+from dataclasses import replace
 from typing import List, Optional
 
 import torch
@@ -246,6 +247,10 @@ class PagedAttention(Mixer):
                                   value_dim=self.dv)
         if self.talking:           # mixed heads score against a token's whole k row: one key head of all kv heads' dims
             need = KVNeed(need.window, (PoolNeed("k", (1, PAGE, self.nkv * self.d)), need.pools[1]))
+        if self.decode_packed:
+            pos = self.position
+            need = replace(need, decode_form=dict(nq=self.nq, nkv=self.nkv, d=self.d, rot=pos.rotary_dim if pos is not None else 0,
+                                                  interleaved=bool(pos is not None and pos.interleaved), biased=self.bias, window=self.window))
         return need
 
     def state_need(self):

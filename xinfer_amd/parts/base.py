@@ -72,9 +72,11 @@ class KVNeed:
     """What a mixer keeps in pages: `window` = 0 keeps every token's entry, w > 0 the last w (pages
     that the window has passed go back to the pool while the request runs); `pools` names the
     pools and the shape of a page in each.  `KVNeed.keys_values` is the pair that attention keeps;
-    a mixer of another kind may keep one pool (a latent), or pools of different widths."""
+    a mixer of another kind may keep one pool (a latent), or pools of different widths.  `decode_form`: what
+    `kernels.decode_lean` asks of a mixer whose steps of single tokens may go in that kernel, as its keyword arguments but the page."""
     window: int = 0
     pools: Tuple[PoolNeed, ...] = ()
+    decode_form: Optional[Dict[str, Any]] = field(default=None, compare=False)
 
     @staticmethod
     def keys_values(num_kv_heads: int, head_dim: int, window: int = 0, v_grouped: bool = False,
@@ -146,7 +148,7 @@ class StepContext:
     ctx_lens_host: Sequence[int] = ()
     max_q_len: int = 0
     max_ctx_len: int = 0
-    similar_lengths: int = False               # host: the mean cached length is at least 0.9 of the longest (True) or 0.4 (kernels.EVEN_LENGTHS)
+    similar_lengths: int = False               # host: the mean cached length is at least 0.9 of the longest (True), or see kernels.EVEN_LENGTHS
     no_slots: Optional[torch.Tensor] = None    # int64 [T] of -1: "store nothing"
     empty_f32: Optional[torch.Tensor] = None   # float32 [1, 0]: tables of "no rotation"
     scratch: Dict[Any, Any] = field(default_factory=dict)   # per-step data that kernels derive once
