@@ -197,6 +197,34 @@ def test_real_layer_sizes_wide_decode_batches(name, live, real_model_dirs):
         assert max(float((got[k] - again[k]).abs().max()) for k in got) < 2e-3 * scale
 
 
+@pytest.mark.parametrize("live,evenness", [(20, 0), (28, 2)])
+def test_recorded_steps_of_uneven_lengths(live, evenness, tmp_path):
+    """One long request beside short ones, whose mean drifts over 0.4 of the longest, and lengths of all kinds: one recording for all steps,
+    keyed by the lengths' class only where that makes another plan (28 requests on 8 kv heads), and the launched steps' logits."""
+    from configs import _cfg
+    from xinfer_amd import kernels
+    from xinfer_amd.engine import ModelRunner, load_model
+    from xinfer_amd.weights import write_random_model
+    config = _cfg(num_hidden_layers=2, hidden_size=128, num_attention_heads=16, num_key_value_heads=8, head_dim=64, intermediate_size=192,
+                  vocab_size=300, rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=True, max_position_embeddings=1024)
+    d, rng, tail = write_random_model(str(tmp_path), config, 11, 0.03, 0.1), random.Random(live), 9
+    lengths = [60 + tail] + [22 + tail] * (live - 1) if evenness == 0 else [20 + 3 * i + tail for i in range(live)]
+    reqs = {f"r{i}": harness.random_prompt(rng, n, 300) for i, n in enumerate(lengths)}
+    pm = plain.PlainModel(d)
+    ref = {rid: pm.logits(toks) for rid, toks in reqs.items()}
+    steps = harness.trace_batch_decode(reqs, tail=tail)
+    model = load_model(d, "bfloat16", "cuda:0")
+    assert kernels.EVEN_LENGTHS == 2 and kernels.even_lengths_matter(8 * live, 1024) == bool(evenness)
+    runner = ModelRunner(model, page_size=64, num_pages=3 * live, max_requests=live, graph_after=3, graph_max_batch=64)
+    assert runner._even_heads == (8,)
+    got = harness.replay(runner, steps)
+    assert list(runner._graphs) == [(live, 1024, evenness)] == list(runner._seen) and runner.graph_replays == tail - 3
+    harness.compare(got, ref, harness.TOL["bfloat16"], f"{live} of uneven lengths")
+    again = harness.replay(ModelRunner(model, page_size=64, num_pages=3 * live, max_requests=live, use_graphs=False), steps)
+    scale = max(float(r.abs().max()) for r in ref.values())
+    assert max(float((got[k] - again[k]).abs().max()) for k in got) < 2e-3 * scale        # as in the batches above
+
+
 def test_mixed_step_with_long_contexts_both_attention_paths(real_model_dirs):
     """A step that brings single tokens of six requests with contexts of some thousand tokens and a
     portion of a seventh, at Qwen3-8B layer sizes: the decode kernel takes the six (their contexts

@@ -279,7 +279,7 @@ def test_busiest_over_share():
 
 def test_lengths_class_looks_at_how_the_sequences_deal_out():
     """Not the mean alone: one full round of long sequences and a few more leave most of the chip idle, whatever the short ones beside them."""
-    of = lambda lengths, heads=(8,), **kw: lengths_class(np.asarray(lengths, np.int32), heads, **kw)
+    of = lambda lengths, heads=(8,), **kw: lengths_class(np.asarray(lengths, np.int32), 1 + max(lengths, default=0), heads, **kw)
     rng = random.Random(6)
     ragged = [rng.randint(90, 2700) for _ in range(61)]
     assert of(ragged) == kernels.EVEN_LENGTHS and of(sorted(ragged)) == kernels.EVEN_LENGTHS
@@ -290,3 +290,21 @@ def test_lengths_class_looks_at_how_the_sequences_deal_out():
     # several numbers of kv heads: every one has to deal out
     uneven = [1800] * 33 + [100] * 12
     assert of(uneven, (8,)) is False and of(uneven, (16,)) is False and of(uneven, (6,)) == kernels.EVEN_LENGTHS and of(uneven, (6, 8)) is False
+
+
+def test_lengths_class_is_told_only_where_a_plan_differs():
+    """The class is part of a recorded step's key: lengths that drift over the line do not record the same kernels again."""
+    of = lambda lengths, span, heads: lengths_class(np.asarray(lengths, np.int32), span, heads)
+    told = 0
+    for B in (16, 20, 27, 28, 32, 48, 61, 64, 200, 256):
+        ragged = [20 + 5 * i for i in range(B)]
+        assert not of(ragged, 8192, ()) and of([500] * B, 1024, ()) is True
+        for span in range(1024, 9 * 1024, 1024):
+            got = of(ragged, span, (8,))
+            assert got in (False, kernels.EVEN_LENGTHS)
+            told += bool(got)
+            differs = kernels.decode_keys_per_workgroup(8 * B, span, kernels.EVEN_LENGTHS) != kernels.decode_keys_per_workgroup(8 * B, span, False)
+            assert bool(got) == differs, (B, span)        # (these lengths deal out)
+            if B < 28 or span > 4096 or (B >= 48 and span <= 2048):
+                assert not got, (B, span)
+    assert told

@@ -61,7 +61,7 @@ def _bind(lib):
         "xi_cm_max_table_len": (i, [vp, i, _I64P]),
         "xi_cm_lengths": (None, [vp, i, _I64P, _I64P]),
         "xi_cm_decode_step": (i, [vp, i, _I64P, _I32P, i, i, i64, i, _I32P, i, _I32P, _I64P, _I32P, _I32P]),
-        "xi_busiest_over_share": (i, [i, _I32P, i]),
+        "xi_busiest_over_share": (i, [i, vp, i]),
         "xi_cm_reserve_many": (i, [vp, i, _I64P, _I32P]),
         "xi_cm_commit_many": (i, [vp, i, _I64P, _I32P]),
         "xi_cm_build_batch": (i, [vp, i, _I64P, _I32P, _I32P, _I32P, _I32P, _I32P, _I32P,
@@ -91,9 +91,10 @@ class BatchArrays:
 
 
 def busiest_over_share(lengths: np.ndarray, columns: int) -> int:
-    """Sequences of these lengths (int32, contiguous) dealt out whole over `columns`, the longest first, each to the one with the fewest keys so
-    far: the keys that the busiest has beyond its share of all."""
-    return int(_bind(load_host()).xi_busiest_over_share(int(lengths.size), lengths.ctypes.data_as(_I32P), int(columns)))
+    """Sequences of these lengths dealt out whole over `columns`, the longest first, each to the one with the fewest keys so far: the keys that
+    the busiest has beyond its share of all."""
+    lengths = np.ascontiguousarray(lengths, dtype=np.int32)
+    return int(_bind(load_host()).xi_busiest_over_share(lengths.size, lengths.ctypes.data, columns))
 
 
 class DecodeStepError(Exception):

@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from ..cache import DecodeStepError, BatchArrays, CacheGroup, PagedCacheManager, busiest_over_share
-from ..kernels import COMPUTE_UNITS, EVEN_LENGTHS, EVEN_SLACK, PINNED_BYTES, decode_lean, on_device
+from ..kernels import COMPUTE_UNITS, EVEN_LENGTHS, EVEN_SLACK, PINNED_BYTES, decode_lean, even_lengths_matter, on_device
 from ..parts import LayerCache, StepContext, state_needs_of
 from .model import CausalLM
 
@@ -40,17 +40,20 @@ class StepError(ValueError):
     pass
 
 
-def lengths_class(ctx_lens: np.ndarray, kv_heads: Sequence[int], similar: Optional[bool] = None) -> int:
-    """How even the cached lengths of a step of single tokens are (int32), for the plans of its attention: True, about equally long (kernels may
-    then give each a workgroup of its own instead of cutting all into equal pieces; `similar` if the caller knows), EVEN_LENGTHS for
-    every one of the numbers of kv heads of the layers whose kernel reads that, or False."""
+def lengths_class(ctx_lens: np.ndarray, span: int, kv_heads: Sequence[int], similar: Optional[bool] = None) -> int:
+    """How even the cached lengths of a step of single tokens are (int32), for the plans that its attention makes for `span` keys: True, about
+    equally long (kernels may then give each a workgroup of its own; `similar` if the caller knows), EVEN_LENGTHS, or False.  `kv_heads`: of the
+    layers whose kernel reads EVEN_LENGTHS.  It is part of a recorded step's key, so it is False wherever no layer's plan would be
+    another one: a step whose lengths drift is then recorded once (a second recording of the same kernels is 8 to 17 ms and
+    a graph's place), and the lengths are looked at only where it matters."""
     if not ctx_lens.size:
         return False
     if similar is None:
         similar = float(ctx_lens.mean()) >= 0.9 * float(ctx_lens.max())
-    if similar or ctx_lens.size < 16 or not kv_heads:
+    if similar or ctx_lens.size < 16:
         return bool(similar)
-    return EVEN_LENGTHS if all(busiest_over_share(ctx_lens, max(1, COMPUTE_UNITS // n)) <= EVEN_SLACK for n in kv_heads) else False
+    heads = [n for n in kv_heads if even_lengths_matter(ctx_lens.size * n, span)]
+    return EVEN_LENGTHS if heads and all(busiest_over_share(ctx_lens, max(1, COMPUTE_UNITS // n)) <= EVEN_SLACK for n in heads) else False
 
 
 class _Staging:
@@ -407,8 +410,8 @@ class ModelRunner:
                              -3: f"request {rid}: its tokens exceed the model's {spec.max_positions} positions",
                              -4: f"a token id is outside the vocabulary of {spec.vocab_size}"}.get(
                                  ex.kind, f"the step could not be prepared ({ex.kind})")) from None
-        similar = lengths_class(host32[4 * B + 1:5 * B + 1], self._even_heads, similar)      # (the lengths just written)
         bucket = context_bucket(longest)
+        similar = lengths_class(host32[4 * B + 1:5 * B + 1], bucket, self._even_heads, similar)      # (the lengths just written)
         g = self._graphs.get((B, bucket, similar))
         if g is None:
             return None
@@ -446,6 +449,7 @@ class ModelRunner:
         tables = v32(6, G * B * P).view(G, B, P)
         slots = d64[o64[1]:o64[1] + G * T].view(G, T)
         q_lens = np.diff(a.cu_q)
+        span = int(a.ctx_lens.max()) if max_ctx_len is None else int(max_ctx_len)
         ctx = StepContext(
             num_tokens=T, num_seqs=B, dtype=self.model.dtype, device=dev,
             positions=v32(1, T), tok_seq=v32(2, T), cu_q=v32(3, B + 1), ctx_lens=v32(4, B),
@@ -454,8 +458,7 @@ class ModelRunner:
             cu_q_host=a.cu_q.tolist() if host_lengths else (),
             ctx_lens_host=a.ctx_lens.tolist() if host_lengths else (),
             max_q_len=int(q_lens.max()),
-            max_ctx_len=int(a.ctx_lens.max()) if max_ctx_len is None else int(max_ctx_len),
-            similar_lengths=lengths_class(a.ctx_lens, self._even_heads if T == B else ()),
+            max_ctx_len=span, similar_lengths=lengths_class(a.ctx_lens, span, self._even_heads if T == B else ()),
             no_slots=d64[o64[2]:o64[2] + T], empty_f32=self._empty_f32)
         return ctx, v32(0, T), v32(5, rows32.size), d32, d64
 
@@ -497,7 +500,7 @@ class ModelRunner:
         B = a.num_seqs
         longest = int(a.ctx_lens.max())
         bucket = context_bucket(longest)
-        key = (B, bucket, lengths_class(a.ctx_lens, self._even_heads))     # what kernels choose their shapes from
+        key = (B, bucket, lengths_class(a.ctx_lens, bucket, self._even_heads))     # what kernels choose their shapes from
         all_rows = np.zeros(B, dtype=np.int32)
         all_rows[:rows32.size] = rows32
         g = self._graphs.get(key)

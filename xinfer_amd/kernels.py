@@ -1244,6 +1244,12 @@ def decode_keys_per_workgroup(pairs: int, span: int, similar: int = False) -> in
 
 
 @functools.lru_cache(maxsize=4096)
+def even_lengths_matter(pairs: int, span: int) -> bool:
+    """Whether EVEN_LENGTHS makes another plan than False."""
+    return _decode_keys_per_workgroup(pairs, span, EVEN_LENGTHS) != _decode_keys_per_workgroup(pairs, span, 0)
+
+
+@functools.lru_cache(maxsize=4096)
 def _decode_keys_per_workgroup(pairs: int, span: int, similar: int) -> int:
     """Keys per workgroup of the split-K decode kernel for `pairs` (sequence, kv head) pairs of
     up to `span` keys (a multiple of 128; more than `span`: a workgroup takes a whole sequence and
