@@ -308,3 +308,10 @@ def test_lengths_class_is_told_only_where_a_plan_differs():
             if B < 28 or span > 4096 or (B >= 48 and span <= 2048):
                 assert not got, (B, span)
     assert told
+
+
+def test_moe_tiles_of_few_rows_where_no_expert_has_many():
+    """Steps of up to 16 tokens have at most 16 rows an expert, however they share out; longer ones may put most pairs on a few experts."""
+    rows = lambda T, top, E: kernels.moe_tile_rows(T * top, E, 768, 1024, True, T)
+    assert rows(8, 2, 8) == rows(16, 4, 8) == rows(1, 8, 1000) == rows(17, 2, 16) == rows(64, 4, 64) == rows(16, 8, 16) == (16, 16)
+    assert rows(16, 5, 8) == rows(17, 2, 8) == rows(32, 2, 8) == rows(65, 4, 64) == rows(128, 8, 128) == rows(64, 8, 64) == (64, 64)

@@ -841,22 +841,27 @@ def moe_tiled_takes(T: int, top: int, E: int, H: int, F: int, gated: bool) -> bo
     return E <= 1024 and bool(takes(ctypes.c_longlong(T), F, H, int(gated))) and bool(takes(P, H, F, 0))
 
 
-MOE_FEW_PAIRS = 8                   # pairs an expert up to which tiles have 16 rows
+MOE_FEW_PAIRS = 8                   # pairs an expert up to which tiles have 16 rows, in steps of up to 16 tokens
+MOE_FEW_PAIRS_SKEWED = 4            # the same in steps of more
 
 
 @functools.lru_cache(maxsize=1024)
-def moe_tile_rows(P: int, E: int, F: int, H: int, gated: bool):
-    """Most rows of a workgroup's tile in the two products of `moe_experts_tiled` for P pairs on E experts: 64, or 0: chosen on the
-    device from the experts' own counts, 128 to 256 (`xi_moe_plan`).  16 up to 8 pairs an expert on average, so that hardly any expert has
-    a second tile that reads its weights again (both products and what stands around them, us, 16 | 64 rows: 8 gated experts of 6144 at
+def moe_tile_rows(P: int, E: int, F: int, H: int, gated: bool, T: int = 0):
+    """Most rows of a workgroup's tile in the two products of `moe_experts_tiled` for P pairs of T tokens (0: as few as there can be) on E experts:
+    64, or 0: chosen on the device from the experts' own counts, 128 to 256 (`xi_moe_plan`).  16 for few pairs (both products and what stands
+    around them, us, 16 | 64 rows, an even share-out: 8 gated experts of 6144 at
     width 4096, 0.25 pairs each 74 | 87, 2 206 | 219, 8 225 | 235, 12 234 | 238, 16 255 | 240; without a gate 2 each 148 | 167, 8 160 | 178, 16
-    181 | 181; 16 of 4096 at 2048, 1 each 86 | 98, 8 117 | 133; 64 gated ones of 768 at 1024, 0.5 each 40 | 41, 4 63 | 69); 64 up to 56, where the
+    181 | 181; 16 of 4096 at 2048, 1 each 86 | 98, 8 117 | 133; 64 gated ones of 768 at 1024, 0.5 each 40 | 41, 4 63 | 69): up to 8 an expert on average in
+    steps of up to 16 tokens, where no expert can have a second tile that reads its weights again (a router's picks of a token are distinct), and
+    up to 4 in longer ones, whose experts may have any share: with half of the pairs on an eighth of the experts 4 pairs each are ahead everywhere
+    (the 8 of 6144 209 | 224, 64 of 768 62 | 67, 128 of 768 at 2048 208 | 220), 8 each are not (32 tokens on the 8 of 6144 243 | 236, all pairs on an eighth
+    of the 64 of 768 28 | 25 and of the 128 84 | 66; that share-out loses at 4 too, 58 | 49 on the 128).  64 up to 56, where the
     weights' bytes bound both; beyond where its rounds of 256 workgroups, with half a tile past an expert's rows on average, take a fifth less time than
     the others' (a round of tiles of h rows by 256: h + 16; of 64 by 128: 64).  Measured on MI355X, both products and what stands
     around them (us, 64 | 0): 8 gated experts of 6144 at width 4096, 64 pairs each 265 | 290, 100 381 | 305, 410 895 | 542, 512 1072 |
     580; without a gate 500 each 730 | 460; 8 of 1536 at width 1024, 125 each 33 | 51, 1,000 each 127 | 86; 16 of 4096 at 2048, 300
     each 365 | 249."""
-    if P <= MOE_FEW_PAIRS * E:
+    if P <= (MOE_FEW_PAIRS if T <= 16 else MOE_FEW_PAIRS_SKEWED) * E:
         return 16, 16
     if P <= 56 * E:
         return 64, 64
@@ -909,7 +914,7 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
             raise KernelError("moe_experts_tiled: an opening is one number a token for rows to add")
     rows = x if x.data_ptr() % 16 == 0 else x.clone()          # (the products want them on 16 bytes)
     P = T * top
-    highs = (int(tile_rows),) * 2 if tile_rows is not None else moe_tile_rows(P, E, F, H, gated)
+    highs = (int(tile_rows),) * 2 if tile_rows is not None else moe_tile_rows(P, E, F, H, gated, T)
     if tile_rows is not None and highs[0] not in (16, 64, 128, 256):
         raise KernelError("moe_experts_tiled: tiles of 16, 64, 128 or 256 rows")
     (high1, most1, columns1), (high2, most2, columns2) = (_moe_tiles(P, E, h, n, g) for h, n, g in zip(highs, (F, H), (gated, False)))
