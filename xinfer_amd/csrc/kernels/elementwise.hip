@@ -431,17 +431,18 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
       wa = *reinterpret_cast<const f4_any*>(w + 4 * cl);
       wb = *reinterpret_cast<const f4_any*>(w + half + 4 * cl);
     }
+    f4_any ba = {0.f, 0.f, 0.f, 0.f}, bb = ba;
+    if (bias) {
+      ba = *reinterpret_cast<const f4_any*>(bias + (size_t)h * d + 4 * cl);
+      bb = *reinterpret_cast<const f4_any*>(bias + (size_t)h * d + half + 4 * cl);
+    }
     const f4_any cs = *reinterpret_cast<const f4_any*>(cos_t + (size_t)pos * half + 4 * cl);
     const f4_any sn = *reinterpret_cast<const f4_any*>(sin_t + (size_t)pos * half + 4 * cl);
     float va[4], vb[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      va[e] = to_float(xa.v[e]);
-      vb[e] = to_float(xb.v[e]);
-      if (bias) {
-        va[e] += bias[(size_t)h * d + 4 * cl + e];
-        vb[e] += bias[(size_t)h * d + half + 4 * cl + e];
-      }
+      va[e] = to_float(xa.v[e]) + ba[e];
+      vb[e] = to_float(xb.v[e]) + bb[e];
     }
     if (w) {
       // The squares in the order of the lanes of eight elements below, so that a head's norm has one value whatever its rotation: an even lane's four
