@@ -315,3 +315,16 @@ def test_moe_tiles_of_few_rows_where_no_expert_has_many():
     rows = lambda T, top, E: kernels.moe_tile_rows(T * top, E, 768, 1024, True, T)
     assert rows(8, 2, 8) == rows(16, 4, 8) == rows(1, 8, 1000) == rows(17, 2, 16) == rows(64, 4, 64) == rows(16, 8, 16) == (16, 16)
     assert rows(16, 5, 8) == rows(17, 2, 8) == rows(32, 2, 8) == rows(65, 4, 64) == rows(128, 8, 128) == rows(64, 8, 64) == (64, 64)
+
+
+def test_thin_products_ask_for_all_of_k_where_it_was_ahead():
+    """Tiles of 512 k that few-row products ask for together: up to 1,024 of K with any rows, 2,048 with up to 8 and 1,536 with more; workgroups of
+    up to four features that add into the stream 2,048, and 3,072 with up to 8 rows.  Longer K, 0, is walked; -1: no such tiles."""
+    depth = kernels.lib().xi_linear_thin_depth
+    for N, adds, most in ((1024, 0, {8: 2048, 16: 1536}), (2048, 0, {8: 2048, 16: 1536}), (2048, 1, {8: 2048, 16: 1536}), (1024, 1, {8: 3072, 16: 2048}),
+                          (256, 1, {8: 3072, 16: 2048}), (4096, 1, {8: 2048, 16: 1536})):
+        for M in (1, 4, 8, 9, 16):
+            for K in range(512, 8192, 512):
+                got = depth(M, N, K, adds)
+                assert (got > 0) == (K <= most[8 if M <= 8 else 16]) and (got == 0 or 512 * got >= K), (N, adds, M, K, got)
+    assert depth(1, 8192, 1024, 0) == -1 and depth(1, 1024, 768, 0) == -1 and depth(1, 1024, 100, 0) == -1

@@ -239,6 +239,27 @@ int xi_linear_thin_features(int N, int K) {
   return thin_features(N);
 }
 
+// A tile of 16 rows of w where the workgroups own at most 16 features and K is a multiple of 512.
+static int thin_tile_rows(int R, int K) { return (R <= 16 && K % 512 == 0) ? 16 : 32; }
+
+// Tiles of 16 rows of w that are asked for together where that is all of K (2, 4 or 6), or 0: K is walked with two on their way.  A workgroup
+// reads all of x too, so that with more rows there is more in flight than it can draw.  Us, weights from memory, walked | whole: N = 2048, 1 row, K = 2048
+// 4.0 | 3.7, 3072 4.6 | 4.8; 16 rows, 1536 4.1 | 4.0, 2048 4.5 | 4.8, 3072 5.5 | 6.4.  Workgroups of up to four features that add into the stream copy
+// four rows of w, which leaves room for more: N = 1024, 1 row, K = 2048 3.5 | 3.3, 3072 4.4 | 4.0; 8 rows, 3072 4.6 | 4.5; 16 rows, 2048 4.1 | 4.1, 3072
+// 5.1 | 5.7.  (K = 4096 there: 1 row 5.2 | 4.5, 8 rows 5.3 | 5.4, 16 rows 6.0 | 6.9; not made.)
+static int thin_depth(int M, int R, int K, bool adds) {
+  const int tiles = K / 512;
+  if (tiles <= 2) return 2;
+  if (adds && R <= 4) return tiles <= 4 ? 4 : tiles <= 6 && M <= 8 ? 6 : 0;
+  return tiles <= (M <= 8 ? 4 : 3) ? 4 : 0;
+}
+
+// The same for a product of these sizes (-1: it has no such tiles).
+int xi_linear_thin_depth(int M, int N, int K, int adds) {
+  const int R = xi_linear_thin_features(N, K);
+  return R && thin_tile_rows(R, K) == 16 ? thin_depth(M, R, K, adds != 0) : -1;
+}
+
 // Workgroups (= parts of a row's sum of squares that xi_linear_thin_fold_out hands on).
 int xi_linear_thin_parts(int N, int K) {
   const int R = xi_linear_thin_features(N, K);
@@ -252,9 +273,6 @@ static int thin_check(const char* what, const void* x, const void* w, int M, int
   XI_CHECK((long long)(N + thin_features(N) - 1) / thin_features(N) < (1ll << 31), "%s: too many workgroups", what);
   return 0;
 }
-
-// A tile of 16 rows of w where the workgroups own at most 16 features and K is a multiple of 512.
-static int thin_tile_rows(int R, int K) { return (R <= 16 && K % 512 == 0) ? 16 : 32; }
 
 #define XI_THIN_LAUNCH_(MODE, TO, TR, yptr, ...)                                                                     \
   do {                                                                                                          \
@@ -270,18 +288,19 @@ static int thin_tile_rows(int R, int K) { return (R <= 16 && K % 512 == 0) ? 16 
     const size_t parts_lds = MODE == 2 ? fold_parts_room(M * fold.parts) * sizeof(float) : 0;                  \
     kern<<<wgs, 256, thin_lds_bytes(TR) + parts_lds, stream>>>((const bf16*)x, (const bf16*)w, (TO*)(yptr), M, N, K, R, rotate, fold); \
   } while (0)
-// tiles of 16 rows of w (512 k): up to six of them are asked for together
-#define XI_THIN_DEPTH(MODE, TO, yptr, XR)                                          \
-  do {                                                                             \
-    constexpr int kLow = MODE == 1 ? 4 : 16;                                       \
-    if (MODE == 1 && R <= 4) {                                                     \
-      if (K <= 2048) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true, kLow);       \
-      else if (K <= 3072) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 6, true, kLow);  \
-      else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, false, kLow);                \
-    } else if (K <= 1024) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, true);               \
-    else if (K <= 2048) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true);          \
-    else if (K <= 3072) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 6, true);          \
-    else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR);                                  \
+// tiles of 16 rows of w (512 k)
+#define XI_THIN_DEPTH(MODE, TO, yptr, XR)                                                             \
+  do {                                                                                                \
+    constexpr int kLow = MODE == 1 ? 4 : 16, kMost = MODE == 1 && XR < 16 ? 6 : 4;                    \
+    const int depth = thin_depth(M, R, K, MODE == 1);                                                 \
+    if (MODE == 1 && R <= 4) {                                                                        \
+      if (depth == 6) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, kMost, true, kLow);                     \
+      else if (depth == 4) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true, kLow);                    \
+      else if (depth == 2) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, true, kLow);                    \
+      else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, false, kLow);                                   \
+    } else if (depth == 4) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 4, true);                          \
+    else if (depth == 2) XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR, 2, true);                            \
+    else XI_THIN_LAUNCH_(MODE, TO, 16, yptr, XR);                                                     \
   } while (0)
 // rows of x in a tile: 4 (tiles of 16 rows of w only: their copying takes 4 rows at once), 8 or 16
 #define XI_THIN_TILE_ROWS(MODE, TO, yptr)                                  \
