@@ -328,3 +328,15 @@ def test_thin_products_ask_for_all_of_k_where_it_was_ahead():
                 got = depth(M, N, K, adds)
                 assert (got > 0) == (K <= most[8 if M <= 8 else 16]) and (got == 0 or 512 * got >= K), (N, adds, M, K, got)
     assert depth(1, 8192, 1024, 0) == -1 and depth(1, 1024, 768, 0) == -1 and depth(1, 1024, 100, 0) == -1
+
+
+def test_round_tiles_of_few_features_leave_strides_of_powers_of_two_alone():
+    ahead = kernels.round_tiles_ahead
+    for M, N in ((3584, 2048), (4096, 2048), (4352, 1920), (3072, 2560)):
+        for K in (5120, 6144, 7168, 10240, 12288, 14336, 17408, 20480):
+            assert ahead(M, N, K), (M, N, K)
+        for K in (4096, 7232, 8192, 8256, 9216, 14400, 15360, 16320, 16384, 16448, 17344, 20544, 24576, 32768):
+            assert not ahead(M, N, K), (M, N, K)
+    for K in (5120, 8192, 15360, 16384, 24576):
+        assert ahead(2048, 4096, K) and ahead(2560, 3072, K)
+    assert not ahead(2048, 4096, 24640) and not ahead(2048, 4096, 32768) and not ahead(2048, 4096, 4096)

@@ -2044,12 +2044,15 @@ ROUND_TILES = (224, 256)            # tiles of 256 rows by 128 features that are
 
 def round_tiles_ahead(M: int, N: int, K: int) -> bool:
     """Whether x [M, K] @ w [N, K]^T goes in tiles of 256 rows by 128 features (shape 1 of `linear_tile`) because they are one full round of
-    the compute units (224 to 256 of them) and K is long, from 5,120 on.  Weights from memory, library / this, over N of 2,048 to 8,192 and the
-    rows that make 224 tiles and more: K = 5,120 1.00 to 1.18, 6,144 1.03 to 1.11, 8,192 0.99 to 1.12, 12,288 1.03 to 1.15, 16,384 1.01 to 1.15,
-    20,480 (the library at half its rate) 1.5 to 1.6.  2,048 rows, us: N=4096 K=6144 91 / 87, K=12288 178 / 167, K=17408 377 / 231.  Not there: K = 4,096 (0.93
-    to 1.14 alone, inside a prompt of 2,048 tokens 59 / 61 us), 200 tiles (0.97 to 1.15) and fewer, N up to 2,048 around K = 16,384 (0.74), two
-    rounds (the library ahead by 5 to 12%)."""
-    return ROUND_TILES[0] <= -(-M // 256) * -(-N // 128) <= ROUND_TILES[1] and 5120 <= K < 1 << 22 and not (N <= 2048 and 14336 < K < 18432)
+    the compute units (224 to 256 of them) and K is long.  Weights from memory, library / this, over N of 1,920 to 8,192 and the rows that make 224
+    tiles and more: from N = 3,072 on, K = 5,120 to 7,168 1.02 to 1.13, 8,192 0.98 to 1.04, 10,240 to 15,360 1.01 to 1.14, 16,384 0.99 to 2.0, 17,408 to 20,480 (the
+    library at half its rate) 1.5 to 1.7, 24,576 1.09 to 1.48, 32,768 0.89 to 1.28 (not taken).  Fewer features: K up to 7,168 1.00 to 1.07, 10,240 to 14,336 1.01
+    to 1.06, 17,408 to 20,480 1.0 to 1.6; between these, rows whose stride is about a power of two, 0.91 to 1.01 around 8,192 and 0.72 to 1.67 around 16,384; beyond 0.79 to
+    1.38.  2,048 rows, us: N=4096 K=6144 91 / 87, K=12288 178 / 167, K=17408 377 / 231.  Not there: K = 4,096 (0.93
+    to 1.14 alone, inside a prompt of 2,048 tokens 59 / 61 us), 200 tiles (0.97 to 1.15) and fewer, two rounds (the library ahead by 5 to 12%)."""
+    if not ROUND_TILES[0] <= -(-M // 256) * -(-N // 128) <= ROUND_TILES[1]:
+        return False
+    return 5120 <= K <= 24576 if N >= 3072 else 5120 <= K <= 7168 or 10240 <= K <= 14336 or 17408 <= K <= 20480
 
 
 def linear_tall(x: torch.Tensor, w: torch.Tensor, rows: int) -> torch.Tensor:
