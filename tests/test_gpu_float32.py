@@ -357,3 +357,26 @@ def test_attention_past_a_waves_pages(page, window, d, news):
     assert float((one - run(matrix=False)).abs().max()) < 2e-5           # as in `test_attention`
     assert torch.equal(run(tile=min(8, news + 1)), one)
     assert torch.equal(run(tile=8, lead=1), one)
+
+
+@pytest.mark.parametrize("nq,nkv,d", [(12, 4, 80), (6, 1, 96), (8, 8, 112), (6, 2, 128)])
+def test_attention_sizes_between_64_and_128(nq, nkv, d):
+    """Head sizes with kernels of their own: tokens by themselves (few and many workgroups) and in tiles the same bits, and those of one lane a key
+    but for the sums' order; the same keys with fewer value dims, which go in the kernel with tests, give those dims' bits."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d)
+    lens, news, page = [33, 200, 64, 17] + [130] * 40, [5, 37, 64, 1] + [1] * 40, 16
+    mp = -(-max(lens) // page)
+    kc, vc = (torch.randn(len(lens) * mp, nkv, page, d, generator=g).to(DEV) for _ in range(2))
+    bt = torch.randperm(len(lens) * mp, generator=g).to(torch.int32).view(len(lens), mp).to(DEV)
+    q = torch.randn(sum(news), nq, d, generator=g).to(DEV)
+    seq = torch.arange(len(lens), dtype=torch.int32).repeat_interleave(torch.tensor(news)).to(DEV)
+    pos = torch.tensor([n - new + i for n, new in zip(lens, news) for i in range(new)], dtype=torch.int32, device=DEV)
+    run = lambda v, rows=slice(None), **kw: kernels.attention_generic(q[rows].contiguous(), kc, v, bt, seq[rows].contiguous(), pos[rows].contiguous(),
+                                                                      d ** -0.5, **kw)
+    one = run(vc, tile=1)
+    assert float((one - run(vc, matrix=False)).abs().max()) < 2e-5           # as in `test_attention`
+    assert torch.equal(run(vc, tile=2), one) and torch.equal(run(vc), one)
+    assert torch.equal(run(vc, slice(0, 8)), one[:8]) and torch.equal(run(vc, slice(106, 112)), one[106:112])
+    less = run(vc[..., :d - 16].contiguous(), tile=1)
+    assert torch.equal(less.view(-1, nq, d - 16), one.view(-1, nq, d)[..., :d - 16])

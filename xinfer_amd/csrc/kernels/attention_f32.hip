@@ -19,7 +19,8 @@
 //
 // A block's K is asked for a block ahead, its V before its scores are made: a wave would wait for the page number, K and V one after the
 // other.  The page numbers of a wave's next 64 blocks are one load, a lane a block (pages in whole blocks; others are looked up key by key);
-// heads of whole tiles (WHOLE) are a kernel without tests around their loads, behind which the compiler waits for more than it needs.
+// heads of whole tiles (WHOLE: 64, 80, 96, 112, 128, 256) are a kernel without tests around their loads, behind which the compiler waits for more
+// than it needs.
 //
 // Measured on MI355X, 32 heads of 128 on 8 kv heads, against a page's number looked up for every block and tests around every load (us):
 // prompts of 200, 127, 54, 172 and 9 tokens 67.6 (79.4), a prompt of 1,024 208 (248), 8 single tokens at up to 330 keys 15.9 (17.3), one at
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attention_f32_kernel(
   const float* qp = q + ((size_t)t * nq + h) * d + 4 * j;
   float* qr = q_s + r * (d + 4) + 4 * j;
   constexpr int kQ = (DT + kWaves - 1) / kWaves;
-  constexpr bool kHold = DT == 8;                   // (in registers from then on)
+  constexpr bool kHold = DT > 4 && DT <= 8;         // (in registers from then on)
   f4 qx[kQ], qh[kHold ? DT : 1];
 #pragma unroll
   for (int i = 0; i < kQ; ++i)
@@ -377,6 +378,11 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
     else if (whole) XI_AF1(DT, false, true);                                                                                  \
     else XI_AF1(DT, false, false);                                                                                            \
   } while (0)
+#define XI_AFW(DT)                                                                                                            \
+  do {                                                                                                                        \
+    if (single) XI_AF1(DT, true, true);                                                                                       \
+    else XI_AF1(DT, false, true);                                                                                             \
+  } while (0)
 #define XI_AF1(DT, SINGLE, WHOLE)                                                                                                    \
   do {                                                                                                                        \
     if (lds > 65536) {     /* always the most this kernel may want: another thread's launch may lie between */                \
@@ -388,7 +394,13 @@ int xi_attention_f32(const float* q, const float* k_cache, const float* v_cache,
         q, k_cache, v_cache, block_tables, max_pages, tok_seq, positions, out, scale, window, page_size, n_tok, lead, tile, nq, nkv, d, dv, softcap, \
         slopes, sinks, values_in_keys, chunk);                                                                                \
   } while (0)
+  // Sizes between 64 and 128 have kernels of their own: in the one for 128 the tests on every load cost more than its other steps give wherever
+  // many single tokens wait for memory: 64 heads of 96 on 8, 32 tokens at 330 keys 22.5 us, 19.5 so (21.3 with a page looked up for every block and the
+  // tests), a prompt of 1,024 378, 317 (368).  Values of another size than the keys stay there: 32 heads of 128 with values of 64, the same 25.2 (23.2).
   if (most <= 64) XI_AF(4);
+  else if (d == dv && d == 80) XI_AFW(5);
+  else if (d == dv && d == 96) XI_AFW(6);
+  else if (d == dv && d == 112) XI_AFW(7);
   else if (most <= 128) XI_AF(8);
   else XI_AF(16);
 #undef XI_AF
