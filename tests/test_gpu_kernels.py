@@ -769,6 +769,26 @@ def test_qk_norm_rope_kv_orders_are_one(d, biased):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("d,rot,interleaved", [(128, 64, False), (64, 32, False), (256, 64, False), (56, 16, False), (128, 128, True), (128, 64, True),
+                                               (96, 40, True), (24, 16, False)])
+def test_qk_norm_rope_kv_turns_alike(d, rot, interleaved):
+    """Heads of which a part turns, in either layout: every product is rounded where the form of one wave per head rounds it, so that without a
+    norm both forms have the same bits."""
+    from xinfer_amd import kernels
+    g = torch.Generator().manual_seed(d + rot)
+    T, page, nq, nkv = 2051, 64, 5, 3
+    qkv = _rand((T, (nq + 2 * nkv) * d), torch.bfloat16, g).to(DEV)
+    cos, sin = (torch.randn(T, rot // 2, generator=g).to(DEV) for _ in range(2))
+    at, both = torch.arange(T, device=DEV), []
+    for least in (1, 10 ** 6):
+        kc = torch.zeros((33, nkv, page, d), dtype=torch.bfloat16, device=DEV)
+        vt = torch.zeros((33, nkv, page // 8, d, 8), dtype=torch.bfloat16, device=DEV)
+        both.append((kernels.qk_norm_rope_kv(qkv, None, None, 1e-6, cos, sin, rot, interleaved, at.to(torch.int32), at, kc, vt, nq, nkv, d,
+                                             v_grouped=True, vector_min_tokens=least), kc, vt))
+    for a, b in zip(*both):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,T,nq,nkv,d,rot,interleaved", [
     (torch.float32, 11, 3, 1, 48, 48, False), (torch.bfloat16, 11, 4, 2, 32, 16, True),
     (torch.bfloat16, 150, 5, 5, 48, 48, False), (torch.bfloat16, 150, 2, 1, 128, 64, True)])

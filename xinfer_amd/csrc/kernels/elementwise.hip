@@ -557,8 +557,8 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
     const float c4[4] = {c0.x, c0.y, c0.z, c0.w}, s4[4] = {s0.x, s0.y, s0.z, s0.w};
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-      o[e] = in_rot ? v[e] * c4[e / 2] - v[e + 1] * s4[e / 2] : v[e];
-      o[e + 1] = in_rot ? v[e] * s4[e / 2] + v[e + 1] * c4[e / 2] : v[e + 1];
+      o[e] = in_rot ? __builtin_fmaf(v[e], c4[e / 2], -(v[e + 1] * s4[e / 2])) : v[e];
+      o[e + 1] = in_rot ? __builtin_fmaf(v[e], s4[e / 2], v[e + 1] * c4[e / 2]) : v[e + 1];
     }
   } else if (interleaved) {
 #pragma unroll
@@ -566,8 +566,8 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
       const int i = 8 * c + e;
       if (i < rot) {
         const float cs = cos_t[(size_t)pos * half + (i >> 1)], sn = sin_t[(size_t)pos * half + (i >> 1)];
-        o[e] = v[e] * cs - v[e + 1] * sn;
-        o[e + 1] = v[e] * sn + v[e + 1] * cs;
+        o[e] = __builtin_fmaf(v[e], cs, -(v[e + 1] * sn));
+        o[e + 1] = __builtin_fmaf(v[e + 1], cs, v[e] * sn);      // (the one form that rounds the other product, as it always has)
       } else {
         o[e] = v[e];
         o[e + 1] = v[e + 1];
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(512) void qk_norm_rope_kvt_bf16_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float pv = __shfl(v[e], partner, kWave);
-      o[e] = !in_rot ? v[e] : (first ? v[e] * cs[e] - pv * sn[e] : pv * sn[e] + v[e] * cs[e]);
+      o[e] = !in_rot ? v[e] : first ? __builtin_fmaf(v[e], cs[e], -(pv * sn[e])) : __builtin_fmaf(pv, sn[e], v[e] * cs[e]);       // (as in qk_row.h)
     }
   }
   if (!on) return;
