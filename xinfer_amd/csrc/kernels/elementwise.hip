@@ -306,8 +306,9 @@ __global__ void qk_norm_rope_kv_kernel(const void* __restrict__ qkv_v, int slice
 // group of lanes), a wave holds 64/(d/8) tokens, the workgroup's waves hold the block.  The
 // workgroup of a V head turns its [tokens, d] tile through LDS so that where eight tokens follow each other
 // in a group of the pool a lane stores their 16 bytes of a dim.  Value heads may have a size of their own, dv.
-// Measured, us (bytes moved at): 2,048 tokens of 32 + 16 heads of 128 under 13.4 (3.7 TB/s and more), 16.2 where a lane held eight elements side by
-// side, whose partners' came from other lanes, V went two bytes at a time and workgroups had 64 tokens; 64 + 16 heads 22.1 (28.0).  Bound by
+// Measured, us (bytes moved at): 2,048 tokens of 32 + 16 heads of 128 12.3 (4.1 TB/s), 16.2 where a lane held eight elements side by
+// side, whose partners' came from other lanes, V went two bytes at a time and workgroups had 64 tokens; 64 + 16 heads 22.1 (27.3), 8,192 tokens of 32 + 16
+// with a bias 56 (70; 82 with a bias of an element at a time).  Bound by
 // vector instructions (conversions, norm, rotation) and the pass's few trips to memory; asking for all of a head at once without the pairs was
 // slower (18.1: the tables' rows are read twice).
 // Rows may be longer than their heads (`width`), the values' first column is `v_col` (behind the keys, or the keys' own: the
@@ -1226,7 +1227,8 @@ int xi_qk_norm_rope_kv(const void* qkv, int dtype, int slices, const float* bias
       ((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16 == 0) {
     const int lph = d / 8, hpw = 64 / lph;
     // Small workgroups, which start as soon as four waves have ended (2,048 tokens of 64 + 16 heads of 128 in workgroups of 4 | 8 | 16 waves 22.1 |
-    // 24.0 | 27.6 us), of whole groups of eight tokens (40 tokens of heads of 96: 32.0 | 34.1 in workgroups of 20); at most 64 tokens.
+    // 24.0 | 27.6 us), of whole groups of eight tokens (40 tokens of heads of 96: 32.0 | 34.1 in workgroups of 20; heads of 24 and 56, of which a wave
+    // holds 21 and 9, make 63 tokens, and the values of a group that two workgroups share go two bytes at a time); at most 64 tokens.
     const int fit = 64 / hpw, n_waves = fit < (hpw % 2 ? 8 : 4) ? fit : hpw % 2 ? 8 : 4;
     const int tpw = n_waves * hpw;
     const unsigned blocks_x = (unsigned)((n_tok + tpw - 1) / tpw);

@@ -1,5 +1,5 @@
-// The parts of the rows' sums of squares that a product behind a folded norm needs at its end (linear_thin.hip, linear_mid.hip,
-// linear_skinny.hip), brought into LDS by loads that write LDS.  They are the first thing such a kernel asks for, and every instruction in
+// The parts of the rows' sums of squares that a product behind a folded norm needs at its end (linear_thin.hip, linear_mid.hip), brought into
+// LDS by loads that write LDS.  They are the first thing such a kernel asks for, and every instruction in
 // front of its first weights is time without traffic: 32 tested loads a thread for one row of 256 parts were 0.9 us of a product of 3.5
 // (1,024 wide), one load a wave is 0.1.
 #pragma once
@@ -21,14 +21,12 @@ __device__ __forceinline__ void fetch_fold_parts(const float* __restrict__ from,
   }
 }
 
-// 1 / rms of the row whose `parts` parts start at `row`: LANES neighbouring lanes share them out, the lane `sub` those from sub on in steps of
-// LANES, in this order, and add theirs up by halves.
-template <int LANES>
+// 1 / rms of the row whose `parts` parts start at `row`: sixteen neighbouring lanes share them out, the lane `sub` those from sub on in steps of
+// sixteen, in this order, and add theirs up by halves.
 __device__ __forceinline__ float fold_inverse(const float* row, int parts, int sub, float inv_h, float eps) {
   float t = 0.f;
 #pragma unroll 8
-  for (int p = sub; p < parts; p += LANES) t += row[p];
-  if constexpr (LANES > 16) t += lane_xor<16>(t);
+  for (int p = sub; p < parts; p += 16) t += row[p];
   t += lane_xor<8>(t);
   t += lane_xor<4>(t);
   t += lane_xor<2>(t);

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
   if constexpr (FOLD) {
     const int token = tid >> 4;
     if (token < M) {
-      const float inv = fold_inverse<16>(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
+      const float inv = fold_inverse(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
       if ((tid & 15) == 0) inv_s[token] = inv;
     }
     __syncthreads();

@@ -7,12 +7,13 @@
 //
 // A workgroup of four waves owns R <= 32 features (R from N alone, so that the workgroups are a
 // multiple of the 256 compute units) and all of K.  It walks K in tiles of 256: all 256 threads
-// copy the w tile [32 rows, 512 bytes each: 32 lanes a row] and the x tile [4, 8 or 16 rows] from
+// copy the w tile [32 rows, 512 bytes each: 32 lanes a row] and the x tile [8 or 16 rows] from
 // memory into registers, two tiles ahead, and from there into LDS (double buffered, one barrier
 // a tile); wave v multiplies k steps 2v and 2v+1 of the tile's eight (v_mfma_f32_16x16x32_bf16,
 // A = 16 rows of w, B = the 16 rows of x), two tiles of 16 features each.  Workgroups of up to
-// 16 features take tiles of [16 rows, 512 k] instead: the same bytes a tile, no rows that
-// nobody multiplies, half the barriers.  At the end the four
+// 16 features take tiles of [16 rows, 512 k] instead (x: 4, 8 or 16 rows): the same bytes a tile, no rows that
+// nobody multiplies, half the barriers, and all of a short K is asked for at the start (`thin_depth`); those of up to 4 features
+// that add into the stream copy 4 rows of w.  At the end the four
 // waves' sums are added through LDS in wave order and stored: plain (MODE 0), adding into the
 // float32 residual stream and handing on round(stream * g) and the rows' sums of squares (MODE
 // 1), or scaling the rows by rsqrt(sum of the parts / K + eps) (MODE 2).
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
   if constexpr (MODE == 2) {
     const int token = tid >> 4;
     if (token < M) {
-      const float inv = fold_inverse<16>(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
+      const float inv = fold_inverse(parts_s + token * fold.parts, fold.parts, tid & 15, fold.inv_h, fold.eps);
       if ((tid & 15) == 0) side[token] = inv;
     }
   }

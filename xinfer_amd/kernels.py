@@ -886,7 +886,7 @@ def moe_experts_tiled(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     [T, X][:, 0]: what `gated_add_` does behind it, in the pass that adds the experts up): the pairs sorted by expert on the device, each expert's rows
     multiplied in tiles of up to `tile_rows` (16, 64, 128 or 256; None: `moe_tile_rows`, one for each product) by the walk of the dense many-row product, the
     activation on the first product's float32 sums.  Nothing is read on the host.  From one token on it is ahead of the other
-    forms: 16 pairs on 8 gated experts of 6144 at width 4096 184 us where the grouped form takes 331 and a pair at a time 441,
+    forms: 16 pairs on 8 gated experts of 6144 at width 4096 206 us where the grouped form takes 331 and a pair at a time 441,
     2,048 tokens 535 to 580 by how they share out, where the vendor library's products an expert take 925."""
     _dev(x, gate_up, down, idx, wt, add)
     _moe_rows(x, add, identity, weigh_input)
