@@ -35,10 +35,10 @@ constexpr int kThinFeatures = 32;        // most rows of w in a workgroup's tile
 constexpr int kThinK = 256;              // k per tile of 32 rows of w (a tile of 16 rows takes 512: the same bytes)
 constexpr int kThinDepth = 2;            // tiles whose loads are in flight
 constexpr int kThinParts = 512;          // most parts of a row's sum of squares
-constexpr size_t thin_lds_bytes(int tr) {     // two buffers of a w tile and an x tile, rows padded by 8 elements
-  return 2 * (size_t)(tr + kThinRows) * (8192 / tr + 8) * sizeof(bf16);
+constexpr size_t thin_lds_bytes(int tr, int wr, int xr) {     // two buffers of wr rows of w and xr of x, padded by 8 elements
+  return 2 * (size_t)(wr + xr) * (8192 / tr + 8) * sizeof(bf16);
 }
-constexpr size_t kThinLdsMost = thin_lds_bytes(16) + kThinRows * kThinParts * sizeof(float);     // and MODE 2's parts
+constexpr size_t kThinLdsMost = thin_lds_bytes(16, 16, kThinRows) + kThinRows * kThinParts * sizeof(float);     // and MODE 2's parts
 
 struct ThinFold {
   float* resid;         // MODE 1: [M, N] float32, updated in place
@@ -218,6 +218,12 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
   }
 }
 
+// The tiles' LDS of a form, by the kernel's own template arguments.
+template <int TR, int XR, int D = kThinDepth, bool WHOLE = false, int WR = TR>
+struct ThinForm {
+  static constexpr size_t kLds = thin_lds_bytes(TR, WR, XR);
+};
+
 // Features per workgroup: the fewest workgroups that are a multiple of the 256 compute units
 // with at most 32 features each.  From N alone.
 static int thin_features(int N) {
@@ -287,7 +293,7 @@ static int thin_check(const char* what, const void* x, const void* w, int M, int
       lds_set = true;                                                                                           \
     }                                                                                                           \
     const size_t parts_lds = MODE == 2 ? fold_parts_room(M * fold.parts) * sizeof(float) : 0;                  \
-    kern<<<wgs, 256, thin_lds_bytes(TR) + parts_lds, stream>>>((const bf16*)x, (const bf16*)w, (TO*)(yptr), M, N, K, R, rotate, fold); \
+    kern<<<wgs, 256, ThinForm<TR, __VA_ARGS__>::kLds + parts_lds, stream>>>((const bf16*)x, (const bf16*)w, (TO*)(yptr), M, N, K, R, rotate, fold); \
   } while (0)
 // tiles of 16 rows of w (512 k)
 #define XI_THIN_DEPTH(MODE, TO, yptr, XR)                                                             \
