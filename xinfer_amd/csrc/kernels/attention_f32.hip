@@ -25,8 +25,9 @@
 // Measured on MI355X, 32 heads of 128 on 8 kv heads, against a page's number looked up for every block and tests around every load (us):
 // prompts of 200, 127, 54, 172 and 9 tokens 67.6 (79.4), a prompt of 1,024 208 (248), 8 single tokens at up to 330 keys 15.9 (17.3), one at
 // 4,096 keys 99 (125); 16 heads on 8, a prompt of 1,024, heads of 64 71 (113), a prompt of 512, heads of 256 118 (182).  One lane a key took 396,
-// 1,990, 54 and 738 for the first four.  Bound by the issue of the matrix and vector instructions of two waves a SIMD, of whose 16 columns a
-// decode step uses the heads of a kv head.
+// 1,990, 54 and 738 for the first four.  Counters: on prompts a unit issues an instruction in half of its busy cycles (vector ones in 36%; matrix cores
+// busy 12%), for 8 single tokens in a third (23%; 20%, of whose 16 columns a decode step uses the heads of a kv head): what bounds it is a block's
+// chain (K, scores, their sums over lanes, V) in the two waves a SIMD that its registers leave room for.
 //
 // A value that a token does not see never reaches it, not even with a weight of 0 (an infinite or
 // undefined one would): in a block that some token of the tile does not see in full, each token's
