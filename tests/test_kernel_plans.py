@@ -3,6 +3,8 @@ along K for the many-row tiled kernel, and how a decode step's keys are shared o
 import os
 import random
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -340,3 +342,26 @@ def test_round_tiles_of_few_features_leave_strides_of_powers_of_two_alone():
     for K in (5120, 8192, 15360, 16384, 24576):
         assert ahead(2048, 4096, K) and ahead(2560, 3072, K)
     assert not ahead(2048, 4096, 24640) and not ahead(2048, 4096, 32768) and not ahead(2048, 4096, 4096)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs the compiler")
+@pytest.mark.parametrize("name", ["linear_thin", "linear_mid"])
+def test_folded_products_wait_for_their_parts(name, tmp_path):
+    """In the compiled kernels the loads that bring the rows' parts into LDS are issued before the first operands, and the count that is
+    waited for behind them is not more than what has been issued since: it waits for the parts."""
+    from xinfer_amd.csrc import build
+    out = tmp_path / "k.s"
+    subprocess.run(["hipcc", *build.HIP_FLAGS, "--offload-device-only", "-S", os.path.join(build.KERNEL_DIR, name + ".hip"), "-o", str(out)], check=True,
+                   capture_output=True, timeout=300)
+    found = 0
+    for kernel, body in re.findall(r"^(_ZN2xi\w+):(.*?)s_endpgm", out.read_text(), re.S | re.M):
+        lines = [line.strip() for line in body.split("\n")]
+        parts = [i for i, line in enumerate(lines) if line.startswith("global_load_lds_dword ")]
+        if not parts:
+            continue
+        found += 1
+        loads = [i for i, line in enumerate(lines) if line.startswith("global_load_dwordx4 ")]
+        wait = next(i for i, line in enumerate(lines) if i > parts[-1] and line.startswith("s_waitcnt vmcnt("))
+        count = int(re.search(r"vmcnt\((\d+)\)", lines[wait])[1])
+        assert min(loads) > parts[-1] and count <= sum(parts[-1] < i < wait for i in loads), kernel
+    assert found

@@ -34,11 +34,15 @@ __device__ __forceinline__ float fold_inverse(const float* row, int parts, int s
   return rsqrtf(t * inv_h + eps);
 }
 
-// All but the last N of this wave's loads have landed.
+// All but the last N of this wave's loads have landed.  N is at most what is issued between those that are waited for and here: a count of more
+// than are on their way waits for none, and loads of read-only operands are the compiler's to move behind an asm (of the slots asked for at a
+// kernel's start one goes into the branch that has a second tile).
 template <int N>
 __device__ __forceinline__ void wait_all_but() {
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 }  // namespace xi

@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256, 1) void linear_mid_kernel(const bf16* __restri
   const int last = nkt - 1;
 #pragma unroll
   for (int s = 0; s < D; ++s) XI_MID_ISSUE(s, s < last ? s : last);
-  if constexpr (FOLD) wait_all_but<D * (WR + XI)>();            // this wave's parts are in LDS (the first tile is waited for anyway)
+  if constexpr (FOLD) wait_all_but<(D - 1) * (WR + XI)>();      // this wave's parts are in LDS
 
   // One tile: registers of slot s to LDS, the slot loaded again D tiles ahead, barrier,
   // products.  One barrier a tile is enough: whoever writes this buffer again, two tiles on, has

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(const bf16* __restrict
   const int last = nkt - 1;
 #pragma unroll
   for (int s = 0; s < D; ++s) XI_THIN_ISSUE(s, s < last ? s : last);
-  if constexpr (MODE == 2) wait_all_but<D * (WP + XP)>();       // this wave's parts are in LDS (the first tile is waited for anyway)
+  if constexpr (MODE == 2) wait_all_but<(D - 1) * (WP + XP)>();       // this wave's parts are in LDS
 
   int buf = 0;
 #define XI_THIN_TILE(s, t)                                                                                \
